@@ -206,7 +206,7 @@ struct ChunkParams {
     ChunkWs ws;
     int64_t T; int H, HV; int64_t N; int64_t NT;       // NT: chunks per sequence (dense input)
     int K, V;                                          // head dims of the caller's tensors (multiples of 8; K, V <= 128, or 128 < K <= 256 with any V)
-    float scale; int gb_dtype; uint32_t flags;
+    float scale; int gb_dtype, beta_dtype; uint32_t flags;
     int64_t NH;
     int want_P;                                        // the prepare kernel also writes P (GDN_FLAG_RECORD_P)
 };

@@ -80,7 +80,7 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
     uint32_t rg = 0, rb = 0;
     if (lane < valid) {
         rg = p.g ? load_scalar_bits(p.g, (tok0 + lane) * HV + hv, p.gb_dtype) : 0;   // (no gate: the plain delta rule)
-        rb = load_scalar_bits(p.beta, (tok0 + lane) * HV + hv, p.gb_dtype);
+        rb = load_scalar_bits(p.beta, (tok0 + lane) * HV + hv, p.beta_dtype);
     }
     f32x4 U[4][4];
 #pragma unroll
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
     // ---- gates: inclusive scan over the chunk, one token per lane; the tables; the bound on the chunk's transition ----
     float beta_tok;
     {
-        float x = scalar_of_bits(rg, p.gb_dtype), b = scalar_of_bits(rb, p.gb_dtype);
+        float x = scalar_of_bits(rg, p.gb_dtype), b = scalar_of_bits(rb, p.beta_dtype);
         if (lane < valid) {                      // optional activations of the raw gate / beta inputs
             if (p.A_log && p.g) x = -__expf(p.A_log[hv]) * softplus_f(x + (p.dt_bias ? p.dt_bias[hv] : 0.f));
             if (p.flags & GDN_FLAG_BETA_SIGMOID) b = sigmoid_f(b) * ((p.flags & GDN_FLAG_NEG_EIGVAL) ? 2.f : 1.f);

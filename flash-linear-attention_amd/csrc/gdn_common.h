@@ -66,6 +66,9 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 template <typename T> __device__ __forceinline__ float to_f32(T x) { return (float)x; }
 template <typename T> __device__ __forceinline__ T from_f32(float x) { return (T)x; }
 
+// (g and beta of different types: GDN_GB_DTYPES)
+inline int beta_dtype_of(int gb_dtype) { return gb_dtype >> 8 ? (gb_dtype >> 8) - 1 : gb_dtype; }
+
 // g/beta may arrive in any float type; they are tiny, so a run-time switch is enough.
 __device__ __forceinline__ float load_scalar(const void* p, int64_t i, int dtype) {
     if (dtype == GDN_DTYPE_F32) return ((const float*)p)[i];

@@ -24,7 +24,7 @@ struct RecurrentParams {
     const void* cu_seqlens; const void* state_slots; const void* num_accepted;
     int64_t slots_stride;
     int64_t T; int H, HV, K, V, NVB;
-    float scale; int gb_dtype; uint32_t flags;
+    float scale; int gb_dtype, beta_dtype; uint32_t flags;
     int xcd_group; int64_t nblocks;      // see xcd_block()
     // gate per key feature given as a raw input (the KDA operator): 0 = gk is the log decay itself,
     // 1: gk <- -e^A softplus(gk + bias), 2: gk <- lower sigmoid(e^A (gk + bias)); A = A_log[head] (mode 1 without
@@ -54,6 +54,18 @@ __device__ __forceinline__ int64_t xcd_block(const RecurrentParams& p) {
         if (blk >= p.nblocks) return -1;
     }
     return blk;
+}
+
+// The bits of element i of a gate or beta (NULL: any bits) without a branch, to be converted where they are used: two halves of 16
+// bits, the same one twice for 16-bit types.  A branch per type would make the wave wait for everything requested so far.
+struct ScalarBits { uint16_t lo, hi; };
+__device__ __forceinline__ ScalarBits fetch_scalar(const void* p, const void* dummy, int64_t i, int dtype) {
+    const bool f32 = dtype == GDN_DTYPE_F32;
+    const uint16_t* at = p ? (const uint16_t*)p + (f32 ? 2 * i : i) : (const uint16_t*)dummy;
+    return ScalarBits{at[0], at[p && f32 ? 1 : 0]};
+}
+__device__ __forceinline__ float scalar_value(ScalarBits b, int dtype) {
+    return scalar_of_bits(dtype == GDN_DTYPE_F32 ? (uint32_t)b.lo | ((uint32_t)b.hi << 16) : b.lo, dtype);
 }
 
 __device__ __forceinline__ float wave_sum(float x) {
@@ -237,10 +249,10 @@ __global__ __launch_bounds__(256) void gdn_recurrent_kernel(RecurrentParams p) {
                 if (p.beta) {
                     if (p.flags & GDN_FLAG_BETA_VECTOR) {
                         const int64_t bi = (tok * HV + ihv) * V + cont_idx;
-                        bb = f32x4{load_scalar(p.beta, bi, p.gb_dtype), load_scalar(p.beta, bi + 1, p.gb_dtype),
-                                   load_scalar(p.beta, bi + 2, p.gb_dtype), load_scalar(p.beta, bi + 3, p.gb_dtype)};
+                        bb = f32x4{load_scalar(p.beta, bi, p.beta_dtype), load_scalar(p.beta, bi + 1, p.beta_dtype),
+                                   load_scalar(p.beta, bi + 2, p.beta_dtype), load_scalar(p.beta, bi + 3, p.beta_dtype)};
                     } else {
-                        const float b = load_scalar(p.beta, tok * HV + ihv, p.gb_dtype);
+                        const float b = load_scalar(p.beta, tok * HV + ihv, p.beta_dtype);
                         bb = f32x4{b, b, b, b};
                     }
                 }
@@ -284,8 +296,8 @@ __global__ __launch_bounds__(256) void gdn_recurrent_kernel(RecurrentParams p) {
                 if (rok) {
                     vv = to_f32(v[(tok * HV + ihv) * V + row]);
                     if (p.beta) {
-                        bb = (p.flags & GDN_FLAG_BETA_VECTOR) ? load_scalar(p.beta, (tok * HV + ihv) * V + row, p.gb_dtype)
-                                                              : load_scalar(p.beta, tok * HV + ihv, p.gb_dtype);
+                        bb = (p.flags & GDN_FLAG_BETA_VECTOR) ? load_scalar(p.beta, (tok * HV + ihv) * V + row, p.beta_dtype)
+                                                              : load_scalar(p.beta, tok * HV + ihv, p.beta_dtype);
                     }
                     if (p.flags & GDN_FLAG_BETA_SIGMOID) bb = bmul * sigmoid_f(bb);
                 }
@@ -306,32 +318,37 @@ __global__ __launch_bounds__(256) void gdn_recurrent_kernel(RecurrentParams p) {
 }
 
 
-// The common decode shape on its own: K = V = 128, K-first states [K][V], one gate and one beta per head, states
-// per sequence or per slot.  Same arithmetic as gdn_recurrent_kernel with the decay e^g applied after the reductions,
+// The common decode shapes on their own: K = 128 or 256, V a multiple of the block of VB columns, K-first states [K][V], one gate
+// and one beta per head, states per sequence or per slot.  Same arithmetic as gdn_recurrent_kernel with the decay e^g applied after
+// the reductions,
 //   S' = e^g S + k d^T,   d = beta (v - e^g S^T k),   o = scale (e^g S^T q + (q.k) d),
 // k and q of a token read from LDS where they are used instead of being held per row.  The token's own rows (q, k,
 // v, gate, beta) are requested BEFORE the state: loads return in issue order, so their norms and the LDS staging are
-// done while the 64 KB of state are still on their way, and what follows the state's arrival is only the two
-// reductions and the update.  Thread (c = tid % 32, r0 = tid / 32) owns value columns 4c .. 4c+3 of key rows r0 + 8i.
-// Launched with enough unused LDS that two workgroups share a CU: more resident workgroups widen the window of
-// memory the chip works on at one time, and the read-modify-write stream gets slower (measured: 1, 2, 3+ workgroups
-// per CU = 208, 183, 191 us for 1 GiB of state traffic).
-constexpr size_t DECODE_LDS_PAD = 64 * 1024;
+// done while the state is still on its way, and what follows the state's arrival is only the two
+// reductions and the update.  Thread (c = tid % (VB/4), r0 = tid / (VB/4)) owns value columns 4c .. 4c+3 of key rows r0 + RP i.
+// Blocks of 32 columns (16 KB of state): measured against 128, 64 and 16 columns at 32 heads of 128 x 128 - 1 sequence 4.4 us (5.5, 4.8,
+// 5.1), 48 sequences 34.9 (38.0, 36.0, 44.0), 256 sequences 170.9 = 6.28 TB/s (174.2, 175.7, 226.7; 64-byte rows at 16 columns).
+// No load of a token or of the state stands behind a branch (fetch_scalar, one test of h0 for all pieces): with a test per piece the
+// compiler waits for each before it requests the next (the same 32 columns: 178.7 us).  Occupancy needs no cap at this size: with
+// unused LDS for 10 down to 5 workgroups per CU the time stays, with 2 it is 256 us.
 
 // GK: a decay per key feature as well (the KDA operator's decode step): S' = diag(e^gk) e^g S + k d^T, so the two
 // reductions run over e^gk k and e^gk q, staged beside k and q, and the update takes a factor per row.
 // PK: a second key p that the prediction uses on the state as it was BEFORE this token's decay (the comba operator's
 // decode step): d = beta (v - S^T p), so that reduction runs over p and takes no e^g.
-template <typename T, bool GK = false, bool PK = false>
+template <typename T, int KD, int VB, bool GK = false, bool PK = false>
 __global__ __launch_bounds__(256, 2) void gdn_decode_kernel(RecurrentParams p) {
     static_assert(!(GK && PK), "one of the two forms at a time");
+    constexpr int TC = VB / 4, RP = 256 / TC, R = KD / RP;      // threads along the columns, rows per pass, pieces of 16 bytes per thread
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c = tid & 31, r0 = tid >> 5;
-    const int64_t inh = xcd_block(p);
-    if (inh < 0) return;
+    const int c = tid % TC, r0 = tid / TC;
+    const int64_t blk = xcd_block(p);
+    if (blk < 0) return;
+    const int ivb = (int)(blk % p.NVB);
+    const int64_t inh = blk / p.NVB;
     const int64_t in = inh / p.HV;
     const int ihv = (int)(inh % p.HV);
-    const int H = p.H, HV = p.HV;
+    const int H = p.H, HV = p.HV, V = p.V;
     const int ih = ihv / (HV / H);
     const bool cu32 = p.flags & GDN_FLAG_CU_INT32;
     int64_t bos, len;
@@ -343,44 +360,44 @@ __global__ __launch_bounds__(256, 2) void gdn_decode_kernel(RecurrentParams p) {
         len = p.T;
     }
     const int64_t slot = p.state_slots ? load_index(p.state_slots, in, p.flags & GDN_FLAG_SLOT_INT32) : in;
-    const int64_t state_off = (slot * HV + ihv) * (int64_t)16384 + 4 * c;
+    const int col = ivb * VB + 4 * c;
+    const int64_t state_off = (slot * HV + ihv) * (int64_t)KD * V + col;
     const T* q = (const T*)p.q; const T* k = (const T*)p.k; const T* v = (const T*)p.v; T* o = (T*)p.o;
     // what a token brings, as it comes from memory
-    struct Token { T q, k, pk; T v[4]; float g, b, gk; };
+    struct Token { T q, k, pk; T v[4]; ScalarBits g, b; float gk; };
     const float a_k = GK && p.gk_act ? (p.A_log ? __expf(p.A_log[ihv]) : (p.gk_act == 2 ? 1.f : __expf(1.f))) : 0.f;
-    const float gk_bias = GK && p.gk_act && p.gk_bias && tid < 128 ? p.gk_bias[ihv * 128 + tid] : 0.f;
+    const float gk_bias = GK && p.gk_act && p.gk_bias && tid < KD ? p.gk_bias[ihv * KD + tid] : 0.f;
     auto fetch = [&](int64_t tok) {
         Token x;
-        x.q = x.k = x.pk = from_f32<T>(0.f);
-        x.gk = 0.f;
-        if (tid < 128) {
-            x.q = q[(tok * H + ih) * 128 + tid]; x.k = k[(tok * H + ih) * 128 + tid];
-            if constexpr (GK) x.gk = p.gk[(tok * HV + ihv) * 128 + tid];
-            if constexpr (PK) x.pk = ((const T*)p.pk)[(tok * H + ih) * 128 + tid];
-        }
-        const T* pv = v + (tok * HV + ihv) * 128 + 4 * c;
+        const int f = tid & (KD - 1);                   // (threads beyond KD read valid elements and do not use them)
+        x.q = q[(tok * H + ih) * KD + f]; x.k = k[(tok * H + ih) * KD + f];
+        if constexpr (GK) x.gk = p.gk[(tok * HV + ihv) * KD + f];
+        if constexpr (PK) x.pk = ((const T*)p.pk)[(tok * H + ih) * KD + f];
+        const T* pv = v + (tok * HV + ihv) * V + col;
 #pragma unroll
         for (int j = 0; j < 4; ++j) x.v[j] = pv[j];
-        x.g = p.g ? load_scalar(p.g, tok * HV + ihv, p.gb_dtype) : 0.f;
-        x.b = p.beta ? load_scalar(p.beta, tok * HV + ihv, p.gb_dtype) : 1.f;
+        x.g = fetch_scalar(p.g, q, tok * HV + ihv, p.gb_dtype);
+        x.b = fetch_scalar(p.beta, q, tok * HV + ihv, p.beta_dtype);
         return x;
     };
     Token cur = {};
     if (len > 0) cur = fetch(bos);
     float a_neg = 0.f, dtb = 0.f;
     if (p.A_log) { a_neg = -__expf(p.A_log[ihv]); if (p.dt_bias) dtb = p.dt_bias[ihv]; }
-    // ---- the state: 16 requests of 16 bytes per thread, a wave instruction covers two whole rows ----
-    f32x4 S[16];
+    // ---- the state: R requests of 16 bytes per thread, a wave instruction covers whole rows of the block ----
+    f32x4 S[R];
+    if (p.h0) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (p.h0) S[i] = __builtin_nontemporal_load((const f32x4*)(p.h0 + state_off + (r0 + 8 * i) * 128));
+        for (int i = 0; i < R; ++i) S[i] = __builtin_nontemporal_load((const f32x4*)(p.h0 + state_off + (int64_t)(r0 + RP * i) * V));
+    } else {
+#pragma unroll
+        for (int i = 0; i < R; ++i) S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    __shared__ float sh_q[2][128], sh_k[2][128];
-    __shared__ float sh_kr[GK ? 2 : 1][GK ? 128 : 1], sh_eg[GK ? 2 : 1][GK ? 128 : 1];     // (GK) k as it is, and e^gk per row
-    __shared__ float sh_p[PK ? 2 : 1][PK ? 128 : 1];
+    __shared__ float sh_q[2][KD], sh_k[2][KD];
+    __shared__ float sh_kr[GK ? 2 : 1][GK ? KD : 1], sh_eg[GK ? 2 : 1][GK ? KD : 1];     // (GK) k as it is, and e^gk per row
+    __shared__ float sh_p[PK ? 2 : 1][PK ? KD : 1];
     __shared__ float sh_red[2][4][4];
-    __shared__ f32x4 sh_part[2][4][2][32];
+    __shared__ f32x4 sh_part[2][4][2][TC];
     const float bmul = (p.flags & GDN_FLAG_NEG_EIGVAL) ? 2.f : 1.f;
 
     for (int64_t t = 0; t < len; ++t) {
@@ -388,7 +405,7 @@ __global__ __launch_bounds__(256, 2) void gdn_decode_kernel(RecurrentParams p) {
         const int64_t tok = bos + t;
         const float qv = to_f32(cur.q), kv = to_f32(cur.k);
         if constexpr (GK) {
-            if (tid < 128) {
+            if (tid < KD) {
                 float x = cur.gk;
                 if (p.gk_act) {
                     x += gk_bias;
@@ -398,83 +415,92 @@ __global__ __launch_bounds__(256, 2) void gdn_decode_kernel(RecurrentParams p) {
                 sh_q[pb][tid] = qv * e; sh_k[pb][tid] = kv * e; sh_kr[pb][tid] = kv; sh_eg[pb][tid] = e;
             }
         } else {
-            if (tid < 128) { sh_q[pb][tid] = qv; sh_k[pb][tid] = kv; }
+            if (tid < KD) { sh_q[pb][tid] = qv; sh_k[pb][tid] = kv; }
         }
         float sqq = wave_sum(qv * qv), skk = wave_sum(kv * kv), sqk = wave_sum(qv * kv);
         if (lane == 0) { sh_red[pb][wave][0] = sqq; sh_red[pb][wave][1] = skk; sh_red[pb][wave][2] = sqk; }
         if constexpr (PK) {
             const float pv = to_f32(cur.pk);
-            if (tid < 128) sh_p[pb][tid] = pv;
+            if (tid < KD) sh_p[pb][tid] = pv;
             const float spp = wave_sum(pv * pv);
             if (lane == 0) sh_red[pb][wave][3] = spp;
         }
         float eg = 1.f;
         if (p.g) {
-            float gt = cur.g;
+            float gt = scalar_value(cur.g, p.gb_dtype);
             if (p.A_log) gt = a_neg * softplus_f(gt + dtb);
             eg = __expf(gt);
         }
-        float bb = cur.b;
+        float bb = p.beta ? scalar_value(cur.b, p.beta_dtype) : 1.f;
         if (p.flags & GDN_FLAG_BETA_SIGMOID) bb = bmul * sigmoid_f(bb);
         const f32x4 vv = {to_f32(cur.v[0]), to_f32(cur.v[1]), to_f32(cur.v[2]), to_f32(cur.v[3])};
         if (t + 1 < len) cur = fetch(tok + 1);          // the next token's rows travel during this one's arithmetic
         __syncthreads();
-        sqq = sh_red[pb][0][0] + sh_red[pb][1][0];      // (q and k live in waves 0 and 1)
-        skk = sh_red[pb][0][1] + sh_red[pb][1][1];
-        sqk = sh_red[pb][0][2] + sh_red[pb][1][2];
+        auto over_waves = [&](int what) {               // (q and k live in the first KD / 64 waves)
+            float x = sh_red[pb][0][what];
+#pragma unroll
+            for (int w = 1; w < KD / 64; ++w) x += sh_red[pb][w][what];
+            return x;
+        };
+        sqq = over_waves(0); skk = over_waves(1); sqk = over_waves(2);
         float rq = p.scale, rk = 1.f, rp = 1.f;
         if (p.flags & GDN_FLAG_QK_L2NORM) {
             rq *= 1.f / sqrtf(sqq + 1e-6f);
             rk = 1.f / sqrtf(skk + 1e-6f);
-            if constexpr (PK) rp = 1.f / sqrtf(sh_red[pb][0][3] + sh_red[pb][1][3] + 1e-6f);
+            if constexpr (PK) rp = 1.f / sqrtf(over_waves(3) + 1e-6f);
         }
         const float qk = sqk * rq * rk;
         // S^T k and S^T q over this thread's rows (k, q unscaled: the row factors come after the reduction)
         f32x4 sk = {0.f, 0.f, 0.f, 0.f}, sq = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            sk += S[i] * (PK ? sh_p[pb][r0 + 8 * i] : sh_k[pb][r0 + 8 * i]);
-            sq += S[i] * sh_q[pb][r0 + 8 * i];
+        for (int i = 0; i < R; ++i) {
+            sk += S[i] * (PK ? sh_p[pb][r0 + RP * i] : sh_k[pb][r0 + RP * i]);
+            sq += S[i] * sh_q[pb][r0 + RP * i];
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) { sk[j] += __shfl_xor(sk[j], 32, 64); sq[j] += __shfl_xor(sq[j], 32, 64); }
-        if (lane < 32) { sh_part[pb][wave][0][c] = sk; sh_part[pb][wave][1][c] = sq; }
+        for (int off = TC; off < 64; off <<= 1)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { sk[j] += __shfl_xor(sk[j], off, 64); sq[j] += __shfl_xor(sq[j], off, 64); }
+        if (lane < TC) { sh_part[pb][wave][0][c] = sk; sh_part[pb][wave][1][c] = sq; }
         __syncthreads();
         sk = (sh_part[pb][0][0][c] + sh_part[pb][1][0][c] + sh_part[pb][2][0][c] + sh_part[pb][3][0][c]) * (PK ? rp : eg * rk);
         sq = (sh_part[pb][0][1][c] + sh_part[pb][1][1][c] + sh_part[pb][2][1][c] + sh_part[pb][3][1][c]) * (eg * rq);
         const f32x4 d = bb * (vv - sk);
         const f32x4 dk = d * rk;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            if constexpr (GK) S[i] = S[i] * (eg * sh_eg[pb][r0 + 8 * i]) + dk * sh_kr[pb][r0 + 8 * i];
-            else S[i] = S[i] * eg + dk * sh_k[pb][r0 + 8 * i];
+        for (int i = 0; i < R; ++i) {
+            if constexpr (GK) S[i] = S[i] * (eg * sh_eg[pb][r0 + RP * i]) + dk * sh_kr[pb][r0 + RP * i];
+            else S[i] = S[i] * eg + dk * sh_k[pb][r0 + RP * i];
         }
         if (r0 == 0) {
             const f32x4 ov = sq + d * qk;
-            T* po = o + (tok * HV + ihv) * 128 + 4 * c;
+            T* po = o + (tok * HV + ihv) * V + col;
             po[0] = from_f32<T>(ov.x); po[1] = from_f32<T>(ov.y); po[2] = from_f32<T>(ov.z); po[3] = from_f32<T>(ov.w);
         }
     }
     if (p.ht) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) __builtin_nontemporal_store(S[i], (f32x4*)(p.ht + state_off + (r0 + 8 * i) * 128));
+        for (int i = 0; i < R; ++i) __builtin_nontemporal_store(S[i], (f32x4*)(p.ht + state_off + (int64_t)(r0 + RP * i) * V));
     }
 }
 
-// The common decode shape with V-first states [V][K] (the layout serving engines keep, `state_v_first`): thread
-// (c = tid % 32, r0 = tid / 32) owns key features 4c .. 4c+3 of value rows r0 + 8i, so S^T k and S^T q are sums along a
-// row: four products per thread and row, then over the 32 lanes that share the row.  The token's rows are requested
-// before the state here as well (k and q as the thread's own four features, v through LDS), two workgroups share a CU.
+// The common decode shapes with V-first states [V][K] (the layout serving engines keep, `state_v_first`), a block of VB value rows per
+// workgroup: thread (c = tid % (KD/4), r0 = tid / (KD/4)) owns key features 4c .. 4c+3 of value rows r0 + RP i, so S^T k and S^T q are
+// sums along a row: four products per thread and row, then over the KD/4 lanes that share the row.  The token's rows are requested
+// before the state here as well (k and q as the thread's own four features, v through LDS).
 // GK: a decay per key feature as well (the KDA operator): here a factor per column, the thread's own four.
-template <typename T, bool GK = false>
+template <typename T, int KD, int VB, bool GK = false>
 __global__ __launch_bounds__(256, 2) void gdn_decode_vfirst_kernel(RecurrentParams p) {
+    constexpr int TC = KD / 4, RP = 256 / TC, R = VB / RP;      // threads along a row, rows per pass, pieces of 16 bytes per thread
     const int tid = threadIdx.x;
-    const int c = tid & 31, r0 = tid >> 5;
-    const int64_t inh = xcd_block(p);
-    if (inh < 0) return;
+    const int c = tid % TC, r0 = tid / TC;
+    const int64_t blk = xcd_block(p);
+    if (blk < 0) return;
+    const int v0 = (int)(blk % p.NVB) * VB;
+    const int64_t inh = blk / p.NVB;
     const int64_t in = inh / p.HV;
     const int ihv = (int)(inh % p.HV);
-    const int H = p.H, HV = p.HV;
+    const int H = p.H, HV = p.HV, V = p.V;
     const int ih = ihv / (HV / H);
     const bool cu32 = p.flags & GDN_FLAG_CU_INT32;
     int64_t bos, len;
@@ -486,41 +512,42 @@ __global__ __launch_bounds__(256, 2) void gdn_decode_vfirst_kernel(RecurrentPara
         len = p.T;
     }
     const int64_t slot = p.state_slots ? load_index(p.state_slots, in, p.flags & GDN_FLAG_SLOT_INT32) : in;
-    const int64_t state_off = (slot * HV + ihv) * (int64_t)16384 + 4 * c;
+    const int64_t state_off = ((slot * HV + ihv) * (int64_t)V + v0) * KD + 4 * c;
     const T* q = (const T*)p.q; const T* k = (const T*)p.k; const T* v = (const T*)p.v; T* o = (T*)p.o;
-    struct Token { T q[4], k[4]; T v; float g, b; f32x4 gk; };
+    struct Token { T q[4], k[4]; T v; ScalarBits g, b; f32x4 gk; };
     const float a_k = GK && p.gk_act ? (p.A_log ? __expf(p.A_log[ihv]) : (p.gk_act == 2 ? 1.f : __expf(1.f))) : 0.f;
     f32x4 gk_bias = {0.f, 0.f, 0.f, 0.f};
-    if (GK && p.gk_act && p.gk_bias) gk_bias = *(const f32x4*)(p.gk_bias + ihv * 128 + 4 * c);
+    if (GK && p.gk_act && p.gk_bias) gk_bias = *(const f32x4*)(p.gk_bias + ihv * KD + 4 * c);
     auto fetch = [&](int64_t tok) {
         Token x;
-        const T* pq = q + (tok * H + ih) * 128 + 4 * c;
-        const T* pk = k + (tok * H + ih) * 128 + 4 * c;
+        const T* pq = q + (tok * H + ih) * KD + 4 * c;
+        const T* pk = k + (tok * H + ih) * KD + 4 * c;
 #pragma unroll
         for (int j = 0; j < 4; ++j) { x.q[j] = pq[j]; x.k[j] = pk[j]; }
         x.gk = f32x4{0.f, 0.f, 0.f, 0.f};
-        if constexpr (GK) x.gk = *(const f32x4*)(p.gk + (tok * HV + ihv) * 128 + 4 * c);
-        x.v = from_f32<T>(0.f);
-        if (tid < 128) x.v = v[(tok * HV + ihv) * 128 + tid];
-        x.g = p.g ? load_scalar(p.g, tok * HV + ihv, p.gb_dtype) : 0.f;
-        x.b = p.beta ? load_scalar(p.beta, tok * HV + ihv, p.gb_dtype) : 1.f;
+        if constexpr (GK) x.gk = *(const f32x4*)(p.gk + (tok * HV + ihv) * KD + 4 * c);
+        x.v = v[(tok * HV + ihv) * V + v0 + (tid & (VB - 1))];
+        x.g = fetch_scalar(p.g, q, tok * HV + ihv, p.gb_dtype);
+        x.b = fetch_scalar(p.beta, q, tok * HV + ihv, p.beta_dtype);
         return x;
     };
     Token cur = {};
     if (len > 0) cur = fetch(bos);
     float a_neg = 0.f, dtb = 0.f;
     if (p.A_log) { a_neg = -__expf(p.A_log[ihv]); if (p.dt_bias) dtb = p.dt_bias[ihv]; }
-    f32x4 S[16];
+    f32x4 S[R];
+    if (p.h0) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (p.h0) S[i] = __builtin_nontemporal_load((const f32x4*)(p.h0 + state_off + (r0 + 8 * i) * 128));
+        for (int i = 0; i < R; ++i) S[i] = __builtin_nontemporal_load((const f32x4*)(p.h0 + state_off + (r0 + RP * i) * KD));
+    } else {
+#pragma unroll
+        for (int i = 0; i < R; ++i) S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    __shared__ float sh_v[2][128];
+    __shared__ float sh_v[2][VB];
     const float bmul = (p.flags & GDN_FLAG_NEG_EIGVAL) ? 2.f : 1.f;
-    auto row_sum = [&](float x) {                               // over the 32 lanes that share a row
+    auto row_sum = [&](float x) {                               // over the TC lanes that share a row
 #pragma unroll
-        for (int off = 1; off < 32; off <<= 1) x += __shfl_xor(x, off, 64);
+        for (int off = 1; off < TC; off <<= 1) x += __shfl_xor(x, off, 64);
         return x;
     };
 
@@ -530,14 +557,14 @@ __global__ __launch_bounds__(256, 2) void gdn_decode_vfirst_kernel(RecurrentPara
         f32x4 qc, kc;
 #pragma unroll
         for (int j = 0; j < 4; ++j) { qc[j] = to_f32(cur.q[j]); kc[j] = to_f32(cur.k[j]); }
-        if (tid < 128) sh_v[pb][tid] = to_f32(cur.v);
+        if (tid < VB) sh_v[pb][tid] = to_f32(cur.v);
         float eg = 1.f;
         if (p.g) {
-            float gt = cur.g;
+            float gt = scalar_value(cur.g, p.gb_dtype);
             if (p.A_log) gt = a_neg * softplus_f(gt + dtb);
             eg = __expf(gt);
         }
-        float bb = cur.b;
+        float bb = p.beta ? scalar_value(cur.b, p.beta_dtype) : 1.f;
         if (p.flags & GDN_FLAG_BETA_SIGMOID) bb = bmul * sigmoid_f(bb);
         f32x4 eg4 = {eg, eg, eg, eg};
         if constexpr (GK) {
@@ -564,19 +591,19 @@ __global__ __launch_bounds__(256, 2) void gdn_decode_vfirst_kernel(RecurrentPara
         kc *= rk; qc *= rq;
         __syncthreads();                                // (v of this token is in LDS)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int row = r0 + 8 * i;
+        for (int i = 0; i < R; ++i) {
+            const int row = r0 + RP * i;
             const f32x4 sdec = S[i] * eg4;
             const f32x4 a = sdec * kc, b = sdec * qc;
             const float sk = row_sum((a.x + a.y) + (a.z + a.w)), sq = row_sum((b.x + b.y) + (b.z + b.w));
             const float d = bb * (sh_v[pb][row] - sk);
             S[i] = sdec + kc * d;
-            if (c == 0) o[(tok * HV + ihv) * 128 + row] = from_f32<T>(sq + d * qk);
+            if (c == 0) o[(tok * HV + ihv) * V + v0 + row] = from_f32<T>(sq + d * qk);
         }
     }
     if (p.ht) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) __builtin_nontemporal_store(S[i], (f32x4*)(p.ht + state_off + (r0 + 8 * i) * 128));
+        for (int i = 0; i < R; ++i) __builtin_nontemporal_store(S[i], (f32x4*)(p.ht + state_off + (r0 + RP * i) * KD));
     }
 }
 
@@ -606,16 +633,15 @@ __global__ __launch_bounds__(256, 2) void gdn_decode_bf16_kernel(RecurrentParams
     const int64_t slot = p.state_slots ? load_index(p.state_slots, in, p.flags & GDN_FLAG_SLOT_INT32) : in;
     const int64_t state_off = (slot * HV + ihv) * (int64_t)16384 + 8 * c;
     const T* q = (const T*)p.q; const T* k = (const T*)p.k; const T* v = (const T*)p.v; T* o = (T*)p.o;
-    struct Token { T q, k; T v[8]; float g, b; };
+    struct Token { T q, k; T v[8]; ScalarBits g, b; };
     auto fetch = [&](int64_t tok) {
         Token x;
-        x.q = x.k = from_f32<T>(0.f);
-        if (tid < 128) { x.q = q[(tok * H + ih) * 128 + tid]; x.k = k[(tok * H + ih) * 128 + tid]; }
+        x.q = q[(tok * H + ih) * 128 + (tid & 127)]; x.k = k[(tok * H + ih) * 128 + (tid & 127)];
         const T* pv = v + (tok * HV + ihv) * 128 + 8 * c;
 #pragma unroll
         for (int j = 0; j < 8; ++j) x.v[j] = pv[j];
-        x.g = p.g ? load_scalar(p.g, tok * HV + ihv, p.gb_dtype) : 0.f;
-        x.b = p.beta ? load_scalar(p.beta, tok * HV + ihv, p.gb_dtype) : 1.f;
+        x.g = fetch_scalar(p.g, q, tok * HV + ihv, p.gb_dtype);
+        x.b = fetch_scalar(p.beta, q, tok * HV + ihv, p.beta_dtype);
         return x;
     };
     Token cur = {};
@@ -649,11 +675,11 @@ __global__ __launch_bounds__(256, 2) void gdn_decode_bf16_kernel(RecurrentParams
         if (lane == 0) { sh_red[pb][wave][0] = sqq; sh_red[pb][wave][1] = skk; sh_red[pb][wave][2] = sqk; }
         float eg = 1.f;
         if (p.g) {
-            float gt = cur.g;
+            float gt = scalar_value(cur.g, p.gb_dtype);
             if (p.A_log) gt = a_neg * softplus_f(gt + dtb);
             eg = __expf(gt);
         }
-        float bb = cur.b;
+        float bb = p.beta ? scalar_value(cur.b, p.beta_dtype) : 1.f;
         if (p.flags & GDN_FLAG_BETA_SIGMOID) bb = bmul * sigmoid_f(bb);
         float vv[8];
 #pragma unroll
@@ -749,6 +775,19 @@ static int launch_vb(const RecurrentParams& p0, int64_t n_states, int vb, hipStr
     return check_launch("gdn_recurrent_kernel");
 }
 
+template <typename T, int KD, int VB>
+static int launch_decode(const RecurrentParams& p0, int64_t n_states, hipStream_t stream) {
+    RecurrentParams p = p0;
+    p.NVB = p.V / VB;
+    const int64_t grid = place(p, n_states * p.NVB, (int64_t)p.HV * p.NVB);
+    const bool vfirst = p.flags & GDN_FLAG_STATE_V_FIRST;
+    void (*kern)(RecurrentParams) = vfirst ? (p.gk ? gdn_decode_vfirst_kernel<T, KD, VB, true> : gdn_decode_vfirst_kernel<T, KD, VB>)
+                                  : p.pk ? gdn_decode_kernel<T, KD, VB, false, true>
+                                  : p.gk ? gdn_decode_kernel<T, KD, VB, true> : gdn_decode_kernel<T, KD, VB>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), 0, stream, p);
+    return check_launch(vfirst ? "gdn_decode_vfirst_kernel" : "gdn_decode_kernel");
+}
+
 template <typename T>
 static int launch_t(const RecurrentParams& p, int64_t n_states, hipStream_t stream) {
     const bool vfirst = p.flags & GDN_FLAG_STATE_V_FIRST;
@@ -758,37 +797,14 @@ static int launch_t(const RecurrentParams& p, int64_t n_states, hipStream_t stre
         hipLaunchKernelGGL(gdn_decode_bf16_kernel<T>, dim3((unsigned)grid), dim3(256), 0, stream, pd);
         return check_launch("gdn_decode_bf16_kernel");
     }
-    if (p.K == 128 && p.V == 128 && vfirst && !p.gv && !p.pk && n_states >= 1024 && (uintptr_t)p.gk_bias % 16 == 0 &&
+    // the common decode shapes have kernels of their own
+    if ((p.K == 128 || p.K == 256) && p.V % 32 == 0 && !p.gv && !(p.pk && p.gk) && !(p.pk && vfirst) && (uintptr_t)p.gk_bias % 16 == 0 &&
         !(p.flags & (GDN_FLAG_BETA_VECTOR | GDN_FLAG_SLOT_PER_TOKEN | GDN_FLAG_STATE_PER_TOKEN))) {
-        RecurrentParams pd = p;
-        const int64_t grid = place(pd, n_states, p.HV);
-        static SmemAttrDone attr_done_vf, attr_done_vf_gk;
-        if (p.gk) {
-            if (int rc = ensure_dynamic_smem((const void*)gdn_decode_vfirst_kernel<T, true>, DECODE_LDS_PAD, attr_done_vf_gk, "hipFuncSetAttribute(decode)")) return rc;
-            hipLaunchKernelGGL((gdn_decode_vfirst_kernel<T, true>), dim3((unsigned)grid), dim3(256), DECODE_LDS_PAD, stream, pd);
-        } else {
-            if (int rc = ensure_dynamic_smem((const void*)gdn_decode_vfirst_kernel<T, false>, DECODE_LDS_PAD, attr_done_vf, "hipFuncSetAttribute(decode)")) return rc;
-            hipLaunchKernelGGL((gdn_decode_vfirst_kernel<T, false>), dim3((unsigned)grid), dim3(256), DECODE_LDS_PAD, stream, pd);
-        }
-        return check_launch("gdn_decode_vfirst_kernel");
-    }
-    // the common decode shape has a kernel of its own (enough states to fill the chip with whole-state workgroups)
-    if (p.K == 128 && p.V == 128 && !vfirst && !p.gv && !(p.pk && p.gk) && n_states >= 1024 &&
-        !(p.flags & (GDN_FLAG_BETA_VECTOR | GDN_FLAG_SLOT_PER_TOKEN | GDN_FLAG_STATE_PER_TOKEN))) {
-        RecurrentParams pd = p;
-        const int64_t grid = place(pd, n_states, p.HV);
-        static SmemAttrDone attr_done, attr_done_gk, attr_done_pk;     // per instantiation
-        if (p.pk) {
-            if (int rc = ensure_dynamic_smem((const void*)gdn_decode_kernel<T, false, true>, DECODE_LDS_PAD, attr_done_pk, "hipFuncSetAttribute(decode)")) return rc;
-            hipLaunchKernelGGL((gdn_decode_kernel<T, false, true>), dim3((unsigned)grid), dim3(256), DECODE_LDS_PAD, stream, pd);
-        } else if (p.gk) {
-            if (int rc = ensure_dynamic_smem((const void*)gdn_decode_kernel<T, true>, DECODE_LDS_PAD, attr_done_gk, "hipFuncSetAttribute(decode)")) return rc;
-            hipLaunchKernelGGL((gdn_decode_kernel<T, true>), dim3((unsigned)grid), dim3(256), DECODE_LDS_PAD, stream, pd);
-        } else {
-            if (int rc = ensure_dynamic_smem((const void*)gdn_decode_kernel<T, false>, DECODE_LDS_PAD, attr_done, "hipFuncSetAttribute(decode)")) return rc;
-            hipLaunchKernelGGL((gdn_decode_kernel<T, false>), dim3((unsigned)grid), dim3(256), DECODE_LDS_PAD, stream, pd);
-        }
-        return check_launch("gdn_decode_kernel");
+        // 32 value columns (or rows) a workgroup, for every number of states from one sequence to 256; V-first states that then
+        // leave CUs without a workgroup go 16 rows at a time (K-first ones would read 64-byte rows).
+        if (vfirst && n_states * (p.V / 32) < 256)
+            return p.K == 128 ? launch_decode<T, 128, 16>(p, n_states, stream) : launch_decode<T, 256, 16>(p, n_states, stream);
+        return p.K == 128 ? launch_decode<T, 128, 32>(p, n_states, stream) : launch_decode<T, 256, 32>(p, n_states, stream);
     }
     // Value block per workgroup: whole rows when there are enough (sequence, head) pairs to
     // fill 256 CUs several times over, narrower blocks otherwise.
@@ -862,7 +878,7 @@ static int recurrent_entry(
     p.A_log = A_log; p.dt_bias = dt_bias; p.h0 = h0; p.ht = ht; p.o = o; p.cu_seqlens = cu_seqlens; p.state_slots = state_slots;
     p.num_accepted = num_accepted; p.slots_stride = slots_stride;
     p.T = T; p.H = (int)H; p.HV = (int)HV; p.K = (int)K; p.V = (int)V; p.NVB = 1;
-    p.scale = scale; p.gb_dtype = gb_dtype; p.flags = flags;
+    p.scale = scale; p.gb_dtype = gb_dtype & 255; p.beta_dtype = beta_dtype_of(gb_dtype); p.flags = flags;
     p.gk_act = gk_act; p.gk_bias = gk_bias; p.gk_lower = gk_lower;
     switch (qkv_dtype) {
         case GDN_DTYPE_BF16: return launch_t<bf16_t>(p, N * HV, s);

@@ -33,6 +33,9 @@ extern "C" {
 #define GDN_DTYPE_BF16 0
 #define GDN_DTYPE_F16  1
 #define GDN_DTYPE_F32  2
+/* gb_dtype of gdn_fused_recurrent_fwd, gdn_fused_recurrent_kda_fwd, gdn_fused_recurrent_comba_fwd and gdn_chunk_fwd* where g and
+ * beta differ in type (one type for both: the plain code) */
+#define GDN_GB_DTYPES(g_dtype, beta_dtype) ((g_dtype) | ((beta_dtype) + 1) << 8)
 
 /* flag bits (the reference's keyword switches) */
 #define GDN_FLAG_QK_L2NORM      (1u << 0)  /* use_qk_l2norm_in_kernel                           */
