@@ -1,4 +1,5 @@
-"""Compiles csrc/*.hip into fla_hip/_C/libgdn_hip.so for gfx950 with hipcc.
+"""Compiles csrc/*.hip into fla_hip/_C/libgdn_hip.so for gfx950 with hipcc, and csrc/host/gdn_host.cpp (host code only) into
+the CPython extension fla_hip/_C/gdn_host.so with g++.
 
     python flash-linear-attention_amd/build.py [--force]
 
@@ -11,6 +12,7 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -18,6 +20,8 @@ CSRC = os.path.join(HERE, 'csrc')
 OUT_DIR = os.path.join(HERE, 'fla_hip', '_C')
 LIB = os.path.join(OUT_DIR, 'libgdn_hip.so')
 OBJ_DIR = os.path.join(HERE, 'build', 'obj')
+HOST_SRC = os.path.join(CSRC, 'host', 'gdn_host.cpp')
+HOST_LIB = os.path.join(OUT_DIR, 'gdn_host.so')
 
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
 FLAGS = [
@@ -47,6 +51,18 @@ def _compile(src, obj):
         sys.stderr.write(err + '\n')
 
 
+def _compile_host():
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = ['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-fvisibility=hidden', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
+           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}',
+           *(f'-I{d}' for d in (f'{root}/include', f'{root}/include/torch/csrc/api/include', '/opt/rocm/include', sysconfig.get_paths()['include'])),
+           HOST_SRC, '-o', HOST_LIB, f'-L{root}/lib', '-ltorch_python', '-ltorch', '-ltorch_cpu', '-lc10', '-lc10_hip', f'-Wl,-rpath,{root}/lib']
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f'g++ failed for {HOST_SRC}:\n{r.stderr}')
+
+
 def build(force: bool = False, verbose: bool = True) -> str:
     os.makedirs(OUT_DIR, exist_ok=True)
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -58,10 +74,15 @@ def build(force: bool = False, verbose: bool = True) -> str:
         objs.append(o)
         if force or _newer([s, *hdrs], o):
             jobs.append((s, o))
-    if verbose and jobs:
-        print(f'[build] compiling {len(jobs)} file(s) for gfx950', flush=True)
-    with ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs)))) as ex:
-        list(ex.map(lambda a: _compile(*a), jobs))
+    host = force or _newer([HOST_SRC, hdrs[-1]], HOST_LIB)
+    if verbose and (jobs or host):
+        print(f'[build] compiling {len(jobs)} file(s) for gfx950' + (' and the host extension' if host else ''), flush=True)
+    with ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs) + host))) as ex:
+        pending = [ex.submit(_compile, *a) for a in jobs]
+        if host:
+            pending.append(ex.submit(_compile_host))
+        for p in pending:
+            p.result()
     if jobs or force or _newer(objs, LIB):
         cmd = [HIPCC, '--offload-arch=gfx950', '-shared', '-fPIC', '-o', LIB, *objs]
         r = subprocess.run(cmd, capture_output=True, text=True)

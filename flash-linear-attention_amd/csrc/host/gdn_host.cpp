@@ -1,0 +1,237 @@
+// The operators' host path as native code (a CPython extension over libtorch): argument checks, output and workspace allocation and
+// the call into libgdn_hip.so for the calls that need no conversion of any kind - every tensor contiguous, aligned, on the current
+// device and of a type and shape the kernels take as it is.  Every function returns None for anything else (wrong arguments
+// included) and changes nothing then: the Python path behind it converts, pads or raises.
+//
+// A call through Python and ctypes took 25 us of host time (decode step) to 60 us (prefill), more than the kernels of a small call.
+#include <Python.h>
+#include <ATen/ATen.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cmath>
+
+#include "../../../include/gdn_hip.h"
+
+namespace {
+
+// ---- entry points of libgdn_hip.so, handed over by the Python binding that has loaded it ----
+decltype(&gdn_fused_recurrent_fwd) p_fused_recurrent_fwd;
+decltype(&gdn_fused_recurrent_kda_fwd) p_fused_recurrent_kda_fwd;
+decltype(&gdn_chunk_fwd) p_chunk_fwd;
+decltype(&gdn_chunk_workspace_bytes) p_chunk_workspace_bytes;
+
+PyObject* bind(PyObject*, PyObject* table) {
+    auto take = [&](const char* name, auto& fn) {
+        PyObject* at = PyDict_GetItemString(table, name);
+        if (!at) { PyErr_Format(PyExc_KeyError, "gdn_host.bind: no address of %s", name); return false; }
+        fn = (std::remove_reference_t<decltype(fn)>)PyLong_AsVoidPtr(at);
+        return !PyErr_Occurred();
+    };
+    if (!take("gdn_fused_recurrent_fwd", p_fused_recurrent_fwd) || !take("gdn_fused_recurrent_kda_fwd", p_fused_recurrent_kda_fwd) ||
+        !take("gdn_chunk_fwd", p_chunk_fwd) || !take("gdn_chunk_workspace_bytes", p_chunk_workspace_bytes))
+        return nullptr;
+    Py_RETURN_NONE;
+}
+
+// ---- arguments ----
+// A tensor argument: absent (None), present, or something else.
+struct Arg {
+    const at::Tensor* t = nullptr;
+    bool bad = false;
+    explicit Arg(PyObject* o) {
+        if (o == Py_None) return;
+        if (THPVariable_Check(o)) t = &THPVariable_Unpack(o);
+        else bad = true;
+    }
+    explicit operator bool() const { return t != nullptr; }
+    const at::Tensor* operator->() const { return t; }
+    void* ptr() const { return t ? t->data_ptr() : nullptr; }
+};
+
+int code_of(at::ScalarType s) {
+    switch (s) {
+        case at::kBFloat16: return GDN_DTYPE_BF16;
+        case at::kHalf: return GDN_DTYPE_F16;
+        case at::kFloat: return GDN_DTYPE_F32;
+        default: return -1;
+    }
+}
+
+bool plain(const Arg& a, c10::Device dev) { return !a.bad && (!a || (a->device() == dev && a->is_contiguous() && a->layout() == at::kStrided)); }
+bool aligned16(const void* p) { return (uintptr_t)p % 16 == 0; }
+bool truth(PyObject* o) { return PyObject_IsTrue(o) == 1; }
+
+// g and beta share a code, or carry one each; -1: a type the kernels do not take
+int gb_code_of(const Arg& g, const Arg& beta) {
+    const int cg = g ? code_of(g->scalar_type()) : -2, cb = beta ? code_of(beta->scalar_type()) : -2;
+    if (cg == -1 || cb == -1) return -1;
+    if (cg == -2) return cb == -2 ? GDN_DTYPE_F32 : cb;
+    return cb == -2 || cb == cg ? cg : GDN_GB_DTYPES(cg, cb);
+}
+
+// q, k [B,T,H,K], v [B,T,HV,V] of one type, on the current GPU
+struct Dims { int64_t B, T, H, HV, K, V; c10::Device dev{c10::kCPU}; int code; };
+bool operands(const Arg& q, const Arg& k, const Arg& v, Dims& d) {
+    if (!q || !k || !v || !q->is_cuda() || q->dim() != 4 || v->dim() != 4 || k->sizes() != q->sizes()) return false;
+    d.dev = q->device();
+    if (!plain(q, d.dev) || !plain(k, d.dev) || !plain(v, d.dev)) return false;
+    if (q->scalar_type() != k->scalar_type() || q->scalar_type() != v->scalar_type()) return false;
+    d.code = code_of(q->scalar_type());
+    d.B = q->size(0); d.T = q->size(1); d.H = q->size(2); d.K = q->size(3); d.HV = v->size(2); d.V = v->size(3);
+    return d.code >= 0 && d.B > 0 && d.T > 0 && d.H > 0 && d.K > 0 && d.HV > 0 && d.V > 0 && v->size(0) == d.B && v->size(1) == d.T &&
+           d.HV % d.H == 0 && d.dev.index() == c10::hip::current_device();
+}
+bool per_head(const Arg& x, const Dims& d) {            // [B,T,HV] (or absent)
+    return !x || (x->numel() == d.B * d.T * d.HV && x->dim() == 3 && x->size(0) == d.B && x->size(1) == d.T);
+}
+bool floats(const Arg& x, int64_t n) { return !x || (x->scalar_type() == at::kFloat && x->numel() == n); }
+bool indices(const Arg& x, int64_t n) {
+    return !x || (x->dim() == 1 && (n < 0 || x->numel() == n) && (x->scalar_type() == at::kLong || x->scalar_type() == at::kInt));
+}
+bool scale_of(PyObject* o, int64_t K, float& scale) {
+    if (o == Py_None) { scale = (float)std::pow((double)K, -0.5); return true; }
+    if (!PyFloat_Check(o) && !PyLong_Check(o)) return false;
+    scale = (float)PyFloat_AsDouble(o);
+    return !PyErr_Occurred();
+}
+at::Tensor empty_on(c10::Device dev, at::ScalarType s, at::IntArrayRef sizes) { return at::empty(sizes, at::TensorOptions().dtype(s).device(dev)); }
+void* stream_of(c10::Device dev) { return (void*)c10::hip::getCurrentHIPStream(dev.index()).stream(); }
+
+PyObject* pair(const at::Tensor& a, const at::Tensor& b) {
+    PyObject* x = THPVariable_Wrap(a);
+    PyObject* y = b.defined() ? THPVariable_Wrap(b) : (Py_INCREF(Py_None), Py_None);
+    PyObject* r = x && y ? PyTuple_Pack(2, x, y) : nullptr;
+    Py_XDECREF(x); Py_XDECREF(y);
+    return r;
+}
+
+// ---- token recurrence ----
+// (q, k, v, g, gk, beta, A_log, dt_bias, scale, initial_state, output_final_state, qk_l2norm, beta_sigmoid, neg_eigval, state_v_first,
+//  cu_seqlens, inplace_final_state, state_slots, kda_gate_mode, lower_bound); gk: the KDA operator's gate (kda_gate_mode 0 .. 2) or
+// the general operator's log decays per key feature (kda_gate_mode None)
+PyObject* fused_recurrent(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 20) { PyErr_SetString(PyExc_TypeError, "gdn_host.fused_recurrent takes 20 arguments"); return nullptr; }
+    const Arg q(a[0]), k(a[1]), v(a[2]), g(a[3]), gk(a[4]), beta(a[5]), A_log(a[6]), dt_bias(a[7]), h0(a[9]), cu(a[15]), slots(a[17]);
+    const bool out_final = truth(a[10]), bsig = truth(a[12]), neg = truth(a[13]), vfirst = truth(a[14]), inplace = truth(a[16]);
+    const bool kda = a[18] != Py_None;
+    Dims d;
+    float scale;
+    if (!operands(q, k, v, d) || !scale_of(a[8], d.K, scale)) Py_RETURN_NONE;
+    for (const Arg* x : {&g, &gk, &beta, &A_log, &dt_bias, &h0, &cu, &slots})
+        if (!plain(*x, d.dev)) Py_RETURN_NONE;
+    if (d.K % 4 || d.V % 4 || d.K > 256 || !per_head(g, d) || !indices(cu, -1) || (neg && !bsig)) Py_RETURN_NONE;
+    uint32_t flags = (truth(a[11]) ? GDN_FLAG_QK_L2NORM : 0) | (bsig ? GDN_FLAG_BETA_SIGMOID : 0) | (neg ? GDN_FLAG_NEG_EIGVAL : 0) |
+                     (vfirst ? GDN_FLAG_STATE_V_FIRST : 0);
+    if (beta && beta->dim() == 4 && beta->sizes() == v->sizes() && d.V > 1) flags |= GDN_FLAG_BETA_VECTOR;
+    else if (!per_head(beta, d)) Py_RETURN_NONE;
+    if (gk && (gk->scalar_type() != at::kFloat || gk->numel() != d.B * d.T * d.HV * d.K || gk->dim() != 4 || gk->size(2) != d.HV ||
+               gk->size(1) != d.T || gk->size(3) != d.K || !aligned16(gk.ptr())))
+        Py_RETURN_NONE;
+    if (!floats(A_log, d.HV) || !floats(dt_bias, kda ? d.HV * d.K : d.HV) || (dt_bias && !A_log && !kda) || (A_log && !g && !kda)) Py_RETURN_NONE;
+    const int gb = gb_code_of(g, beta);
+    if (gb < 0) Py_RETURN_NONE;
+    const int64_t N = cu ? cu->numel() - 1 : d.B;
+    if (N < 1 || (cu && d.B != 1)) Py_RETURN_NONE;
+    if (cu && cu->scalar_type() == at::kInt) flags |= GDN_FLAG_CU_INT32;
+    if (slots) {
+        if (!inplace || !h0 || !indices(slots, N)) Py_RETURN_NONE;
+        if (slots->scalar_type() == at::kInt) flags |= GDN_FLAG_SLOT_INT32;
+    }
+    if (inplace && !h0) Py_RETURN_NONE;
+    const int64_t rows = vfirst ? d.V : d.K, cols = vfirst ? d.K : d.V;
+    if (h0) {
+        if (h0->dim() != 4 || (!slots && h0->size(0) != N) || h0->size(1) != d.HV || h0->size(2) != rows || h0->size(3) != cols || !aligned16(h0.ptr()))
+            Py_RETURN_NONE;
+        if (h0->scalar_type() == at::kBFloat16) {
+            if (!inplace || d.K != 128 || d.V != 128 || vfirst || gk || kda || (flags & GDN_FLAG_BETA_VECTOR)) Py_RETURN_NONE;
+            flags |= GDN_FLAG_STATE_BF16;
+        } else if (h0->scalar_type() != at::kFloat) Py_RETURN_NONE;
+    }
+    float lower = 0.f;
+    int mode = 0;
+    if (kda) {
+        if (g || !gk) Py_RETURN_NONE;
+        mode = (int)PyLong_AsLong(a[18]);
+        lower = (float)PyFloat_AsDouble(a[19]);
+        if (PyErr_Occurred()) return nullptr;
+    }
+    const at::Tensor o = empty_on(d.dev, v->scalar_type(), v->sizes());
+    at::Tensor ht;
+    if (inplace) ht = *h0.t;
+    else if (out_final) ht = empty_on(d.dev, at::kFloat, {N, d.HV, rows, cols});
+    void* stream = stream_of(d.dev);
+    float* pht = ht.defined() ? (float*)ht.data_ptr() : nullptr;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    if (kda)
+        rc = p_fused_recurrent_kda_fwd(q.ptr(), k.ptr(), v.ptr(), (const float*)gk.ptr(), beta.ptr(), (const float*)A_log.ptr(), (const float*)dt_bias.ptr(),
+                                       lower, mode, (const float*)h0.ptr(), pht, o.data_ptr(), cu.ptr(), slots.ptr(), nullptr, 1,
+                                       d.B, d.T, d.H, d.HV, d.K, d.V, N, scale, d.code, gb, flags, stream);
+    else
+        rc = p_fused_recurrent_fwd(q.ptr(), k.ptr(), v.ptr(), g.ptr(), beta.ptr(), (const float*)gk.ptr(), nullptr, (const float*)A_log.ptr(),
+                                   (const float*)dt_bias.ptr(), (const float*)h0.ptr(), pht, o.data_ptr(), cu.ptr(), slots.ptr(), nullptr, 1,
+                                   d.B, d.T, d.H, d.HV, d.K, d.V, N, scale, d.code, gb, flags, stream);
+    Py_END_ALLOW_THREADS
+    if (rc != GDN_OK) Py_RETURN_NONE;               // (refused before any launch: the Python path raises)
+    return pair(o, ht);
+}
+
+// ---- chunked forward ----
+// (q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, chunk_indices, scan_tables, A_log, dt_bias,
+//  flags); chunk_indices, scan_tables: the tables of checked boundaries, in cu_seqlens' type
+PyObject* chunk_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 15) { PyErr_SetString(PyExc_TypeError, "gdn_host.chunk_fwd takes 15 arguments"); return nullptr; }
+    const Arg q(a[0]), k(a[1]), v(a[2]), g(a[3]), beta(a[4]), h0(a[6]), cu(a[9]), table(a[10]), offsets(a[11]), A_log(a[12]), dt_bias(a[13]);
+    const bool vfirst = truth(a[8]);
+    Dims d;
+    float scale;
+    if (!operands(q, k, v, d) || d.code == GDN_DTYPE_F32 || !scale_of(a[5], d.K, scale)) Py_RETURN_NONE;
+    for (const Arg* x : {&g, &beta, &h0, &cu, &table, &offsets, &A_log, &dt_bias})
+        if (!plain(*x, d.dev)) Py_RETURN_NONE;
+    if (d.K % 8 || d.V % 8 || d.K > 256 || (d.K <= 128 && d.V > 128) || !beta || !per_head(g, d) || !per_head(beta, d) || !indices(cu, -1)) Py_RETURN_NONE;
+    if (!aligned16(q.ptr()) || !aligned16(k.ptr()) || !aligned16(v.ptr()) || !floats(A_log, d.HV) || !floats(dt_bias, d.HV)) Py_RETURN_NONE;
+    if ((A_log && !g) || (dt_bias && !A_log)) Py_RETURN_NONE;
+    const int gb = gb_code_of(g, beta);
+    if (gb < 0) Py_RETURN_NONE;
+    const int64_t N = cu ? cu->numel() - 1 : d.B;
+    if (N < 1 || (cu && (d.B != 1 || !table || !offsets || table->dim() != 2 || table->scalar_type() != cu->scalar_type() ||
+                         offsets->scalar_type() != cu->scalar_type() || offsets->numel() != 2 * N + 1)))
+        Py_RETURN_NONE;
+    const int64_t num_chunks = cu ? table->size(0) : d.B * ((d.T + 63) / 64);
+    const int64_t rows = vfirst ? d.V : d.K, cols = vfirst ? d.K : d.V;
+    if (h0 && (h0->scalar_type() != at::kFloat || h0->dim() != 4 || h0->size(0) != N || h0->size(1) != d.HV || h0->size(2) != rows ||
+               h0->size(3) != cols || !aligned16(h0.ptr())))
+        Py_RETURN_NONE;
+    uint32_t flags = (uint32_t)PyLong_AsUnsignedLong(a[14]);
+    if (PyErr_Occurred()) return nullptr;
+    if (vfirst) flags |= GDN_FLAG_STATE_V_FIRST;
+    if (cu) flags |= GDN_FLAG_SEQ_ORDER | (cu->scalar_type() == at::kInt ? GDN_FLAG_CU_INT32 : 0);
+    const size_t ws_bytes = p_chunk_workspace_bytes(N, d.T, num_chunks, d.H, d.HV, d.K, d.V, cu ? 1 : 0, flags);
+    if (ws_bytes == 0) Py_RETURN_NONE;
+    const at::Tensor o = empty_on(d.dev, v->scalar_type(), v->sizes());
+    at::Tensor ht;
+    if (truth(a[7])) ht = empty_on(d.dev, at::kFloat, {N, d.HV, rows, cols});
+    const at::Tensor ws = empty_on(d.dev, at::kByte, {(int64_t)ws_bytes});
+    void* stream = stream_of(d.dev);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = p_chunk_fwd(q.ptr(), k.ptr(), v.ptr(), g.ptr(), beta.ptr(), (const float*)A_log.ptr(), (const float*)dt_bias.ptr(), (const float*)h0.ptr(),
+                     ht.defined() ? (float*)ht.data_ptr() : nullptr, o.data_ptr(), cu.ptr(), table.ptr(), offsets.ptr(), ws.data_ptr(), ws_bytes,
+                     d.B, d.T, d.H, d.HV, d.K, d.V, N, num_chunks, scale, d.code, gb, flags, stream);
+    Py_END_ALLOW_THREADS
+    if (rc != GDN_OK) Py_RETURN_NONE;
+    return pair(o, ht);
+}
+
+PyMethodDef methods[] = {
+    {"bind", bind, METH_O, "bind({name: address}) - entry points of libgdn_hip.so"},
+    {"fused_recurrent", (PyCFunction)(void*)fused_recurrent, METH_FASTCALL, "token recurrence; None: not a call for the native path"},
+    {"chunk_fwd", (PyCFunction)(void*)chunk_fwd, METH_FASTCALL, "chunked forward; None: not a call for the native path"},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "gdn_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_gdn_host() { return PyModule_Create(&module); }

@@ -2,12 +2,15 @@
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_uint32, c_void_p
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get('FLA_HIP_LIBRARY') or os.path.join(_HERE, '_C', 'libgdn_hip.so')
+
+HOST_PATH = os.path.join(_HERE, '_C', 'gdn_host.so')
 
 ABI_VERSION = 13
 
@@ -190,6 +193,29 @@ def load() -> ctypes.CDLL:
             raise GDNLibraryError(f'{LIB_PATH} has ABI version {got}, expected {ABI_VERSION}; rebuild it')
         _lib = lib
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The host path's native code (csrc/host/gdn_host.cpp), bound to the library's entry points.  Built with it and, like it,
+    without a stand-in."""
+    global _host
+    if _host is not None:
+        return _host
+    lib = load()
+    with _lock:
+        if _host is None:
+            if not os.path.exists(HOST_PATH):
+                raise GDNLibraryError(f'{HOST_PATH} is missing. Build it with `python {os.path.join(os.path.dirname(_HERE), "build.py")}`.')
+            import torch  # noqa: F401  (the extension's symbols)
+            spec = importlib.util.spec_from_file_location('gdn_host', HOST_PATH)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            module.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in SIGNATURES})
+            _host = module
+    return _host
 
 
 def last_error() -> str:

@@ -123,7 +123,7 @@ def dispatch(operation: str) -> Callable[[Callable], Callable]:
         def wrapper(*args, **kwargs) -> Any:
             BackendRegistry.ensure_initialized(operation)
             registry = BackendRegistry._registries.get(operation)
-            if registry is None:
+            if registry is None or not registry._backends:
                 return func(*args, **kwargs)
             for be in registry._get_sorted_backends():
                 if not (be.is_available() and be.is_enabled()):

@@ -25,7 +25,7 @@ from fla_hip.ops.gated_delta_rule._common import (
     require_gpu,
     unify_gate_beta,
 )
-from fla_hip.ops.utils.index import check_cu_seqlens, prepare_chunk_indices, prepare_scan_tables
+from fla_hip.ops.utils.index import check_cu_seqlens, packed_tables, prepare_chunk_indices, prepare_scan_tables
 from fla_hip.utils import input_guard
 
 # The HIP kernels work on 64-token chunks.  The result of the operator does not depend on
@@ -163,8 +163,39 @@ class ChunkLaunch:
         return o.to(self.out_dtype), ht
 
 
-@input_guard
+def _native_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, cu_seqlens_cpu, A_log, dt_bias,
+                qk_l2norm, beta_sigmoid, neg_eigval):
+    """The forward through the native host path, or None where a tensor needs a conversion first."""
+    mode = os.environ.get('FLA_HIP_SCAN_MODE')
+    flags = (_lib.FLAG_QK_L2NORM if qk_l2norm else 0) | (_SCAN_MODE_FLAGS.get(mode, 0) if mode else 0)
+    if beta_sigmoid:
+        flags |= _lib.FLAG_BETA_SIGMOID | (_lib.FLAG_NEG_EIGVAL if neg_eigval else 0)
+    chunk_indices = scan_tables = None
+    if cu_seqlens is not None:
+        if not cu_seqlens.is_cuda or cu_seqlens.dtype not in (torch.int32, torch.int64):
+            return None
+        _, _, chunk_indices, scan_tables = packed_tables(cu_seqlens, k.shape[1], _KERNEL_CHUNK, cu_seqlens_cpu)
+    return _lib.host().chunk_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, chunk_indices,
+                                 scan_tables, A_log, dt_bias, flags)
+
+
 def chunk_gated_delta_rule_fwd(
+    q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first=False, cu_seqlens=None, cu_seqlens_cpu=None,
+    chunk_indices=None, chunk_size=64, A_log=None, dt_bias=None, use_qk_l2norm_in_kernel=False, use_beta_sigmoid_in_kernel=False,
+    allow_neg_eigval=False,
+):
+    """See ``_chunk_fwd_general``, which takes what the native host path leaves (anything that needs a conversion)."""
+    out = _native_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, cu_seqlens_cpu, A_log,
+                      dt_bias, use_qk_l2norm_in_kernel, use_beta_sigmoid_in_kernel, allow_neg_eigval)
+    if out is not None:
+        return out
+    return _chunk_fwd_general(
+        q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, cu_seqlens_cpu, chunk_indices,
+        chunk_size, A_log, dt_bias, use_qk_l2norm_in_kernel, use_beta_sigmoid_in_kernel, allow_neg_eigval)
+
+
+@input_guard
+def _chunk_fwd_general(
     q: torch.Tensor,
     k: torch.Tensor,
     v: torch.Tensor,

@@ -23,8 +23,28 @@ from fla_hip.ops.utils.index import max_seq_len
 from fla_hip.utils import input_guard
 
 
-@input_guard
 def fused_recurrent_gated_delta_rule_fwd(
+    q, k, v, g=None, gk=None, gv=None, beta=None, A_log=None, dt_bias=None, scale=None, initial_state=None,
+    output_final_state=False, use_qk_l2norm_in_kernel=False, use_beta_sigmoid_in_kernel=False, allow_neg_eigval=False,
+    state_v_first=False, cu_seqlens=None, inplace_final_state=False, ssm_state_indices=None, num_accepted_tokens=None,
+    kda_gate_mode=None, lower_bound=0.0,
+):
+    """See ``_fused_recurrent_general``, which takes what the native host path leaves (anything that needs a conversion)."""
+    if gv is None and num_accepted_tokens is None and scale is not None:
+        out = _lib.host().fused_recurrent(
+            q, k, v, g, gk, beta, A_log, dt_bias, scale, initial_state, output_final_state, use_qk_l2norm_in_kernel,
+            use_beta_sigmoid_in_kernel, allow_neg_eigval, state_v_first, cu_seqlens, inplace_final_state, ssm_state_indices,
+            kda_gate_mode, lower_bound)
+        if out is not None:
+            return out
+    return _fused_recurrent_general(
+        q, k, v, g, gk, gv, beta, A_log, dt_bias, scale, initial_state, output_final_state, use_qk_l2norm_in_kernel,
+        use_beta_sigmoid_in_kernel, allow_neg_eigval, state_v_first, cu_seqlens, inplace_final_state, ssm_state_indices,
+        num_accepted_tokens, kda_gate_mode, lower_bound)
+
+
+@input_guard
+def _fused_recurrent_general(
     q: torch.Tensor,
     k: torch.Tensor,
     v: torch.Tensor,
@@ -268,6 +288,15 @@ def fused_recurrent_gated_delta_rule(
     ssm_state_indices = kwargs.pop('ssm_state_indices', None)
     num_accepted_tokens = kwargs.pop('num_accepted_tokens', None)
 
+    # (the native path takes only what passes every check below)
+    if gv is None and num_accepted_tokens is None and not (use_gate_in_kernel and (A_log is None or g is None)):
+        out = _lib.host().fused_recurrent(
+            q, k, v, g, gk, beta, A_log if use_gate_in_kernel else None, dt_bias if use_gate_in_kernel else None, scale, initial_state,
+            output_final_state, use_qk_l2norm_in_kernel, use_beta_sigmoid_in_kernel, allow_neg_eigval, state_v_first, cu_seqlens,
+            inplace_final_state, ssm_state_indices, None, 0.0)
+        if out is not None:
+            return out
+
     if q.shape[2] != k.shape[2]:
         raise ValueError(f'q and k must have the same number of heads, got {q.shape[2]} and {k.shape[2]}')
     if v.shape[2] % q.shape[2] != 0:
@@ -297,7 +326,7 @@ def fused_recurrent_gated_delta_rule(
                                 or initial_state.dtype not in (torch.float32, torch.bfloat16)):
         raise ValueError('`inplace_final_state=True` requires a contiguous fp32 (or bf16) `initial_state`.')
 
-    return fused_recurrent_gated_delta_rule_fwd(
+    return _fused_recurrent_general(
         q, k, v, g, gk, gv, beta, A_log, dt_bias, scale, initial_state, output_final_state,
         use_qk_l2norm_in_kernel, use_beta_sigmoid_in_kernel, allow_neg_eigval, state_v_first, cu_seqlens,
         inplace_final_state, ssm_state_indices, num_accepted_tokens)

@@ -96,3 +96,19 @@ def prepare_scan_tables(cu_seqlens: torch.Tensor, chunk_size: int,
     out[1:counts.numel() + 1] = torch.cumsum(counts, 0)
     out[counts.numel() + 1:] = torch.argsort(counts, descending=True, stable=True)
     return out.to(device=cu_seqlens.device, dtype=cu_seqlens.dtype)
+
+
+@tensor_cache
+def _packed_tables(cu_seqlens: torch.Tensor, chunk_size: int, cu_seqlens_cpu: torch.Tensor | None = None) -> tuple:
+    return (*_cu_summary(cu_seqlens, cu_seqlens_cpu)[:2], prepare_chunk_indices(cu_seqlens, chunk_size, cu_seqlens_cpu=cu_seqlens_cpu),
+            prepare_scan_tables(cu_seqlens, chunk_size, cu_seqlens_cpu=cu_seqlens_cpu))
+
+
+def packed_tables(cu_seqlens: torch.Tensor, total_tokens: int, chunk_size: int, cu_seqlens_cpu: torch.Tensor | None = None) -> tuple:
+    """Everything a packed call needs from its checked boundaries in one memoised lookup: (first, last boundary,
+    ``prepare_chunk_indices``, ``prepare_scan_tables``).  The check against ``total_tokens`` is ``check_cu_seqlens``'."""
+    hit = _packed_tables.lookup(cu_seqlens, chunk_size, cu_seqlens_cpu)
+    if hit is None or not hit[1] <= total_tokens:
+        check_cu_seqlens(cu_seqlens, total_tokens, cu_seqlens_cpu)
+        hit = _packed_tables(cu_seqlens, chunk_size, cu_seqlens_cpu)
+    return hit

@@ -33,23 +33,35 @@ def tensor_cache(fn: Callable[..., Any]) -> Callable[..., Any]:
         # (tensors created in inference mode keep no version counter: calls with one are not memoised)
         return tuple(None if x.is_inference() else x._version for x in (*args, *kwargs.values()) if isinstance(x, torch.Tensor))
 
-    @functools.wraps(fn)
-    def wrapper(*args, **kwargs):
+    def find(args, kwargs):
         if FLA_DISABLE_TENSOR_CACHE or os.environ.get('FLA_DISABLE_TENSOR_CACHE') == '1':
-            return fn(*args, **kwargs)
+            return None, None
         now = versions(args, kwargs)
         if None in now:
-            return fn(*args, **kwargs)
+            return None, None
         for a0, k0, v0, r0 in entries:
             if len(a0) == len(args) and k0.keys() == kwargs.keys() \
                     and all(x is y for x, y in zip(args, a0)) \
                     and all(kwargs[key] is k0[key] for key in kwargs) \
                     and v0 == now:
-                return r0
+                return now, r0
+        return now, None
+
+    @functools.wraps(fn)
+    def wrapper(*args, **kwargs):
+        now, out = find(args, kwargs)
+        if out is not None:
+            return out
         out = fn(*args, **kwargs)
-        entries.append((args, kwargs, now, out))
+        if now is not None:
+            entries.append((args, kwargs, now, out))
         return out
 
+    def lookup(*args):
+        """The memoised result of a call with positional arguments, or None: never computes."""
+        return find(args, {})[1]
+
+    wrapper.lookup = lookup
     return wrapper
 
 

@@ -1,0 +1,43 @@
+"""The native host path and the decode kernels behind it: blocks of 32 (16) value columns at the edges of their range, gates and betas of
+different types, and the same bits as the general Python path where both can run a call."""
+import pytest
+import torch
+
+from oracle import gdn_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('N,T,H,HV,K,V,vfirst', [
+    (1, 1, 1, 1, 128, 32, False), (1, 1, 1, 1, 128, 32, True), (1, 3, 16, 32, 128, 128, True), (70, 1, 16, 32, 128, 128, True),
+    (70, 1, 16, 32, 128, 128, False), (2, 2, 2, 4, 256, 96, False), (3, 1, 6, 6, 256, 512, True), (20, 1, 6, 6, 256, 512, True)])
+def test_decode_blocks(N, T, H, HV, K, V, vfirst):
+    from fla_hip.ops.gated_delta_rule import fused_recurrent_gated_delta_rule
+    q, k, v, g, beta, h0 = O.make_inputs(N, T, H, HV, K, V, seed=N + K, gate_div=2.0, h0_std=0.3, dtype=torch.bfloat16)
+    beta = beta.bfloat16()
+    ref_o, ref_h = O.recurrent_gated_delta_rule(q, k, v, g, beta.float(), None, h0, True)
+    h = h0.transpose(-1, -2).contiguous() if vfirst else h0.clone()
+    o, ht = fused_recurrent_gated_delta_rule(q.cuda(), k.cuda(), v.cuda(), g.cuda(), beta=beta.cuda(), initial_state=h.cuda(),
+                                             output_final_state=True, state_v_first=vfirst)
+    ht = ht.transpose(-1, -2) if vfirst else ht
+    assert O.get_err_ratio(ref_o, o.float().cpu()) < 5e-3
+    assert O.get_err_ratio(ref_h, ht.cpu()) < 1e-5
+
+
+@pytest.mark.parametrize('cu', [None, [0, 5, 70, 70, 200]])
+def test_native_path_gives_the_general_path_s_bits(cu):
+    from fla_hip.ops.gated_delta_rule import chunk as C
+    from fla_hip.ops.gated_delta_rule import fused_recurrent as R
+    N = 2 if cu is None else len(cu) - 1
+    q, k, v, g, beta, h0 = (x.cuda() for x in O.make_inputs(2 if cu is None else 1, 200, 2, 4, 128, 128, seed=3, gate_div=4.0, h0_std=0.3, N=N,
+                                                            dtype=torch.bfloat16))
+    cu_t = None if cu is None else torch.tensor(cu, device='cuda', dtype=torch.int32)
+    args = (q, k, v, g, beta, 0.1, h0, True, False, cu_t)
+    kw = dict(use_qk_l2norm_in_kernel=True)
+    native = C._native_fwd(*args, None, None, None, True, False, False)
+    assert native is not None
+    general = C._chunk_fwd_general(*args, **kw)
+    assert all(torch.equal(a, b) for a, b in zip(native, general))
+    rargs = (q, k, v, g, None, None, beta, None, None, 0.1, h0, True)
+    native, general = R.fused_recurrent_gated_delta_rule_fwd(*rargs, cu_seqlens=cu_t, **kw), R._fused_recurrent_general(*rargs, cu_seqlens=cu_t, **kw)
+    assert all(torch.equal(a, b) for a, b in zip(native, general))
