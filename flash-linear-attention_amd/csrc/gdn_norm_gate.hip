@@ -213,7 +213,11 @@ static int launch_norm_gate(const NormGateParams& p, bool aligned, hipStream_t s
     if (p.T == 0) return GDN_OK;
     const int64_t pieces = p.D / VEC;                         // 16-byte pieces per row (when D % VEC == 0)
     if (aligned && p.D % VEC == 0 && pieces <= 64 * 8) {
-        if (pieces <= 8) launch_rows<T, 8, 1, 4>(p, stream);
+        // (a decode step: too few rows for four at a time to reach every CU)
+        if (pieces == 64 && p.T <= 4096) launch_rows<T, 64, 1, 1>(p, stream);
+        else if (pieces == 32 && p.T <= 8192) launch_rows<T, 32, 1, 1>(p, stream);
+        else if (pieces == 16 && p.T <= 16384) launch_rows<T, 16, 1, 1>(p, stream);
+        else if (pieces <= 8) launch_rows<T, 8, 1, 4>(p, stream);
         else if (pieces <= 16) launch_rows<T, 16, 1, 4>(p, stream);
         else if (pieces <= 32) launch_rows<T, 32, 1, 4>(p, stream);
         else if (pieces <= 64) launch_rows<T, 64, 1, 4>(p, stream);

@@ -21,6 +21,8 @@ decltype(&gdn_fused_recurrent_fwd) p_fused_recurrent_fwd;
 decltype(&gdn_fused_recurrent_kda_fwd) p_fused_recurrent_kda_fwd;
 decltype(&gdn_chunk_fwd) p_chunk_fwd;
 decltype(&gdn_chunk_workspace_bytes) p_chunk_workspace_bytes;
+decltype(&gdn_step_linear) p_step_linear;
+decltype(&gdn_norm_gated_fwd) p_norm_gated_fwd;
 
 PyObject* bind(PyObject*, PyObject* table) {
     auto take = [&](const char* name, auto& fn) {
@@ -30,7 +32,8 @@ PyObject* bind(PyObject*, PyObject* table) {
         return !PyErr_Occurred();
     };
     if (!take("gdn_fused_recurrent_fwd", p_fused_recurrent_fwd) || !take("gdn_fused_recurrent_kda_fwd", p_fused_recurrent_kda_fwd) ||
-        !take("gdn_chunk_fwd", p_chunk_fwd) || !take("gdn_chunk_workspace_bytes", p_chunk_workspace_bytes))
+        !take("gdn_chunk_fwd", p_chunk_fwd) || !take("gdn_chunk_workspace_bytes", p_chunk_workspace_bytes) ||
+        !take("gdn_step_linear", p_step_linear) || !take("gdn_norm_gated_fwd", p_norm_gated_fwd))
         return nullptr;
     Py_RETURN_NONE;
 }
@@ -225,7 +228,83 @@ PyObject* chunk_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return pair(o, ht);
 }
 
+// ---- one decode step of the layer ----
+// (x [N,1,hidden], q, k, v, a, b, g, o weights, A_log, dt_bias, (q, k, v conv weights [D,1,W]), (q, k, v conv biases), (q, k, v conv
+//  states [N,D,W]), recurrent state [N,HV,V,K], norm weight, norm eps, neg_eigval, num_heads): four launches - the six projections
+// with the convolutions' update and the gate's and beta's activations, the recurrence on the state where it is, the gated norm, the
+// output projection.  The states are updated in place.
+PyObject* layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 18) { PyErr_SetString(PyExc_TypeError, "gdn_host.layer_step takes 18 arguments"); return nullptr; }
+    const Arg x(a[0]), qw(a[1]), kw(a[2]), vw(a[3]), aw(a[4]), bw(a[5]), gw(a[6]), ow(a[7]), A_log(a[8]), dt_bias(a[9]), state(a[13]), norm_w(a[14]);
+    if (!x || !x->is_cuda() || x->dim() != 3 || x->size(1) != 1) Py_RETURN_NONE;
+    const c10::Device dev = x->device();
+    const at::ScalarType type = x->scalar_type();
+    const int code = code_of(type);
+    if ((code != GDN_DTYPE_BF16 && code != GDN_DTYPE_F16) || dev.index() != c10::hip::current_device()) Py_RETURN_NONE;
+    const int64_t N = x->size(0), hidden = x->size(2), H = PyLong_AsLongLong(a[17]);
+    if (PyErr_Occurred()) return nullptr;
+    for (const Arg* t : {&x, &qw, &kw, &vw, &aw, &bw, &gw, &ow, &A_log, &dt_bias, &state, &norm_w})
+        if (!*t || !plain(*t, dev) || !aligned16(t->ptr())) Py_RETURN_NONE;
+    for (const Arg* t : {&qw, &kw, &vw, &aw, &bw, &gw})
+        if (t->t->scalar_type() != type || t->t->dim() != 2 || t->t->size(1) != hidden) Py_RETURN_NONE;
+    if (state->scalar_type() != at::kFloat || state->dim() != 4 || state->size(0) != N) Py_RETURN_NONE;
+    const int64_t HV = state->size(1), V = state->size(2), K = state->size(3), kd = H * K, vd = HV * V;
+    if (N < 1 || N > 128 || H < 1 || HV % H || K % 4 || V % 8 || K > 256 || hidden % 256 || vd % 256 || qw->size(0) != kd || kw->size(0) != kd || vw->size(0) != vd ||
+        gw->size(0) != vd || aw->size(0) != HV || bw->size(0) != HV || ow->scalar_type() != type || ow->dim() != 2 || ow->size(1) != vd ||
+        A_log->numel() != HV || dt_bias->numel() != HV || A_log->scalar_type() != dt_bias->scalar_type() || norm_w->numel() != V)
+        Py_RETURN_NONE;
+    const int gate_code = code_of(A_log->scalar_type()), norm_code = code_of(norm_w->scalar_type());
+    if (gate_code < 0 || norm_code < 0) Py_RETURN_NONE;
+    const int64_t out_cols = ow->size(0);
+    gdn_step_segment seg[6] = {};
+    for (int i = 10; i < 13; ++i)
+        if (!PyTuple_Check(a[i]) || PyTuple_GET_SIZE(a[i]) != 3) Py_RETURN_NONE;
+    for (int i = 0; i < 3; ++i) {
+        const Arg w(PyTuple_GetItem(a[10], i)), bias(PyTuple_GetItem(a[11], i)), st(PyTuple_GetItem(a[12], i));
+        const int64_t D = i < 2 ? kd : vd;
+        if (!w || !st || !plain(w, dev) || !plain(bias, dev) || !plain(st, dev) || w->scalar_type() != type || st->scalar_type() != type) Py_RETURN_NONE;
+        const int64_t W = w->size(-1);
+        if (W < 1 || W > 8 || w->numel() != D * W || st->dim() != 3 || st->size(0) != N || st->size(1) != D || st->size(2) != W ||
+            (bias && (bias->scalar_type() != type || bias->numel() != D)) || !aligned16(w.ptr()) || !aligned16(st.ptr()))
+            Py_RETURN_NONE;
+        const Arg& pw = i == 0 ? qw : i == 1 ? kw : vw;
+        seg[i] = {pw.ptr(), D, nullptr, w.ptr(), bias.ptr(), st.ptr(), nullptr, nullptr, GDN_STEP_CONV, (int)W, 0, 0};
+    }
+    seg[3] = {gw.ptr(), vd, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, GDN_STEP_PLAIN, 0, 0, 0};
+    seg[4] = {aw.ptr(), HV, nullptr, nullptr, nullptr, nullptr, A_log.ptr(), dt_bias.ptr(), GDN_STEP_GATE, 0, gate_code, 0};
+    seg[5] = {bw.ptr(), HV, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, truth(a[16]) ? GDN_STEP_BETA2 : GDN_STEP_BETA, 0, 0, 0};
+    const float eps = (float)PyFloat_AsDouble(a[15]);
+    if (PyErr_Occurred()) return nullptr;
+    const at::Tensor out = empty_on(dev, type, {N, 1, out_cols});
+    // one allocation for everything in between, each part 256-byte aligned
+    int64_t at_byte = 0;
+    auto take = [&](int64_t bytes) { const int64_t at = at_byte; at_byte += (bytes + 255) / 256 * 256; return at; };
+    const int64_t o_q = take(N * kd * 2), o_k = take(N * kd * 2), o_v = take(N * vd * 2), o_gate = take(N * vd * 2), o_o = take(N * vd * 2),
+                  o_y = take(N * vd * 2), o_g = take(N * HV * 4), o_b = take(N * HV * 4);
+    const at::Tensor ws = empty_on(dev, at::kByte, {at_byte});
+    char* base = (char*)ws.data_ptr();
+    seg[0].out = base + o_q; seg[1].out = base + o_k; seg[2].out = base + o_v; seg[3].out = base + o_gate; seg[4].out = base + o_g; seg[5].out = base + o_b;
+    gdn_step_segment last = {};
+    last.weight = ow.ptr(); last.cols = out_cols; last.out = out.data_ptr(); last.kind = GDN_STEP_PLAIN;
+    void* stream = stream_of(dev);
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = p_step_linear(x.ptr(), N, hidden, seg, 6, code, stream);
+    if (rc == GDN_OK)
+        rc = p_fused_recurrent_fwd(base + o_q, base + o_k, base + o_v, base + o_g, base + o_b, nullptr, nullptr, nullptr, nullptr, (const float*)state.ptr(),
+                                   (float*)state.ptr(), base + o_o, nullptr, nullptr, nullptr, 1, N, 1, H, HV, K, V, N, (float)std::pow((double)K, -0.5), code,
+                                   GDN_DTYPE_F32, GDN_FLAG_QK_L2NORM | GDN_FLAG_STATE_V_FIRST, stream);
+    if (rc == GDN_OK)
+        rc = p_norm_gated_fwd(base + o_o, base + o_gate, norm_w.ptr(), nullptr, nullptr, base + o_y, nullptr, nullptr, nullptr, N * HV, V, eps, code, norm_code,
+                              GDN_DTYPE_F32, GDN_DTYPE_F32, GDN_ACT_SILU, 1, stream);
+    if (rc == GDN_OK) rc = p_step_linear(base + o_y, N, vd, &last, 1, code, stream);
+    Py_END_ALLOW_THREADS
+    if (rc != GDN_OK) { PyErr_Format(PyExc_RuntimeError, "gdn_host.layer_step: status %d", rc); return nullptr; }
+    return THPVariable_Wrap(out);
+}
+
 PyMethodDef methods[] = {
+    {"layer_step", (PyCFunction)(void*)layer_step, METH_FASTCALL, "one decode step of the layer; None: not a call for the native path"},
     {"bind", bind, METH_O, "bind({name: address}) - entry points of libgdn_hip.so"},
     {"fused_recurrent", (PyCFunction)(void*)fused_recurrent, METH_FASTCALL, "token recurrence; None: not a call for the native path"},
     {"chunk_fwd", (PyCFunction)(void*)chunk_fwd, METH_FASTCALL, "chunked forward; None: not a call for the native path"},

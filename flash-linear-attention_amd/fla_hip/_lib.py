@@ -157,6 +157,7 @@ SIGNATURES['gdn_norm_gated_bwd'] = (c_int, [
     c_void_p, c_void_p, c_void_p,                      # mean rstd dresidual
     c_void_p, c_void_p, c_void_p, c_void_p,            # dx dg dw_part db_part
     c_int64, c_int64, c_int64, c_int64, c_int, c_int, c_int, c_int, c_void_p])   # T D ld parts ...
+SIGNATURES['gdn_step_linear'] = (c_int, [c_void_p, c_int64, c_int64, c_void_p, c_int, c_int, c_void_p])     # x N hidden segments nseg dtype
 SIGNATURES['gdn_calib_rmw'] = (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p])
 CHUNK_STATIC_WORKSPACE_BYTES = 64 << 20
 CONV_BWD_TILES_PER_PART = 8

@@ -22,8 +22,13 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from fla_hip import _lib
 from fla_hip.modules import FusedRMSNormGated, ShortConvolution
 from fla_hip.ops.gated_delta_rule import chunk_gated_delta_rule, fused_recurrent_gated_delta_rule
+
+
+_STEP_LINEARS = ('q_proj', 'k_proj', 'v_proj', 'a_proj', 'b_proj', 'g_proj', 'o_proj')
+_STEP_CONVS = ('q_conv1d', 'k_conv1d', 'v_conv1d')
 
 
 class LayerCache:
@@ -138,6 +143,37 @@ class GatedDeltaNet(nn.Module):
         with torch.no_grad():
             return self._forward(hidden_states, attention_mask, past_key_values, use_cache, **kwargs)
 
+    def _step(self, hidden_states, past_key_values):
+        """One token per sequence on a filled cache through the native host path (``gdn_host.layer_step``: four launches), or None
+        where the layer is not its plain self - another module in a projection's place, hooks, autocast, a state to be converted."""
+        if past_key_values is None or len(past_key_values) <= self.layer_idx or not (self.use_gate and self.use_short_conv):
+            return None
+        entry = past_key_values[self.layer_idx]
+        state, conv = entry.get('recurrent_state'), entry.get('conv_state')
+        if state is None or conv is None or torch.is_autocast_enabled():
+            return None
+        mods = self._modules
+        linears = [mods[n] for n in _STEP_LINEARS]
+        convs = [mods[n] for n in _STEP_CONVS]
+        norm = mods['o_norm']
+        for m in linears:
+            if type(m) is not nn.Linear or m.bias is not None or m._forward_hooks or m._forward_pre_hooks:
+                return None
+        for m in convs:
+            if type(m) is not ShortConvolution or m.activation is None or m._forward_hooks or m._forward_pre_hooks:
+                return None
+        if type(norm) is not FusedRMSNormGated or norm.activation == 'sigmoid' or norm._forward_hooks or norm._forward_pre_hooks:
+            return None
+        weights = [m._parameters.get('weight') for m in (*linears, *convs, norm)]
+        if any(type(w) is not nn.Parameter for w in weights):
+            return None
+        o = _lib.host().layer_step(
+            hidden_states, *weights[:7], self._parameters['A_log'], self._parameters['dt_bias'], tuple(weights[7:10]),
+            tuple(m._parameters['bias'] for m in convs), tuple(conv), state, weights[10], norm.eps, self.allow_neg_eigval, self.num_heads)
+        if o is not None:
+            past_key_values.update(layer_idx=self.layer_idx, recurrent_state=state, conv_state=conv, offset=1)
+        return o
+
     def _forward(self, hidden_states, attention_mask, past_key_values, use_cache, **kwargs):
         if attention_mask is not None:
             assert attention_mask.dim() == 2, 'attention_mask must be a 0-1 matrix [batch_size, seq_len] (0 = padding)'
@@ -148,6 +184,10 @@ class GatedDeltaNet(nn.Module):
         if self.training and mode != 'chunk':
             raise AssertionError('Only chunk mode is supported in training.')
 
+        if q_len == 1 and not self.training and use_cache and attention_mask is None and kwargs.get('cu_seqlens') is None:
+            o = self._step(hidden_states, past_key_values)
+            if o is not None:
+                return o, None, past_key_values
         last_state = None
         if past_key_values is not None and len(past_key_values) > self.layer_idx:
             last_state = past_key_values[self.layer_idx]

@@ -108,6 +108,30 @@ int gdn_fused_recurrent_fwd(
     float scale, int qkv_dtype, int gb_dtype, uint32_t flags, void* stream);
 
 /*
+ * The projections of one decode step of the layer (fla/layers/gated_deltanet.py:246-300 with one token per sequence) in one launch:
+ * for every segment y = x weight^T (x [N][hidden], weight [cols][hidden], all in `dtype`, bf16 or f16), rounded to `dtype`, then by kind
+ *   GDN_STEP_PLAIN  out [N][cols] = y
+ *   GDN_STEP_CONV   the one-token update of a causal convolution with SiLU (gdn_causal_conv1d_update): conv_state [N][cols][conv_size]
+ *                   moves one place to the left and takes y, out = silu(sum conv_state conv_weight + conv_bias)
+ *   GDN_STEP_GATE   out (fp32) = -exp(A_log) softplus(y + dt_bias), A_log, dt_bias [cols] in gate_dtype (dt_bias may be NULL)
+ *   GDN_STEP_BETA   out (fp32) = sigmoid(y); GDN_STEP_BETA2: twice that
+ * N from 1 to 128, hidden a multiple of 256.
+ */
+#define GDN_STEP_SEGMENTS 6
+#define GDN_STEP_PLAIN 0
+#define GDN_STEP_CONV  1
+#define GDN_STEP_GATE  2
+#define GDN_STEP_BETA  3
+#define GDN_STEP_BETA2 4
+typedef struct {
+    const void* weight; int64_t cols; void* out;
+    const void* conv_weight; const void* conv_bias; void* conv_state;
+    const void* A_log; const void* dt_bias;
+    int kind, conv_size, gate_dtype, reserved;
+} gdn_step_segment;
+int gdn_step_linear(const void* x, int64_t N, int64_t hidden, const gdn_step_segment* segs, int nseg, int dtype, void* stream);
+
+/*
  * Replaces fla/ops/delta_rule/fused_recurrent.py:313-385 (fused_recurrent_delta_rule_bwd and its kernel :111-266): the
  * backward of the token recurrence of the delta rule without gates,
  *   u_t = v_t - S^T k_t;  S <- S + k_t (beta_t u_t)^T;  o_t = scale S^T q_t.

@@ -41,3 +41,33 @@ def test_native_path_gives_the_general_path_s_bits(cu):
     rargs = (q, k, v, g, None, None, beta, None, None, 0.1, h0, True)
     native, general = R.fused_recurrent_gated_delta_rule_fwd(*rargs, cu_seqlens=cu_t, **kw), R._fused_recurrent_general(*rargs, cu_seqlens=cu_t, **kw)
     assert all(torch.equal(a, b) for a, b in zip(native, general))
+
+
+@pytest.mark.parametrize('N,hidden,heads,v_heads,D,expand,conv,neg', [
+    (1, 256, 2, 2, 128, 1, 4, False), (3, 512, 2, 4, 128, 2, 3, True), (16, 2048, 6, 6, 256, 2, 4, False), (17, 1024, 4, 4, 256, 1, 4, False),
+    (33, 1024, 8, 8, 128, 1, 4, True), (65, 512, 4, 4, 64, 1, 4, False), (128, 512, 4, 4, 128, 1, 2, False)])
+def test_layer_step_in_four_launches(N, hidden, heads, v_heads, D, expand, conv, neg, monkeypatch):
+    """The native decode step of the layer against the same step module by module: output and every state, two steps in a row."""
+    from fla_hip.layers import GatedDeltaNet
+    from fla_hip.layers.gated_deltanet import LayerCache
+    torch.manual_seed(N)
+    layer = GatedDeltaNet(hidden_size=hidden, expand_v=expand, head_dim=D, num_heads=heads, num_v_heads=v_heads, conv_size=conv, conv_bias=neg,
+                          allow_neg_eigval=neg, layer_idx=0).cuda().bfloat16().eval()
+    caches = []
+    state = 0.1 * torch.randn(N, v_heads, layer.head_v_dim, D, device='cuda')
+    convs = [torch.randn(N, d, conv, device='cuda', dtype=torch.bfloat16) for d in (layer.key_dim, layer.key_dim, layer.value_dim)]
+    for _ in range(2):
+        caches.append(LayerCache())
+        caches[-1].update(layer_idx=0, recurrent_state=state.clone(), conv_state=tuple(c.clone() for c in convs))
+    for step in range(2):
+        x = torch.randn(N, 1, hidden, device='cuda', dtype=torch.bfloat16)
+        assert layer._step(x, None) is None
+        got = layer._step(x, caches[0])
+        assert got is not None
+        with monkeypatch.context() as m:
+            m.setattr(GatedDeltaNet, '_step', lambda *a: None)
+            want, _, _ = layer(x, past_key_values=caches[1], use_cache=True)
+        assert O.get_err_ratio(want.float(), got.float()) < 5e-3
+        assert O.get_err_ratio(caches[1][0]['recurrent_state'], caches[0][0]['recurrent_state']) < 2e-3
+        for a, b in zip(caches[1][0]['conv_state'], caches[0][0]['conv_state']):
+            assert O.get_err_ratio(a.float(), b.float()) < 2e-3
