@@ -90,6 +90,7 @@ struct BwdParams {
     // to `warm_cap` chunks outside its range where the chunks' transition bounds say that this is forgotten by the time its own
     // range begins (gdn_chunk_common.h, WARM_LOG2); a head with a segment that cannot is walked whole by the workgroups of segment 0.
     int nseg, seg_chunks, warm_cap;
+    int parts;                           // dq and dk leave as this many partial rows per token and q/k head (a divisor of HV / H)
 };
 
 // The mirror image of warm_chunks() for the scan that runs backwards: how many chunks AFTER chunk it1 - 1 a run must start from a
@@ -154,9 +155,7 @@ __device__ __forceinline__ void l2norm_tile_rows(TileRegs<BD>& r, T* out, float*
         float f[8], ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) { f[e] = (float)x[e]; ss += f[e] * f[e]; }
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) ss += __shfl_xor(ss, off, 64);
-        const float rs = rsqrtf(ss + 1e-6f);
+        const float rs = rsqrtf(sum_over_c16(ss) + 1e-6f);
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = (T)(f[e] * rs);
         r.x[i] = __builtin_bit_cast(u32x4, x);
@@ -1851,6 +1850,8 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2w_kernel(BwdParams p, int64
     }
 }
 
+#include "gdn_chunk_bwd_unit.h"
+
 template <typename T, int KT, bool COMBA = false>
 static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t stream) {
     BwdParams p = p_in;
@@ -1933,7 +1934,21 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
         {l2 ? (const void*)gdn_bwd_dqkw_kernel<T, 1, true> : (const void*)gdn_bwd_dqkw_kernel<T, KT>, bwd_dqkw_smem<KT>(), "gdn_bwd_dqkw_kernel", units < 256u ? units : 256u},
         wy,
     };
+    K unit = {nullptr, 0, "gdn_bwd_unit_kernel", 0};
+    int64_t items = 0;
+    if constexpr (!COMBA && KT == 1) {
+        p.parts = p.HV / p.H;
+        items = num_chunks * p.H * p.parts;
+        unit = {l2 ? (const void*)gdn_bwd_unit_kernel<T, BD * KT, BD, 8, true> : (const void*)gdn_bwd_unit_kernel<T, BD * KT, BD, 8, false>, bwd_unit_smem<BD * KT, BD, 8>(), "gdn_bwd_unit_kernel", (unsigned)std::min<int64_t>(items, 256)};
+    }
     for (int i = 0; i < 5; ++i) {
+        if (!COMBA && KT == 1 && i == 3) {
+            if (int rc = ensure_dynamic_smem_for(unit.f, unit.smem, unit.name)) return rc;
+            void* args[] = {(void*)&p, (void*)&items};
+            if (hipLaunchKernel(unit.f, dim3(unit.grid), dim3(512), args, unit.smem, stream) != hipSuccess) return check_launch(unit.name);
+            if (int rc = check_launch(unit.name)) return rc;
+            break;
+        }
         if (ks[i].grid == 0) continue;
         if (int rc = ensure_dynamic_smem_for(ks[i].f, ks[i].smem, ks[i].name)) return rc;
         void* args[] = {(void*)&p, (void*)&second_arg[i]};

@@ -92,6 +92,14 @@ __device__ __forceinline__ int64_t load_index(const void* p, int64_t i, bool is_
     return is_i32 ? (int64_t)((const int32_t*)p)[i] : ((const int64_t*)p)[i];
 }
 
+// The same for an index that is the same in every lane, from a table no kernel in flight writes: scalar loads, which do not stand in
+// the queue of the vector loads (a wave that walks over units would wait for its whole prefetch before it knew the next unit).
+__device__ __forceinline__ int64_t load_index_uniform(const void* p, int64_t i, bool is_i32) {
+    typedef const __attribute__((address_space(4))) int32_t* c32;
+    typedef const __attribute__((address_space(4))) int64_t* c64;
+    return is_i32 ? (int64_t)((c32)(uintptr_t)p)[i] : ((c64)(uintptr_t)p)[i];
+}
+
 __device__ __forceinline__ float softplus_f(float x) {
     // log(1 + e^x) with the usual linear tail (torch threshold 20)
     return x > 20.f ? x : log1pf(__expf(x));

@@ -23,8 +23,8 @@ template <typename P>
 __device__ __forceinline__ ChunkAt chunk_at(const P& p, int64_t ci) {
     const bool cu32 = p.flags & GDN_FLAG_CU_INT32;
     if (p.cu_seqlens) {
-        const int64_t n = load_index(p.chunk_table, 2 * ci, cu32), it = load_index(p.chunk_table, 2 * ci + 1, cu32);
-        const int64_t bos = load_index(p.cu_seqlens, n, cu32), eos = load_index(p.cu_seqlens, n + 1, cu32);
+        const int64_t n = load_index_uniform(p.chunk_table, 2 * ci, cu32), it = load_index_uniform(p.chunk_table, 2 * ci + 1, cu32);
+        const int64_t bos = load_index_uniform(p.cu_seqlens, n, cu32), eos = load_index_uniform(p.cu_seqlens, n + 1, cu32);
         const int64_t t0 = bos + it * CH;
         return ChunkAt{t0, (int)min((int64_t)CH, eos - t0)};
     }
@@ -46,9 +46,9 @@ __device__ __forceinline__ SeqAt seq_at(const P& p, int64_t n) {
     const bool cu32 = p.flags & GDN_FLAG_CU_INT32;
     SeqAt s;
     if (p.cu_seqlens) {
-        s.bos = load_index(p.cu_seqlens, n, cu32);
-        s.len = load_index(p.cu_seqlens, n + 1, cu32) - s.bos;
-        s.cbase = load_index(p.chunk_offsets, n, cu32);
+        s.bos = load_index_uniform(p.cu_seqlens, n, cu32);
+        s.len = load_index_uniform(p.cu_seqlens, n + 1, cu32) - s.bos;
+        s.cbase = load_index_uniform(p.chunk_offsets, n, cu32);
     } else {
         s.bos = n * p.T; s.len = p.T; s.cbase = n * p.NT;
     }
@@ -140,19 +140,28 @@ template <typename T>
 __device__ __forceinline__ typename Mma<T>::V4 pack4(f32x4 x) {
     return typename Mma<T>::V4{(T)x[0], (T)x[1], (T)x[2], (T)x[3]};
 }
+// Sums across lanes without LDS traffic (a ds_bpermute each, some hundred cycles apart, bounded the kernels that walk over units):
+// rows of 16 lanes trade places with v_permlane16_swap / v_permlane32_swap (which need two wait states after the write of their
+// operands), lanes inside a row with DPP.
 __device__ __forceinline__ float sum_over_g(float x) {          // over the four lanes that share c16
-    x += __shfl_xor(x, 16, 64);
-    return x + __shfl_xor(x, 32, 64);
+    float y = x;
+    asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(x), "+v"(y));
+    x += y;
+    y = x;
+    asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "+v"(y));
+    return x + y;
+}
+template <int CTRL> __device__ __forceinline__ float add_dpp(float x) {
+    return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, true));
 }
 __device__ __forceinline__ float sum_over_c16(float x) {        // over the sixteen lanes that share g
-    x += __shfl_xor(x, 1, 64); x += __shfl_xor(x, 2, 64); x += __shfl_xor(x, 4, 64);
-    return x + __shfl_xor(x, 8, 64);
+    x = add_dpp<0xB1>(x);                                       // quad_perm [1,0,3,2]
+    x = add_dpp<0x4E>(x);                                       // quad_perm [2,3,0,1]
+    x = add_dpp<0x141>(x);                                      // row_half_mirror: the other quad of the eight
+    return add_dpp<0x140>(x);                                   // row_mirror: the other eight
 }
 // x summed over the four lanes of a quad (lanes 4n .. 4n+3), in every one of them
-__device__ __forceinline__ float sum_over_quad(float x) {
-    x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, true));   // quad_perm [1,0,3,2]
-    return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x4E, 0xF, 0xF, true));   // [2,3,0,1]
-}
+__device__ __forceinline__ float sum_over_quad(float x) { return add_dpp<0x4E>(add_dpp<0xB1>(x)); }
 #define ZERO4 (f32x4{0.f, 0.f, 0.f, 0.f})
 
 
