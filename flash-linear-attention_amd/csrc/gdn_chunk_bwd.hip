@@ -90,6 +90,7 @@ struct BwdParams {
     // to `warm_cap` chunks outside its range where the chunks' transition bounds say that this is forgotten by the time its own
     // range begins (gdn_chunk_common.h, WARM_LOG2); a head with a segment that cannot is walked whole by the workgroups of segment 0.
     int nseg, seg_chunks, warm_cap;
+    int64_t tokens;                      // rows of q and k per head
     int parts;                           // dq and dk leave as this many partial rows per token and q/k head (a divisor of HV / H)
 };
 
@@ -129,6 +130,11 @@ __device__ __forceinline__ ScanPlan scan_plan(const BwdParams& p, const SeqAt& s
     }
     if (sp.whole) { sp.f0 = 0; sp.f1 = sq.nc; sp.fw = sp.rw = 0; }
     return sp;
+}
+
+// The i-th sequence in the order the scans take them: the longest first where the caller has sorted them (GDN_FLAG_SEQ_ORDER).
+__device__ __forceinline__ int64_t seq_in_order(const BwdParams& p, int64_t i) {
+    return p.cu_seqlens && (p.flags & GDN_FLAG_SEQ_ORDER) ? load_index_uniform(p.chunk_offsets, p.N + 1 + i, p.flags & GDN_FLAG_CU_INT32) : i;
 }
 
 // steps of the longer of the two scans of a workgroup
@@ -208,11 +214,12 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_prepare_kernel(BwdParams p, in
         const int tid = tid_opaque, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = lane & 15, g = lane >> 4;
         if constexpr (L2) {
             const UnitAt at = unit_at(p, u);
-            const int hv = at.hv;                      // (== the q/k head)
             const ChunkAt c = at.c;
-            l2norm_tile_rows<T>(rK, (T*)p.k + (c.tok0 * p.H + hv) * KD, (float*)p.k_rstd + c.tok0 * p.H + hv, p.H, c.valid, tid);
-            l2norm_tile_rows<T>(rQ, (T*)p.q + (c.tok0 * p.H + hv) * KD, (float*)p.q_rstd + c.tok0 * p.H + hv, p.H, c.valid, tid);
-            if constexpr (COMBA) l2norm_tile_rows<T>(rP, (T*)p.pk + (c.tok0 * p.H + hv) * KD, (float*)p.p_rstd + c.tok0 * p.H + hv, p.H, c.valid, tid);
+            const int64_t row0 = c.tok0 * p.H + at.hq;
+            const int keep = at.hq * (p.HV / p.H) == at.hv ? c.valid : 0;      // (the first of the value heads that share the rows leaves them)
+            l2norm_tile_rows<T>(rK, (T*)p.k + row0 * KD, (float*)p.k_rstd + row0, p.H, keep, tid);
+            l2norm_tile_rows<T>(rQ, (T*)p.q + row0 * KD, (float*)p.q_rstd + row0, p.H, keep, tid);
+            if constexpr (COMBA) l2norm_tile_rows<T>(rP, (T*)p.pk + row0 * KD, (float*)p.p_rstd + row0, p.H, keep, tid);
         }
         put_tile<KD>(sK, PK, rK, tid);
         put_tile<KD>(sQ, PK, rQ, tid);
@@ -555,7 +562,7 @@ __device__ __forceinline__ void bwd_state_body(const BwdParams& p, char* smem, c
     const int64_t run = (int64_t)(bid / (8 * NVS)) * 8 + bid % 8;
     if (run >= p.N * p.HV) return;
     const int vs = (bid / 8) % NVS, hv = (int)(run % p.HV), hq = hv / (p.HV / p.H);
-    const int64_t n = run / p.HV;
+    const int64_t n = seq_in_order(p, run / p.HV);
     const SeqAt sq = seq_at(p, n);
     const int vcol0 = vs * VBT;
     const ScanPlan plan = scan_plan(p, sq, hv, seg, lane);
@@ -680,10 +687,10 @@ __device__ __forceinline__ void bwd_state_body(const BwdParams& p, char* smem, c
 // (all 128 value columns of a head: eight waves, two per SIMD, share one set of tiles)
 template <int VBT> constexpr int scan_waves() { return VBT == BD ? 8 : 4; }
 
-template <typename T, int VBT, int KT, bool KDA = false>
+template <typename T, int VBT, int KT>
 __global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_state_kernel(BwdParams p) {
     extern __shared__ __align__(16) char smem[];
-    bwd_state_body<T, VBT, KT, 1, scan_waves<VBT>(), KDA>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
+    bwd_state_body<T, VBT, KT, 1, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
 }
 
 // KDA: k and q arrive as KG and QG (decays and the scale on them), P row-major instead of transposed, the gradient of the
@@ -707,7 +714,7 @@ __device__ __forceinline__ void bwd_dstate_body(const BwdParams& p, char* smem, 
     const int64_t run = (int64_t)(bid / (8 * NVS)) * 8 + bid % 8;
     if (run >= p.N * p.HV) return;
     const int vs = (bid / 8) % NVS, hv = (int)(run % p.HV), hq = hv / (p.HV / p.H);
-    const int64_t n = run / p.HV;
+    const int64_t n = seq_in_order(p, run / p.HV);
     const SeqAt sq = seq_at(p, n);
     const int vcol0 = vs * VBT;
     const ScanPlan plan = scan_plan(p, sq, hv, seg, lane);
@@ -872,10 +879,10 @@ __device__ __forceinline__ void bwd_dstate_body(const BwdParams& p, char* smem, 
     }
 }
 
-template <typename T, int VBT, int KT, bool KDA = false>
+template <typename T, int VBT, int KT>
 __global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_dstate_kernel(BwdParams p) {
     extern __shared__ __align__(16) char smem[];
-    bwd_dstate_body<T, VBT, KT, 1, scan_waves<VBT>(), KDA>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
+    bwd_dstate_body<T, VBT, KT, 1, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
 }
 
 // Both scans in one workgroup of eight waves: waves 0-3 walk the chunks forwards (S, v_new), waves 4-7 backwards (dS, dv_new).
@@ -885,48 +892,47 @@ __global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_dstate_kernel(
 // gdn_bwd_scans_apart_kernel below.
 template <int VBT, int KT> constexpr size_t bwd_scans_smem() { return bwd_state_smem<VBT, KT>() + bwd_dstate_smem<VBT, KT>(); }
 
-template <typename T, int VBT, int KT, bool KDA = false>
+template <typename T, int VBT, int KT>
 __global__ __launch_bounds__(512) void gdn_bwd_scans_kernel(BwdParams p) {
     extern __shared__ __align__(16) char smem[];
     static_assert(bwd_state_smem<VBT, KT>() % 16 == 0, "the second set of tiles starts 16-byte aligned");
-    if (threadIdx.x < 256) bwd_state_body<T, VBT, KT, 1, 4, KDA>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
-    else bwd_dstate_body<T, VBT, KT, 1, 4, KDA>(p, smem + bwd_state_smem<VBT, KT>(), threadIdx.x - 256, blockIdx.x, gridDim.x);
+    if (threadIdx.x < 256) bwd_state_body<T, VBT, KT, 1, 4>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
+    else bwd_dstate_body<T, VBT, KT, 1, 4>(p, smem + bwd_state_smem<VBT, KT>(), threadIdx.x - 256, blockIdx.x, gridDim.x);
 }
 
-// Both scans in one launch, in workgroups of their own: the first `nstate` workgroups walk forwards, the others backwards.
-// For calls whose two scans together need no more workgroups than there are CUs: the launch then takes the time of the
-// longer scan instead of their sum.
+// Both scans in one launch, in workgroups of their own: the first `nrev` workgroups walk backwards (the longer steps), the others
+// forwards.  Where the two together need no more workgroups than there are CUs the launch takes the time of the longer scan; where
+// they need more, the CUs that one scan's last round would leave idle go on with the other (16000 packed tokens in 12 sequences, 32
+// heads: the step 1355 us with one scan after the other, 1245 us with both in a launch, longest sequences first).
 template <int VBT, int KT> constexpr size_t bwd_scans_apart_smem() {
     return bwd_state_smem<VBT, KT>() > bwd_dstate_smem<VBT, KT>() ? bwd_state_smem<VBT, KT>() : bwd_dstate_smem<VBT, KT>();
 }
 template <typename T, int VBT, int KT, bool KDA = false>
-__global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_scans_apart_kernel(BwdParams p, int64_t nstate) {
+__global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_scans_apart_kernel(BwdParams p, int64_t nrev) {
     extern __shared__ __align__(16) char smem[];
-    if (blockIdx.x >= nstate) bwd_dstate_body<T, VBT, KT, 1, scan_waves<VBT>(), KDA>(p, smem, threadIdx.x, blockIdx.x - (unsigned)nstate, gridDim.x - (unsigned)nstate);
-    else bwd_state_body<T, VBT, KT, 1, scan_waves<VBT>(), KDA>(p, smem, threadIdx.x, blockIdx.x, (unsigned)nstate);
+    if (blockIdx.x < nrev) bwd_dstate_body<T, VBT, KT, 1, scan_waves<VBT>(), KDA>(p, smem, threadIdx.x, blockIdx.x, (unsigned)nrev);
+    else bwd_state_body<T, VBT, KT, 1, scan_waves<VBT>(), KDA>(p, smem, threadIdx.x, blockIdx.x - (unsigned)nrev, gridDim.x - (unsigned)nrev);
 }
 
 // ---------------------------------------------------------------------------------------------
-// dq, dw and the first parts of dk and dgam.  Per block kb of 128 key features wave w owns features 128kb + 32w .. + 31
-// (two tiles a2) of all 64 tokens (four tiles t): lane (c16, g) holds token 16t + c16 and features
-// 128kb + 16(2w+a2) + 4g .. +3.
+// (comba) dq, dw and the first parts of dk and dgam.  Wave w owns key features 32w .. + 31 (two tiles a2) of all 64 tokens (four
+// tiles t): lane (c16, g) holds token 16t + c16 and features 16(2w+a2) + 4g .. +3.
 // ---------------------------------------------------------------------------------------------
-// One workgroup per CU walks over the units and fetches everything the next unit needs (five tiles and, with one block of key
-// features, its fragments of S and dS) into registers while it works on the current one.
+// One workgroup per CU walks over the units and fetches everything the next unit needs (five tiles and its
+// fragments of S and dS) into registers while it works on the current one.
 // L2: dq goes back through the l2 normalisation of q before it is written (its rows wait in registers for the row sums of q . dq).
-template <int KT> constexpr size_t bwd_dqkw_smem() { return (3 * 64 * P128 + 2 * 64 * (BD * KT + 8) + 64 * P64) * 2 + 640 * 4; }
+constexpr size_t BWD_DQKW_SMEM = (5 * 64 * P128 + 64 * P64) * 2 + 640 * 4;
 
-template <typename T, int KT, bool L2 = false>
+template <typename T, bool L2 = false>
 __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64_t units) {
     typedef typename Mma<T>::V8 V8;
     typedef typename Mma<T>::V4 V4;
-    constexpr int KD = BD * KT, PK = KD + 8;
+    constexpr int KD = BD, PK = KD + 8;
     extern __shared__ __align__(16) char smem[];
     T* sDO = (T*)smem; T* sVn = sDO + 64 * P128; T* sDvn = sVn + 64 * P128; T* sK = sDvn + 64 * P128; T* sQ = sK + 64 * PK;
     T* sDP = sQ + 64 * PK;
     float* sGam = (float*)(sDP + 64 * P64); float* sDg = sGam + 64;    // sDg [4][64]: a row per wave, added up in a fixed order (same bits every run)
     float* sQd = sDg + 256; float* sRq = sQd + 256;                    // (L2) q . dq per wave and token; the tokens' factors
-    static_assert(!L2 || KT == 1, "the rows of dq wait in the registers of one block of key features");
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c16 = lane & 15, g = lane >> 4;
 
     TileRegs<BD> rDO, rVn, rDvn;
@@ -940,7 +946,7 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
         fetch_tile<BD>(rDO, (const T*)p.dout + (c.tok0 * p.HV + hv) * BD, (int64_t)p.HV * BD, c.valid, tid);
         fetch_tile<BD>(rVn, (const T*)p.ws.Vn + u * 64 * BD, BD, 64, tid);
         fetch_tile<BD>(rDvn, (const T*)p.ws.dVn + u * 64 * BD, BD, 64, tid);
-        if constexpr (KT == 1) {
+        {
             const T* Hu = (const T*)p.ws.Hs + u * KD * BD;
             const T* dHu = (const T*)p.ws.dHs + u * KD * BD;
 #pragma unroll
@@ -952,10 +958,8 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
                     rdS[a2][s] = *(const V8*)(dHu + kk * BD + 32 * s + 8 * g);
                 }
         }
-        if constexpr (KT == 1) {
-            fetch_tile<KD>(rK, (const T*)p.k + (c.tok0 * p.H + hq) * KD, (int64_t)p.H * KD, c.valid, tid);
-            fetch_tile<KD>(rQ, (const T*)p.q + (c.tok0 * p.H + hq) * KD, (int64_t)p.H * KD, c.valid, tid);
-        }
+        fetch_tile<KD>(rK, (const T*)p.k + (c.tok0 * p.H + hq) * KD, (int64_t)p.H * KD, c.valid, tid);
+        fetch_tile<KD>(rQ, (const T*)p.q + (c.tok0 * p.H + hq) * KD, (int64_t)p.H * KD, c.valid, tid);
         if (tid < 64) rGam = p.ws.Gam[u * 64 + tid];
         if constexpr (L2) rRq = tid < c.valid ? p.q_rstd[(c.tok0 + tid) * p.H + hq] : 0.f;
     };
@@ -964,11 +968,6 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
         const UnitAt at = unit_at(p, u);
         const int hv = at.hv;
         const ChunkAt c = at.c;
-        if constexpr (KT > 1) {                                 // (no registers to spare for fetching the wide tiles ahead)
-            const int hq = at.hq;
-            fetch_tile<KD>(rK, (const T*)p.k + (c.tok0 * p.H + hq) * KD, (int64_t)p.H * KD, c.valid, tid);
-            fetch_tile<KD>(rQ, (const T*)p.q + (c.tok0 * p.H + hq) * KD, (int64_t)p.H * KD, c.valid, tid);
-        }
         put_tile<BD>(sDO, P128, rDO, tid);
         put_tile<BD>(sVn, P128, rVn, tid);
         put_tile<BD>(sDvn, P128, rDvn, tid);
@@ -978,7 +977,7 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
         if constexpr (L2) { if (tid < 64) sRq[tid] = rRq; }
         sDg[tid] = 0.f;
         V8 sf[2][4], df[2][4];
-        if constexpr (KT == 1) {
+        {
 #pragma unroll
             for (int a2 = 0; a2 < 2; ++a2)
 #pragma unroll
@@ -989,21 +988,7 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
 
         float sdot = 0.f, dglast = 0.f;
         f32x4 dq_rows[L2 ? 2 : 1][4];
-#pragma unroll 1
-        for (int kb = 0; kb < KT; ++kb) {                       // (a real loop: one block's accumulators at a time)
-            if (KT > 1) {
-                // (two blocks of key features: no registers to spare for fetching these ahead, they come straight from memory)
-                const T* Hu = (const T*)p.ws.Hs + u * KD * BD;
-                const T* dHu = (const T*)p.ws.dHs + u * KD * BD;
-#pragma unroll
-                for (int a2 = 0; a2 < 2; ++a2)
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const int kk = BD * kb + 16 * (2 * w + a2) + c16;
-                        sf[a2][s] = *(const V8*)(Hu + kk * BD + 32 * s + 8 * g);
-                        df[a2][s] = *(const V8*)(dHu + kk * BD + 32 * s + 8 * g);
-                    }
-            }
+        {
             // Operand fragments are fetched from LDS once per use across the two feature tiles of this wave.
             f32x4 G1[2][4], dKS[2][4], dWt[2][4], dPt[4];
 #pragma unroll
@@ -1018,8 +1003,7 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
                 for (int a2 = 0; a2 < 2; ++a2)
 #pragma unroll
                     for (int e = 0; e < 8; ++e) sdot += (float)sf[a2][s][e] * (float)df[a2][s][e];
-                V8 own;
-                if (kb == 0) own = frag_rows(sDO, P128, 16 * w, 32 * s, lane);      // this wave's 16 token rows of do, for dP
+                const V8 own = frag_rows(sDO, P128, 16 * w, 32 * s, lane);      // this wave's 16 token rows of do, for dP
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const V8 bdo = frag_rows(sDO, P128, 16 * t, 32 * s, lane), bdv = frag_rows(sDvn, P128, 16 * t, 32 * s, lane),
@@ -1030,7 +1014,7 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
                         dWt[a2][t] = Mma<T>::run(sf[a2][s], bdv, dWt[a2][t]);
                         dKS[a2][t] = Mma<T>::run(df[a2][s], bvn, dKS[a2][t]);
                     }
-                    if (kb == 0 && t <= w) dPt[t] = Mma<T>::run(own, bvn, dPt[t]);
+                    if (t <= w) dPt[t] = Mma<T>::run(own, bvn, dPt[t]);
                 }
             }
             {
@@ -1039,9 +1023,9 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
                 for (int a2 = 0; a2 < 2; ++a2)
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
-                        *(V4*)(dWu + (16 * t + c16) * KD + BD * kb + 16 * (2 * w + a2) + 4 * g) = pack4<T>(-dWt[a2][t]);
+                        *(V4*)(dWu + (16 * t + c16) * KD + 16 * (2 * w + a2) + 4 * g) = pack4<T>(-dWt[a2][t]);
             }
-            if (kb == 0) {
+            {
                 // dP o D for this wave's 16 token rows, as an operand tile
                 float gi[4];
 #pragma unroll
@@ -1065,8 +1049,8 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
             for (int a2 = 0; a2 < 2; ++a2)
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
-                    fk[a2][s] = frag_cols(sK, PK, 32 * s, BD * kb + 16 * (2 * w + a2), lane);
-                    fq[a2][s] = frag_cols(sQ, PK, 32 * s, BD * kb + 16 * (2 * w + a2), lane);
+                    fk[a2][s] = frag_cols(sK, PK, 32 * s, 16 * (2 * w + a2), lane);
+                    fq[a2][s] = frag_cols(sQ, PK, 32 * s, 16 * (2 * w + a2), lane);
                 }
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
@@ -1077,7 +1061,7 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
                 V4 q4[2], k4[2];
 #pragma unroll
                 for (int a2 = 0; a2 < 2; ++a2) {
-                    const int n16 = BD * kb + 16 * (2 * w + a2);
+                    const int n16 = 16 * (2 * w + a2);
                     dq[a2] = G1[a2][t] * fqs;
                     dk[a2] = dKS[a2][t] * fks;
                     q4[a2] = *(const V4*)(sQ + x * PK + n16 + 4 * g);
@@ -1113,7 +1097,7 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
                 if (x < c.valid) {
 #pragma unroll
                     for (int a2 = 0; a2 < 2; ++a2) {
-                        const int n16 = BD * kb + 16 * (2 * w + a2);
+                        const int n16 = 16 * (2 * w + a2);
                         if constexpr (!L2) *(V4*)((T*)p.dq + ((c.tok0 + x) * p.HV + hv) * KD + n16 + 4 * g) = pack4<T>(dq[a2]);
                         *(V4*)((T*)p.dk + ((c.tok0 + x) * p.HV + hv) * KD + n16 + 4 * g) = pack4<T>(dk[a2]);
                     }
@@ -1148,7 +1132,7 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
 }
 
 // ---------------------------------------------------------------------------------------------
-// back through w = X (e^gam k), u = X v, X = A diag(beta), A = (I + diag(beta) stril(k k^T o D))^-1
+// (comba) back through w = X (e^gam0 p), u = X v, X = A diag(beta), A = (I + diag(beta) stril(k k^T o D))^-1
 // ---------------------------------------------------------------------------------------------
 // Workgroups walk over the units (chunk, v-head), the next unit's tiles on their way into registers meanwhile: dX = tril(dw (e^gam k)^T
 // + du v^T), dA = stril(dX diag(beta)); dv = beta (A^T du); d(e^gam k) = beta (A^T dw), into dk, dbeta, dgam; Y = dA A^T,
@@ -1160,24 +1144,24 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
 // (dX's second term, k k^T, the first part of dk; comba: with the rows of p in a third place) - with the second set on its way
 // into registers during the first half and the next unit's first pair during the second; Y = dA A^T takes dw's place once dw is done with.
 // L2: dk goes back through the l2 normalisation of k before it is written.
-template <bool COMBA = false> constexpr size_t bwd_wy2_smem() { return ((2 + (COMBA ? 1 : 0)) * 64 * P128 + 2 * 64 * P64) * 2 + (960 + 640) * 4; }
+constexpr size_t BWD_WY2_SMEM = (3 * 64 * P128 + 2 * 64 * P64) * 2 + (960 + 640) * 4;
 
-template <typename T, bool L2 = false, bool COMBA = false>
+template <typename T, bool L2 = false>
 __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_t units) {
-    static_assert(2 * bwd_wy2_smem<COMBA>() <= 160 * 1024, "two workgroups per CU");
+    static_assert(2 * BWD_WY2_SMEM <= 160 * 1024, "two workgroups per CU");
     typedef typename Mma<T>::V8 V8;
     typedef typename Mma<T>::V4 V4;
     constexpr int KD = BD, PK = P128, NA = 2;
     extern __shared__ __align__(16) char smem[];
     T* sX0 = (T*)smem; T* sX1 = sX0 + 64 * P128;               // dv_new | v, then dw | k
     T* sA = sX1 + 64 * P128; T* sM1 = sA + 64 * P64; T* sP = sM1 + 64 * P64;     // (comba) rows of the second key
-    float* sGam = (float*)(sP + (COMBA ? 64 * P128 : 0)); float* sBeta = sGam + 64; float* sDg = sBeta + 64; float* sDb = sDg + 256;
+    float* sGam = (float*)(sP + 64 * P128); float* sBeta = sGam + 64; float* sDg = sBeta + 64; float* sDb = sDg + 256;
     float* sKd = sDb + 256; float* sRk = sKd + 256;              // (L2) k . dk per wave and token; the tokens' factors
     float* sDg0 = sRk + 64; float* sGam0 = sDg0 + 256;           // (comba)
     float* sPd = sGam0 + 64; float* sRp = sPd + 256;             // (comba, L2) p . dp per wave and token; the tokens' factors
     T* sDvn = sX0; T* sV = sX1; T* sDW = sX0; T* sK = sX1; T* sM2 = sX0;
-    T* sRows = COMBA ? sP : sK;
-    float* sGamRow = COMBA ? sGam0 : sGam; float* sDgRow = COMBA ? sDg0 : sDg;
+    T* sRows = sP;
+    float* sGamRow = sGam0; float* sDgRow = sDg0;
 
     TileRegs<BD> rDvn, rV, rDW, rK, rP;
     TileRegs<CH> rA;
@@ -1194,9 +1178,9 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
             rGam = p.ws.Gam[u * 64 + tid];
             rBeta = tid < c.valid ? load_scalar_bits(p.beta, (c.tok0 + tid) * p.HV + hv, p.gb_dtype) : 0;
             rDg = p.ws.Dgam[u * 64 + tid];
-            if constexpr (COMBA) rGam0 = p.ws.Gam0[u * 64 + tid];
+            rGam0 = p.ws.Gam0[u * 64 + tid];
             if constexpr (L2) rRk = tid < c.valid ? p.k_rstd[(c.tok0 + tid) * p.H + hv] : 0.f;
-            if constexpr (L2 && COMBA) rRp = tid < c.valid ? p.p_rstd[(c.tok0 + tid) * p.H + hv] : 0.f;
+            if constexpr (L2) rRp = tid < c.valid ? p.p_rstd[(c.tok0 + tid) * p.H + hv] : 0.f;
         }
     };
     fetch_first(blockIdx.x, threadIdx.x);
@@ -1213,14 +1197,14 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
         put_tile<BD>(sDvn, P128, rDvn, tid);
         put_tile<BD>(sV, P128, rV, tid);
         put_tile<CH>(sA, P64, rA, tid);
-        if (tid < 64) { sGam[tid] = rGam; sBeta[tid] = scalar_of_bits(rBeta, p.gb_dtype); if constexpr (L2) sRk[tid] = rRk; if constexpr (COMBA) sGam0[tid] = rGam0; if constexpr (L2 && COMBA) sRp[tid] = rRp; }
+        if (tid < 64) { sGam[tid] = rGam; sBeta[tid] = scalar_of_bits(rBeta, p.gb_dtype); if constexpr (L2) sRk[tid] = rRk; sGam0[tid] = rGam0; if constexpr (L2) sRp[tid] = rRp; }
         sDg[tid] = tid < 64 ? rDg : 0.f;
         sDb[tid] = 0.f;
-        if constexpr (COMBA) sDg0[tid] = 0.f;
+        sDg0[tid] = 0.f;
         // the second pair of this unit, and what the previous kernel left in dk at this lane's places
         fetch_tile<KD>(rDW, (const T*)p.ws.dWm + u * 64 * KD, KD, 64, tid);
         fetch_tile<KD>(rK, (const T*)p.k + (c.tok0 * p.H + hq) * KD, (int64_t)p.H * KD, c.valid, tid);
-        if constexpr (COMBA) fetch_tile<KD>(rP, (const T*)p.pk + (c.tok0 * p.H + hq) * KD, (int64_t)p.H * KD, c.valid, tid);
+        fetch_tile<KD>(rP, (const T*)p.pk + (c.tok0 * p.H + hq) * KD, (int64_t)p.H * KD, c.valid, tid);
         V4 dk_old[NA][4];
 #pragma unroll
         for (int a2 = 0; a2 < NA; ++a2)
@@ -1285,7 +1269,7 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
         lds_barrier();                                          // (dv_new and v are done with)
         put_tile<KD>(sDW, PK, rDW, tid);
         put_tile<KD>(sK, PK, rK, tid);
-        if constexpr (COMBA) put_tile<KD>(sP, PK, rP, tid);
+        put_tile<KD>(sP, PK, rP, tid);
         lds_barrier();
         if (u + gridDim.x < units) fetch_first(u + gridDim.x, tid);
 
@@ -1307,8 +1291,7 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
 #pragma unroll
                     for (int s = 0; s < 4; ++s) {
                         const V8 bk = frag_rows(sK, PK, 16 * tj, 32 * s, lane);
-                        if constexpr (COMBA) dXw = Mma<T>::run(fw[s], frag_rows(sP, PK, 16 * tj, 32 * s, lane), dXw);
-                        else dXw = Mma<T>::run(fw[s], bk, dXw);
+                        dXw = Mma<T>::run(fw[s], frag_rows(sP, PK, 16 * tj, 32 * s, lane), dXw);
                         kkT[tj] = Mma<T>::run(fk[s], bk, kkT[tj]);
                     }
                 }
@@ -1322,7 +1305,7 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
             }
         }
         // d(e^gam k) = beta (A^T dw): into dk, dbeta, dgam  (comba: d(e^gam0 p), into dp, dbeta, dgam0)
-        f32x4 dk[NA][4], dpk[COMBA ? NA : 1][4];
+        f32x4 dk[NA][4], dpk[NA][4];
         {
             V8 fA[4][2];
             float ej[4], bj[4];
@@ -1355,8 +1338,7 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
                     for (int r = 0; r < 4; ++r) dot += ak[r] * (float)k4[r];
                     dot = sum_over_g(dot);
                     if (g == 0) { atomicAdd(&sDb[64 * w + j], ej[t] * dot); atomicAdd(&sDgRow[64 * w + j], bj[t] * ej[t] * dot); }
-                    if constexpr (COMBA) { dpk[a2][t] = ak * (bj[t] * ej[t]); dk[a2][t] = ZERO4; }
-                    else dk[a2][t] = ak * (bj[t] * ej[t]);
+                    { dpk[a2][t] = ak * (bj[t] * ej[t]); dk[a2][t] = ZERO4; }
                 }
             }
         }
@@ -1422,13 +1404,13 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
         lds_barrier();
         // dk += E k + E^T k, on top of what the previous kernel left  (comba: dp += E k, dk += E^T p)
         {
-            V8 fk[NA][2], fp[COMBA ? NA : 1][2];
+            V8 fk[NA][2], fp[NA][2];
 #pragma unroll
             for (int a2 = 0; a2 < NA; ++a2)
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
                     fk[a2][s] = frag_cols(sK, PK, 32 * s, feat(a2), lane);
-                    if constexpr (COMBA) fp[a2][s] = frag_cols(sP, PK, 32 * s, feat(a2), lane);
+                    fp[a2][s] = frag_cols(sP, PK, 32 * s, feat(a2), lane);
                 }
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
@@ -1438,16 +1420,14 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
                         const V8 e = frag_rows(sM1, P64, 16 * t, 32 * s, lane);
 #pragma unroll
                         for (int a2 = 0; a2 < NA; ++a2) {
-                            if constexpr (COMBA) dpk[a2][t] = Mma<T>::run(fk[a2][s], e, dpk[a2][t]);
-                            else dk[a2][t] = Mma<T>::run(fk[a2][s], e, dk[a2][t]);
+                            dpk[a2][t] = Mma<T>::run(fk[a2][s], e, dpk[a2][t]);
                         }
                     }
                     if (32 * s + 31 >= 16 * t) {                // E[i][l], i > l
                         const V8 e = frag_cols(sM1, P64, 32 * s, 16 * t, lane);
 #pragma unroll
                         for (int a2 = 0; a2 < NA; ++a2) {
-                            if constexpr (COMBA) dk[a2][t] = Mma<T>::run(fp[a2][s], e, dk[a2][t]);
-                            else dk[a2][t] = Mma<T>::run(fk[a2][s], e, dk[a2][t]);
+                            dk[a2][t] = Mma<T>::run(fp[a2][s], e, dk[a2][t]);
                         }
                     }
                 }
@@ -1462,7 +1442,7 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
                     }
                     kdk = sum_over_g(kdk);
                     if (g == 0) sKd[64 * w + x] = kdk;
-                    if constexpr (COMBA) {
+                    {
                         float pdp = 0.f;
 #pragma unroll
                         for (int a2 = 0; a2 < NA; ++a2) {
@@ -1480,7 +1460,7 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
 #pragma unroll
                         for (int r = 0; r < 4; ++r) acc[r] += (float)dk_old[a2][t][r];
                         *(V4*)((T*)p.dk + ((c.tok0 + x) * p.HV + hv) * KD + feat(a2) + 4 * g) = pack4<T>(acc);
-                        if constexpr (COMBA) *(V4*)((T*)p.dp + ((c.tok0 + x) * p.HV + hv) * KD + feat(a2) + 4 * g) = pack4<T>(dpk[a2][t]);
+                        *(V4*)((T*)p.dp + ((c.tok0 + x) * p.HV + hv) * KD + feat(a2) + 4 * g) = pack4<T>(dpk[a2][t]);
                     }
                 }
             }
@@ -1501,7 +1481,7 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
                         *(V4*)((T*)p.dk + ((c.tok0 + x) * p.HV + hv) * KD + feat(a2) + 4 * g) = pack4<T>(out);
                     }
                 }
-                if constexpr (COMBA) {
+                {
                     const float dotp = (sPd[x] + sPd[64 + x]) + (sPd[128 + x] + sPd[192 + x]), rp = sRp[x];
                     if (x < c.valid) {
 #pragma unroll
@@ -1520,327 +1500,13 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
             float x = (sDg[lane] + sDg[64 + lane]) + (sDg[128 + lane] + sDg[192 + lane]);
             // (comba) dg_t = sum_{s >= t} dgam_s + sum_{s > t} dgam0_s: one reverse cumulative sum of both, less the token's own dgam0
             float own0 = 0.f;
-            if constexpr (COMBA) { own0 = (sDg0[lane] + sDg0[64 + lane]) + (sDg0[128 + lane] + sDg0[192 + lane]); x += own0; }
+            { own0 = (sDg0[lane] + sDg0[64 + lane]) + (sDg0[128 + lane] + sDg0[192 + lane]); x += own0; }
 #pragma unroll
             for (int off = 1; off < 64; off <<= 1) {
                 const float y = __shfl_down(x, off, 64);
                 if (lane + off < 64) x += y;
             }
             x -= own0;
-            if (lane < c.valid) {
-                p.dg[(c.tok0 + lane) * p.HV + hv] = x;
-                p.dbeta[(c.tok0 + lane) * p.HV + hv] = (sDb[lane] + sDb[64 + lane]) + (sDb[128 + lane] + sDb[192 + lane]);
-            }
-        }
-        lds_barrier();
-    }
-}
-
-// The same in two halves for two blocks of key features, still two workgroups per CU: the second half takes dw and k one block of
-// 128 features at a time through the same two tile places (the products with dw and k add up over the blocks; d(e^gam k) of a
-// block needs that block only), and the last step goes over the blocks again, k's first block fetched a second time.
-constexpr size_t BWD_WY2W_SMEM = (2 * 64 * P128 + 2 * 64 * P64) * 2 + 640 * 4;
-
-template <typename T>
-__global__ __launch_bounds__(256, 2) void gdn_bwd_wy2w_kernel(BwdParams p, int64_t units) {
-    static_assert(2 * BWD_WY2W_SMEM <= 160 * 1024, "two workgroups per CU");
-    typedef typename Mma<T>::V8 V8;
-    typedef typename Mma<T>::V4 V4;
-    constexpr int KD = 2 * BD, PK = P128, NA = 2;
-    extern __shared__ __align__(16) char smem[];
-    T* sX0 = (T*)smem; T* sX1 = sX0 + 64 * P128;               // dv_new | v, then a block of dw | k
-    T* sA = sX1 + 64 * P128; T* sM1 = sA + 64 * P64;
-    float* sGam = (float*)(sM1 + 64 * P64); float* sBeta = sGam + 64; float* sDg = sBeta + 64; float* sDb = sDg + 256;
-    T* sDvn = sX0; T* sV = sX1; T* sDW = sX0; T* sK = sX1; T* sM2 = sX0;
-
-    TileRegs<BD> rDvn, rV, rDW, rK;
-    TileRegs<CH> rA;
-    float rGam = 0.f, rDg = 0.f;
-    uint32_t rBeta = 0;                                          // (raw bits: converted when the unit's turn comes)
-    auto fetch_first = [&](int64_t u, int tid) {
-        const UnitAt at = unit_at(p, u);
-        const ChunkAt c = at.c;
-        fetch_tile<BD>(rDvn, (const T*)p.ws.dVn + u * 64 * BD, BD, 64, tid);
-        fetch_tile<BD>(rV, (const T*)p.v + (c.tok0 * p.HV + at.hv) * BD, (int64_t)p.HV * BD, c.valid, tid);
-        fetch_tile<CH>(rA, (const T*)p.ws.Am + u * 64 * 64, 64, 64, tid);
-        if (tid < 64) {
-            rGam = p.ws.Gam[u * 64 + tid];
-            rBeta = tid < c.valid ? load_scalar_bits(p.beta, (c.tok0 + tid) * p.HV + at.hv, p.gb_dtype) : 0;
-            rDg = p.ws.Dgam[u * 64 + tid];
-        }
-    };
-    fetch_first(blockIdx.x, threadIdx.x);
-    for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
-        // (everything derived from the lane number is derived again per unit from a copy the compiler cannot see through:
-        // hoisted out of this loop, the addresses of its unrolled body would sit in registers, or spill, for its whole length)
-        int tid_opaque = threadIdx.x;
-        asm volatile("" : "+v"(tid_opaque));
-        const int tid = tid_opaque, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = lane & 15, g = lane >> 4;
-        auto feat = [&](int a) { return 16 * (2 * w + a); };    // first key feature, inside a block, of this wave's tile a
-        const UnitAt at = unit_at(p, u);
-        const int hv = at.hv, hq = at.hq;
-        const ChunkAt c = at.c;
-        auto fetch_dw = [&](int kb) { fetch_tile<BD>(rDW, (const T*)p.ws.dWm + u * 64 * KD + BD * kb, KD, 64, tid); };
-        auto fetch_k = [&](int kb) { fetch_tile<BD>(rK, (const T*)p.k + (c.tok0 * p.H + hq) * KD + BD * kb, (int64_t)p.H * KD, c.valid, tid); };
-        put_tile<BD>(sDvn, P128, rDvn, tid);
-        put_tile<BD>(sV, P128, rV, tid);
-        put_tile<CH>(sA, P64, rA, tid);
-        if (tid < 64) { sGam[tid] = rGam; sBeta[tid] = scalar_of_bits(rBeta, p.gb_dtype); }
-        sDg[tid] = tid < 64 ? rDg : 0.f;
-        sDb[tid] = 0.f;
-        fetch_dw(0);
-        fetch_k(0);
-        lds_barrier();
-
-        // ---- first half: dX's first term du v^T (this wave's 16 rows i; lane: column j, rows 4g + r), and dv = beta (A^T du) ----
-        f32x4 dXv[4];
-        {
-            V8 fa[4];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) fa[s] = frag_rows(sDvn, P128, 16 * w, 32 * s, lane);
-#pragma unroll
-            for (int tj = 0; tj < 4; ++tj) {
-                dXv[tj] = ZERO4;
-                if (tj <= w) {
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) dXv[tj] = Mma<T>::run(fa[s], frag_rows(sV, P128, 16 * tj, 32 * s, lane), dXv[tj]);
-                }
-            }
-        }
-        {
-            V8 fA[4][2];                                        // A^T operand of token tile t, step s (zero where A is)
-            float bj[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-#pragma unroll
-                for (int s = 0; s < 2; ++s)
-                    if (32 * s + 31 >= 16 * t) fA[t][s] = frag_cols(sA, P64, 32 * s, 16 * t, lane);
-                bj[t] = sBeta[16 * t + c16];
-            }
-#pragma unroll
-            for (int a2 = 0; a2 < 2; ++a2) {                    // value columns 16(2w+a2) ..
-                const int n16 = 16 * (2 * w + a2);
-                V8 fdv[2];
-#pragma unroll
-                for (int s = 0; s < 2; ++s) fdv[s] = frag_cols(sDvn, P128, 32 * s, n16, lane);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    f32x4 av = ZERO4;
-#pragma unroll
-                    for (int s = 0; s < 2; ++s) {
-                        if (32 * s + 31 < 16 * t) continue;     // A[i][j] = 0 for i < j
-                        av = Mma<T>::run(fdv[s], fA[t][s], av);
-                    }
-                    const int j = 16 * t + c16;
-                    const V4 v4 = *(const V4*)(sV + j * P128 + n16 + 4 * g);
-                    float dbv = 0.f;
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) dbv += av[r] * (float)v4[r];
-                    dbv = sum_over_g(dbv);
-                    if (g == 0) atomicAdd(&sDb[64 * w + j], dbv);
-                    if (j < c.valid) *(V4*)((T*)p.dv + ((c.tok0 + j) * p.HV + hv) * BD + n16 + 4 * g) = pack4<T>(av * bj[t]);
-                }
-            }
-        }
-
-        // ---- second half, a block of key features at a time: dX's second term dw (e^gam k)^T and k k^T add up over the blocks;
-        // d(e^gam k) = beta (A^T dw) of a block goes into that block's dk, and into dbeta, dgam ----
-        f32x4 dXw[4], kkT[4], dk[2][NA][4];
-#pragma unroll
-        for (int tj = 0; tj < 4; ++tj) dXw[tj] = kkT[tj] = ZERO4;
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            lds_barrier();                                      // (the two tile places are done with)
-            put_tile<BD>(sDW, PK, rDW, tid);
-            put_tile<BD>(sK, PK, rK, tid);
-            lds_barrier();
-            if (kb == 0) { fetch_dw(1); fetch_k(1); }
-            else {
-                if (u + gridDim.x < units) fetch_first(u + gridDim.x, tid);
-                fetch_k(0);                                     // (for the last step)
-            }
-            {
-                V8 fw[4], fk[4];
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    fw[s] = frag_rows(sDW, PK, 16 * w, 32 * s, lane);
-                    fk[s] = frag_rows(sK, PK, 16 * w, 32 * s, lane);
-                }
-#pragma unroll
-                for (int tj = 0; tj < 4; ++tj) {
-                    if (tj <= w) {
-#pragma unroll
-                        for (int s = 0; s < 4; ++s) {
-                            const V8 bk = frag_rows(sK, PK, 16 * tj, 32 * s, lane);
-                            dXw[tj] = Mma<T>::run(fw[s], bk, dXw[tj]);
-                            kkT[tj] = Mma<T>::run(fk[s], bk, kkT[tj]);
-                        }
-                    }
-                }
-            }
-            {
-                V8 fA[4][2];
-                float ej[4], bj[4];
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-#pragma unroll
-                    for (int s = 0; s < 2; ++s)
-                        if (32 * s + 31 >= 16 * t) fA[t][s] = frag_cols(sA, P64, 32 * s, 16 * t, lane);
-                    ej[t] = __expf(sGam[16 * t + c16]);
-                    bj[t] = sBeta[16 * t + c16];
-                }
-#pragma unroll
-                for (int a2 = 0; a2 < NA; ++a2) {               // key features 128 kb + feat(a2) ..
-                    const int n16 = feat(a2);
-                    V8 fdw[2];
-#pragma unroll
-                    for (int s = 0; s < 2; ++s) fdw[s] = frag_cols(sDW, PK, 32 * s, n16, lane);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        f32x4 ak = ZERO4;
-#pragma unroll
-                        for (int s = 0; s < 2; ++s) {
-                            if (32 * s + 31 < 16 * t) continue;
-                            ak = Mma<T>::run(fdw[s], fA[t][s], ak);
-                        }
-                        const int j = 16 * t + c16;
-                        const V4 k4 = *(const V4*)(sK + j * PK + n16 + 4 * g);
-                        float dot = 0.f;
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) dot += ak[r] * (float)k4[r];
-                        dot = sum_over_g(dot);
-                        if (g == 0) { atomicAdd(&sDb[64 * w + j], ej[t] * dot); atomicAdd(&sDg[64 * w + j], bj[t] * ej[t] * dot); }
-                        dk[kb][a2][t] = ak * (bj[t] * ej[t]);
-                    }
-                }
-            }
-        }
-        // dA = stril(dX diag(beta))
-#pragma unroll
-        for (int tj = 0; tj < 4; ++tj) {
-            const int j = 16 * tj + c16;
-            const float ej = __expf(sGam[j]), bj = sBeta[j];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = 16 * w + 4 * g + r;
-                sM1[i * P64 + j] = (T)(i > j ? (dXv[tj][r] + ej * dXw[tj][r]) * bj : 0.f);
-            }
-        }
-        lds_barrier();
-        // Y = dA A^T  (into dw's place)
-        {
-            V8 fd[2];
-#pragma unroll
-            for (int s = 0; s < 2; ++s) fd[s] = frag_rows(sM1, P64, 16 * w, 32 * s, lane);
-#pragma unroll
-            for (int tl = 0; tl < 4; ++tl) {
-                f32x4 acc = ZERO4;
-#pragma unroll
-                for (int s = 0; s < 2; ++s) acc = Mma<T>::run(fd[s], frag_rows(sA, P64, 16 * tl, 32 * s, lane), acc);
-                const int l = 16 * tl + c16;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) sM2[(16 * w + 4 * g + r) * P64 + l] = (T)acc[r];
-            }
-        }
-        lds_barrier();
-        // dL = -stril(A^T Y);  E = diag(beta) dL o D as an operand tile;  dbeta, dgam from L = diag(beta) stril(k k^T o D)
-        {
-            float dbi[4] = {0.f, 0.f, 0.f, 0.f}, rowF[4] = {0.f, 0.f, 0.f, 0.f}, gi[4], bi[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) { gi[r] = sGam[16 * w + 4 * g + r]; bi[r] = sBeta[16 * w + 4 * g + r]; }
-            V8 fAt[2];
-#pragma unroll
-            for (int s = 0; s < 2; ++s) fAt[s] = frag_cols(sA, P64, 32 * s, 16 * w, lane);
-#pragma unroll
-            for (int tl = 0; tl < 4; ++tl) {
-                f32x4 acc = ZERO4;
-                if (tl <= w) {
-#pragma unroll
-                    for (int s = 0; s < 2; ++s) acc = Mma<T>::run(fAt[s], frag_cols(sM2, P64, 32 * s, 16 * tl, lane), acc);
-                }
-                const f32x4 kk = kkT[tl];
-                const int l = 16 * tl + c16;
-                const float gl = sGam[l];
-                float colF = 0.f;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int i = 16 * w + 4 * g + r;
-                    float E = 0.f;
-                    if (i > l) {
-                        const float d = __expf(gi[r] - gl), dL = -acc[r];
-                        dbi[r] += dL * kk[r] * d;
-                        E = dL * bi[r] * d;
-                        const float F = E * kk[r];
-                        rowF[r] += F;
-                        colF += F;
-                    }
-                    sM1[i * P64 + l] = (T)E;
-                }
-                colF = sum_over_g(colF);
-                if (g == 0 && tl <= w) atomicAdd(&sDg[64 * w + l], -colF);
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float a = sum_over_c16(dbi[r]), b = sum_over_c16(rowF[r]);
-                if (c16 == 0) { atomicAdd(&sDb[64 * w + 16 * w + 4 * g + r], a); atomicAdd(&sDg[64 * w + 16 * w + 4 * g + r], b); }
-            }
-        }
-        // dk += E k + E^T k, on top of what the previous kernel left: the second block (its rows of k are in place), then the first
-#pragma unroll
-        for (int kb = 1; kb >= 0; --kb) {
-            V4 dk_old[NA][4];
-#pragma unroll
-            for (int a2 = 0; a2 < NA; ++a2)
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int x = 16 * t + c16;
-                    dk_old[a2][t] = V4{(T)0.f, (T)0.f, (T)0.f, (T)0.f};
-                    if (x < c.valid) dk_old[a2][t] = *(const V4*)((const T*)p.dk + ((c.tok0 + x) * p.HV + hv) * KD + BD * kb + feat(a2) + 4 * g);
-                }
-            lds_barrier();                                      // (E is complete; second round: the second block's rows are done with)
-            if (kb == 0) {
-                put_tile<BD>(sK, PK, rK, tid);
-                lds_barrier();
-            }
-            V8 fk[NA][2];
-#pragma unroll
-            for (int a2 = 0; a2 < NA; ++a2)
-#pragma unroll
-                for (int s = 0; s < 2; ++s) fk[a2][s] = frag_cols(sK, PK, 32 * s, feat(a2), lane);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-#pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    if (32 * s <= 16 * t + 15) {                // E[i][l], l < i
-                        const V8 e = frag_rows(sM1, P64, 16 * t, 32 * s, lane);
-#pragma unroll
-                        for (int a2 = 0; a2 < NA; ++a2) dk[kb][a2][t] = Mma<T>::run(fk[a2][s], e, dk[kb][a2][t]);
-                    }
-                    if (32 * s + 31 >= 16 * t) {                // E[i][l], i > l
-                        const V8 e = frag_cols(sM1, P64, 32 * s, 16 * t, lane);
-#pragma unroll
-                        for (int a2 = 0; a2 < NA; ++a2) dk[kb][a2][t] = Mma<T>::run(fk[a2][s], e, dk[kb][a2][t]);
-                    }
-                }
-                const int x = 16 * t + c16;
-                if (x < c.valid) {
-#pragma unroll
-                    for (int a2 = 0; a2 < NA; ++a2) {
-                        f32x4 acc = dk[kb][a2][t];
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[r] += (float)dk_old[a2][t][r];
-                        *(V4*)((T*)p.dk + ((c.tok0 + x) * p.HV + hv) * KD + BD * kb + feat(a2) + 4 * g) = pack4<T>(acc);
-                    }
-                }
-            }
-        }
-        if (w == 0) {
-            float x = (sDg[lane] + sDg[64 + lane]) + (sDg[128 + lane] + sDg[192 + lane]);
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const float y = __shfl_down(x, off, 64);
-                if (lane + off < 64) x += y;
-            }
             if (lane < c.valid) {
                 p.dg[(c.tok0 + lane) * p.HV + hv] = x;
                 p.dbeta[(c.tok0 + lane) * p.HV + hv] = (sDb[lane] + sDb[64 + lane]) + (sDb[128 + lane] + sDb[192 + lane]);
@@ -1864,24 +1530,8 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
     const int vbt_d = KT == 1 ? vbt : runs1 >= 128 ? 64 : 32;
     const unsigned units = (unsigned)(num_chunks * p.HV);
     auto runs = [&](int v) { return (unsigned)((runs1 + 7) / 8 * 8 * (BD / v)); };
-    struct K { const void* f; size_t smem; const char* name; unsigned grid; };
-    K state, dstate;
-    if (vbt == 32) state = {(const void*)gdn_bwd_state_kernel<T, 32, KT>, bwd_state_smem<32, KT>(), "gdn_bwd_state_kernel", runs(32)};
-    else if (vbt == 64) state = {(const void*)gdn_bwd_state_kernel<T, 64, KT>, bwd_state_smem<64, KT>(), "gdn_bwd_state_kernel", runs(64)};
-    else state = {(const void*)gdn_bwd_state_kernel<T, 128, KT>, bwd_state_smem<128, KT>(), "gdn_bwd_state_kernel", runs(128)};
-    if (vbt_d == 32) dstate = {(const void*)gdn_bwd_dstate_kernel<T, 32, KT>, bwd_dstate_smem<32, KT>(), "gdn_bwd_dstate_kernel", runs(32)};
-    else if (vbt_d == 64) dstate = {(const void*)gdn_bwd_dstate_kernel<T, 64, KT>, bwd_dstate_smem<64, KT>(), "gdn_bwd_dstate_kernel", runs(64)};
-    else if constexpr (KT == 1) dstate = {(const void*)gdn_bwd_dstate_kernel<T, 128, KT>, bwd_dstate_smem<128, KT>(), "gdn_bwd_dstate_kernel", runs(128)};
-    unsigned threads[5] = {256, vbt == BD ? 512u : 256u, vbt_d == BD ? 512u : 256u, 256, 256};
-    if constexpr (KT == 1) {
-        // both scans side by side in one launch (the second entry then has nothing to launch): what time segments run in, where
-        // every CU has a workgroup already
-        if (vbt == 32) {
-            state = {(const void*)gdn_bwd_scans_kernel<T, 32, KT>, bwd_scans_smem<32, KT>(), "gdn_bwd_scans_kernel", runs(32)};
-            threads[1] = 512;
-            dstate.grid = 0;
-        }
-    }
+    struct K { const void* f; size_t smem; const char* name; unsigned grid, threads; };
+    K state, dstate = {nullptr, 0, "gdn_bwd_dstate_kernel", 0, 0};
     // Time segments for the two scans (one block of key features, dense input): long sequences on few heads leave CUs without a
     // workgroup; never more workgroups than CUs, segments of 8 chunks or more, and at least 24 steps saved per workgroup
     // (a warm-up of typical length must pay).  GDN_FLAG_SCAN_WIDE asks for whole sequences, GDN_FLAG_SCAN_SEGMENTS for segments of 4.
@@ -1894,65 +1544,64 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
                 p.nseg = nseg;
                 p.seg_chunks = (int)((p.NT + nseg - 1) / nseg);
                 p.warm_cap = std::min(WARM_CAP_MAX, p.seg_chunks + p.seg_chunks / 4 + 6);
-                state.grid *= nseg;                             // (vbt = 32: the two scans side by side)
             }
         }
     }
     int64_t second_arg[5] = {units, units, units, units, units};    // (the kernels that walk over the units take their number)
-    if (vbt == 32 && vbt_d == 32 && dstate.grid != 0 && state.grid + dstate.grid <= 256u) {
-        // both scans in one launch, each in workgroups of its own (the second entry then has nothing to launch)
-        second_arg[1] = state.grid;
-        state = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, KT>, bwd_scans_apart_smem<32, KT>(), "gdn_bwd_scans_apart_kernel", state.grid + dstate.grid};
-        dstate.grid = 0;
-    }
-    if constexpr (KT == 1) {
-        // Whole sequences on up to 128 runs: both scans in one launch, every workgroup with a CU to itself, as many value columns
-        // each as that allows.  What a CU moves per step bounds the step (some 22 GB/s per CU, loads and stores together, whatever
-        // shares the CU): 32 KB + c/2 for c columns of the forward scan, 56 KB + c/2 of the reverse one - side by side in one
-        // workgroup the two add up, apart the longer one counts.
-        if (p.nseg == 1 && runs1 <= 128) {
-            const int va = runs1 <= 32 ? 32 : runs1 <= 64 ? 64 : 128;
-            second_arg[1] = runs(va);
-            threads[1] = va == BD ? 512u : 256u;
-            if (va == 32) state = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, KT>, bwd_scans_apart_smem<32, KT>(), "gdn_bwd_scans_apart_kernel", 2 * runs(32)};
-            else if (va == 64) state = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, KT>, bwd_scans_apart_smem<64, KT>(), "gdn_bwd_scans_apart_kernel", 2 * runs(64)};
-            else state = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, KT>, bwd_scans_apart_smem<128, KT>(), "gdn_bwd_scans_apart_kernel", 2 * runs(128)};
-            dstate.grid = 0;
-        }
-    }
-    const bool l2 = KT == 1 && p.q_raw;                     // (the entry has checked H == HV)
-    K prep;
-    if constexpr (KT == 1) prep = {l2 ? (const void*)gdn_bwd_prepare_kernel<T, COMBA, true> : (const void*)gdn_bwd_prepare_kernel<T, COMBA>, bwd_prep_smem<COMBA>(), "gdn_bwd_prepare_kernel", units < 512u ? units : 512u};
-    else prep = {(const void*)gdn_bwd_prepare2w_kernel<T>, BWD_PREP2W_SMEM, "gdn_bwd_prepare2w_kernel", units < 512u ? units : 512u};
-    K wy;
-    if constexpr (KT == 1) wy = {l2 ? (const void*)gdn_bwd_wy2_kernel<T, true, COMBA> : (const void*)gdn_bwd_wy2_kernel<T, false, COMBA>, bwd_wy2_smem<COMBA>(), "gdn_bwd_wy2_kernel", units < 512u ? units : 512u};
-    else wy = {(const void*)gdn_bwd_wy2w_kernel<T>, BWD_WY2W_SMEM, "gdn_bwd_wy2w_kernel", units < 512u ? units : 512u};
-    const K ks[5] = {
-        prep,
-        state,
-        dstate,
-        {l2 ? (const void*)gdn_bwd_dqkw_kernel<T, 1, true> : (const void*)gdn_bwd_dqkw_kernel<T, KT>, bwd_dqkw_smem<KT>(), "gdn_bwd_dqkw_kernel", units < 256u ? units : 256u},
-        wy,
+    auto apart = [&](const void* f, size_t smem, int v) {
+        second_arg[1] = runs(v);
+        state = {f, smem, "gdn_bwd_scans_apart_kernel", 2 * runs(v), v == BD ? 512u : 256u};
     };
-    K unit = {nullptr, 0, "gdn_bwd_unit_kernel", 0};
-    int64_t items = 0;
-    if constexpr (!COMBA && KT == 1) {
-        p.parts = p.HV / p.H;
-        items = num_chunks * p.H * p.parts;
-        unit = {l2 ? (const void*)gdn_bwd_unit_kernel<T, BD * KT, BD, 8, true> : (const void*)gdn_bwd_unit_kernel<T, BD * KT, BD, 8, false>, bwd_unit_smem<BD * KT, BD, 8>(), "gdn_bwd_unit_kernel", (unsigned)std::min<int64_t>(items, 256)};
-    }
-    for (int i = 0; i < 5; ++i) {
-        if (!COMBA && KT == 1 && i == 3) {
-            if (int rc = ensure_dynamic_smem_for(unit.f, unit.smem, unit.name)) return rc;
-            void* args[] = {(void*)&p, (void*)&items};
-            if (hipLaunchKernel(unit.f, dim3(unit.grid), dim3(512), args, unit.smem, stream) != hipSuccess) return check_launch(unit.name);
-            if (int rc = check_launch(unit.name)) return rc;
-            break;
+    if constexpr (KT == 1) {
+        if (p.nseg > 1)                                         // both scans side by side in a workgroup: every CU has one already
+            state = {(const void*)gdn_bwd_scans_kernel<T, 32, KT>, bwd_scans_smem<32, KT>(), "gdn_bwd_scans_kernel", runs(32) * p.nseg, 512};
+        // Whole sequences: both scans in one launch, up to 128 runs every workgroup with a CU to itself, as many value columns each as
+        // that allows.  What a CU moves per step bounds the step (some 22 GB/s per CU, loads and stores together, whatever shares the
+        // CU): 32 KB + c/2 for c columns of the forward scan, 56 KB + c/2 of the reverse one - side by side in one workgroup the two
+        // add up, apart the longer one counts.
+        else if (runs1 <= 32) apart((const void*)gdn_bwd_scans_apart_kernel<T, 32, KT>, bwd_scans_apart_smem<32, KT>(), 32);
+        else if (runs1 <= 64) apart((const void*)gdn_bwd_scans_apart_kernel<T, 64, KT>, bwd_scans_apart_smem<64, KT>(), 64);
+        else apart((const void*)gdn_bwd_scans_apart_kernel<T, 128, KT>, bwd_scans_apart_smem<128, KT>(), 128);
+    } else {
+        if (runs1 <= 32) apart((const void*)gdn_bwd_scans_apart_kernel<T, 32, KT>, bwd_scans_apart_smem<32, KT>(), 32);
+        else {
+            if (vbt == 32) state = {(const void*)gdn_bwd_state_kernel<T, 32, KT>, bwd_state_smem<32, KT>(), "gdn_bwd_state_kernel", runs(32), 256};
+            else if (vbt == 64) state = {(const void*)gdn_bwd_state_kernel<T, 64, KT>, bwd_state_smem<64, KT>(), "gdn_bwd_state_kernel", runs(64), 256};
+            else state = {(const void*)gdn_bwd_state_kernel<T, 128, KT>, bwd_state_smem<128, KT>(), "gdn_bwd_state_kernel", runs(128), 512};
+            if (vbt_d == 32) dstate = {(const void*)gdn_bwd_dstate_kernel<T, 32, KT>, bwd_dstate_smem<32, KT>(), "gdn_bwd_dstate_kernel", runs(32), 256};
+            else dstate = {(const void*)gdn_bwd_dstate_kernel<T, 64, KT>, bwd_dstate_smem<64, KT>(), "gdn_bwd_dstate_kernel", runs(64), 256};
         }
+    }
+    const bool l2 = p.q_raw != nullptr;
+    if constexpr (KT == 2) {
+        // (rows of two blocks do not pass through one tile of the prepare kernel: normalised in passes of their own)
+        if (l2) {
+            const int dtype = std::is_same<T, bf16_t>::value ? GDN_DTYPE_BF16 : GDN_DTYPE_F16;
+            const int64_t rows = p.tokens * p.H;
+            if (int rc = gdn_l2norm_fwd(p.q_raw, (void*)p.q, (float*)p.q_rstd, rows, BD * KT, BD * KT, dtype, stream)) return rc;
+            if (int rc = gdn_l2norm_fwd(p.k_raw, (void*)p.k, (float*)p.k_rstd, rows, BD * KT, BD * KT, dtype, stream)) return rc;
+        }
+    }
+    K prep;
+    if constexpr (KT == 1) prep = {l2 ? (const void*)gdn_bwd_prepare_kernel<T, COMBA, true> : (const void*)gdn_bwd_prepare_kernel<T, COMBA>, bwd_prep_smem<COMBA>(), "gdn_bwd_prepare_kernel", units < 512u ? units : 512u, 256};
+    else prep = {(const void*)gdn_bwd_prepare2w_kernel<T>, BWD_PREP2W_SMEM, "gdn_bwd_prepare2w_kernel", units < 512u ? units : 512u, 256};
+    K dqkw{}, wy{}, unit{};
+    if constexpr (COMBA) {
+        dqkw = {l2 ? (const void*)gdn_bwd_dqkw_kernel<T, true> : (const void*)gdn_bwd_dqkw_kernel<T>, BWD_DQKW_SMEM, "gdn_bwd_dqkw_kernel", units < 256u ? units : 256u, 256};
+        wy = {l2 ? (const void*)gdn_bwd_wy2_kernel<T, true> : (const void*)gdn_bwd_wy2_kernel<T, false>, BWD_WY2_SMEM, "gdn_bwd_wy2_kernel", units < 512u ? units : 512u, 256};
+    } else {
+        // (with the normalisation inside, dq and dk need the sum over the value heads before it can be taken back)
+        p.parts = l2 ? 1 : p.HV / p.H;
+        second_arg[3] = num_chunks * p.H * p.parts;
+        unit = {l2 ? (const void*)gdn_bwd_unit_kernel<T, BD * KT, BD, 8, true> : (const void*)gdn_bwd_unit_kernel<T, BD * KT, BD, 8, false>,
+                bwd_unit_smem<BD * KT, BD, 8>(), "gdn_bwd_unit_kernel", (unsigned)std::min<int64_t>(second_arg[3], 256), 512};
+    }
+    const K ks[5] = {prep, state, dstate, COMBA ? dqkw : unit, wy};
+    for (int i = 0; i < 5; ++i) {
         if (ks[i].grid == 0) continue;
         if (int rc = ensure_dynamic_smem_for(ks[i].f, ks[i].smem, ks[i].name)) return rc;
         void* args[] = {(void*)&p, (void*)&second_arg[i]};
-        if (hipLaunchKernel(ks[i].f, dim3(ks[i].grid), dim3(threads[i]), args, ks[i].smem, stream) != hipSuccess) return check_launch(ks[i].name);
+        if (hipLaunchKernel(ks[i].f, dim3(ks[i].grid), dim3(ks[i].threads), args, ks[i].smem, stream) != hipSuccess) return check_launch(ks[i].name);
         if (int rc = check_launch(ks[i].name)) return rc;
     }
     return GDN_OK;
@@ -1985,7 +1634,7 @@ static int chunk_bwd_entry(
                   "%s: K = 128%s and V = 128 only (got K=%lld V=%lld); pad smaller head dims with zeros", who, comba ? "" : " or 256",
                   (long long)K, (long long)V);
     GDN_CHECK_ARG(qkv_dtype == GDN_DTYPE_BF16 || qkv_dtype == GDN_DTYPE_F16, GDN_ERR_UNSUPPORTED, "%s: q/k/v/do must be bf16 or f16", who);
-    GDN_CHECK_ARG((flags & ~(uint32_t)(GDN_FLAG_CU_INT32 | GDN_FLAG_SCAN_WIDE | GDN_FLAG_SCAN_SEGMENTS)) == 0, GDN_ERR_UNSUPPORTED,
+    GDN_CHECK_ARG((flags & ~(uint32_t)(GDN_FLAG_CU_INT32 | GDN_FLAG_SEQ_ORDER | GDN_FLAG_SCAN_WIDE | GDN_FLAG_SCAN_SEGMENTS)) == 0, GDN_ERR_UNSUPPORTED,
                   "%s: only GDN_FLAG_CU_INT32 and the two flags that steer the scans' time segments are understood here (activations and the state layout are the caller's)", who);
     GDN_CHECK_ARG(HV <= 65535 && num_chunks * HV < (1ll << 31) && N * HV * 4 < (1ll << 31), GDN_ERR_UNSUPPORTED,
                   "%s: too many heads or chunks for one launch", who);
@@ -2004,14 +1653,13 @@ static int chunk_bwd_entry(
     GDN_CHECK_ARG(q && k && v && beta && dout && dq && dk && dv && dg && dbeta, GDN_ERR_INVALID,
                   "%s: q, k, v, beta, do, dq, dk, dv, dg, dbeta must not be NULL", who);
     GDN_CHECK_ARG(!comba || (pk && dp && g), GDN_ERR_INVALID, "%s: p, g and dp must not be NULL", who);
-    GDN_CHECK_ARG(!l2 || (H == HV && K == BD), GDN_ERR_UNSUPPORTED,
-                  "%s: the l2 normalisation is taken in here for H == HV and K = 128 only", who);
+    GDN_CHECK_ARG(!l2 || !comba || H == HV, GDN_ERR_UNSUPPORTED, "%s: the l2 normalisation is taken in here for H == HV only", who);
     for (const void* x : {q, k, pk, v, dout, (const void*)h0, (const void*)dht, (const void*)dq, (const void*)dk, (const void*)dp, (const void*)dv, (const void*)dh0})
         GDN_CHECK_ARG(((uintptr_t)x % 16) == 0, GDN_ERR_INVALID, "%s: tensors must be 16-byte aligned", who);
     GDN_CHECK_ARG(((uintptr_t)workspace % 256) == 0, GDN_ERR_INVALID, "%s: the workspace must be 256-byte aligned", who);
     BwdParams p;
     size_t need = bwd_ws_layout(num_chunks * HV, K, (char*)workspace, &p.ws);
-    const size_t rows_bytes = ws_align((size_t)(B * T * H) * BD * 2), factors_bytes = ws_align((size_t)(B * T * H) * 4);
+    const size_t rows_bytes = ws_align((size_t)(B * T * H) * K * 2), factors_bytes = ws_align((size_t)(B * T * H) * 4);
     const size_t l2_at = need;
     if (l2) need += (comba ? 3 : 2) * (rows_bytes + factors_bytes);
     GDN_CHECK_ARG(workspace && workspace_bytes >= need, GDN_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who,
@@ -2032,7 +1680,7 @@ static int chunk_bwd_entry(
     p.q = q; p.k = k; p.v = v; p.g = g; p.beta = beta; p.h0 = h0; p.dout = dout; p.dht = dht;
     p.dq = dq; p.dk = dk; p.dv = dv; p.dg = dg; p.dbeta = dbeta; p.dh0 = dh0; p.pk = pk; p.dp = dp; p.dgk = nullptr;
     p.cu_seqlens = cu_seqlens; p.chunk_table = chunk_table; p.chunk_offsets = chunk_offsets;
-    p.T = T; p.H = (int)H; p.HV = (int)HV; p.N = N; p.NT = (T + CH - 1) / CH;
+    p.T = T; p.H = (int)H; p.HV = (int)HV; p.N = N; p.NT = (T + CH - 1) / CH; p.tokens = B * T;
     p.scale = scale; p.gb_dtype = gb_dtype; p.flags = flags;
     p.nseg = 1; p.seg_chunks = (int)p.NT; p.warm_cap = 0;
     if (comba) return qkv_dtype == GDN_DTYPE_BF16 ? launch_bwd<bf16_t, 1, true>(p, num_chunks, s) : launch_bwd<f16_t, 1, true>(p, num_chunks, s);
@@ -2054,10 +1702,28 @@ extern "C" int gdn_chunk_bwd(
                            scale, qkv_dtype, gb_dtype, flags, stream);
 }
 
+extern "C" size_t gdn_chunk_bwd_qk_l2norm_grouped_workspace_bytes(int64_t num_chunks, int64_t H, int64_t HV, int64_t K, int64_t tokens) {
+    if (num_chunks < 0 || H < 1 || HV < 1 || (K != 128 && K != 256) || tokens < 0) return 0;
+    return gdn::bwd_ws_layout(num_chunks * HV, K, nullptr, nullptr) + 2 * gdn::ws_align((size_t)(tokens * H) * K * 2) +
+           2 * gdn::ws_align((size_t)(tokens * H) * 4);
+}
+
+extern "C" int gdn_chunk_bwd_qk_l2norm_grouped(
+    const void* q, const void* k, const void* v, const void* g, const void* beta,
+    const float* h0, const void* dout, const float* dht,
+    void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0,
+    const void* cu_seqlens, const void* chunk_table, const void* chunk_offsets,
+    void* workspace, size_t workspace_bytes,
+    int64_t B, int64_t T, int64_t H, int64_t HV, int64_t K, int64_t V,
+    int64_t N, int64_t num_chunks,
+    float scale, int qkv_dtype, int gb_dtype, uint32_t flags, void* stream) {
+    return chunk_bwd_entry("gdn_chunk_bwd_qk_l2norm_grouped", false, true, q, k, nullptr, v, g, beta, h0, dout, dht, dq, dk, nullptr, dv, dg, dbeta, dh0,
+                           cu_seqlens, chunk_table, chunk_offsets, workspace, workspace_bytes, B, T, H, HV, K, V, N, num_chunks,
+                           scale, qkv_dtype, gb_dtype, flags, stream);
+}
+
 extern "C" size_t gdn_chunk_bwd_qk_l2norm_workspace_bytes(int64_t num_chunks, int64_t HV, int64_t K, int64_t tokens) {
-    if (num_chunks < 0 || HV < 1 || K != 128 || tokens < 0) return 0;
-    return gdn::bwd_ws_layout(num_chunks * HV, K, nullptr, nullptr) + 2 * gdn::ws_align((size_t)(tokens * HV) * gdn::BD * 2) +
-           2 * gdn::ws_align((size_t)(tokens * HV) * 4);
+    return K == 128 ? gdn_chunk_bwd_qk_l2norm_grouped_workspace_bytes(num_chunks, HV, HV, K, tokens) : 0;
 }
 
 extern "C" int gdn_chunk_bwd_qk_l2norm(
@@ -2069,6 +1735,8 @@ extern "C" int gdn_chunk_bwd_qk_l2norm(
     int64_t B, int64_t T, int64_t H, int64_t HV, int64_t K, int64_t V,
     int64_t N, int64_t num_chunks,
     float scale, int qkv_dtype, int gb_dtype, uint32_t flags, void* stream) {
+    using namespace gdn;
+    GDN_CHECK_ARG(H == HV && K == BD, GDN_ERR_UNSUPPORTED, "gdn_chunk_bwd_qk_l2norm: H == HV and K = 128 only (gdn_chunk_bwd_qk_l2norm_grouped takes the others)");
     return chunk_bwd_entry("gdn_chunk_bwd_qk_l2norm", false, true, q, k, nullptr, v, g, beta, h0, dout, dht, dq, dk, nullptr, dv, dg, dbeta, dh0,
                            cu_seqlens, chunk_table, chunk_offsets, workspace, workspace_bytes, B, T, H, HV, K, V, N, num_chunks,
                            scale, qkv_dtype, gb_dtype, flags, stream);
@@ -2129,7 +1797,7 @@ extern "C" int gdn_chunk_kda_bwd(
     GDN_CHECK_ARG(K == BD && V == BD, GDN_ERR_UNSUPPORTED, "%s: K = V = 128 only (got K=%lld V=%lld); pad smaller head dims with zeros",
                   who, (long long)K, (long long)V);
     GDN_CHECK_ARG(qkv_dtype == GDN_DTYPE_BF16 || qkv_dtype == GDN_DTYPE_F16, GDN_ERR_UNSUPPORTED, "%s: q/k/v/do must be bf16 or f16", who);
-    GDN_CHECK_ARG((flags & ~(uint32_t)GDN_FLAG_CU_INT32) == 0, GDN_ERR_UNSUPPORTED,
+    GDN_CHECK_ARG((flags & ~(uint32_t)(GDN_FLAG_CU_INT32 | GDN_FLAG_SEQ_ORDER)) == 0, GDN_ERR_UNSUPPORTED,
                   "%s: only GDN_FLAG_CU_INT32 is understood here (activations and the state layout are the caller's)", who);
     GDN_CHECK_ARG(HV <= 65535 && num_chunks * HV < (1ll << 31) && N * HV * 4 < (1ll << 31), GDN_ERR_UNSUPPORTED,
                   "%s: too many heads or chunks for one launch", who);

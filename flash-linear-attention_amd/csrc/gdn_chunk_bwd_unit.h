@@ -9,8 +9,12 @@
 // One workgroup takes the value heads of a q/k head (or an even share of them, `parts`) of one chunk in turn, with k and q in LDS and
 // dq, dk in fp32 registers over all of them.  What used to be two kernels moved 312 KB per chunk and value head at 128 x 128 (dw, the
 // first half of dk, dv_new, k twice, per-head dq and dk); this one moves 168 KB + 96 KB per q/k head.  Eight waves, one workgroup per
-// CU (64-wide heads: four waves, two workgroups): wave w owns the key features 16 NA w .. of all 64 tokens, the tiles of the 64 x 64
-// lower triangles are dealt out one by one.  The next value head's tiles and state fragments are requested in the middle of a head.
+// CU: wave w owns the key features 16 NA w .. of all 64 tokens, the tiles of the 64 x 64
+// lower triangles are dealt out one by one.  The next value head's tiles and state fragments are requested in the middle of a head
+// (always, the last time for nothing: behind a condition the registers of the last request stay alive through the whole head).
+// 16000 packed tokens, 16 q/k and 32 value heads of 128: 650 us as two kernels, 490 us; with the heads of a group added up and the l2
+// normalisation taken back in here 500 us, and 132 us of passes around it gone.  8 x 2048 tokens, 32 heads of 256 x 256: 2230 us with
+// those passes, 1830 us (state fragments requested a head ahead there: 1920 us, for want of registers).
 
 // lower triangle of 4 x 4 tiles, row by row
 __device__ __forceinline__ int tri_row(int idx) { return idx < 1 ? 0 : idx < 3 ? 1 : idx < 6 ? 2 : 3; }
@@ -134,11 +138,11 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
             }
             // what comes next is requested a few tiles at a time over the phases of this head: a wave stands at a load for which
             // the CU's path to the L2 (some 25 bytes per clock) has no room yet
-            const bool last = hi + 1 == heads, ahead = !last || more;
+            const bool last = hi + 1 == heads;
             const Item& to = last ? nx : at;
             const int to_hv = last ? nx.hv0 : hv + 1;
             lds_barrier();
-            if (ahead) fetch_out(to, to_hv, tid);
+            if constexpr (!LEAN) fetch_out(to, to_hv, tid);
 
             // dP o D, tile by tile
 #pragma unroll
@@ -162,13 +166,17 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
             lds_barrier();
 
             // dq, dk of the output and the state update, dw (kept until do and v_new are done with)
-            if (ahead) fetch_in(to, to_hv, tid);
+            if constexpr (!LEAN) fetch_in(to, to_hv, tid);
             float dglast = 0.f, dgx[4] = {0.f, 0.f, 0.f, 0.f}, dbx[4] = {0.f, 0.f, 0.f, 0.f};    // this lane's share of dgam, dbeta of token 16t + c16
             f32x4 sd = ZERO4;                                    // diagonal: <S, dS> of this wave's rows
             V4 dw[NA][4];
 #pragma unroll
             for (int a = 0; a < NA; ++a) {
-                if constexpr (LEAN) fetch_state(at, hv, a, w, lane);
+                if constexpr (LEAN) {                           // (the lane number anew: one tile's fragments at a time)
+                    int lane_a = lane;
+                    asm volatile("" : "+v"(lane_a));
+                    fetch_state(at, hv, a, w, lane_a);
+                }
                 f32x4 G1[4], dKS[4], dWt[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t) G1[t] = dKS[t] = dWt[t] = ZERO4;
@@ -254,7 +262,9 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
 #pragma unroll
                 for (int t = 0; t < 4; ++t) *(V4*)(sDW + (16 * t + c16) * PK + feat(a) + 4 * g) = dw[a][t];
             lds_barrier();
-            if (ahead) { fetch_rest(to, to_hv, tid); if constexpr (!LEAN) fetch_state(to, to_hv, 0, w, lane); }
+            if constexpr (LEAN) { fetch_out(to, to_hv, tid); fetch_in(to, to_hv, tid); }
+            fetch_rest(to, to_hv, tid);
+            if constexpr (!LEAN) fetch_state(to, to_hv, 0, w, lane);
             // dX's second term dw (e^gam k)^T, dA = stril(dX diag(beta)), k k^T of the same tiles
             f32x4 kk[NTRI];
 #pragma unroll
@@ -267,6 +277,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
                     f32x4 dXw = ZERO4;
 #pragma unroll
                     for (int s = 0; s < SK; ++s) {
+                        if (LEAN && s % 2 == 0) __builtin_amdgcn_sched_barrier(0);
                         const V8 bk = frag_rows(sK, PK, 16 * tj, 32 * s, lane);
                         dXw = Mma<T>::run(frag_rows(sDW, PK, 16 * ti, 32 * s, lane), bk, dXw);
                         kk[n] = Mma<T>::run(frag_rows(sK, PK, 16 * ti, 32 * s, lane), bk, kk[n]);
@@ -400,7 +411,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
             int tid_opaque = threadIdx.x;
             asm volatile("" : "+v"(tid_opaque));
             const int tid = tid_opaque, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = lane & 15, g = lane >> 4;
-            if (LEAN && more) fetch_qk(nx, tid);
+            if constexpr (LEAN) fetch_qk(nx, tid);
             if constexpr (L2) {
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {

@@ -596,30 +596,22 @@ static int launch_bwd_kda(const BwdParams& p, const KdaParams& kp, int64_t num_c
     const unsigned units = (unsigned)(num_chunks * p.HV);
     auto runs = [&](int v) { return (unsigned)((runs1 + 7) / 8 * 8 * (BD / v)); };
     struct K { const void* f; size_t smem; const char* name; unsigned grid, threads; };
-    K state, dstate;
-    int64_t nstate = 0;
-    if (runs1 <= 128) {
-        // both scans in one launch, every workgroup with a CU to itself, as many value columns each as that allows
-        const int va = runs1 <= 32 ? 32 : runs1 <= 64 ? 64 : 128;
-        nstate = runs(va);
-        if (va == 32) state = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 1, true>, bwd_scans_apart_smem<32, 1>(), "gdn_bwd_scans_apart_kernel", 2 * runs(32), 256};
-        else if (va == 64) state = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 1, true>, bwd_scans_apart_smem<64, 1>(), "gdn_bwd_scans_apart_kernel", 2 * runs(64), 256};
-        else state = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, 1, true>, bwd_scans_apart_smem<128, 1>(), "gdn_bwd_scans_apart_kernel", 2 * runs(128), 512};
-        dstate = {nullptr, 0, "", 0, 0};
-    } else {
-        state = {(const void*)gdn_bwd_state_kernel<T, 128, 1, true>, bwd_state_smem<128, 1>(), "gdn_bwd_state_kernel", runs(128), 512};
-        dstate = {(const void*)gdn_bwd_dstate_kernel<T, 128, 1, true>, bwd_dstate_smem<128, 1>(), "gdn_bwd_dstate_kernel", runs(128), 512};
-    }
-    const K ks[4] = {
-        state, dstate,
+    K state;
+    // both scans in one launch, up to 128 runs every workgroup with a CU to itself, as many value columns each as that allows
+    const int va = runs1 <= 32 ? 32 : runs1 <= 64 ? 64 : 128;
+    const int64_t nrev = runs(va);
+    if (va == 32) state = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 1, true>, bwd_scans_apart_smem<32, 1>(), "gdn_bwd_scans_apart_kernel", 2 * runs(32), 256};
+    else if (va == 64) state = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 1, true>, bwd_scans_apart_smem<64, 1>(), "gdn_bwd_scans_apart_kernel", 2 * runs(64), 256};
+    else state = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, 1, true>, bwd_scans_apart_smem<128, 1>(), "gdn_bwd_scans_apart_kernel", 2 * runs(128), 512};
+    const K ks[3] = {
+        state,
         {(const void*)gdn_bwd_dqkw_kda_kernel<T>, BWD_DQKW_KDA_SMEM, "gdn_bwd_dqkw_kda_kernel", units < 256u ? units : 256u, 256},
         {(const void*)gdn_bwd_wy_kda_kernel<T>, BWD_WY_KDA_SMEM, "gdn_bwd_wy_kda_kernel", units < 256u ? units : 256u, 256},
     };
     int64_t nunits = units;
-    for (int i = 0; i < 4; ++i) {
-        if (ks[i].grid == 0) continue;
+    for (int i = 0; i < 3; ++i) {
         if (int rc = ensure_dynamic_smem_for(ks[i].f, ks[i].smem, ks[i].name)) return rc;
-        void* args[] = {(void*)&p, i == 0 && nstate ? (void*)&nstate : (void*)&nunits};
+        void* args[] = {(void*)&p, i == 0 ? (void*)&nrev : (void*)&nunits};
         if (hipLaunchKernel(ks[i].f, dim3(ks[i].grid), dim3(ks[i].threads), args, ks[i].smem, stream) != hipSuccess) return check_launch(ks[i].name);
         if (int rc = check_launch(ks[i].name)) return rc;
     }

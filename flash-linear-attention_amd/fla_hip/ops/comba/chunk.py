@@ -176,6 +176,7 @@ def chunk_comba_bwd(q, k, v, p, g, beta, scale, initial_state, do, dht, cu_seqle
         check_cu_seqlens(cu_seqlens, T, cu_seqlens_cpu)
         chunk_table = prepare_chunk_indices(cu_seqlens, _CHUNK, cu_seqlens_cpu=cu_seqlens_cpu)
         chunk_table = chunk_table.to(device=dev, dtype=cu_seqlens.dtype).contiguous()
+        flags |= _lib.FLAG_SEQ_ORDER
         chunk_offsets = prepare_scan_tables(cu_seqlens, _CHUNK, cu_seqlens_cpu=cu_seqlens_cpu)
         num_chunks = chunk_table.shape[0]
         # tokens of a packed tensor outside every sequence are never written: they get zero gradients

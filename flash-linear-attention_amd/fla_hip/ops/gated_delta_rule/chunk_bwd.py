@@ -47,8 +47,8 @@ def chunk_gated_delta_rule_bwd(
     ``initial_state``).  With ``q_rstd``, ``k_rstd`` (the factors ``l2norm_fwd`` returns next to the normalised rows
     passed as q and k) dq and dk are the gradients of the rows before normalisation: the reference's ``l2norm_bwd``
     (chunk.py:385-387) happens in the kernel that also adds up the value heads of a q/k head.  With ``qk_l2norm`` q and k
-    are the rows BEFORE their l2 normalisation and dq, dk the gradients of those: one C call (``gdn_chunk_bwd_qk_l2norm``)
-    where every value head has a q/k head of its own and K <= 128, ``l2norm_fwd`` and the route above otherwise."""
+    are the rows BEFORE their l2 normalisation and dq, dk the gradients of those: one C call
+    (``gdn_chunk_bwd_qk_l2norm_grouped``), which also adds up the value heads of a q/k head."""
     dev = require_gpu(q, k, v, beta, do)
     check_operand_shapes(q, k, v, g=g, beta=beta)
     if do.shape != v.shape:
@@ -59,11 +59,6 @@ def chunk_gated_delta_rule_bwd(
         raise NotImplementedError(f'the backward kernels cover key head dims up to {2 * _DIM} (got K={K})')
     KD = _DIM if K <= _DIM else 2 * _DIM
     N = B if cu_seqlens is None else len(cu_seqlens) - 1
-    inside = qk_l2norm and H == HV and KD == _DIM and V <= _DIM
-    if qk_l2norm and not inside:
-        q, q_rstd = l2norm_fwd(q)
-        k, k_rstd = l2norm_fwd(k)
-        q, k = q[..., :K], k[..., :K]                  # (l2norm_fwd pads rows to a multiple of 8)
     nb = (V + _DIM - 1) // _DIM
     if nb > 1:
         # value columns are independent: a head with V > 128 is nb heads of 128 columns that share q, k, g, beta
@@ -81,7 +76,7 @@ def chunk_gated_delta_rule_bwd(
         h2, d2 = split(initial_state), split(dht)
         dq, dk, dv2, db2, dg2, dh2 = chunk_gated_delta_rule_bwd(
             q, k, v2, g2, beta.repeat_interleave(nb, dim=2), scale, h2, do2, d2, state_v_first,
-            cu_seqlens, cu_seqlens_cpu, chunk_indices, chunk_size, q_rstd, k_rstd)
+            cu_seqlens, cu_seqlens_cpu, chunk_indices, chunk_size, q_rstd, k_rstd, qk_l2norm)
         # (dq, dk come back per q/k head: already summed over the value heads)
         dv = dv2.reshape(B, T, HV, nb * _DIM)[..., :V]
         db, dg = db2.reshape(B, T, HV, nb).sum(-1), dg2.reshape(B, T, HV, nb).sum(-1)
@@ -126,6 +121,7 @@ def chunk_gated_delta_rule_bwd(
         check_cu_seqlens(cu_seqlens, T, cu_seqlens_cpu)
         chunk_indices = prepare_chunk_indices(cu_seqlens, _CHUNK, cu_seqlens_cpu=cu_seqlens_cpu)      # (derived here, never taken over)
         chunk_table = chunk_indices.to(device=dev, dtype=cu_seqlens.dtype).contiguous()
+        flags |= _lib.FLAG_SEQ_ORDER
         chunk_offsets = prepare_scan_tables(cu_seqlens, _CHUNK, cu_seqlens_cpu=cu_seqlens_cpu)
         num_chunks = chunk_table.shape[0]
     else:
@@ -139,21 +135,22 @@ def chunk_gated_delta_rule_bwd(
         first, last = cu_bounds(cu_seqlens, cu_seqlens_cpu)
         if first != 0 or last != T:
             alloc = torch.zeros
-    dq = alloc(B, T, HV, KD, dtype=work, device=dev)
-    dk = alloc(B, T, HV, KD, dtype=work, device=dev)
+    rows = H if qk_l2norm else HV                       # dq and dk leave per q/k head or per value head
+    dq = alloc(B, T, rows, KD, dtype=work, device=dev)
+    dk = alloc(B, T, rows, KD, dtype=work, device=dev)
     dv = alloc(B, T, HV, _DIM, dtype=work, device=dev)
     dg = alloc(B, T, HV, dtype=torch.float32, device=dev)
     db = alloc(B, T, HV, dtype=torch.float32, device=dev)
     dh0 = torch.empty(N, HV, KD, _DIM, dtype=torch.float32, device=dev) if initial_state is not None else None
     lib = _lib.load()
-    ws_bytes = lib.gdn_chunk_bwd_qk_l2norm_workspace_bytes(num_chunks, HV, KD, B * T) if inside else lib.gdn_chunk_bwd_workspace_bytes(num_chunks, HV, KD)
+    ws_bytes = lib.gdn_chunk_bwd_qk_l2norm_grouped_workspace_bytes(num_chunks, H, HV, KD, B * T) if qk_l2norm else lib.gdn_chunk_bwd_workspace_bytes(num_chunks, HV, KD)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     tail = (ptr(vw), ptr(gw), ptr(bw), ptr(h0), ptr(dow), ptr(dhtw),
             ptr(dq), ptr(dk), ptr(dv), ptr(dg), ptr(db), ptr(dh0),
             ptr(cu_seqlens), ptr(chunk_table), ptr(chunk_offsets), ptr(workspace), ws_bytes,
             B, T, H, HV, KD, _DIM, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags,
             current_stream_ptr(dev))
-    _lib.check((lib.gdn_chunk_bwd_qk_l2norm if inside else lib.gdn_chunk_bwd)(ptr(qw), ptr(kw), *tail))
+    _lib.check((lib.gdn_chunk_bwd_qk_l2norm_grouped if qk_l2norm else lib.gdn_chunk_bwd)(ptr(qw), ptr(kw), *tail))
     dq = _finish(lib, dq, qw, q_rstd, H, K, out_dtype)
     dk = _finish(lib, dk, kw, k_rstd, H, K, out_dtype)
     dv = dv[..., :V].to(out_dtype)
@@ -164,7 +161,7 @@ def chunk_gated_delta_rule_bwd(
 
 
 def _finish(lib, dxh: torch.Tensor, y: torch.Tensor, rstd: torch.Tensor | None, H: int, K: int, out_dtype) -> torch.Tensor:
-    """dq or dk per value head ``[B,T,HV,KD]`` -> per q/k head ``[B,T,H,K]``: the sum over the value heads of a
+    """dq or dk per value head (or already per q/k head) ``[B,T,HV,KD]`` -> per q/k head ``[B,T,H,K]``: the sum over the value heads of a
     q/k head and, with ``rstd``, the way back through the l2 normalisation (``y``: the normalised rows, KD wide)."""
     B, T, HV, D = dxh.shape
     if rstd is None and HV == H and K == D:

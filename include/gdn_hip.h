@@ -309,9 +309,20 @@ int gdn_chunk_bwd(
  * dx = (dy - y (y . dy)) rstd per row to their fp32 results before they write them.
  * Arguments as for gdn_chunk_bwd, except:
  *   workspace: at least gdn_chunk_bwd_qk_l2norm_workspace_bytes(num_chunks, HV, K, B * T) bytes (0: unsupported K)
- *   H == HV and K = 128 only (GDN_ERR_UNSUPPORTED otherwise: call gdn_l2norm_fwd, gdn_chunk_bwd, then gdn_l2norm_bwd,
- *   which also adds up the value heads of a q/k head).
+ *   H == HV and K = 128 only (GDN_ERR_UNSUPPORTED otherwise).
+ * gdn_chunk_bwd_qk_l2norm_grouped takes any HV that is a multiple of H and K = 128 or 256; dq and dk come back per q/k head,
+ * [B,T,H,K]: the value heads of a q/k head are added up in fp32 inside.
  */
+size_t gdn_chunk_bwd_qk_l2norm_grouped_workspace_bytes(int64_t num_chunks, int64_t H, int64_t HV, int64_t K, int64_t tokens);
+int gdn_chunk_bwd_qk_l2norm_grouped(
+    const void* q, const void* k, const void* v, const void* g, const void* beta,
+    const float* h0, const void* dout, const float* dht,
+    void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0,
+    const void* cu_seqlens, const void* chunk_table, const void* chunk_offsets,
+    void* workspace, size_t workspace_bytes,
+    int64_t B, int64_t T, int64_t H, int64_t HV, int64_t K, int64_t V,
+    int64_t N, int64_t num_chunks,
+    float scale, int qkv_dtype, int gb_dtype, uint32_t flags, void* stream);
 size_t gdn_chunk_bwd_qk_l2norm_workspace_bytes(int64_t num_chunks, int64_t HV, int64_t K, int64_t tokens);
 int gdn_chunk_bwd_qk_l2norm(
     const void* q, const void* k, const void* v, const void* g, const void* beta,
