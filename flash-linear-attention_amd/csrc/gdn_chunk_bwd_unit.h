@@ -6,7 +6,8 @@
 //   Y = dA A^T, dL = -stril(A^T Y), E = diag(beta) dL o D;   dk += E k + E^T k;   dbeta, dgam from every factor, dg = the reverse
 //   cumulative sum of dgam inside the chunk.
 //
-// One workgroup takes the value heads of a q/k head (or an even share of them, `parts`) of one chunk in turn, with k and q in LDS and
+// One workgroup takes the value heads of a q/k head (or an even share of them, `parts`; with more value columns than VD their blocks
+// count as heads) of one chunk in turn, with k and q in LDS and
 // dq, dk in fp32 registers over all of them.  What used to be two kernels moved 312 KB per chunk and value head at 128 x 128 (dw, the
 // first half of dk, dv_new, k twice, per-head dq and dk); this one moves 168 KB + 96 KB per q/k head.  Eight waves, one workgroup per
 // CU: wave w owns the key features 16 NA w .. of all 64 tokens, the tiles of the 64 x 64
@@ -53,8 +54,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
     TileRegs<CH, NTH> rA;
     TileRegs<KD, NTH> rK, rQ;
     V8 sf[SV], df[SV];
-    float rGam = 0.f, rRq = 0.f, rRk = 0.f;
-    uint32_t rBeta = 0;
+    float rGam = 0.f, rBeta = 0.f, rRq = 0.f, rRk = 0.f;
+    const int HVg = p.HV / p.nb;
     auto fetch_state = [&](const Item& at, int hv, int a, int w, int lane) {     // feature tile a of this wave
         const int64_t u = at.ch * p.HV + hv;
         const int64_t off = u * KD * VD + (16 * (NA * w + a) + (lane & 15)) * VD + 8 * (lane >> 4);
@@ -72,12 +73,9 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
         fetch_tile<VD, NTH>(rV, (const T*)p.v + (at.c.tok0 * p.HV + hv) * VD, (int64_t)p.HV * VD, at.c.valid, tid);
     };
     auto fetch_rest = [&](const Item& at, int hv, int tid) {
-        const int64_t u = at.ch * p.HV + hv;
-        fetch_tile<CH, NTH>(rA, (const T*)p.ws.Am + u * 64 * 64, 64, 64, tid);
-        if (tid < 64) {
-            rGam = p.ws.Gam[u * 64 + tid];
-            rBeta = tid < at.c.valid ? load_scalar_bits(p.beta, (at.c.tok0 + tid) * p.HV + hv, p.gb_dtype) : 0;
-        }
+        const int64_t ug = at.ch * HVg + hv / p.nb;
+        fetch_tile<CH, NTH>(rA, (const T*)p.ws.Am + ug * 64 * 64, 64, 64, tid);
+        if (tid < 64) { rGam = p.ws.Gam[ug * 64 + tid]; rBeta = p.ws.Bet[ug * 64 + tid]; }
     };
     auto fetch_qk = [&](const Item& at, int tid) {
         fetch_tile<KD, NTH>(rK, (const T*)p.k + (at.c.tok0 * p.H + at.hq) * KD, (int64_t)p.H * KD, at.c.valid, tid);
@@ -112,6 +110,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
             put_tile<KD, NTH>(sQ, PK, rQ, tid);
             if constexpr (L2) { if (tid < 64) { sRq[tid] = rRq; sRk[tid] = rRk; } }
         }
+        float dg_sum = 0.f, db_sum = 0.f;
         f32x4 dq[NA][4], dk[NA][4];
 #pragma unroll
         for (int a = 0; a < NA; ++a)
@@ -132,7 +131,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
             put_tile<VD, NTH>(sV, PV, rV, tid);
             put_tile<CH, NTH>(sA, P64, rA, tid);
             if (tid < 64) {
-                sGam[tid] = rGam; sBeta[tid] = scalar_of_bits(rBeta, p.gb_dtype);
+                sGam[tid] = rGam; sBeta[tid] = rBeta;
                 sEg[tid] = __expf(rGam);
                 sEl[tid] = __expf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, rGam), 63)) - rGam);
             }
@@ -399,9 +398,12 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
                     const float y = __shfl_down(x, off, 64);
                     if (lane + off < 64) x += y;
                 }
-                if (lane < at.c.valid) {
-                    p.dg[(at.c.tok0 + lane) * p.HV + hv] = x;
-                    p.dbeta[(at.c.tok0 + lane) * p.HV + hv] = b;
+                // (the blocks of a value head one after the other: their sums leave together)
+                const int blk = hv % p.nb;
+                dg_sum = blk ? dg_sum + x : x; db_sum = blk ? db_sum + b : b;
+                if (blk == p.nb - 1 && lane < at.c.valid) {
+                    p.dg[(at.c.tok0 + lane) * HVg + hv / p.nb] = dg_sum;
+                    p.dbeta[(at.c.tok0 + lane) * HVg + hv / p.nb] = db_sum;
                 }
             }
             lds_barrier();

@@ -592,28 +592,11 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_wy_kda_kernel(BwdParams p, int
 template <typename T>
 static int launch_bwd_kda(const BwdParams& p, const KdaParams& kp, int64_t num_chunks, int qkv_dtype, hipStream_t stream) {
     if (int rc = launch_kda_prepare(kp, num_chunks, qkv_dtype, stream)) return rc;
-    const int64_t runs1 = p.N * p.HV;
-    const unsigned units = (unsigned)(num_chunks * p.HV);
-    auto runs = [&](int v) { return (unsigned)((runs1 + 7) / 8 * 8 * (BD / v)); };
-    struct K { const void* f; size_t smem; const char* name; unsigned grid, threads; };
-    K state;
-    // both scans in one launch, up to 128 runs every workgroup with a CU to itself, as many value columns each as that allows
-    const int va = runs1 <= 32 ? 32 : runs1 <= 64 ? 64 : 128;
-    const int64_t nrev = runs(va);
-    if (va == 32) state = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 1, true>, bwd_scans_apart_smem<32, 1>(), "gdn_bwd_scans_apart_kernel", 2 * runs(32), 256};
-    else if (va == 64) state = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 1, true>, bwd_scans_apart_smem<64, 1>(), "gdn_bwd_scans_apart_kernel", 2 * runs(64), 256};
-    else state = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, 1, true>, bwd_scans_apart_smem<128, 1>(), "gdn_bwd_scans_apart_kernel", 2 * runs(128), 512};
-    const K ks[3] = {
-        state,
-        {(const void*)gdn_bwd_dqkw_kda_kernel<T>, BWD_DQKW_KDA_SMEM, "gdn_bwd_dqkw_kda_kernel", units < 256u ? units : 256u, 256},
-        {(const void*)gdn_bwd_wy_kda_kernel<T>, BWD_WY_KDA_SMEM, "gdn_bwd_wy_kda_kernel", units < 256u ? units : 256u, 256},
+    const unsigned units = (unsigned)(num_chunks * p.HV), grid = units < 256u ? units : 256u;
+    const BwdLaunch ks[3] = {
+        scans_128<T, FORM_KDA>(p),
+        {(const void*)gdn_bwd_dqkw_kda_kernel<T>, BWD_DQKW_KDA_SMEM, "gdn_bwd_dqkw_kda_kernel", grid, 256, units},
+        {(const void*)gdn_bwd_wy_kda_kernel<T>, BWD_WY_KDA_SMEM, "gdn_bwd_wy_kda_kernel", grid, 256, units},
     };
-    int64_t nunits = units;
-    for (int i = 0; i < 3; ++i) {
-        if (int rc = ensure_dynamic_smem_for(ks[i].f, ks[i].smem, ks[i].name)) return rc;
-        void* args[] = {(void*)&p, i == 0 ? (void*)&nrev : (void*)&nunits};
-        if (hipLaunchKernel(ks[i].f, dim3(ks[i].grid), dim3(ks[i].threads), args, ks[i].smem, stream) != hipSuccess) return check_launch(ks[i].name);
-        if (int rc = check_launch(ks[i].name)) return rc;
-    }
-    return GDN_OK;
+    return launch_all(p, ks, 3, stream);
 }

@@ -13,23 +13,15 @@
 //     lane (c16, g) holds 8 features of token row c16), so K K^T needs no LDS; the value heads of a q/k head sit in
 //     neighbouring waves and read the same lines.
 //   * Everything is kept TRANSPOSED: the raw tile (a, b), a <= b, holds (k_j . k_i) for rows j of t-tile a and columns i
-//     of t-tile b, gated it is U = L^T, and T = X^T = (I + U)^-1 is upper triangular.  A tile in accumulator layout
-//     (lane (c16, g): rows 4g..4g+3, column c16) serves directly as the RIGHT factor of a product on the fp32 matrix
-//     cores (step e contracts over the indices {4g + e}), the left factor comes from LDS by rows, and the result is
-//     again in accumulator layout.  The transposed X in accumulator layout is also exactly the order of the Xb operand
-//     fragments (row c16, columns 4g + e): results go from registers to memory.
-//   * Diagonal 16x16 blocks: lane group g inverts block g by substitution, one row of X per lane (all 64 lanes busy).
-//     Merges: T(lo,hi) = -(T(lo,lo) U(lo,hi)) T(hi,hi) on 16-tiles, then on 32-blocks with the zero tiles left out: the gated
-//     tiles U are right factors and never leave the registers, only the products T U pass through LDS.
-#include "gdn_chunk_common.h"
+//     of t-tile b, gated it is U = L^T, and T = X^T = (I + U)^-1 is upper triangular (gdn_chunk_inverse.h).  The transposed X in
+//     accumulator layout is also exactly the order of the Xb operand fragments (row c16, columns 4g + e): results go from
+//     registers to memory.
+#include "gdn_chunk_inverse.h"
 
 namespace gdn {
 
-// LDS per wave: seven 16x16 fp32 tiles that serve as left factors.  The diagonal blocks of L (by rows) and the three gate
-// tables lie where the transposed diagonal blocks of X go afterwards, |k|^2 and 1/|q| where the first products go
-// afterwards: 8.75 KB, four workgroups per CU.
-constexpr int TP = 20;                                       // pitch (floats) of a 16x16 fp32 tile in LDS
-constexpr int PW_FLOATS = 7 * 16 * TP;                       // 2240 floats per wave
+// The three gate tables lie where the transposed diagonal blocks of X go afterwards, |k|^2 and 1/|q| where the first products go
+// afterwards: 8.75 KB per wave, four workgroups per CU.
 constexpr int PW_WAVES = 4;                                  // waves per workgroup: small workgroups keep the CU's wave slots filled
 constexpr size_t PREP_SMEM = (size_t)PW_WAVES * PW_FLOATS * 4;
 
@@ -45,14 +37,9 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
     if (u >= units) return;
     float* base = (float*)smem + w * PW_FLOATS;
     float* tiles = base;
-    // left factors: the transposed diagonal blocks T(0,0) .. T(3,3) and the intermediate products V = T U; the gated
-    // tiles U themselves stay in registers as right factors
-    constexpr int I_T00 = 0, I_T11 = 1, I_T22 = 2, I_T33 = 3, I_V01 = 4, I_V23 = 5, I_T01 = I_V01;
-    constexpr int I_V02 = I_T22, I_V03 = I_T33, I_V12 = I_V23, I_V13 = 6;      // (T(2,2), T(3,3), V(2,3) are in registers by then)
     float* sLd = tiles;                                      // [4][16 i][16 j] diagonal blocks of L, by rows (until the T(g,g) are written)
     float* sG = tiles + 1024; float* sBN = sG + 64; float* sNK = sG + 128;      // gate tables (likewise)
     float* sK2 = tiles + 4 * 16 * TP; float* sNQ = sK2 + 64; // (until the gated tiles are written)
-    auto tile = [&](int i) { return tiles + i * 16 * TP; };
     auto lds_sync = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };   // (LDS operations of a wave execute in order)
 
     const int H = p.H, HV = p.HV, G = HV / H, K = p.K;
@@ -265,63 +252,11 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
             else U[a][b] = val;                                                        // stays in registers: a right factor
         }
     lds_sync();
-    // ---- diagonal blocks: X (I + L) = I by rows, from the right.  Lane c16 of group g owns row c16 of block g; as soon as
-    // x_i is known it is folded into the pending sums of all earlier columns (a dependent chain of 16 short steps) ----
-    {
-        const float* ld = sLd + g * 256;
-        float x[16], acc[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-#pragma unroll
-        for (int i = 15; i >= 0; --i) {
-            x[i] = ((i == c16) ? 1.f : 0.f) - acc[i];
-            float row[16];
-#pragma unroll
-            for (int q4 = 0; q4 < (i + 3) / 4; ++q4) *(f32x4*)(row + 4 * q4) = *(const f32x4*)(ld + i * 16 + 4 * q4);
-#pragma unroll
-            for (int j = 0; j < i; ++j) acc[j] += row[j] * x[i];
-        }
-        // T(g,g) = X_gg^T as a left factor: [row j][column c16]
-        float* tt = tile(I_T00 + g);             // (group g: block g)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) tt[j * TP + c16] = x[j];
-    }
-    lds_sync();
-    auto acc_layout = [&](int i) {               // a tile of LDS in accumulator layout
-        const float* t = tile(i);
-        return f32x4{t[(4 * g) * TP + c16], t[(4 * g + 1) * TP + c16], t[(4 * g + 2) * TP + c16], t[(4 * g + 3) * TP + c16]};
-    };
-    // acc + A B: A a tile of LDS by rows, B in accumulator layout
-    auto mul = [&](int ia, f32x4 B, f32x4 acc) {
-        const f32x4 a = *(const f32x4*)(tile(ia) + c16 * TP + 4 * g);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], B[e], acc, 0, 0, 0);
-        return acc;
-    };
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    auto put = [&](int i, f32x4 v) {             // a tile in accumulator layout to LDS, by rows
-#pragma unroll
-        for (int r = 0; r < 4; ++r) tile(i)[(4 * g + r) * TP + c16] = v[r];
-    };
-    const f32x4 T00 = acc_layout(I_T00), T11 = acc_layout(I_T11), T22 = acc_layout(I_T22), T33 = acc_layout(I_T33);
-    // ---- merge 16 -> 32: T(lo,hi) = -(T(lo,lo) U(lo,hi)) T(hi,hi) ----
-    put(I_V01, mul(I_T00, U[0][1], zero));
-    put(I_V23, mul(I_T22, U[2][3], zero));
-    lds_sync();
-    const f32x4 T01 = -mul(I_V01, T11, zero);
-    const f32x4 T23 = -mul(I_V23, T33, zero);
-    put(I_T01, T01);
-    lds_sync();
-    // ---- merge 32 -> 64: V = T[0:32][0:32] U[0:32][32:64], T[0:32][32:64] = -V T[32:64][32:64] (zero tiles left out) ----
-    put(I_V02, mul(I_T00, U[0][2], mul(I_T01, U[1][2], zero)));
-    put(I_V03, mul(I_T00, U[0][3], mul(I_T01, U[1][3], zero)));
-    put(I_V12, mul(I_T11, U[1][2], zero));
-    put(I_V13, mul(I_T11, U[1][3], zero));
-    lds_sync();
-    const f32x4 T02 = -mul(I_V02, T22, zero), T03 = -mul(I_V03, T33, mul(I_V02, T23, zero));
-    const f32x4 T12 = -mul(I_V12, T22, zero), T13 = -mul(I_V13, T33, mul(I_V12, T23, zero));
+    f32x4 X[4][4];
+    inverse_transposed(tiles, U, X, c16, g);
     // ---- Xb = X diag(beta) as operand fragments: rows of t-tile tt, columns {32sp + 4g + e} and {32sp + 16 + 4g + e} ----
     {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
         char* rec = p.ws.Rec + (ci * HV + hv) * REC_BYTES;
         auto emit = [&](int tt, int sp, f32x4 lo, f32x4 hi, bool has_hi) {
             V8 frag;
@@ -332,12 +267,12 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
             }
             store_frag<T>(rec + REC_X, tt, sp, lane, frag);
         };
-        emit(0, 0, T00, zero, false);
-        emit(1, 0, T01, T11, true);
-        emit(2, 0, T02, T12, true);
-        emit(2, 1, T22, zero, false);
-        emit(3, 0, T03, T13, true);
-        emit(3, 1, T23, T33, true);
+        emit(0, 0, X[0][0], zero, false);
+        emit(1, 0, X[0][1], X[1][1], true);
+        emit(2, 0, X[0][2], X[1][2], true);
+        emit(2, 1, X[2][2], zero, false);
+        emit(3, 0, X[0][3], X[1][3], true);
+        emit(3, 1, X[2][3], X[3][3], true);
     }
 }
 

@@ -108,8 +108,8 @@ SIGNATURES['gdn_chunk_bwd'] = (c_int, [
     c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,   # B T H HV K V N num_chunks
     c_float, c_int, c_int, c_uint32, c_void_p])
 SIGNATURES['gdn_chunk_bwd_qk_l2norm_workspace_bytes'] = (c_size_t, [c_int64, c_int64, c_int64, c_int64])
-SIGNATURES['gdn_chunk_bwd_qk_l2norm_grouped_workspace_bytes'] = (c_size_t, [c_int64] * 5)      # num_chunks H HV K tokens
-SIGNATURES['gdn_chunk_bwd_qk_l2norm_grouped'] = SIGNATURES['gdn_chunk_bwd']      # (the same for grouped heads and K = 256)
+SIGNATURES['gdn_chunk_bwd_heads_workspace_bytes'] = (c_size_t, [c_int64] * 6 + [c_uint32])      # num_chunks H HV K V tokens flags
+SIGNATURES['gdn_chunk_bwd_heads'] = (c_int, SIGNATURES['gdn_chunk_bwd'][1][:5] + [c_void_p, c_void_p] + SIGNATURES['gdn_chunk_bwd'][1][5:])      # A_log dt_bias behind beta
 SIGNATURES['gdn_chunk_bwd_qk_l2norm'] = SIGNATURES['gdn_chunk_bwd']      # (q, k before their l2 normalisation)
 SIGNATURES['gdn_chunk_comba_bwd'] = (c_int, [
     c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,  # q k p v g beta

@@ -16,7 +16,7 @@ from fla_hip.ops.gated_delta_rule._common import aligned16, as_f32, check_operan
 from fla_hip.ops.utils.index import check_cu_seqlens, cu_bounds, prepare_chunk_indices, prepare_scan_tables
 
 _CHUNK = 64
-_DIM = 128          # value columns of the backward kernels; key features: 128 or 256 (other head dims are zero-padded)
+_DIM = 128          # block of value columns of the backward kernels
 
 
 def _pad_last(x: torch.Tensor, size: int) -> torch.Tensor:
@@ -46,9 +46,9 @@ def chunk_gated_delta_rule_bwd(
     Returns ``(dq, dk, dv, dbeta, dg, dh0)``: dq, dk, dv in q's dtype, dbeta, dg fp32, dh0 fp32 (None without
     ``initial_state``).  With ``q_rstd``, ``k_rstd`` (the factors ``l2norm_fwd`` returns next to the normalised rows
     passed as q and k) dq and dk are the gradients of the rows before normalisation: the reference's ``l2norm_bwd``
-    (chunk.py:385-387) happens in the kernel that also adds up the value heads of a q/k head.  With ``qk_l2norm`` q and k
+    (chunk.py:385-387) in a kernel of its own.  With ``qk_l2norm`` q and k
     are the rows BEFORE their l2 normalisation and dq, dk the gradients of those: one C call
-    (``gdn_chunk_bwd_qk_l2norm_grouped``), which also adds up the value heads of a q/k head."""
+    (``gdn_chunk_bwd_heads``), which also adds up the value heads of a q/k head."""
     dev = require_gpu(q, k, v, beta, do)
     check_operand_shapes(q, k, v, g=g, beta=beta)
     if do.shape != v.shape:
@@ -57,42 +57,14 @@ def chunk_gated_delta_rule_bwd(
     HV, V = v.shape[2], v.shape[3]
     if K > 2 * _DIM:
         raise NotImplementedError(f'the backward kernels cover key head dims up to {2 * _DIM} (got K={K})')
-    KD = _DIM if K <= _DIM else 2 * _DIM
+    # the kernels' dims: 64 x 64, or 128 or 256 key features with value columns in blocks of 128
+    KD, VD = (64, 64) if K <= 64 and V <= 64 else (_DIM if K <= _DIM else 2 * _DIM, (V + _DIM - 1) // _DIM * _DIM)
     N = B if cu_seqlens is None else len(cu_seqlens) - 1
-    nb = (V + _DIM - 1) // _DIM
-    if nb > 1:
-        # value columns are independent: a head with V > 128 is nb heads of 128 columns that share q, k, g, beta
-        v2 = _pad_last(v, nb * _DIM).reshape(B, T, HV * nb, _DIM)
-        do2 = _pad_last(do, nb * _DIM).reshape(B, T, HV * nb, _DIM)
-        g2 = None if g is None else g.repeat_interleave(nb, dim=2)
-        h2 = d2 = None
-
-        def split(s):       # [N, HV, K, V] -> [N, HV*nb, K, 128]  (V-first: [N, HV, V, K] -> [N, HV*nb, 128, K])
-            if s is None:
-                return None
-            if state_v_first:
-                return F.pad(s, (0, 0, 0, nb * _DIM - V)).reshape(N, HV * nb, _DIM, K)
-            return _pad_last(s, nb * _DIM).reshape(N, HV, K, nb, _DIM).permute(0, 1, 3, 2, 4).reshape(N, HV * nb, K, _DIM)
-        h2, d2 = split(initial_state), split(dht)
-        dq, dk, dv2, db2, dg2, dh2 = chunk_gated_delta_rule_bwd(
-            q, k, v2, g2, beta.repeat_interleave(nb, dim=2), scale, h2, do2, d2, state_v_first,
-            cu_seqlens, cu_seqlens_cpu, chunk_indices, chunk_size, q_rstd, k_rstd, qk_l2norm)
-        # (dq, dk come back per q/k head: already summed over the value heads)
-        dv = dv2.reshape(B, T, HV, nb * _DIM)[..., :V]
-        db, dg = db2.reshape(B, T, HV, nb).sum(-1), dg2.reshape(B, T, HV, nb).sum(-1)
-        dh0 = None
-        if dh2 is not None:
-            if state_v_first:
-                dh0 = dh2.reshape(N, HV, nb * _DIM, K)[:, :, :V]
-            else:
-                dh0 = dh2.reshape(N, HV, nb, K, _DIM).permute(0, 1, 3, 2, 4).reshape(N, HV, K, nb * _DIM)[..., :V]
-            dh0 = dh0.contiguous()
-        return dq, dk, dv.contiguous(), db, dg, dh0
 
     out_dtype = q.dtype
     work = q.dtype if q.dtype in (torch.bfloat16, torch.float16) else torch.bfloat16
     qw, kw = (aligned16(_pad_last(x.to(work), KD).contiguous()) for x in (q, k))
-    vw, dow = (aligned16(_pad_last(x.to(work), _DIM).contiguous()) for x in (v, do))
+    vw, dow = (aligned16(_pad_last(x.to(work), VD).contiguous()) for x in (v, do))
     gw = None if g is None else as_f32(g).contiguous()
     bw = as_f32(beta).contiguous()
 
@@ -105,7 +77,7 @@ def chunk_gated_delta_rule_bwd(
         s = as_f32(s)
         if state_v_first:
             s = s.transpose(-1, -2)
-        return aligned16(pad_last_two(s, KD, _DIM).contiguous())
+        return aligned16(pad_last_two(s, KD, VD).contiguous())
     h0, dhtw = state_in(initial_state), state_in(dht)
 
     # FLA_HIP_BWD_SCAN_MODE forces one form of the two scans (default: automatic): whole sequences ('wide') or time segments
@@ -135,22 +107,23 @@ def chunk_gated_delta_rule_bwd(
         first, last = cu_bounds(cu_seqlens, cu_seqlens_cpu)
         if first != 0 or last != T:
             alloc = torch.zeros
-    rows = H if qk_l2norm else HV                       # dq and dk leave per q/k head or per value head
-    dq = alloc(B, T, rows, KD, dtype=work, device=dev)
-    dk = alloc(B, T, rows, KD, dtype=work, device=dev)
-    dv = alloc(B, T, HV, _DIM, dtype=work, device=dev)
+    dq = alloc(B, T, H, KD, dtype=work, device=dev)
+    dk = alloc(B, T, H, KD, dtype=work, device=dev)
+    dv = alloc(B, T, HV, VD, dtype=work, device=dev)
     dg = alloc(B, T, HV, dtype=torch.float32, device=dev)
     db = alloc(B, T, HV, dtype=torch.float32, device=dev)
-    dh0 = torch.empty(N, HV, KD, _DIM, dtype=torch.float32, device=dev) if initial_state is not None else None
+    dh0 = torch.empty(N, HV, KD, VD, dtype=torch.float32, device=dev) if initial_state is not None else None
     lib = _lib.load()
-    ws_bytes = lib.gdn_chunk_bwd_qk_l2norm_grouped_workspace_bytes(num_chunks, H, HV, KD, B * T) if qk_l2norm else lib.gdn_chunk_bwd_workspace_bytes(num_chunks, HV, KD)
+    if qk_l2norm:
+        flags |= _lib.FLAG_QK_L2NORM
+    ws_bytes = lib.gdn_chunk_bwd_heads_workspace_bytes(num_chunks, H, HV, KD, VD, B * T, flags)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    tail = (ptr(vw), ptr(gw), ptr(bw), ptr(h0), ptr(dow), ptr(dhtw),
-            ptr(dq), ptr(dk), ptr(dv), ptr(dg), ptr(db), ptr(dh0),
-            ptr(cu_seqlens), ptr(chunk_table), ptr(chunk_offsets), ptr(workspace), ws_bytes,
-            B, T, H, HV, KD, _DIM, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags,
-            current_stream_ptr(dev))
-    _lib.check((lib.gdn_chunk_bwd_qk_l2norm_grouped if qk_l2norm else lib.gdn_chunk_bwd)(ptr(qw), ptr(kw), *tail))
+    _lib.check(lib.gdn_chunk_bwd_heads(
+        ptr(qw), ptr(kw), ptr(vw), ptr(gw), ptr(bw), None, None, ptr(h0), ptr(dow), ptr(dhtw),
+        ptr(dq), ptr(dk), ptr(dv), ptr(dg), ptr(db), ptr(dh0),
+        ptr(cu_seqlens), ptr(chunk_table), ptr(chunk_offsets), ptr(workspace), ws_bytes,
+        B, T, H, HV, KD, VD, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags,
+        current_stream_ptr(dev)))
     dq = _finish(lib, dq, qw, q_rstd, H, K, out_dtype)
     dk = _finish(lib, dk, kw, k_rstd, H, K, out_dtype)
     dv = dv[..., :V].to(out_dtype)

@@ -310,11 +310,9 @@ int gdn_chunk_bwd(
  * Arguments as for gdn_chunk_bwd, except:
  *   workspace: at least gdn_chunk_bwd_qk_l2norm_workspace_bytes(num_chunks, HV, K, B * T) bytes (0: unsupported K)
  *   H == HV and K = 128 only (GDN_ERR_UNSUPPORTED otherwise).
- * gdn_chunk_bwd_qk_l2norm_grouped takes any HV that is a multiple of H and K = 128 or 256; dq and dk come back per q/k head,
- * [B,T,H,K]: the value heads of a q/k head are added up in fp32 inside.
  */
-size_t gdn_chunk_bwd_qk_l2norm_grouped_workspace_bytes(int64_t num_chunks, int64_t H, int64_t HV, int64_t K, int64_t tokens);
-int gdn_chunk_bwd_qk_l2norm_grouped(
+size_t gdn_chunk_bwd_qk_l2norm_workspace_bytes(int64_t num_chunks, int64_t HV, int64_t K, int64_t tokens);
+int gdn_chunk_bwd_qk_l2norm(
     const void* q, const void* k, const void* v, const void* g, const void* beta,
     const float* h0, const void* dout, const float* dht,
     void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0,
@@ -323,9 +321,22 @@ int gdn_chunk_bwd_qk_l2norm_grouped(
     int64_t B, int64_t T, int64_t H, int64_t HV, int64_t K, int64_t V,
     int64_t N, int64_t num_chunks,
     float scale, int qkv_dtype, int gb_dtype, uint32_t flags, void* stream);
-size_t gdn_chunk_bwd_qk_l2norm_workspace_bytes(int64_t num_chunks, int64_t HV, int64_t K, int64_t tokens);
-int gdn_chunk_bwd_qk_l2norm(
+
+/*
+ * gdn_chunk_bwd for every head layout and with the forward's activations taken inside.  Arguments as for gdn_chunk_bwd, except:
+ *   K = V = 64, or K = 128 or 256 with V any multiple of 128 (value columns beyond 128 in blocks: v, do, dv, the states and their
+ *   gradients keep their layouts)
+ *   dq, dk [B,T,H,K]: the value heads of a q/k head are added up in fp32 inside
+ *   A_log, dt_bias [HV] fp32 or NULL: the gate is -exp(A_log) softplus(g + dt_bias) (A_log NULL: g itself); dg is the gradient of that
+ *   gate, not of its input; with GDN_FLAG_BETA_SIGMOID (GDN_FLAG_NEG_EIGVAL) dbeta likewise that of (twice) the sigmoid of beta
+ *   flags: also GDN_FLAG_QK_L2NORM (dq, dk: gradients of the rows before normalisation), GDN_FLAG_BETA_SIGMOID, GDN_FLAG_NEG_EIGVAL,
+ *   GDN_FLAG_SEQ_ORDER; gb_dtype may be GDN_GB_DTYPES(g, beta)
+ *   workspace: at least gdn_chunk_bwd_heads_workspace_bytes(num_chunks, H, HV, K, V, B * T, flags) bytes (0: unsupported K, V)
+ */
+size_t gdn_chunk_bwd_heads_workspace_bytes(int64_t num_chunks, int64_t H, int64_t HV, int64_t K, int64_t V, int64_t tokens, uint32_t flags);
+int gdn_chunk_bwd_heads(
     const void* q, const void* k, const void* v, const void* g, const void* beta,
+    const float* A_log, const float* dt_bias,
     const float* h0, const void* dout, const float* dht,
     void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0,
     const void* cu_seqlens, const void* chunk_table, const void* chunk_offsets,
