@@ -21,6 +21,7 @@ OUT_DIR = os.path.join(HERE, 'fla_hip', '_C')
 LIB = os.path.join(OUT_DIR, 'libgdn_hip.so')
 OBJ_DIR = os.path.join(HERE, 'build', 'obj')
 HOST_SRC = os.path.join(CSRC, 'host', 'gdn_host.cpp')
+HOST_HDR = os.path.join(CSRC, 'host', 'gdn_host_train.h')
 HOST_LIB = os.path.join(OUT_DIR, 'gdn_host.so')
 
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
@@ -74,7 +75,7 @@ def build(force: bool = False, verbose: bool = True) -> str:
         objs.append(o)
         if force or _newer([s, *hdrs], o):
             jobs.append((s, o))
-    host = force or _newer([HOST_SRC, hdrs[-1]], HOST_LIB)
+    host = force or _newer([HOST_SRC, HOST_HDR, hdrs[-1]], HOST_LIB)
     if verbose and (jobs or host):
         print(f'[build] compiling {len(jobs)} file(s) for gfx950' + (' and the host extension' if host else ''), flush=True)
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs) + host))) as ex:

@@ -31,6 +31,8 @@ struct ConvBwdParams {
     const void* cu_seqlens; const void* tile_table;
     int64_t B, T, D, N, NT, num_tiles;
     int64_t stride_n, stride_t;        // of x, in elements (channel stride 1)
+    int64_t stride_dx;                 // rows of dx, in elements
+    int per_part;                      // tiles of a workgroup's run
     int W, w_dtype, state_dtype, act;
     bool cu32;
 };
@@ -188,11 +190,10 @@ __device__ __forceinline__ void conv_bwd_dx(const ConvBwdParams& p, const ConvBw
                                             const float (&dz)[CB_TOK + W - 1][CB_VEC]) {
     constexpr int VEC = CB_VEC;
     typedef T vec_t __attribute__((ext_vector_type(VEC)));
-    const int D = (int)p.D;
     const int64_t t0 = g.it * CB_TILE + ty * CB_TOK, len = g.len;
     if ((g.it + 1) * CB_TILE <= len - (p.dht ? W : 0)) {   // a whole tile that the final state does not reach
-        char* row = (char*)((T*)p.dx + (g.bos + g.it * CB_TILE) * D);
-        const uint32_t off = (uint32_t)((ty * CB_TOK) * D + c0) * (uint32_t)sizeof(T);
+        char* row = (char*)((T*)p.dx + (g.bos + g.it * CB_TILE) * p.stride_dx);
+        const uint32_t off = (uint32_t)((ty * CB_TOK) * (int)p.stride_dx + c0) * (uint32_t)sizeof(T);
 #pragma unroll
         for (int i = 0; i < CB_TOK; ++i) {
             vec_t out;
@@ -203,11 +204,11 @@ __device__ __forceinline__ void conv_bwd_dx(const ConvBwdParams& p, const ConvBw
                 for (int j = 0; j < W; ++j) a += wgt[j][e] * dz[i + (W - 1) - j][e];
                 out[e] = (T)a;
             }
-            *(vec_t*)(row + (int64_t)i * D * (int64_t)sizeof(T) + off) = out;
+            *(vec_t*)(row + (int64_t)i * p.stride_dx * (int64_t)sizeof(T) + off) = out;
         }
         return;
     }
-    T* dxs = (T*)p.dx + g.bos * D + c0;
+    T* dxs = (T*)p.dx + g.bos * p.stride_dx + c0;
 #pragma unroll
     for (int i = 0; i < CB_TOK; ++i) {
         const int64_t u = t0 + i;
@@ -219,14 +220,14 @@ __device__ __forceinline__ void conv_bwd_dx(const ConvBwdParams& p, const ConvBw
             float a = 0.f;
 #pragma unroll
             for (int j = 0; j < W; ++j) a += wgt[j][e] * dz[i + (W - 1) - j][e];
-            if (in_final) a += (float)((const T*)p.dht)[(g.n * D + c0 + e) * (int64_t)W + (u - (len - W))];
+            if (in_final) a += (float)((const T*)p.dht)[(g.n * p.D + c0 + e) * (int64_t)W + (u - (len - W))];
             out[e] = (T)a;
         }
-        *(vec_t*)(dxs + u * D) = out;
+        *(vec_t*)(dxs + u * p.stride_dx) = out;
     }
 }
 
-// A workgroup takes GDN_CONV_BWD_TILES_PER_PART consecutive tiles of its channels and keeps the sums for the parameters in
+// A workgroup takes `per_part` consecutive tiles of its channels and keeps the sums for the parameters in
 // registers across them: one row of partial sums per such run.  Each of its four waves owns a quarter of the run's
 // positions and walks over it in strips of CB_TOK positions, LAST FIRST, with the rows of the next strip on their way into
 // registers while it works on the current one; the waves never wait for each other and nothing passes through LDS.
@@ -255,7 +256,7 @@ __global__ __launch_bounds__(CB_CX * CB_TY, 2) void causal_conv1d_bwd_kernel(Con
             wgt[j][e] = live ? load_scalar(p.weight, (int64_t)(c0 + e) * W + j, p.w_dtype) : 0.f;
         }
     }
-    const int64_t tile0 = part * GDN_CONV_BWD_TILES_PER_PART, tile_end = min(p.num_tiles, tile0 + GDN_CONV_BWD_TILES_PER_PART);
+    const int64_t tile0 = part * p.per_part, tile_end = min(p.num_tiles, tile0 + p.per_part);
     const int per_wave = (int)(tile_end - tile0) * (STRIPS / CB_TY);     // strips per wave
     const int s_last = (wave + 1) * per_wave - 1;               // strip s of the run: tile tile0 + s / STRIPS, positions CB_TOK (s % STRIPS) ...
     const ConvBwdTile ga = conv_bwd_tile(p, tile0 + (s_last - (per_wave - 1)) / STRIPS), gb = conv_bwd_tile(p, tile0 + s_last / STRIPS);
@@ -271,7 +272,8 @@ __global__ __launch_bounds__(CB_CX * CB_TY, 2) void causal_conv1d_bwd_kernel(Con
         const uint32_t coff = (uint32_t)c0 * (uint32_t)sizeof(T);
         const char* xseq = (const char*)((const T*)p.x + (p.cu_seqlens ? gb.bos * p.stride_t : gb.n * p.stride_n));
         const char* dyseq = (const char*)((const T*)p.dy + gb.bos * D);
-        char* dxseq = (char*)((T*)p.dx + gb.bos * D);
+        char* dxseq = (char*)((T*)p.dx + gb.bos * p.stride_dx);
+        const int64_t dxstep = p.stride_dx * (int64_t)sizeof(T);
         vec_t xr[CB_TOK + W - 1], dyr[CB_TOK], xn[CB_TOK], dyn[CB_TOK];
 #pragma unroll
         for (int k = 0; k < CB_TOK + W - 1; ++k) xr[k] = *(const vec_t*)(xseq + (pos - (W - 1) + k) * xstep + coff);
@@ -350,7 +352,7 @@ __global__ __launch_bounds__(CB_CX * CB_TY, 2) void causal_conv1d_bwd_kernel(Con
                     for (int j = 0; j < W; ++j) a += wgt[j][e] * dz[i + (W - 1) - j][e];
                     out[e] = (T)a;
                 }
-                *(vec_t*)(dxseq + (pos + i) * dstep + coff) = out;
+                *(vec_t*)(dxseq + (pos + i) * dxstep + coff) = out;
             }
             if constexpr (decltype(ahead)::value) {
 #pragma unroll
@@ -480,7 +482,7 @@ template <typename T>
 static int launch_conv_bwd(const ConvBwdParams& p, hipStream_t stream) {
     constexpr int VEC = CB_VEC;
     if (p.dx && p.num_tiles > 0) {
-        const int64_t parts = (p.num_tiles + GDN_CONV_BWD_TILES_PER_PART - 1) / GDN_CONV_BWD_TILES_PER_PART;
+        const int64_t parts = (p.num_tiles + p.per_part - 1) / p.per_part;
         const int64_t blocks = ((p.D + CB_CX * VEC - 1) / (CB_CX * VEC)) * parts;
         if (blocks >= (1ll << 31)) {
             set_error("gdn_causal_conv1d_bwd: %lld workgroups exceed the grid limit", (long long)blocks);
@@ -639,6 +641,88 @@ static int launch_norm_bwd(const NormGateBwdParams& p, int64_t parts, hipStream_
     return check_launch("norm_gated_bwd_kernel");
 }
 
+// ---------------------------------------------------------------------------------------------
+// the gate and the beta of the operator back through their activations
+//   gate = -exp(A_log) softplus(x), x = g + dt_bias:  dg = dgate (-exp(A_log) sigmoid(x));  dA_log = sum dgate gate;  ddt_bias = sum dg
+//   beta = c sigmoid(b):  db = dbeta beta (1 - beta / c)
+// A thread keeps one head and walks over the tokens; its two sums leave each workgroup as a row of partial sums.
+// ---------------------------------------------------------------------------------------------
+struct GateBwdParams {
+    const float* dgate; const float* dbeta; const void* g; const void* b; const float* A_log; const float* dt_bias;
+    void* dg; void* db; float* part;               // part [parts][2][HV]: dA_log, ddt_bias
+    int64_t rows, HV, ld_g, ld_b, ld_dg, ld_db;    // elements from token to token
+    int64_t zero_from, zero_to;                    // columns of dg's rows to clear (padding of a wider matrix)
+    int g_dtype, b_dtype;
+    float beta_max;                                // 1 or 2; 0: dbeta is handed on as it is
+};
+__device__ __forceinline__ void store_scalar(void* p, int64_t i, float x, int dtype) {
+    if (dtype == GDN_DTYPE_F32) ((float*)p)[i] = x;
+    else if (dtype == GDN_DTYPE_BF16) ((bf16_t*)p)[i] = (bf16_t)x;
+    else ((f16_t*)p)[i] = (f16_t)x;
+}
+__global__ __launch_bounds__(256) void gate_bwd_kernel(GateBwdParams p) {
+    __shared__ float red[2][256];
+    const int64_t HV = p.HV;
+    const int per = HV >= 256 ? 1 : (int)(256 / HV);                 // tokens a workgroup takes at a time
+    for (int64_t c0 = 0; c0 < HV; c0 += 256) {                       // (one round unless there are more than 256 heads)
+        const int width = (int)min((int64_t)256, HV - c0), sub = threadIdx.x / width, hv = (int)(c0 + threadIdx.x % width);
+        const bool live = sub < per;
+        float sA = 0.f, sd = 0.f;
+        if (live) {
+            const float ea = p.A_log ? __expf(p.A_log[hv]) : 0.f, dt = p.dt_bias ? p.dt_bias[hv] : 0.f;
+            for (int64_t r = (int64_t)blockIdx.x * per + sub; r < p.rows; r += (int64_t)gridDim.x * per) {
+                const int64_t i = r * HV + hv;
+                if (p.dg) {
+                    float d = p.dgate[i];
+                    if (p.A_log) {
+                        const float x = load_scalar(p.g, r * p.ld_g + hv, p.g_dtype) + dt;
+                        sA += d * (-ea * softplus_f(x));
+                        d *= -ea * sigmoid_f(x);
+                        sd += d;
+                    }
+                    store_scalar(p.dg, r * p.ld_dg + hv, d, p.g_dtype);
+                }
+                float d = p.dbeta[i];
+                if (p.beta_max > 0.f) {
+                    const float s = sigmoid_f(load_scalar(p.b, r * p.ld_b + hv, p.b_dtype));
+                    d *= p.beta_max * s * (1.f - s);
+                }
+                store_scalar(p.db, r * p.ld_db + hv, d, p.b_dtype);
+            }
+        }
+        if (p.part) {
+            red[0][threadIdx.x] = sA; red[1][threadIdx.x] = sd;
+            __syncthreads();
+            if (threadIdx.x < width) {
+                for (int n = 1; n < per; ++n) { sA += red[0][threadIdx.x + n * width]; sd += red[1][threadIdx.x + n * width]; }
+                p.part[((int64_t)blockIdx.x * 2 + 0) * HV + hv] = sA;
+                p.part[((int64_t)blockIdx.x * 2 + 1) * HV + hv] = sd;
+            }
+            __syncthreads();
+        }
+    }
+    const int64_t wz = p.zero_to - p.zero_from;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < p.rows * wz; i += (int64_t)gridDim.x * 256)
+        store_scalar(p.dg, (i / wz) * p.ld_dg + p.zero_from + i % wz, 0.f, p.g_dtype);
+}
+
+// out[n] = sum of the rows of part [rows][n] in fp32, in a fixed order: what the backward kernels leave as partial sums.
+template <typename T>
+__global__ __launch_bounds__(256) void sum_rows_kernel(const float* part, T* out, int64_t rows, int64_t n) {
+    __shared__ float red[4][64];
+    const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
+    const int64_t at = (int64_t)blockIdx.x * 64 + c;
+    float a = 0.f, b = 0.f;
+    if (at < n) {
+        int64_t r = r0;
+        for (; r + 4 < rows; r += 8) { a += part[r * n + at]; b += part[(r + 4) * n + at]; }
+        if (r < rows) a += part[r * n + at];
+    }
+    red[r0][c] = a + b;
+    __syncthreads();
+    if (r0 == 0 && at < n) out[at] = (T)((red[0][c] + red[1][c]) + (red[2][c] + red[3][c]));
+}
+
 }  // namespace gdn
 
 using namespace gdn;
@@ -646,11 +730,12 @@ using namespace gdn;
 static bool known_dtype(int d) { return d == GDN_DTYPE_BF16 || d == GDN_DTYPE_F16 || d == GDN_DTYPE_F32; }
 static bool aligned16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
-extern "C" int gdn_causal_conv1d_bwd(
+extern "C" int gdn_causal_conv1d_bwd_runs(
     const void* x, const void* weight, const void* bias, const void* initial_state, const void* dy, const void* dht,
     void* dx, float* dw_part, float* db_part, float* dh0,
     const void* cu_seqlens, const void* tile_table,
     int64_t B, int64_t T, int64_t D, int64_t W, int64_t N, int64_t num_tiles, int64_t stride_x_n, int64_t stride_x_t,
+    int64_t stride_dx_t, int64_t tiles_per_part,
     int x_dtype, int w_dtype, int state_dtype, int activation, uint32_t flags, void* stream) {
     const char* who = "gdn_causal_conv1d_bwd";
     GDN_CHECK_ARG(B >= 0 && T >= 0 && D >= 1 && N >= 0 && num_tiles >= 0, GDN_ERR_INVALID, "%s: bad sizes B=%lld T=%lld D=%lld N=%lld", who,
@@ -669,21 +754,33 @@ extern "C" int gdn_causal_conv1d_bwd(
     GDN_CHECK_ARG(D < (1ll << 31) && stride_x_t >= D, GDN_ERR_INVALID, "%s: token stride %lld below D", who, (long long)stride_x_t);
     GDN_CHECK_ARG(stride_x_t <= (1ll << 24), GDN_ERR_UNSUPPORTED, "%s: token stride %lld above 2^24 elements (a lane's offset inside a tile of 64 tokens is kept in 32 bits)",
                   who, (long long)stride_x_t);
+    GDN_CHECK_ARG(stride_dx_t >= D && stride_dx_t <= (1ll << 24) && tiles_per_part >= 1 && tiles_per_part <= 64, GDN_ERR_INVALID,
+                  "%s: bad token stride of dx (%lld) or length of a run (%lld tiles)", who, (long long)stride_dx_t, (long long)tiles_per_part);
     const uintptr_t pair = (uintptr_t)CB_VEC * (x_dtype == GDN_DTYPE_F32 ? 4 : 2);     // a thread reads its channels in one piece
-    GDN_CHECK_ARG(D % CB_VEC == 0 && stride_x_t % CB_VEC == 0 && stride_x_n % CB_VEC == 0 && (uintptr_t)x % pair == 0 && (uintptr_t)dy % pair == 0 &&
+    GDN_CHECK_ARG(D % CB_VEC == 0 && stride_x_t % CB_VEC == 0 && stride_x_n % CB_VEC == 0 && stride_dx_t % CB_VEC == 0 && (uintptr_t)x % pair == 0 && (uintptr_t)dy % pair == 0 &&
                   (uintptr_t)dx % pair == 0, GDN_ERR_UNSUPPORTED, "%s: D and the strides of x must be multiples of %d and rows must start on %d-byte boundaries", who, CB_VEC, (int)pair);
     ConvBwdParams p{};
     p.x = x; p.weight = weight; p.bias = bias; p.initial_state = initial_state; p.dy = dy; p.dht = dht;
     p.dx = dx; p.dw_part = dw_part; p.db_part = db_part; p.dh0 = dh0;
     p.cu_seqlens = cu_seqlens; p.tile_table = tile_table;
     p.B = B; p.T = T; p.D = D; p.N = N; p.NT = (T + 63) / 64; p.num_tiles = num_tiles;
-    p.stride_n = stride_x_n; p.stride_t = stride_x_t;
+    p.stride_n = stride_x_n; p.stride_t = stride_x_t; p.stride_dx = stride_dx_t; p.per_part = (int)tiles_per_part;
     p.W = (int)W; p.w_dtype = w_dtype; p.state_dtype = state_dtype; p.act = activation;
     p.cu32 = (flags & GDN_FLAG_CU_INT32) != 0;
     hipStream_t s = (hipStream_t)stream;
     if (x_dtype == GDN_DTYPE_BF16) return launch_conv_bwd<bf16_t>(p, s);
     if (x_dtype == GDN_DTYPE_F16) return launch_conv_bwd<f16_t>(p, s);
     return launch_conv_bwd<float>(p, s);
+}
+
+extern "C" int gdn_causal_conv1d_bwd(
+    const void* x, const void* weight, const void* bias, const void* initial_state, const void* dy, const void* dht,
+    void* dx, float* dw_part, float* db_part, float* dh0,
+    const void* cu_seqlens, const void* tile_table,
+    int64_t B, int64_t T, int64_t D, int64_t W, int64_t N, int64_t num_tiles, int64_t stride_x_n, int64_t stride_x_t,
+    int x_dtype, int w_dtype, int state_dtype, int activation, uint32_t flags, void* stream) {
+    return gdn_causal_conv1d_bwd_runs(x, weight, bias, initial_state, dy, dht, dx, dw_part, db_part, dh0, cu_seqlens, tile_table, B, T, D, W, N, num_tiles,
+                                      stride_x_n, stride_x_t, D, GDN_CONV_BWD_TILES_PER_PART, x_dtype, w_dtype, state_dtype, activation, flags, stream);
 }
 
 extern "C" int gdn_norm_gated_bwd(
@@ -710,4 +807,32 @@ extern "C" int gdn_norm_gated_bwd(
     if (x_dtype == GDN_DTYPE_BF16) return launch_norm_bwd<bf16_t>(p, parts, s);
     if (x_dtype == GDN_DTYPE_F16) return launch_norm_bwd<f16_t>(p, parts, s);
     return launch_norm_bwd<float>(p, parts, s);
+}
+
+extern "C" int gdn_gate_bwd(
+    const float* dgate, const float* dbeta, const void* g, const void* b, const float* A_log, const float* dt_bias,
+    void* dg, void* db, float* part, int64_t rows, int64_t HV, int64_t parts,
+    int64_t ld_g, int64_t ld_b, int64_t ld_dg, int64_t ld_db, int64_t zero_from, int64_t zero_to,
+    int g_dtype, int b_dtype, float beta_max, void* stream) {
+    const char* who = "gdn_gate_bwd";
+    GDN_CHECK_ARG(rows >= 0 && HV >= 1 && parts >= 1 && parts <= 65535 && zero_to >= zero_from, GDN_ERR_INVALID, "%s: bad sizes", who);
+    GDN_CHECK_ARG(known_dtype(g_dtype) && known_dtype(b_dtype), GDN_ERR_UNSUPPORTED, "%s: unknown dtype", who);
+    GDN_CHECK_ARG(rows == 0 || (dbeta && db && (!dg || dgate) && (!A_log || (g && dg)) && (beta_max == 0.f || b)), GDN_ERR_INVALID, "%s: a tensor is missing", who);
+    GDN_CHECK_ARG(ld_g >= HV && ld_b >= HV && ld_dg >= HV && ld_db >= HV && (zero_to == zero_from || (dg && zero_to <= ld_dg)), GDN_ERR_INVALID, "%s: bad row lengths", who);
+    GateBwdParams p{dgate, dbeta, g, b, A_log, dt_bias, dg, db, part, rows, HV, ld_g, ld_b, ld_dg, ld_db, zero_from, zero_to, g_dtype, b_dtype, beta_max};
+    hipLaunchKernelGGL(gate_bwd_kernel, dim3((unsigned)parts), dim3(256), 0, (hipStream_t)stream, p);
+    return check_launch("gate_bwd_kernel");
+}
+
+extern "C" int gdn_sum_rows(const float* part, void* out, int64_t rows, int64_t n, int out_dtype, void* stream) {
+    const char* who = "gdn_sum_rows";
+    GDN_CHECK_ARG(rows >= 0 && n >= 0 && n < (1ll << 36) && known_dtype(out_dtype), GDN_ERR_INVALID, "%s: bad sizes or dtype", who);
+    if (n == 0) return GDN_OK;
+    GDN_CHECK_ARG(out && (part || rows == 0), GDN_ERR_INVALID, "%s: NULL tensor", who);
+    const dim3 grid((unsigned)((n + 63) / 64));
+    hipStream_t s = (hipStream_t)stream;
+    if (out_dtype == GDN_DTYPE_BF16) hipLaunchKernelGGL(sum_rows_kernel<bf16_t>, grid, dim3(256), 0, s, part, (bf16_t*)out, rows, n);
+    else if (out_dtype == GDN_DTYPE_F16) hipLaunchKernelGGL(sum_rows_kernel<f16_t>, grid, dim3(256), 0, s, part, (f16_t*)out, rows, n);
+    else hipLaunchKernelGGL(sum_rows_kernel<float>, grid, dim3(256), 0, s, part, (float*)out, rows, n);
+    return check_launch("sum_rows_kernel");
 }

@@ -8,9 +8,14 @@
 #include <ATen/ATen.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <c10/core/DeviceGuard.h>
+#include <pybind11/pybind11.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cmath>
+#include <vector>
 
 #include "../../../include/gdn_hip.h"
 
@@ -23,6 +28,14 @@ decltype(&gdn_chunk_fwd) p_chunk_fwd;
 decltype(&gdn_chunk_workspace_bytes) p_chunk_workspace_bytes;
 decltype(&gdn_step_linear) p_step_linear;
 decltype(&gdn_norm_gated_fwd) p_norm_gated_fwd;
+decltype(&gdn_norm_gated_bwd) p_norm_gated_bwd;
+decltype(&gdn_chunk_bwd_heads) p_chunk_bwd_heads;
+decltype(&gdn_chunk_bwd_heads_workspace_bytes) p_chunk_bwd_heads_workspace_bytes;
+decltype(&gdn_causal_conv1d_fwd) p_conv_fwd;
+decltype(&gdn_causal_conv1d_bwd_runs) p_conv_bwd_runs;
+decltype(&gdn_gate_bwd) p_gate_bwd;
+decltype(&gdn_sum_rows) p_sum_rows;
+decltype(&gdn_last_error) p_last_error;
 
 PyObject* bind(PyObject*, PyObject* table) {
     auto take = [&](const char* name, auto& fn) {
@@ -33,7 +46,10 @@ PyObject* bind(PyObject*, PyObject* table) {
     };
     if (!take("gdn_fused_recurrent_fwd", p_fused_recurrent_fwd) || !take("gdn_fused_recurrent_kda_fwd", p_fused_recurrent_kda_fwd) ||
         !take("gdn_chunk_fwd", p_chunk_fwd) || !take("gdn_chunk_workspace_bytes", p_chunk_workspace_bytes) ||
-        !take("gdn_step_linear", p_step_linear) || !take("gdn_norm_gated_fwd", p_norm_gated_fwd))
+        !take("gdn_step_linear", p_step_linear) || !take("gdn_norm_gated_fwd", p_norm_gated_fwd) || !take("gdn_norm_gated_bwd", p_norm_gated_bwd) ||
+        !take("gdn_chunk_bwd_heads", p_chunk_bwd_heads) || !take("gdn_chunk_bwd_heads_workspace_bytes", p_chunk_bwd_heads_workspace_bytes) ||
+        !take("gdn_causal_conv1d_fwd", p_conv_fwd) || !take("gdn_causal_conv1d_bwd_runs", p_conv_bwd_runs) || !take("gdn_gate_bwd", p_gate_bwd) ||
+        !take("gdn_sum_rows", p_sum_rows) || !take("gdn_last_error", p_last_error))
         return nullptr;
     Py_RETURN_NONE;
 }
@@ -184,45 +200,61 @@ PyObject* fused_recurrent(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // ---- chunked forward ----
 // (q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, chunk_indices, scan_tables, A_log, dt_bias,
 //  flags); chunk_indices, scan_tables: the tables of checked boundaries, in cu_seqlens' type
-PyObject* chunk_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
-    if (n != 15) { PyErr_SetString(PyExc_TypeError, "gdn_host.chunk_fwd takes 15 arguments"); return nullptr; }
-    const Arg q(a[0]), k(a[1]), v(a[2]), g(a[3]), beta(a[4]), h0(a[6]), cu(a[9]), table(a[10]), offsets(a[11]), A_log(a[12]), dt_bias(a[13]);
-    const bool vfirst = truth(a[8]);
+struct ChunkArgs {
+    Arg q{Py_None}, k{Py_None}, v{Py_None}, g{Py_None}, beta{Py_None}, h0{Py_None}, cu{Py_None}, table{Py_None}, offsets{Py_None}, A_log{Py_None}, dt_bias{Py_None};
     Dims d;
     float scale;
-    if (!operands(q, k, v, d) || d.code == GDN_DTYPE_F32 || !scale_of(a[5], d.K, scale)) Py_RETURN_NONE;
-    for (const Arg* x : {&g, &beta, &h0, &cu, &table, &offsets, &A_log, &dt_bias})
-        if (!plain(*x, d.dev)) Py_RETURN_NONE;
-    if (d.K % 8 || d.V % 8 || d.K > 256 || (d.K <= 128 && d.V > 128) || !beta || !per_head(g, d) || !per_head(beta, d) || !indices(cu, -1)) Py_RETURN_NONE;
-    if (!aligned16(q.ptr()) || !aligned16(k.ptr()) || !aligned16(v.ptr()) || !floats(A_log, d.HV) || !floats(dt_bias, d.HV)) Py_RETURN_NONE;
-    if ((A_log && !g) || (dt_bias && !A_log)) Py_RETURN_NONE;
-    const int gb = gb_code_of(g, beta);
-    if (gb < 0) Py_RETURN_NONE;
-    const int64_t N = cu ? cu->numel() - 1 : d.B;
-    if (N < 1 || (cu && (d.B != 1 || !table || !offsets || table->dim() != 2 || table->scalar_type() != cu->scalar_type() ||
-                         offsets->scalar_type() != cu->scalar_type() || offsets->numel() != 2 * N + 1)))
-        Py_RETURN_NONE;
-    const int64_t num_chunks = cu ? table->size(0) : d.B * ((d.T + 63) / 64);
-    const int64_t rows = vfirst ? d.V : d.K, cols = vfirst ? d.K : d.V;
-    if (h0 && (h0->scalar_type() != at::kFloat || h0->dim() != 4 || h0->size(0) != N || h0->size(1) != d.HV || h0->size(2) != rows ||
-               h0->size(3) != cols || !aligned16(h0.ptr())))
-        Py_RETURN_NONE;
-    uint32_t flags = (uint32_t)PyLong_AsUnsignedLong(a[14]);
-    if (PyErr_Occurred()) return nullptr;
-    if (vfirst) flags |= GDN_FLAG_STATE_V_FIRST;
-    if (cu) flags |= GDN_FLAG_SEQ_ORDER | (cu->scalar_type() == at::kInt ? GDN_FLAG_CU_INT32 : 0);
-    const size_t ws_bytes = p_chunk_workspace_bytes(N, d.T, num_chunks, d.H, d.HV, d.K, d.V, cu ? 1 : 0, flags);
+    int gb;
+    int64_t N, num_chunks, rows, cols;
+    uint32_t flags;
+};
+// false: not a call for the native path (or an error is set)
+bool chunk_args(PyObject* const* a, ChunkArgs& x) {
+    x.q = Arg(a[0]); x.k = Arg(a[1]); x.v = Arg(a[2]); x.g = Arg(a[3]); x.beta = Arg(a[4]); x.h0 = Arg(a[6]); x.cu = Arg(a[9]); x.table = Arg(a[10]);
+    x.offsets = Arg(a[11]); x.A_log = Arg(a[12]); x.dt_bias = Arg(a[13]);
+    const Arg &q = x.q, &k = x.k, &v = x.v, &g = x.g, &beta = x.beta, &h0 = x.h0, &cu = x.cu, &table = x.table, &offsets = x.offsets, &A_log = x.A_log, &dt_bias = x.dt_bias;
+    Dims& d = x.d;
+    const bool vfirst = truth(a[8]);
+    if (!operands(q, k, v, d) || d.code == GDN_DTYPE_F32 || !scale_of(a[5], d.K, x.scale)) return false;
+    for (const Arg* t : {&g, &beta, &h0, &cu, &table, &offsets, &A_log, &dt_bias})
+        if (!plain(*t, d.dev)) return false;
+    if (d.K % 8 || d.V % 8 || d.K > 256 || (d.K <= 128 && d.V > 128) || !beta || !per_head(g, d) || !per_head(beta, d) || !indices(cu, -1)) return false;
+    if (!aligned16(q.ptr()) || !aligned16(k.ptr()) || !aligned16(v.ptr()) || !floats(A_log, d.HV) || !floats(dt_bias, d.HV)) return false;
+    if ((A_log && !g) || (dt_bias && !A_log)) return false;
+    x.gb = gb_code_of(g, beta);
+    if (x.gb < 0) return false;
+    x.N = cu ? cu->numel() - 1 : d.B;
+    if (x.N < 1 || (cu && (d.B != 1 || !table || !offsets || table->dim() != 2 || table->scalar_type() != cu->scalar_type() ||
+                           offsets->scalar_type() != cu->scalar_type() || offsets->numel() != 2 * x.N + 1)))
+        return false;
+    x.num_chunks = cu ? table->size(0) : d.B * ((d.T + 63) / 64);
+    x.rows = vfirst ? d.V : d.K; x.cols = vfirst ? d.K : d.V;
+    if (h0 && (h0->scalar_type() != at::kFloat || h0->dim() != 4 || h0->size(0) != x.N || h0->size(1) != d.HV || h0->size(2) != x.rows ||
+               h0->size(3) != x.cols || !aligned16(h0.ptr())))
+        return false;
+    x.flags = (uint32_t)PyLong_AsUnsignedLong(a[14]);
+    if (PyErr_Occurred()) return false;
+    if (vfirst) x.flags |= GDN_FLAG_STATE_V_FIRST;
+    if (cu) x.flags |= GDN_FLAG_SEQ_ORDER | (cu->scalar_type() == at::kInt ? GDN_FLAG_CU_INT32 : 0);
+    return true;
+}
+PyObject* chunk_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    if (n != 15) { PyErr_SetString(PyExc_TypeError, "gdn_host.chunk_fwd takes 15 arguments"); return nullptr; }
+    ChunkArgs x;
+    if (!chunk_args(a, x)) { if (PyErr_Occurred()) return nullptr; Py_RETURN_NONE; }
+    const Dims& d = x.d;
+    const size_t ws_bytes = p_chunk_workspace_bytes(x.N, d.T, x.num_chunks, d.H, d.HV, d.K, d.V, x.cu ? 1 : 0, x.flags);
     if (ws_bytes == 0) Py_RETURN_NONE;
-    const at::Tensor o = empty_on(d.dev, v->scalar_type(), v->sizes());
+    const at::Tensor o = empty_on(d.dev, x.v->scalar_type(), x.v->sizes());
     at::Tensor ht;
-    if (truth(a[7])) ht = empty_on(d.dev, at::kFloat, {N, d.HV, rows, cols});
+    if (truth(a[7])) ht = empty_on(d.dev, at::kFloat, {x.N, d.HV, x.rows, x.cols});
     const at::Tensor ws = empty_on(d.dev, at::kByte, {(int64_t)ws_bytes});
     void* stream = stream_of(d.dev);
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = p_chunk_fwd(q.ptr(), k.ptr(), v.ptr(), g.ptr(), beta.ptr(), (const float*)A_log.ptr(), (const float*)dt_bias.ptr(), (const float*)h0.ptr(),
-                     ht.defined() ? (float*)ht.data_ptr() : nullptr, o.data_ptr(), cu.ptr(), table.ptr(), offsets.ptr(), ws.data_ptr(), ws_bytes,
-                     d.B, d.T, d.H, d.HV, d.K, d.V, N, num_chunks, scale, d.code, gb, flags, stream);
+    rc = p_chunk_fwd(x.q.ptr(), x.k.ptr(), x.v.ptr(), x.g.ptr(), x.beta.ptr(), (const float*)x.A_log.ptr(), (const float*)x.dt_bias.ptr(), (const float*)x.h0.ptr(),
+                     ht.defined() ? (float*)ht.data_ptr() : nullptr, o.data_ptr(), x.cu.ptr(), x.table.ptr(), x.offsets.ptr(), ws.data_ptr(), ws_bytes,
+                     d.B, d.T, d.H, d.HV, d.K, d.V, x.N, x.num_chunks, x.scale, d.code, x.gb, x.flags, stream);
     Py_END_ALLOW_THREADS
     if (rc != GDN_OK) Py_RETURN_NONE;
     return pair(o, ht);
@@ -303,7 +335,11 @@ PyObject* layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return THPVariable_Wrap(out);
 }
 
+#include "gdn_host_train.h"
+
 PyMethodDef methods[] = {
+    {"chunk_train", (PyCFunction)(void*)chunk_train, METH_FASTCALL, "chunked operator with gradients; None: not a call for the native path"},
+    {"layer_train", (PyCFunction)(void*)layer_train, METH_FASTCALL, "the layer's forward with gradients; None: not a call for the native path"},
     {"layer_step", (PyCFunction)(void*)layer_step, METH_FASTCALL, "one decode step of the layer; None: not a call for the native path"},
     {"bind", bind, METH_O, "bind({name: address}) - entry points of libgdn_hip.so"},
     {"fused_recurrent", (PyCFunction)(void*)fused_recurrent, METH_FASTCALL, "token recurrence; None: not a call for the native path"},

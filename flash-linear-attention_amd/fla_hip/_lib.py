@@ -154,6 +154,9 @@ SIGNATURES['gdn_causal_conv1d_bwd'] = (c_int, [
     c_void_p, c_void_p,                                # cu_seqlens tile_table
     c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,   # B T D W N num_tiles stride_x_n stride_x_t
     c_int, c_int, c_int, c_int, c_uint32, c_void_p])
+SIGNATURES['gdn_causal_conv1d_bwd_runs'] = (c_int, SIGNATURES['gdn_causal_conv1d_bwd'][1][:20] + [c_int64, c_int64] + SIGNATURES['gdn_causal_conv1d_bwd'][1][20:])
+SIGNATURES['gdn_gate_bwd'] = (c_int, [c_void_p] * 9 + [c_int64] * 9 + [c_int, c_int, c_float, c_void_p])
+SIGNATURES['gdn_sum_rows'] = (c_int, [c_void_p, c_void_p, c_int64, c_int64, c_int, c_void_p])
 SIGNATURES['gdn_norm_gated_bwd'] = (c_int, [
     c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,  # dy x g weight bias
     c_void_p, c_void_p, c_void_p,                      # mean rstd dresidual

@@ -31,6 +31,10 @@ _STEP_LINEARS = ('q_proj', 'k_proj', 'v_proj', 'a_proj', 'b_proj', 'g_proj', 'o_
 _STEP_CONVS = ('q_conv1d', 'k_conv1d', 'v_conv1d')
 
 
+def _hooked(m: nn.Module) -> bool:
+    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+
+
 class LayerCache:
     """Per-layer states of a stack of layers: ``cache[i]`` is layer i's dict, ``update`` replaces entries in it."""
 
@@ -143,30 +147,48 @@ class GatedDeltaNet(nn.Module):
         with torch.no_grad():
             return self._forward(hidden_states, attention_mask, past_key_values, use_cache, **kwargs)
 
-    def _step(self, hidden_states, past_key_values):
-        """One token per sequence on a filled cache through the native host path (``gdn_host.layer_step``: four launches), or None
-        where the layer is not its plain self - another module in a projection's place, hooks, autocast, a state to be converted."""
-        if past_key_values is None or len(past_key_values) <= self.layer_idx or not (self.use_gate and self.use_short_conv):
-            return None
-        entry = past_key_values[self.layer_idx]
-        state, conv = entry.get('recurrent_state'), entry.get('conv_state')
-        if state is None or conv is None or torch.is_autocast_enabled():
+    def _plain(self):
+        """(weights of the projections, the convolutions and the norm; the convolutions; the norm) where the layer is its plain self, or
+        None: another module in a projection's place, hooks, autocast."""
+        if not (self.use_gate and self.use_short_conv) or torch.is_autocast_enabled():
             return None
         mods = self._modules
         linears = [mods[n] for n in _STEP_LINEARS]
         convs = [mods[n] for n in _STEP_CONVS]
         norm = mods['o_norm']
         for m in linears:
-            if type(m) is not nn.Linear or m.bias is not None or m._forward_hooks or m._forward_pre_hooks:
+            if type(m) is not nn.Linear or m.bias is not None or _hooked(m):
                 return None
         for m in convs:
-            if type(m) is not ShortConvolution or m.activation is None or m._forward_hooks or m._forward_pre_hooks:
+            if type(m) is not ShortConvolution or m.activation is None or _hooked(m):
                 return None
-        if type(norm) is not FusedRMSNormGated or norm.activation == 'sigmoid' or norm._forward_hooks or norm._forward_pre_hooks:
+        if type(norm) is not FusedRMSNormGated or norm.activation == 'sigmoid' or _hooked(norm):
             return None
         weights = [m._parameters.get('weight') for m in (*linears, *convs, norm)]
-        if any(type(w) is not nn.Parameter for w in weights):
+        return None if any(type(w) is not nn.Parameter for w in weights) else (weights, convs, norm)
+
+    def _train(self, hidden_states):
+        """Whole dense sequences without a cache through the native training path (``gdn_host.layer_train``), or None."""
+        plain = self._plain()
+        if plain is None or any(m._parameters.get('bias') is not None for m in plain[1]):
             return None
+        w, _, norm = plain
+        return _lib.host().layer_train(hidden_states, *w[:7], tuple(w[7:10]), self._parameters['A_log'], self._parameters['dt_bias'], w[10], norm.eps,
+                                       self.allow_neg_eigval, self.num_heads)
+
+    def _step(self, hidden_states, past_key_values):
+        """One token per sequence on a filled cache through the native host path (``gdn_host.layer_step``: four launches), or None
+        where the layer is not its plain self - another module in a projection's place, hooks, autocast, a state to be converted."""
+        if past_key_values is None or len(past_key_values) <= self.layer_idx:
+            return None
+        entry = past_key_values[self.layer_idx]
+        state, conv = entry.get('recurrent_state'), entry.get('conv_state')
+        if state is None or conv is None:
+            return None
+        plain = self._plain()
+        if plain is None:
+            return None
+        weights, convs, norm = plain
         o = _lib.host().layer_step(
             hidden_states, *weights[:7], self._parameters['A_log'], self._parameters['dt_bias'], tuple(weights[7:10]),
             tuple(m._parameters['bias'] for m in convs), tuple(conv), state, weights[10], norm.eps, self.allow_neg_eigval, self.num_heads)
@@ -188,6 +210,11 @@ class GatedDeltaNet(nn.Module):
             o = self._step(hidden_states, past_key_values)
             if o is not None:
                 return o, None, past_key_values
+        if self.training and past_key_values is None and not use_cache and attention_mask is None and kwargs.get('cu_seqlens') is None \
+                and torch.is_grad_enabled():
+            o = self._train(hidden_states)
+            if o is not None:
+                return o, None, None
         last_state = None
         if past_key_values is not None and len(past_key_values) > self.layer_idx:
             last_state = past_key_values[self.layer_idx]

@@ -114,3 +114,10 @@ def forward_only(what: str, *activations: torch.Tensor | None) -> None:
     result that silently carries none.  Parameters are not looked at: inference outside ``torch.no_grad()`` is fine."""
     if torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in activations):
         raise NotImplementedError(f'{what} has no backward in fla_hip: run it under torch.no_grad() or on detached inputs')
+
+
+def sum_rows(part: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """``part.sum(0)`` of an fp32 tensor of partial sums, in ``dtype`` (added up in fp32, in a fixed order)."""
+    out = torch.empty(part.shape[1:], dtype=dtype, device=part.device)
+    _lib.check(_lib.load().gdn_sum_rows(ptr(part), ptr(out), part.shape[0], out.numel(), dtype_code(dtype), current_stream_ptr(part.device)))
+    return out

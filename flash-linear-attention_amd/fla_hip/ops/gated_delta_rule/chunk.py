@@ -164,19 +164,21 @@ class ChunkLaunch:
 
 
 def _native_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, cu_seqlens_cpu, A_log, dt_bias,
-                qk_l2norm, beta_sigmoid, neg_eigval):
-    """The forward through the native host path, or None where a tensor needs a conversion first."""
+                 qk_l2norm, beta_sigmoid, neg_eigval, train=False):
+    """The forward (``train``: with gradients) through the native host path, or None where a tensor needs a conversion first."""
     mode = os.environ.get('FLA_HIP_SCAN_MODE')
     flags = (_lib.FLAG_QK_L2NORM if qk_l2norm else 0) | (_SCAN_MODE_FLAGS.get(mode, 0) if mode else 0)
     if beta_sigmoid:
         flags |= _lib.FLAG_BETA_SIGMOID | (_lib.FLAG_NEG_EIGVAL if neg_eigval else 0)
     chunk_indices = scan_tables = None
+    whole = True
     if cu_seqlens is not None:
         if not cu_seqlens.is_cuda or cu_seqlens.dtype not in (torch.int32, torch.int64):
             return None
-        _, _, chunk_indices, scan_tables = packed_tables(cu_seqlens, k.shape[1], _KERNEL_CHUNK, cu_seqlens_cpu)
-    return _lib.host().chunk_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, chunk_indices,
-                                 scan_tables, A_log, dt_bias, flags)
+        first, last, chunk_indices, scan_tables = packed_tables(cu_seqlens, k.shape[1], _KERNEL_CHUNK, cu_seqlens_cpu)
+        whole = first == 0 and last == k.shape[1]
+    args = (q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, chunk_indices, scan_tables, A_log, dt_bias, flags)
+    return _lib.host().chunk_train(*args, whole) if train else _lib.host().chunk_fwd(*args)
 
 
 def chunk_gated_delta_rule_fwd(
@@ -343,6 +345,12 @@ def chunk_gated_delta_rule(
     if torch.is_grad_enabled() and any(
             x is not None and x.requires_grad for x in (q, k, v, g, beta, initial_state, A_log, dt_bias)):
         # training: the same forward kernels inside an autograd function (chunk.py:260-395)
+        if not os.environ.get('FLA_HIP_BWD_SCAN_MODE'):
+            out = _native_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, cu_seqlens_cpu,
+                               A_log if use_gate_in_kernel else None, dt_bias if use_gate_in_kernel else None, use_qk_l2norm_in_kernel,
+                               use_beta_sigmoid_in_kernel, allow_neg_eigval, train=True)
+            if out is not None:
+                return out
         from fla_hip.ops.gated_delta_rule.chunk_bwd import ChunkGatedDeltaRuleFunction
         return ChunkGatedDeltaRuleFunction.apply(
             q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, cu_seqlens_cpu,

@@ -41,6 +41,10 @@ def chunk_gated_delta_rule_bwd(
     q_rstd: torch.Tensor | None = None,
     k_rstd: torch.Tensor | None = None,
     qk_l2norm: bool = False,
+    A_log: torch.Tensor | None = None,
+    dt_bias: torch.Tensor | None = None,
+    beta_sigmoid: bool = False,
+    neg_eigval: bool = False,
 ):
     """q, k ``[B,T,H,K]``, v, do ``[B,T,HV,V]``, g (log decay), beta ``[B,T,HV]`` as the recurrence uses them.
     Returns ``(dq, dk, dv, dbeta, dg, dh0)``: dq, dk, dv in q's dtype, dbeta, dg fp32, dh0 fp32 (None without
@@ -48,7 +52,9 @@ def chunk_gated_delta_rule_bwd(
     passed as q and k) dq and dk are the gradients of the rows before normalisation: the reference's ``l2norm_bwd``
     (chunk.py:385-387) in a kernel of its own.  With ``qk_l2norm`` q and k
     are the rows BEFORE their l2 normalisation and dq, dk the gradients of those: one C call
-    (``gdn_chunk_bwd_heads``), which also adds up the value heads of a q/k head."""
+    (``gdn_chunk_bwd_heads``), which also adds up the value heads of a q/k head.  With ``A_log`` (and ``dt_bias``, both ``[HV]`` fp32)
+    or ``beta_sigmoid`` g and beta are the inputs of those activations; dg and dbeta stay the gradients of their results
+    (``gate_bwd`` goes on from there)."""
     dev = require_gpu(q, k, v, beta, do)
     check_operand_shapes(q, k, v, g=g, beta=beta)
     if do.shape != v.shape:
@@ -116,10 +122,12 @@ def chunk_gated_delta_rule_bwd(
     lib = _lib.load()
     if qk_l2norm:
         flags |= _lib.FLAG_QK_L2NORM
+    if beta_sigmoid:
+        flags |= _lib.FLAG_BETA_SIGMOID | (_lib.FLAG_NEG_EIGVAL if neg_eigval else 0)
     ws_bytes = lib.gdn_chunk_bwd_heads_workspace_bytes(num_chunks, H, HV, KD, VD, B * T, flags)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     _lib.check(lib.gdn_chunk_bwd_heads(
-        ptr(qw), ptr(kw), ptr(vw), ptr(gw), ptr(bw), None, None, ptr(h0), ptr(dow), ptr(dhtw),
+        ptr(qw), ptr(kw), ptr(vw), ptr(gw), ptr(bw), ptr(A_log), ptr(dt_bias), ptr(h0), ptr(dow), ptr(dhtw),
         ptr(dq), ptr(dk), ptr(dv), ptr(dg), ptr(db), ptr(dh0),
         ptr(cu_seqlens), ptr(chunk_table), ptr(chunk_offsets), ptr(workspace), ws_bytes,
         B, T, H, HV, KD, VD, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags,
@@ -131,6 +139,30 @@ def chunk_gated_delta_rule_bwd(
         dh0 = dh0[..., :K, :V]
         dh0 = (dh0.transpose(-1, -2) if state_v_first else dh0).contiguous()
     return dq, dk, dv, db, dg, dh0
+
+
+def gate_bwd(dgate, dbeta, g, beta, A_log, dt_bias, beta_max):
+    """The gradients of the gate ``-exp(A_log) softplus(g + dt_bias)`` (``g`` None: of no gate, ``dgate`` comes back) and of
+    ``beta_max sigmoid(beta)`` (0: none) with respect to g and beta, in their types; and ``[parts, 2, HV]`` partial sums of the
+    gradients of A_log and dt_bias (fla/ops/gated_delta_rule/gate.py:109-160)."""
+    dev = dbeta.device
+    HV = dbeta.shape[-1]
+    rows = dbeta.numel() // HV
+    with_gate = g is not None
+    if with_gate:
+        g = g if g.dtype in (torch.bfloat16, torch.float16, torch.float32) else g.float()
+        g = g.contiguous()
+    beta = beta if beta.dtype in (torch.bfloat16, torch.float16, torch.float32) else beta.float()
+    beta = beta.contiguous()
+    parts = max(1, min(256, rows * HV // 2048))
+    dg = torch.empty_like(g) if with_gate else None
+    db = torch.empty_like(beta)
+    part = torch.empty(parts, 2, HV, dtype=torch.float32, device=dev) if with_gate else None
+    _lib.check(_lib.load().gdn_gate_bwd(
+        ptr(dgate) if with_gate else None, ptr(dbeta), ptr(g) if with_gate else None, ptr(beta), ptr(A_log) if with_gate else None,
+        ptr(dt_bias), ptr(dg), ptr(db), ptr(part), rows, HV, parts, HV, HV, HV, HV, 0, 0,
+        dtype_code(g.dtype) if with_gate else _lib.DTYPE_F32, dtype_code(beta.dtype), beta_max, current_stream_ptr(dev)))
+    return dg if with_gate else dgate, db, part
 
 
 def _finish(lib, dxh: torch.Tensor, y: torch.Tensor, rstd: torch.Tensor | None, H: int, K: int, out_dtype) -> torch.Tensor:
@@ -187,29 +219,21 @@ class ChunkGatedDeltaRuleFunction(torch.autograd.Function):
         q, k, v, g, beta_raw, h0, cu_seqlens, cu_seqlens_cpu, chunk_indices, A_log, dt_bias = ctx.saved_tensors
         scale, state_v_first, l2, gate, bsig, neg, chunk_size = ctx.opts
         K = q.shape[-1]
-        beta = beta_raw
-        if bsig:
-            beta = torch.sigmoid(beta_raw.float()) * (2.0 if neg else 1.0)
-        g_in = g
-        if gate:
-            # g = -exp(A_log) softplus(g + dt_bias)   (fla/ops/gated_delta_rule/gate.py:21-46)
-            x = g_in.float() if dt_bias is None else g_in.float() + dt_bias.float()
-            g = -A_log.float().exp() * F.softplus(x)
+        A32 = A_log.float().reshape(-1).contiguous() if gate else None
+        dt32 = dt_bias.float().reshape(-1).contiguous() if gate and dt_bias is not None else None
         dq, dk, dv, db, dg, dh0 = chunk_gated_delta_rule_bwd(
-            q, k, v, g, beta, scale, h0, do.contiguous(), dht, state_v_first, cu_seqlens, cu_seqlens_cpu,
-            chunk_indices, chunk_size, qk_l2norm=l2)
-        if bsig:
-            s = torch.sigmoid(beta_raw.float())
-            db = db * s * (1 - s) * (2.0 if neg else 1.0)
+            q, k, v, g, beta_raw, scale, h0, do.contiguous(), dht, state_v_first, cu_seqlens, cu_seqlens_cpu,
+            chunk_indices, chunk_size, qk_l2norm=l2, A_log=A32, dt_bias=dt32, beta_sigmoid=bsig, neg_eigval=neg)
         dA_log = ddt_bias = None
-        if gate:
-            # (gate.py:109-160)  dg/dx = -exp(A_log) sigmoid(x),  dg/dA_log = g
-            dA_log = (dg * g).sum((0, 1)).to(A_log.dtype).reshape(A_log.shape)
-            dg = dg * (-A_log.float().exp() * torch.sigmoid(x))
-            if dt_bias is not None:
-                ddt_bias = dg.sum((0, 1)).to(dt_bias.dtype).reshape(dt_bias.shape)
-        if g_in is not None:
-            dg = dg.to(g_in.dtype)
+        if gate or bsig:
+            dg, db, part = gate_bwd(dg, db, g if gate else None, beta_raw, A32, dt32, (2.0 if neg else 1.0) if bsig else 0.0)
+            if gate:
+                sums = part.sum(0)
+                dA_log = sums[0].to(A_log.dtype).reshape(A_log.shape)
+                if dt_bias is not None:
+                    ddt_bias = sums[1].to(dt_bias.dtype).reshape(dt_bias.shape)
+        if g is not None:
+            dg = dg.to(g.dtype)
         else:
             dg = None
         return (dq[..., :K].to(q.dtype), dk[..., :K].to(k.dtype), dv.to(v.dtype), dg, db.to(beta_raw.dtype), None, dh0, None, None, None,

@@ -580,6 +580,35 @@ int gdn_causal_conv1d_bwd(
     int x_dtype, int w_dtype, int state_dtype, int activation, uint32_t flags, void* stream);
 
 /*
+ * The same with rows of dx stride_dx_t elements apart (a slice of a wider gradient is written in place) and runs of tiles_per_part
+ * tiles: dw_part [parts,D,W], db_part [parts,D] with parts = ceil(num_tiles / tiles_per_part), 1 <= tiles_per_part <= 64.
+ */
+int gdn_causal_conv1d_bwd_runs(
+    const void* x, const void* weight, const void* bias, const void* initial_state, const void* dy, const void* dht,
+    void* dx, float* dw_part, float* db_part, float* dh0,
+    const void* cu_seqlens, const void* tile_table,
+    int64_t B, int64_t T, int64_t D, int64_t W, int64_t N, int64_t num_tiles, int64_t stride_x_n, int64_t stride_x_t,
+    int64_t stride_dx_t, int64_t tiles_per_part,
+    int x_dtype, int w_dtype, int state_dtype, int activation, uint32_t flags, void* stream);
+
+/*
+ * The gradients gdn_chunk_bwd_heads leaves of the gate and of beta, back through their activations (fla/ops/gated_delta_rule/gate.py:109-160,
+ * the derivative of the sigmoid in chunk.py:385-393).
+ *   dgate, dbeta [rows,HV] fp32; g, b: the raw inputs, rows ld_g, ld_b elements apart; A_log, dt_bias [HV] fp32 or NULL (A_log NULL:
+ *   dgate is handed on); beta_max 1 or 2: beta was that times the sigmoid of b, 0: dbeta is handed on
+ *   dg (or NULL: no gate), db: rows ld_dg, ld_db elements apart, in g_dtype, b_dtype; columns zero_from .. zero_to - 1 of dg's rows are cleared
+ *   part [parts,2,HV] fp32 or NULL: partial sums of dA_log and ddt_bias, one row per workgroup (gdn_sum_rows adds them up)
+ */
+int gdn_gate_bwd(
+    const float* dgate, const float* dbeta, const void* g, const void* b, const float* A_log, const float* dt_bias,
+    void* dg, void* db, float* part, int64_t rows, int64_t HV, int64_t parts,
+    int64_t ld_g, int64_t ld_b, int64_t ld_dg, int64_t ld_db, int64_t zero_from, int64_t zero_to,
+    int g_dtype, int b_dtype, float beta_max, void* stream);
+
+/* out[n] (out_dtype) = the rows of part [rows,n] fp32 added up in fp32, in a fixed order. */
+int gdn_sum_rows(const float* part, void* out, int64_t rows, int64_t n, int out_dtype, void* stream);
+
+/*
  * Backward of gdn_norm_gated_fwd.  Replaces layer_norm_gated_bwd (fla/modules/fused_norm_gate.py:541-650, kernels :192-453).
  *   dy, x, g, dx, dg: T rows of D features x_dtype, ld elements apart (ld >= D a multiple of 16 / sizeof(element), up to 2048;
  *   dy must read as zero from D on); x is what was normalised (the forward's residual_out when there was a residual);
