@@ -24,7 +24,7 @@ static int launch_chunk(const ChunkParams& p0, int64_t num_chunks, int stages, h
         return (stages & STAGE_SCAN) ? launch_wide256<T>(p, stream) : GDN_OK;
     }
     const int64_t G = p.HV / p.H;
-    const int nseg = plan_segments(p.N, p.HV, p.NT, num_chunks, p.cu_seqlens == nullptr, p.flags);
+    const int nseg = plan_segments(p.N, p.HV, p.NT, num_chunks, p.cu_seqlens == nullptr, p.flags, p.K, p.V);
     const bool segments = nseg > 0;
     // (head dims up to 64 have a one-run kernel with a quarter-size state; the two-run kernel would do the full 128 x 128 work)
     const bool small = p.K <= 64 && p.V <= 64;
@@ -37,7 +37,11 @@ static int launch_chunk(const ChunkParams& p0, int64_t num_chunks, int stages, h
     };
     const bool pass2_pairs = segments && use_pair(pair_full_ok, p.NH * nseg);
     const bool whole_pairs = !segments && use_pair(pair_full_ok, p.NH);
-    p.want_P = (p.flags & GDN_FLAG_RECORD_P) != 0;       // every scan kernel forms P itself
+    // (the scan kernels form P themselves, except in halves: those read it, and q's norms, from the records)
+    const bool halves = !segments && !whole_pairs && halves_fit(p.NH, p.K, p.V, p.flags);
+    p.halves = halves;
+    p.want_P = halves || (p.flags & GDN_FLAG_RECORD_P) != 0;
+    if (halves) p.flags &= ~FLAG_Q_NORM_IN_SCAN;
     if (stages & STAGE_PREPARE) {
         int rc = launch_prepare<T>(p, num_chunks, stream);
         if (rc) return rc;
@@ -86,7 +90,7 @@ static size_t chunk_workspace_need(int64_t N, int64_t T, int64_t num_chunks, int
         const int nseg = plan_segments256(N, H, HV, V, (T + CH - 1) / CH, !packed, flags);
         return ws_layout(num_chunks, HV, nseg > 1 ? (int64_t)nseg * N * HV : 0, base, ws, seg256_floats(V));
     }
-    const int nseg = plan_segments(N, HV, (T + CH - 1) / CH, num_chunks, !packed, flags);
+    const int nseg = plan_segments(N, HV, (T + CH - 1) / CH, num_chunks, !packed, flags, K, V);
     return ws_layout(num_chunks, HV, (int64_t)nseg * N * HV, base, ws);
 }
 

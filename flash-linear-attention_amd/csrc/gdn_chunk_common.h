@@ -145,6 +145,14 @@ constexpr int64_t SEG_SLOTS_MAX = 640;            // upper bound on (sequences *
 
 inline size_t ws_align(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// Whole sequences in two halves of 64 value columns, a workgroup each (gdn_chunk_wide.hip, HALF), where twice the runs still fit the
+// chip: a step of half a run takes 1.6 us, one of a whole run 2.7 - 3.2.  Not where the caller asks for one form of the scan.  Up to 36
+// chunks they also beat time segments, whose steps are those of whole runs, with a warm-up of some 8 of them and two more launches, or
+// the exact path's twice as many (1 x 2048 tokens, 32 heads, 4 segments: 98 us with heads that forget slowly).
+inline bool halves_fit(int64_t NH, int64_t K, int64_t V, uint32_t flags) {
+    return K == 128 && V == 128 && NH <= 128 && !(flags & (GDN_FLAG_SCAN_WIDE | GDN_FLAG_SCAN_SEGMENTS | GDN_FLAG_SCAN_PAIR | GDN_FLAG_RECORD_P));
+}
+
 // Number of time segments the sequential stage cuts every sequence into (0: whole sequences, one
 // workgroup per sequence and head).  With few (sequence, head) runs and long dense sequences, time is
 // cut so that every CU has a workgroup - never more workgroups than CUs: a second round of workgroups
@@ -153,9 +161,10 @@ inline size_t ws_align(size_t x) { return (x + 255) & ~(size_t)255; }
 // (one pass over half the chunks plus the warm-up); with exact start states only (first pass, merge,
 // second pass) it takes three.  Either way the steps saved per workgroup must outweigh a warm-up of typical
 // length plus the two launches that find nothing to do: 24 chunks or more.  Shared by the workspace size and the launch.
-inline int plan_segments(int64_t N, int64_t HV, int64_t NT, int64_t num_chunks, bool dense, uint32_t flags) {
+inline int plan_segments(int64_t N, int64_t HV, int64_t NT, int64_t num_chunks, bool dense, uint32_t flags, int64_t K, int64_t V) {
     const int64_t NH = N * HV;
     int nseg = 0;
+    if (halves_fit(NH, K, V, flags) && NT <= 36) return 0;
     if (dense && NH > 0) {
         // (GDN_FLAG_SCAN_SEGMENTS asks for segments wherever they are possible at all: segments of 4 chunks)
         nseg = (int)std::min<int64_t>(256 / NH, NT / ((flags & GDN_FLAG_SCAN_SEGMENTS) ? 4 : 8));
@@ -208,6 +217,7 @@ struct ChunkParams {
     int K, V;                                          // head dims of the caller's tensors (multiples of 8; K, V <= 128, or 128 < K <= 256 with any V)
     float scale; int gb_dtype, beta_dtype; uint32_t flags;
     int64_t NH;
+    bool halves;                                       // two workgroups per run, 64 value columns each
     int want_P;                                        // the prepare kernel also writes P (GDN_FLAG_RECORD_P)
 };
 

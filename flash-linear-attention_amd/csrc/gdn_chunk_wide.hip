@@ -52,19 +52,35 @@ constexpr int OT_BYTES = 64 * OT_PITCH;           // 17 408 B
 constexpr int PCOUNT_OFF = KBUF + 3 * 16384 + OT_BYTES;       // one counter: P fragments published so far
 constexpr size_t WIDE_SMEM = PCOUNT_OFF + 16;                // 156 688 B of the CU's 163 840: one workgroup per CU
 constexpr int WIDE_NN = 2;                        // 16-column tiles per compute wave
+#ifndef WIDE_XB
+#define WIDE_XB 8
+#endif
 #ifndef WIDE_RING
 #define WIDE_RING 3                               // operand fragments in flight per compute wave
 #endif
 constexpr int CW = 8 / WIDE_NN;                   // compute waves
 constexpr int WIDE_THREADS = (CW + 4) * 64;
 
-template <typename T, bool FULL, bool DIMS128, bool SMALL>
+// HALF: three buffers (chunk % 3) for k, q and the 64 columns of v, so that everything is requested two steps ahead (a step of half the
+// length leaves no time for a copy issued one ahead), two for the records (Xb, P, the first table), a narrower output tile.  v: blocks
+// of 4 rows x 8 pieces, laid out like the first half of the blocks above, two to a copy.
+constexpr int HALF_Q = 3 * 16384, HALF_V = 6 * 16384, HALF_V_BYTES = 8192, HALF_REC = HALF_V + 3 * HALF_V_BYTES;
+constexpr int HALF_NREC = REC_PIECES_X + REC_PIECES_P + 1, HALF_OT = HALF_REC + 2 * HALF_NREC * 1024, HALF_OT_PITCH = 144;
+constexpr size_t HALF_SMEM = HALF_OT + 64 * HALF_OT_PITCH;
+
+template <typename T, bool FULL, bool DIMS128, bool SMALL, bool HALF = false>
 __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParams p, SegmentPlan sp) {
     // Head dims: DIMS128 fixes K = V = 128 at compile time (every copy is whole, nothing is masked); otherwise they
     // are the caller's multiples of 8 and the tiles' features past them are zero (q, k) or never stored (v, o, state).
     // SMALL (K, V <= 64, e.g. the reference's D = 64 shapes): a quarter of the state - 64 key rows, 16 value columns
     // per compute wave - with the LDS layout unchanged, so that nothing is multiplied by the zero features.
     static_assert(!(DIMS128 && SMALL), "one or the other");
+    // HALF (whole sequences, up to 128 of them and their heads): two workgroups share a run, 64 value columns each, one 16-column tile
+    // per compute wave - half the instruction stream of a step, which is what a chip with idle CUs waits for.  The copy waves' share of
+    // forming P would then be the longest part of a step: P comes with the records (the prepare kernel forms it for all chunks at once),
+    // and the output wave copies them.  A step takes 3900 cycles alone on its CU (6000 for a whole run), 2300 of them the LDS' share:
+    // every wave reads all of k and q.  1500 tokens, 32 heads: 87 -> 57 us a call; 333 tokens: 33.5 -> 28 us.
+    static_assert(!HALF || (DIMS128 && FULL), "whole runs of 128 x 128");
     const int K = DIMS128 ? 128 : p.K, V = DIMS128 ? 128 : p.V;
     constexpr int KS = SMALL ? 2 : 4;                 // pairs of 16-row key tiles (32 key features each)
     typedef typename Mma<T>::V8 V8;
@@ -94,11 +110,11 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
     const float* src = nullptr;
     float* dst = nullptr;
     if (sp.kind == WIDE_WHOLE) {
-        const int64_t group = (slot / G) * 8 + xcd;                 // (sequence, q/k head)
+        const int64_t member = HALF ? slot >> 1 : slot, group = (member / G) * 8 + xcd;                 // (sequence, q/k head)
         if (group >= p.N * H) return;
         int64_t nseq = group / H;
         if (p.flags & GDN_FLAG_SEQ_ORDER) nseq = load_index(p.chunk_offsets, p.N + 1 + nseq, cu32);     // longest sequences start first
-        inh = nseq * HV + (group % H) * G + slot % G; seg = 0;
+        inh = nseq * HV + (group % H) * G + member % G; seg = 0;
         src = p.h0 ? p.h0 + inh * (int64_t)(K * V) : nullptr; src_user = true;
         dst = p.ht ? p.ht + inh * (int64_t)(K * V) : nullptr; dst_user = true;
     } else if (sp.kind == WIDE_PASS1) {
@@ -143,6 +159,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         }
         if (seg == sp.nseg - 1 && p.ht) { dst = p.ht + inh * (int64_t)(K * V); dst_user = true; }
     }
+    const int col0 = HALF ? 64 * (int)(slot & 1) : 0;       // first value column of this workgroup
     const int64_t n = inh / HV;
     const int hv = (int)(inh % HV);
     const int h = hv / (HV / H);
@@ -162,12 +179,13 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
     const int64_t it1 = min(nt, (int64_t)seg * sp.seg_chunks + sp.seg_chunks);
     const int64_t nsteps = it1 - it0;                       // may be <= 0 for an empty sequence
     const int64_t lastc = it1 - 1;
-    char* otile = smem + KBUF + 3 * 16384;                  // [64 token rows][OT_PITCH]
+    char* otile = smem + (HALF ? HALF_OT : KBUF + 3 * 16384);       // [64 token rows][OTP]
+    constexpr int OTP = HALF ? HALF_OT_PITCH : OT_PITCH;
     // The copy waves form P of a chunk while the compute waves are busy with the first products of its step and
     // announce it by adding to this counter (4 per step); a compute wave looks at the counter before it fetches P.
     // No barrier: one in the middle of a step costs the compute waves the slack between them.
     volatile int* pcount = (volatile int*)(smem + PCOUNT_OFF);
-    if (tid == 0) *pcount = 0;                              // (published by the barrier B0)
+    if (!HALF && tid == 0) *pcount = 0;                              // (published by the barrier B0)
 
     // =====================================================================================
     // Copy waves.  Step i (chunk it = it0 + i, stage cur = i & 1) has two phases, separated by
@@ -196,7 +214,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         // is spread over the lanes exactly like the operand fragment the compute waves read.  A counter in LDS announces it
         // (announce_P). ----
         auto produce_P = [&](const char* st, const char* kbuf) {
-            if constexpr (FULL) {
+            if constexpr (FULL && !HALF) {
                 __builtin_amdgcn_s_setprio(3);
                 const int pw = w - CW;
                 const V8* sK = (const V8*)kbuf;
@@ -244,7 +262,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         };
         // ... and announces it: this wave's fragments of step i are in LDS (its LDS operations complete in order)
         auto announce_P = [&]() {
-            if constexpr (FULL) {
+            if constexpr (FULL && !HALF) {
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 if (lane == 0) __hip_atomic_fetch_add((int*)pcount, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 __builtin_amdgcn_s_setprio(0);
@@ -301,7 +319,37 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
                     else gather_1k_to_lds(rec + j * 1024, lane * 16, lds_stage + STG_REC + j * 1024);
                 }
         };
-        if (w == CW) {
+        // HALF: k, q and v a wave each, the copy of chunk i+2 issued at the start of step i (its buffer was last read in step i-1) and
+        // awaited at the end of step i+1
+        if (HALF && w < CW + 3) {
+            auto walk = [&](auto issue, auto count) {
+                issue((int64_t)0);
+                issue((int64_t)1);
+                wait_vm_at_most<decltype(count)::value>();
+                lds_barrier();                                              // B0
+                for (int64_t i = 0; i < nsteps; ++i) {
+                    issue(i + 2);
+                    lds_barrier();                                          // B1
+                    wait_vm_at_most<decltype(count)::value>();
+                    lds_barrier();                                          // B2
+                }
+            };
+            if (w == CW) walk([&](int64_t i) { gather_blocks((const T*)p.k, min(it0 + i, lastc), 0, 16, lds0 + (int)(i % 3) * 16384); }, std::integral_constant<int, 16>{});
+            else if (w == CW + 1) walk([&](int64_t i) { gather_blocks((const T*)p.q, min(it0 + i, lastc), 0, 16, lds0 + HALF_Q + (int)(i % 3) * 16384); }, std::integral_constant<int, 16>{});
+            else if (w == CW + 2) {
+                const int s5 = lane & 31;                                   // slot inside a block of 4 rows x 8 pieces
+                walk([&](int64_t i) {
+                    const int64_t it = min(it0 + i, lastc);
+                    const int valid = (int)min((int64_t)CH, len - it * CH);
+                    const char* base = (const char*)((const T*)p.v + ((bos + it * CH) * HV + hv) * V);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const int b = 2 * j + (lane >> 5), row = min(4 * b + ((s5 & 15) >> 2), valid - 1), c = 4 * (s5 >> 4) + ((s5 - b) & 3);
+                        gather_1k_to_lds(base, (uint32_t)row * row_bytes + 16 * c + 2 * col0, lds0 + HALF_V + (int)(i % 3) * HALF_V_BYTES + j * 1024);
+                    }
+                }, std::integral_constant<int, 8>{});
+            }
+        } else if (w == CW) {
             // ---- k: the copy of chunk i+2 is issued at the start of step i (its buffer was last read
             // in step i-1) and awaited at the end of step i+1 ----
             auto issue_k = [&](int64_t i) {                                 // i counts from the first chunk of this run
@@ -320,29 +368,29 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
                 lds_barrier();                                              // B2
             }
         } else if (w <= CW + 2) {
-            // ---- q + Xb + tables (wave CW+1) and v (wave CW+2).  Pieces
+            // ---- q (state-only runs: Xb and the first table) (wave CW+1) and v (wave CW+2).  Pieces
             // [0, XB) of chunk c are issued in phase B of step c-2, the rest in phase A of step c-1.
             const bool qside = (w == CW + 1);
-            constexpr int XB = 8;
+            constexpr int XB = WIDE_XB;
             auto issue = [&](int64_t it, int stage, bool early) {
                 const uint32_t st = lds0 + stage * STG_BYTES;
                 const bool warming = it - it0 < warm;               // a chunk of the warm-up: no output, so neither q nor P
                 if (qside) {
                     if constexpr (FULL) {
-                        // 16 q pieces, then Xb (5) and the tables (2)
-                        if (early) gather_blocks((const T*)p.q, it, 0, 8, st + STG_Q, warming);
-                        else { gather_blocks((const T*)p.q, it, 8, 16, st + STG_Q, warming); copy_rec(it, 0, REC_PIECES_X, st); copy_rec(it, REC_PIECE_TAB, REC_PIECE_TAB + 1, st); copy_rec(it, REC_PIECE_TAB2, REC_PIECE_TAB2 + 1, st, warming); }
+                        // 16 q pieces (the output wave copies the records)
+                        if (early) gather_blocks((const T*)p.q, it, 0, XB, st + STG_Q, warming);
+                        else gather_blocks((const T*)p.q, it, XB, 16, st + STG_Q, warming);
                     } else {
                         if (early) { copy_rec(it, 0, REC_PIECES_X, st); copy_rec(it, REC_PIECE_TAB, REC_PIECE_TAB + 1, st); }      // all 6 pieces
                     }
                 } else {
-                    if (early) { if (!v_zero) gather_blocks((const T*)p.v, it, 0, 8, st + STG_V); }      // (v is not read when it counts as zero)
+                    if (early) { if (!v_zero) gather_blocks((const T*)p.v, it, 0, XB, st + STG_V); }      // (v is not read when it counts as zero)
                     else {
-                        if (!v_zero) gather_blocks((const T*)p.v, it, 8, 16, st + STG_V);
+                        if (!v_zero) gather_blocks((const T*)p.v, it, XB, 16, st + STG_V);
                     }
                 }
             };
-            // number of pieces issued early: 8, except 6 for the q side of a state-only run
+            // number of pieces issued early: XB, except 6 for the q side of a state-only run
             auto wait_early_only = [&]() {
                 if (!FULL && qside) wait_vm_at_most<REC_PIECES_X + 1>();
                 else wait_vm_at_most<XB>();
@@ -364,31 +412,53 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
                 lds_barrier();                                              // B2
             }
         } else {
-            // ---- output rows: one instruction stores 4 token rows of 256 bytes ----
+            // ---- output rows: one instruction stores 4 token rows of 256 bytes (HALF: 8 of 128) - and, in full runs, the records: that of
+            // chunk it + 1 is issued in phase A of step it and awaited at its end.  That wait leaves the newer stores outstanding (every
+            // one of them is issued inside the loop: its chunks are whole).  Nothing is issued between the step's two barriers: a copy
+            // takes some hundred cycles to issue, and every wave would wait for it there. ----
+            constexpr int NREC = HALF ? HALF_NREC : REC_PIECES_X + 2, NROW = HALF ? 8 : 16;     // record pieces; store instructions per tile
+            auto issue_rec = [&](int64_t it, int stage) {
+                if constexpr (HALF) copy_rec(it, 0, NREC, lds0 + HALF_REC - STG_REC + stage * (HALF_NREC * 1024));
+                else {
+                    const uint32_t st = lds0 + stage * STG_BYTES;
+                    copy_rec(it, 0, REC_PIECES_X, st);
+                    copy_rec(it, REC_PIECE_TAB, REC_PIECE_TAB + 1, st);
+                    copy_rec(it, REC_PIECE_TAB2, REC_PIECE_TAB2 + 1, st, it - it0 < warm);
+                }
+            };
+            const int orow0 = HALF ? lane >> 3 : g, opiece = HALF ? lane & 7 : c16;
             T* og = (T*)p.o;
-            u32x4 orow[16];                                                 // output tile of the previous chunk
+            u32x4 orow[NROW];                                               // output tile of the previous chunk
             auto store_rows = [&](int64_t it) {
                 const int valid = (int)min((int64_t)CH, len - it * CH);
-                int64_t stride = (int64_t)HV * V * 4;                     // elements between rows 4 apart
-                asm volatile("" : "+s"(stride));                            // keep the 16 row addresses out of long-lived registers
-                T* dstp = og + ((bos + it * CH + g) * HV + hv) * V + c16 * 8;
-                const bool col_ok = c16 * 8 < V;                          // (value columns past V exist in the tile only)
+                int64_t stride = (int64_t)HV * V * (64 / NROW);           // elements between rows 4 (8) apart
+                asm volatile("" : "+s"(stride));                            // keep the row addresses out of long-lived registers
+                T* dstp = og + ((bos + it * CH + orow0) * HV + hv) * V + col0 + opiece * 8;
+                const bool col_ok = HALF || c16 * 8 < V;                  // (value columns past V exist in the tile only)
 #pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    if (4 * j + g < valid && col_ok) *(u32x4*)dstp = orow[j];
+                for (int j = 0; j < NROW; ++j) {
+                    if ((64 / NROW) * j + orow0 < valid && col_ok) *(u32x4*)dstp = orow[j];
                     dstp += stride;
                 }
             };
+            if constexpr (FULL) {
+                issue_rec(it0, 0);
+                wait_vm_at_most<0>();
+            }
             lds_barrier();                                                  // B0
             for (int64_t i = 0; i < nsteps; ++i) {
                 if (i >= warm) produce_P(smem + (i & 1) * STG_BYTES, smem + KBUF + (int)(i % 3) * 16384);
                 announce_P();
-                if constexpr (FULL) { if (i > warm) store_rows(it0 + i - 1); }
+                if constexpr (FULL) {
+                    issue_rec(min(it0 + i + 1, lastc), (int)(i & 1) ^ 1);
+                    if (i > warm) store_rows(it0 + i - 1);
+                }
                 lds_barrier();                                              // B1
                 if constexpr (FULL) {
 #pragma unroll
-                    for (int j = 0; j < 16; ++j) orow[j] = *(const u32x4*)(otile + (4 * j + g) * OT_PITCH + c16 * 16);
+                    for (int j = 0; j < NROW; ++j) orow[j] = *(const u32x4*)(otile + ((64 / NROW) * j + orow0) * OTP + opiece * 16);
                 }
+                if constexpr (FULL) { if (i > warm) wait_vm_at_most<NROW>(); else wait_vm_at_most<0>(); }
                 lds_barrier();                                              // B2 (waits for the tile reads)
             }
             if constexpr (FULL) { if (nsteps > warm) store_rows(lastc); }
@@ -401,13 +471,13 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
     // Compute waves
     // =====================================================================================
     // ---- state: all key rows (permuted, see above), value columns 16w .. 16w+15, C/D layout ----
-    constexpr int NN = SMALL ? 1 : WIDE_NN;           // 16-column tiles per compute wave
+    constexpr int NN = SMALL || HALF ? 1 : WIDE_NN;           // 16-column tiles per compute wave
     f32x4 S[2 * KS][NN];
 #pragma unroll
     for (int m = 0; m < 2 * KS; ++m)
 #pragma unroll
     for (int nn = 0; nn < NN; ++nn) {
-        const int kk = 32 * (m >> 1) + 8 * g + 4 * (m & 1), vc = 16 * (NN * w + nn) + c16;
+        const int kk = 32 * (m >> 1) + 8 * g + 4 * (m & 1), vc = col0 + 16 * (NN * w + nn) + c16;
         f32x4 s = {0.f, 0.f, 0.f, 0.f};
         if (init == 1) {
 #pragma unroll
@@ -443,7 +513,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
 #pragma unroll
     for (int nn = 0; nn < NN; ++nn) {
         const int c = 2 * (NN * w + nn) + (tr_j >> 1);
-        v_tr[nn] = (g * 64 + 16 * (c >> 2) + 4 * tr_i + ((c + g) & 3)) * 8 + 4 * (tr_j & 1);
+        v_tr[nn] = (g * (HALF ? 32 : 64) + 16 * (c >> 2) + 4 * tr_i + ((c + g) & 3)) * 8 + 4 * (tr_j & 1);
     }
 
     // One step, written as a fixed sequence of small scheduling regions (the compiler may reorder
@@ -452,27 +522,30 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
     // window of three operand fragments), and the thin, dependent part of a step (D -> v_new ->
     // output of a pair of t-tiles) is cut into pieces that each share a region with four
     // independent matrix instructions (products of the next tiles, or the state update).
-    auto step = [&](const char* st, const char* kbuf, int p_target) {
+    auto step = [&](const char* kbuf, const char* qbuf, const char* vbuf, const char* rec, int p_target) {
         const V8* sK = (const V8*)kbuf;
-        const V8* sQ = (const V8*)(st + STG_Q);
-        const T* sV = (const T*)(st + STG_V);
+        const V8* sQ = (const V8*)qbuf;
+        const T* sV = (const T*)vbuf;
         const T* sKt = (const T*)kbuf;
-        const char* sX = st + STG_X;
-        const char* sP = st + STG_P;
-        const float* sTab = (const float*)(st + STG_TAB);
-        auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+        const char* sX = rec + REC_X;
+        const char* sP = rec + REC_P;
+        const float* sTab = (const float*)(rec + REC_TAB);
+        auto fence = [] { if constexpr (!HALF) __builtin_amdgcn_sched_barrier(0); };      // (HALF: the compiler's own order is 1 % faster)
 
         // fragment f = (t-tile f/4, key tiles (2s, 2s+1) with s = f%4) of k and q, in a ring of RING register sets
-        constexpr int RING = WIDE_RING;
+        constexpr int RING = HALF ? 6 : WIDE_RING;
         V8 ak[RING], aq[RING];
+        // (HALF: the t-tiles of a pair take turns, so that neighbouring matrix instructions do not wait for each other's sums)
+        auto tile_of = [](int f) { return HALF ? 2 * (f >> 3) + (f & 1) : f / KS; };
+        auto pair_of = [](int f) { return HALF ? (f & 7) >> 1 : f % KS; };
         auto F = [&](int f) {
-            ak[f % RING] = sK[(f / KS) * 256 + 16 * (f % KS) + a_off];
-            if constexpr (FULL) aq[f % RING] = sQ[(f / KS) * 256 + 16 * (f % KS) + a_off];
+            ak[f % RING] = sK[tile_of(f) * 256 + 16 * pair_of(f) + a_off];
+            if constexpr (FULL) aq[f % RING] = sQ[tile_of(f) * 256 + 16 * pair_of(f) + a_off];
         };
         f32x4 ks[4][NN], ao[4][NN];
         V8 Sb[KS][NN];
         auto M = [&](int f) {                   // (k S) and (q S)^T contributions of fragment f
-            const int tt = f / KS, sx = f % KS;
+            const int tt = tile_of(f), sx = pair_of(f);
 #pragma unroll
             for (int nn = 0; nn < NN; ++nn) {
                 ks[tt][nn] = Mma<T>::run(ak[f % RING], Sb[sx][nn], sx ? ks[tt][nn] : f32x4{0.f, 0.f, 0.f, 0.f});
@@ -483,7 +556,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         V8 ax[4][2], ap[4][2];                  // Xb and P fragments [t-tile][column pair]
         auto FV = [&](int tt) {
 #pragma unroll
-            for (int nn = 0; nn < NN; ++nn) vv[tt][nn] = Mma<T>::tr_read(sV + tt * 2048 + v_tr[nn]);
+            for (int nn = 0; nn < NN; ++nn) vv[tt][nn] = Mma<T>::tr_read(sV + tt * (HALF ? 1024 : 2048) + v_tr[nn]);
         };
         auto FX = [&](int tt) {
 #pragma unroll
@@ -552,7 +625,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
                     V4 o4;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) o4[r] = from_f32<T>(oacc[tt][nn][r]);
-                    *(V4*)(otile + (16 * tt + c16) * OT_PITCH + (16 * (NN * w + nn) + 4 * g) * 2) = o4;
+                    *(V4*)(otile + (16 * tt + c16) * OTP + (16 * (NN * w + nn) + 4 * g) * 2) = o4;
                 }
             }
         };
@@ -580,7 +653,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         fence();
         auto wait_P = [&]() {
             // P of this chunk: normally long there (the copy waves form it first thing in a step, at raised priority)
-            if constexpr (FULL) { while (*pcount < p_target) __builtin_amdgcn_s_sleep(1); }
+            if constexpr (FULL && !HALF) { while (*pcount < p_target) __builtin_amdgcn_s_sleep(1); }
         };
         auto fold = [&]() {                     // the decay fold: rare, a scalar branch so that it is not if-converted into the common path
             if (__builtin_amdgcn_readfirstlane((int)lazy) == 0) {
@@ -658,7 +731,10 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
     if (nsteps > 0) {
         lds_barrier();                                          // B0: the copy waves have filled stage 0
         for (int64_t i = 0; i < nsteps; ++i) {
-            step(smem + (i & 1) * STG_BYTES, smem + KBUF + (int)(i % 3) * 16384, 4 * ((int)i + 1));
+            const char* st = smem + (i & 1) * STG_BYTES;
+            const int b3 = (int)(i % 3);
+            if constexpr (HALF) step(smem + b3 * 16384, smem + HALF_Q + b3 * 16384, smem + HALF_V + b3 * HALF_V_BYTES, smem + HALF_REC + (int)(i & 1) * (HALF_NREC * 1024), 0);
+            else step(smem + KBUF + b3 * 16384, st + STG_Q, st + STG_V, st + STG_REC, 4 * ((int)i + 1));
         }
     }
 
@@ -677,7 +753,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         for (int m = 0; m < 2 * KS; ++m)
 #pragma unroll
         for (int nn = 0; nn < NN; ++nn) {
-            const int kk = 32 * (m >> 1) + 8 * g + 4 * (m & 1), vc = 16 * (NN * w + nn) + c16;
+            const int kk = 32 * (m >> 1) + 8 * g + 4 * (m & 1), vc = col0 + 16 * (NN * w + nn) + c16;
             const f32x4 s = S[m][nn] * gamma;
             const int sk = dst_user ? (vfirst ? 1 : V) : 128, sv = dst_user ? (vfirst ? K : 1) : 1;
             if (kk < (dst_user ? K : 128) && vc < (dst_user ? V : 128)) {
@@ -769,13 +845,13 @@ __global__ __launch_bounds__(256) void gdn_segment_merge_kernel(SegmentPlan sp, 
     }
 }
 
-template <typename T, bool FULL, bool DIMS128, bool SMALL>
+template <typename T, bool FULL, bool DIMS128, bool SMALL, bool HALF = false>
 static int launch_wide_dims(const ChunkParams& p, const SegmentPlan& sp, int64_t blocks, hipStream_t stream) {
-    auto kern = gdn_chunk_wide_kernel<T, FULL, DIMS128, SMALL>;
+    auto kern = gdn_chunk_wide_kernel<T, FULL, DIMS128, SMALL, HALF>;
     static SmemAttrDone attr_done;       // per instantiation
-    if (int rc = ensure_dynamic_smem((const void*)kern, WIDE_SMEM, attr_done, "hipFuncSetAttribute(wide)")) return rc;
+    if (int rc = ensure_dynamic_smem((const void*)kern, HALF ? HALF_SMEM : WIDE_SMEM, attr_done, "hipFuncSetAttribute(wide)")) return rc;
     if (blocks <= 0) return GDN_OK;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(WIDE_THREADS), WIDE_SMEM, stream, p, sp);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(WIDE_THREADS), HALF ? HALF_SMEM : WIDE_SMEM, stream, p, sp);
     return check_launch("gdn_chunk_wide_kernel");
 }
 
@@ -795,6 +871,7 @@ int launch_wide(const ChunkParams& p, SegmentPlan sp, hipStream_t stream) {
     if (sp.kind == WIDE_WHOLE) {
         sp.nseg = 1;
         sp.seg_chunks = 1 << 30;
+        if (p.halves) return launch_wide_dims<T, true, true, false, true>(p, sp, (p.N * p.H + 7) / 8 * 8 * G * 2, stream);
         return launch_wide_kind<T, true>(p, sp, (p.N * p.H + 7) / 8 * 8 * G, stream);
     }
     return launch_wide_kind<T, true>(p, sp, (p.N * p.H * sp.nseg + 7) / 8 * 8 * G, stream);
