@@ -53,7 +53,7 @@ constexpr int PCOUNT_OFF = KBUF + 3 * 16384 + OT_BYTES;       // one counter: P 
 constexpr size_t WIDE_SMEM = PCOUNT_OFF + 16;                // 156 688 B of the CU's 163 840: one workgroup per CU
 constexpr int WIDE_NN = 2;                        // 16-column tiles per compute wave
 #ifndef WIDE_XB
-#define WIDE_XB 8
+#define WIDE_XB 6
 #endif
 #ifndef WIDE_RING
 #define WIDE_RING 3                               // operand fragments in flight per compute wave
