@@ -1,7 +1,8 @@
 // The operators' host path as native code (a CPython extension over libtorch): argument checks, output and workspace allocation and
 // the call into libgdn_hip.so for the calls that need no conversion of any kind - every tensor contiguous, aligned, on the current
 // device and of a type and shape the kernels take as it is.  Every function returns None for anything else (wrong arguments
-// included) and changes nothing then: the Python path behind it converts, pads or raises.
+// included) and changes nothing then: the Python path behind it converts, pads or raises.  What fails inside (no memory left, a library
+// call refused) leaves as a Python exception of the type torch itself would raise: every entry is a body in torch's own translation.
 //
 // A call through Python and ctypes took 25 us of host time (decode step) to 60 us (prefill), more than the kernels of a small call.
 #include <Python.h>
@@ -9,7 +10,7 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/core/DeviceGuard.h>
-#include <pybind11/pybind11.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -38,6 +39,7 @@ decltype(&gdn_sum_rows) p_sum_rows;
 decltype(&gdn_last_error) p_last_error;
 
 PyObject* bind(PyObject*, PyObject* table) {
+    HANDLE_TH_ERRORS
     auto take = [&](const char* name, auto& fn) {
         PyObject* at = PyDict_GetItemString(table, name);
         if (!at) { PyErr_Format(PyExc_KeyError, "gdn_host.bind: no address of %s", name); return false; }
@@ -52,16 +54,34 @@ PyObject* bind(PyObject*, PyObject* table) {
         !take("gdn_sum_rows", p_sum_rows) || !take("gdn_last_error", p_last_error))
         return nullptr;
     Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
 }
 
+// The interpreter runs other threads while this lives (exceptions on their way out take it back).
+struct NoGil {
+    PyThreadState* state = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(state); }
+    NoGil() = default;
+    NoGil(const NoGil&) = delete;
+    NoGil& operator=(const NoGil&) = delete;
+};
+
 // ---- arguments ----
+// Strided memory behind it: not the tensors of tracing, vmap and the other transforms, of subclasses with a dispatch of their own, and
+// none that is sparse, nested or to be negated when it is read (the Python path says what becomes of those).
+bool has_memory(const at::Tensor& t) {
+    return t.layout() == at::kStrided && !t.is_neg() && !t.is_nested() && t.has_storage() &&
+           !t.key_set().has_any(c10::DispatchKeySet{c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                                    c10::DispatchKey::Functionalize, c10::DispatchKey::ZeroTensor});
+}
+
 // A tensor argument: absent (None), present, or something else.
 struct Arg {
     const at::Tensor* t = nullptr;
     bool bad = false;
     explicit Arg(PyObject* o) {
         if (o == Py_None) return;
-        if (THPVariable_Check(o)) t = &THPVariable_Unpack(o);
+        if (THPVariable_Check(o) && has_memory(THPVariable_Unpack(o))) t = &THPVariable_Unpack(o);
         else bad = true;
     }
     explicit operator bool() const { return t != nullptr; }
@@ -78,7 +98,7 @@ int code_of(at::ScalarType s) {
     }
 }
 
-bool plain(const Arg& a, c10::Device dev) { return !a.bad && (!a || (a->device() == dev && a->is_contiguous() && a->layout() == at::kStrided)); }
+bool plain(const Arg& a, c10::Device dev) { return !a.bad && (!a || (a->device() == dev && a->is_contiguous())); }
 bool aligned16(const void* p) { return (uintptr_t)p % 16 == 0; }
 bool truth(PyObject* o) { return PyObject_IsTrue(o) == 1; }
 
@@ -131,6 +151,7 @@ PyObject* pair(const at::Tensor& a, const at::Tensor& b) {
 //  cu_seqlens, inplace_final_state, state_slots, kda_gate_mode, lower_bound); gk: the KDA operator's gate (kda_gate_mode 0 .. 2) or
 // the general operator's log decays per key feature (kda_gate_mode None)
 PyObject* fused_recurrent(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     if (n != 20) { PyErr_SetString(PyExc_TypeError, "gdn_host.fused_recurrent takes 20 arguments"); return nullptr; }
     const Arg q(a[0]), k(a[1]), v(a[2]), g(a[3]), gk(a[4]), beta(a[5]), A_log(a[6]), dt_bias(a[7]), h0(a[9]), cu(a[15]), slots(a[17]);
     const bool out_final = truth(a[10]), bsig = truth(a[12]), neg = truth(a[13]), vfirst = truth(a[14]), inplace = truth(a[16]);
@@ -183,18 +204,20 @@ PyObject* fused_recurrent(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void* stream = stream_of(d.dev);
     float* pht = ht.defined() ? (float*)ht.data_ptr() : nullptr;
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    if (kda)
-        rc = p_fused_recurrent_kda_fwd(q.ptr(), k.ptr(), v.ptr(), (const float*)gk.ptr(), beta.ptr(), (const float*)A_log.ptr(), (const float*)dt_bias.ptr(),
-                                       lower, mode, (const float*)h0.ptr(), pht, o.data_ptr(), cu.ptr(), slots.ptr(), nullptr, 1,
+    {
+        const NoGil free;
+        if (kda)
+            rc = p_fused_recurrent_kda_fwd(q.ptr(), k.ptr(), v.ptr(), (const float*)gk.ptr(), beta.ptr(), (const float*)A_log.ptr(), (const float*)dt_bias.ptr(),
+                                           lower, mode, (const float*)h0.ptr(), pht, o.data_ptr(), cu.ptr(), slots.ptr(), nullptr, 1,
+                                           d.B, d.T, d.H, d.HV, d.K, d.V, N, scale, d.code, gb, flags, stream);
+        else
+            rc = p_fused_recurrent_fwd(q.ptr(), k.ptr(), v.ptr(), g.ptr(), beta.ptr(), (const float*)gk.ptr(), nullptr, (const float*)A_log.ptr(),
+                                       (const float*)dt_bias.ptr(), (const float*)h0.ptr(), pht, o.data_ptr(), cu.ptr(), slots.ptr(), nullptr, 1,
                                        d.B, d.T, d.H, d.HV, d.K, d.V, N, scale, d.code, gb, flags, stream);
-    else
-        rc = p_fused_recurrent_fwd(q.ptr(), k.ptr(), v.ptr(), g.ptr(), beta.ptr(), (const float*)gk.ptr(), nullptr, (const float*)A_log.ptr(),
-                                   (const float*)dt_bias.ptr(), (const float*)h0.ptr(), pht, o.data_ptr(), cu.ptr(), slots.ptr(), nullptr, 1,
-                                   d.B, d.T, d.H, d.HV, d.K, d.V, N, scale, d.code, gb, flags, stream);
-    Py_END_ALLOW_THREADS
+    }
     if (rc != GDN_OK) Py_RETURN_NONE;               // (refused before any launch: the Python path raises)
     return pair(o, ht);
+    END_HANDLE_TH_ERRORS
 }
 
 // ---- chunked forward ----
@@ -239,6 +262,7 @@ bool chunk_args(PyObject* const* a, ChunkArgs& x) {
     return true;
 }
 PyObject* chunk_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     if (n != 15) { PyErr_SetString(PyExc_TypeError, "gdn_host.chunk_fwd takes 15 arguments"); return nullptr; }
     ChunkArgs x;
     if (!chunk_args(a, x)) { if (PyErr_Occurred()) return nullptr; Py_RETURN_NONE; }
@@ -251,13 +275,15 @@ PyObject* chunk_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const at::Tensor ws = empty_on(d.dev, at::kByte, {(int64_t)ws_bytes});
     void* stream = stream_of(d.dev);
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = p_chunk_fwd(x.q.ptr(), x.k.ptr(), x.v.ptr(), x.g.ptr(), x.beta.ptr(), (const float*)x.A_log.ptr(), (const float*)x.dt_bias.ptr(), (const float*)x.h0.ptr(),
-                     ht.defined() ? (float*)ht.data_ptr() : nullptr, o.data_ptr(), x.cu.ptr(), x.table.ptr(), x.offsets.ptr(), ws.data_ptr(), ws_bytes,
-                     d.B, d.T, d.H, d.HV, d.K, d.V, x.N, x.num_chunks, x.scale, d.code, x.gb, x.flags, stream);
-    Py_END_ALLOW_THREADS
+    {
+        const NoGil free;
+        rc = p_chunk_fwd(x.q.ptr(), x.k.ptr(), x.v.ptr(), x.g.ptr(), x.beta.ptr(), (const float*)x.A_log.ptr(), (const float*)x.dt_bias.ptr(), (const float*)x.h0.ptr(),
+                         ht.defined() ? (float*)ht.data_ptr() : nullptr, o.data_ptr(), x.cu.ptr(), x.table.ptr(), x.offsets.ptr(), ws.data_ptr(), ws_bytes,
+                         d.B, d.T, d.H, d.HV, d.K, d.V, x.N, x.num_chunks, x.scale, d.code, x.gb, x.flags, stream);
+    }
     if (rc != GDN_OK) Py_RETURN_NONE;
     return pair(o, ht);
+    END_HANDLE_TH_ERRORS
 }
 
 // ---- one decode step of the layer ----
@@ -266,6 +292,7 @@ PyObject* chunk_fwd(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // with the convolutions' update and the gate's and beta's activations, the recurrence on the state where it is, the gated norm, the
 // output projection.  The states are updated in place.
 PyObject* layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     if (n != 18) { PyErr_SetString(PyExc_TypeError, "gdn_host.layer_step takes 18 arguments"); return nullptr; }
     const Arg x(a[0]), qw(a[1]), kw(a[2]), vw(a[3]), aw(a[4]), bw(a[5]), gw(a[6]), ow(a[7]), A_log(a[8]), dt_bias(a[9]), state(a[13]), norm_w(a[14]);
     if (!x || !x->is_cuda() || x->dim() != 3 || x->size(1) != 1) Py_RETURN_NONE;
@@ -320,19 +347,21 @@ PyObject* layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
     last.weight = ow.ptr(); last.cols = out_cols; last.out = out.data_ptr(); last.kind = GDN_STEP_PLAIN;
     void* stream = stream_of(dev);
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = p_step_linear(x.ptr(), N, hidden, seg, 6, code, stream);
-    if (rc == GDN_OK)
-        rc = p_fused_recurrent_fwd(base + o_q, base + o_k, base + o_v, base + o_g, base + o_b, nullptr, nullptr, nullptr, nullptr, (const float*)state.ptr(),
-                                   (float*)state.ptr(), base + o_o, nullptr, nullptr, nullptr, 1, N, 1, H, HV, K, V, N, (float)std::pow((double)K, -0.5), code,
-                                   GDN_DTYPE_F32, GDN_FLAG_QK_L2NORM | GDN_FLAG_STATE_V_FIRST, stream);
-    if (rc == GDN_OK)
-        rc = p_norm_gated_fwd(base + o_o, base + o_gate, norm_w.ptr(), nullptr, nullptr, base + o_y, nullptr, nullptr, nullptr, N * HV, V, eps, code, norm_code,
-                              GDN_DTYPE_F32, GDN_DTYPE_F32, GDN_ACT_SILU, 1, stream);
-    if (rc == GDN_OK) rc = p_step_linear(base + o_y, N, vd, &last, 1, code, stream);
-    Py_END_ALLOW_THREADS
+    {
+        const NoGil free;
+        rc = p_step_linear(x.ptr(), N, hidden, seg, 6, code, stream);
+        if (rc == GDN_OK)
+            rc = p_fused_recurrent_fwd(base + o_q, base + o_k, base + o_v, base + o_g, base + o_b, nullptr, nullptr, nullptr, nullptr, (const float*)state.ptr(),
+                                       (float*)state.ptr(), base + o_o, nullptr, nullptr, nullptr, 1, N, 1, H, HV, K, V, N, (float)std::pow((double)K, -0.5), code,
+                                       GDN_DTYPE_F32, GDN_FLAG_QK_L2NORM | GDN_FLAG_STATE_V_FIRST, stream);
+        if (rc == GDN_OK)
+            rc = p_norm_gated_fwd(base + o_o, base + o_gate, norm_w.ptr(), nullptr, nullptr, base + o_y, nullptr, nullptr, nullptr, N * HV, V, eps, code, norm_code,
+                                  GDN_DTYPE_F32, GDN_DTYPE_F32, GDN_ACT_SILU, 1, stream);
+        if (rc == GDN_OK) rc = p_step_linear(base + o_y, N, vd, &last, 1, code, stream);
+    }
     if (rc != GDN_OK) { PyErr_Format(PyExc_RuntimeError, "gdn_host.layer_step: status %d", rc); return nullptr; }
     return THPVariable_Wrap(out);
+    END_HANDLE_TH_ERRORS
 }
 
 #include "gdn_host_train.h"

@@ -6,7 +6,11 @@ using torch::autograd::Variable;
 using torch::autograd::variable_list;
 
 void check_rc(int rc, const char* what) {
-    TORCH_CHECK(rc == GDN_OK, what, ": libgdn_hip status ", rc, ": ", p_last_error ? p_last_error() : "");
+    if (rc == GDN_OK) return;
+    const char* why = p_last_error ? p_last_error() : "";            // (types as _lib.check gives them)
+    TORCH_CHECK_VALUE(rc != GDN_ERR_INVALID, what, ": ", why);
+    TORCH_CHECK_NOT_IMPLEMENTED(rc != GDN_ERR_UNSUPPORTED, what, ": ", why);
+    TORCH_CHECK(false, what, ": libgdn_hip status ", rc, ": ", why);
 }
 template <typename T = void>
 T* ptr_of(const at::Tensor& t) { return t.defined() ? (T*)t.data_ptr() : nullptr; }
@@ -131,6 +135,7 @@ struct ChunkTrain : torch::autograd::Function<ChunkTrain> {
 // (q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens, chunk_indices, scan_tables, A_log, dt_bias,
 //  flags, whole); as chunk_fwd, for calls that need gradients.  None: not a call for the native path
 PyObject* chunk_train(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     if (n != 16) { PyErr_SetString(PyExc_TypeError, "gdn_host.chunk_train takes 16 arguments"); return nullptr; }
     ChunkArgs x;
     if (!chunk_args(a, x)) { if (PyErr_Occurred()) return nullptr; Py_RETURN_NONE; }
@@ -139,11 +144,12 @@ PyObject* chunk_train(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const ChunkCall c{d.B, d.T, d.H, d.HV, d.K, d.V, x.N, x.num_chunks, x.scale, x.flags, truth(a[7]), truth(a[8]), truth(a[15])};
     auto var = [](const Arg& t) { return t ? ChunkTrain::Maybe(*t.t) : ChunkTrain::Maybe(); };
     variable_list r;
-    try {
-        pybind11::gil_scoped_release no_gil;
+    {
+        const NoGil free;
         r = ChunkTrain::apply(*x.q.t, *x.k.t, *x.v.t, var(x.g), *x.beta.t, var(x.h0), var(x.A_log), var(x.dt_bias), var(x.cu), var(x.table), var(x.offsets), c);
-    } catch (const std::exception& e) { PyErr_SetString(PyExc_RuntimeError, e.what()); return nullptr; }
+    }
     return pair(r[0], r.size() > 1 ? r[1] : at::Tensor());
+    END_HANDLE_TH_ERRORS
 }
 
 // ---- the layer ----
@@ -275,6 +281,7 @@ struct LayerTrain : torch::autograd::Function<LayerTrain> {
 // (x, q, k, v, a, b, g, o weights, (q, k, v conv weights [D,1,W]), A_log, dt_bias, norm weight, norm eps, neg_eigval, num_heads): the
 // layer's forward on whole dense sequences without a cache.  None: not a call for the native path
 PyObject* layer_train(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
     if (n != 15) { PyErr_SetString(PyExc_TypeError, "gdn_host.layer_train takes 15 arguments"); return nullptr; }
     variable_list in(LayerTrain::INPUTS);
     if (!PyTuple_Check(a[8]) || PyTuple_GET_SIZE(a[8]) != 3) Py_RETURN_NONE;
@@ -309,9 +316,10 @@ PyObject* layer_train(PyObject*, PyObject* const* a, Py_ssize_t n) {
         nw.dim() != 1 || nw.numel() != V || code_of(nw.scalar_type()) < 0)
         Py_RETURN_NONE;
     variable_list r;
-    try {
-        pybind11::gil_scoped_release no_gil;
+    {
+        const NoGil free;
         r = LayerTrain::apply(at::TensorList(in), heads, truth(a[13]), eps);
-    } catch (const std::exception& e) { PyErr_SetString(PyExc_RuntimeError, e.what()); return nullptr; }
+    }
     return THPVariable_Wrap(r[0]);
+    END_HANDLE_TH_ERRORS
 }
