@@ -52,9 +52,6 @@ constexpr int OT_BYTES = 64 * OT_PITCH;           // 17 408 B
 constexpr int PCOUNT_OFF = KBUF + 3 * 16384 + OT_BYTES;       // one counter: P fragments published so far
 constexpr size_t WIDE_SMEM = PCOUNT_OFF + 16;                // 156 688 B of the CU's 163 840: one workgroup per CU
 constexpr int WIDE_NN = 2;                        // 16-column tiles per compute wave
-#ifndef WIDE_XB
-#define WIDE_XB 6
-#endif
 #ifndef WIDE_RING
 #define WIDE_RING 3                               // operand fragments in flight per compute wave
 #endif
@@ -319,6 +316,15 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
                     else gather_1k_to_lds(rec + j * 1024, lane * 16, lds_stage + STG_REC + j * 1024);
                 }
         };
+        // The records of a full run: copied by the output wave, or, where REC_Q, by q's.  In the 64 x 64 form a step is short and the
+        // output wave, with its share of P and the stores, has no room left for them: 8 x 1024 tokens, 8 heads 46.2 us there, 42.9 us on
+        // q's wave; 20000 packed tokens, 32 heads 154.0 and 149.9 us.
+        constexpr bool REC_Q = FULL && SMALL;
+        auto copy_records = [&](int64_t it, uint32_t st) {
+            copy_rec(it, 0, REC_PIECES_X, st);
+            copy_rec(it, REC_PIECE_TAB, REC_PIECE_TAB + 1, st);
+            copy_rec(it, REC_PIECE_TAB2, REC_PIECE_TAB2 + 1, st, it - it0 < warm);
+        };
         // HALF: k, q and v a wave each, the copy of chunk i+2 issued at the start of step i (its buffer was last read in step i-1) and
         // awaited at the end of step i+1
         if (HALF && w < CW + 3) {
@@ -371,15 +377,17 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
             // ---- q (state-only runs: Xb and the first table) (wave CW+1) and v (wave CW+2).  Pieces
             // [0, XB) of chunk c are issued in phase B of step c-2, the rest in phase A of step c-1.
             const bool qside = (w == CW + 1);
-            constexpr int XB = WIDE_XB;
+            // (128 x 128, 6 against 8: 32768 tokens with 32 slowly forgetting heads 565 -> 555 us, 9000 tokens with 8 heads 86.3 -> 84.8, dense
+            // and packed whole runs of 32 heads 0.4 % less, 16000 tokens in 9 packed sequences 212.5 -> 215 us.  64 x 64: 8, with the records.)
+            constexpr int XB = SMALL ? 8 : 6;
             auto issue = [&](int64_t it, int stage, bool early) {
                 const uint32_t st = lds0 + stage * STG_BYTES;
                 const bool warming = it - it0 < warm;               // a chunk of the warm-up: no output, so neither q nor P
                 if (qside) {
                     if constexpr (FULL) {
-                        // 16 q pieces (the output wave copies the records)
+                        // 16 q pieces (and, where REC_Q, the records)
                         if (early) gather_blocks((const T*)p.q, it, 0, XB, st + STG_Q, warming);
-                        else gather_blocks((const T*)p.q, it, XB, 16, st + STG_Q, warming);
+                        else { gather_blocks((const T*)p.q, it, XB, 16, st + STG_Q, warming); if constexpr (REC_Q) copy_records(it, st); }
                     } else {
                         if (early) { copy_rec(it, 0, REC_PIECES_X, st); copy_rec(it, REC_PIECE_TAB, REC_PIECE_TAB + 1, st); }      // all 6 pieces
                     }
@@ -419,12 +427,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
             constexpr int NREC = HALF ? HALF_NREC : REC_PIECES_X + 2, NROW = HALF ? 8 : 16;     // record pieces; store instructions per tile
             auto issue_rec = [&](int64_t it, int stage) {
                 if constexpr (HALF) copy_rec(it, 0, NREC, lds0 + HALF_REC - STG_REC + stage * (HALF_NREC * 1024));
-                else {
-                    const uint32_t st = lds0 + stage * STG_BYTES;
-                    copy_rec(it, 0, REC_PIECES_X, st);
-                    copy_rec(it, REC_PIECE_TAB, REC_PIECE_TAB + 1, st);
-                    copy_rec(it, REC_PIECE_TAB2, REC_PIECE_TAB2 + 1, st, it - it0 < warm);
-                }
+                else copy_records(it, lds0 + stage * STG_BYTES);
             };
             const int orow0 = HALF ? lane >> 3 : g, opiece = HALF ? lane & 7 : c16;
             T* og = (T*)p.o;
@@ -441,7 +444,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
                     dstp += stride;
                 }
             };
-            if constexpr (FULL) {
+            if constexpr (FULL && !REC_Q) {
                 issue_rec(it0, 0);
                 wait_vm_at_most<0>();
             }
@@ -449,16 +452,14 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
             for (int64_t i = 0; i < nsteps; ++i) {
                 if (i >= warm) produce_P(smem + (i & 1) * STG_BYTES, smem + KBUF + (int)(i % 3) * 16384);
                 announce_P();
-                if constexpr (FULL) {
-                    issue_rec(min(it0 + i + 1, lastc), (int)(i & 1) ^ 1);
-                    if (i > warm) store_rows(it0 + i - 1);
-                }
+                if constexpr (FULL && !REC_Q) issue_rec(min(it0 + i + 1, lastc), (int)(i & 1) ^ 1);
+                if constexpr (FULL) { if (i > warm) store_rows(it0 + i - 1); }
                 lds_barrier();                                              // B1
                 if constexpr (FULL) {
 #pragma unroll
                     for (int j = 0; j < NROW; ++j) orow[j] = *(const u32x4*)(otile + ((64 / NROW) * j + orow0) * OTP + opiece * 16);
                 }
-                if constexpr (FULL) { if (i > warm) wait_vm_at_most<NROW>(); else wait_vm_at_most<0>(); }
+                if constexpr (FULL && !REC_Q) { if (i > warm) wait_vm_at_most<NROW>(); else wait_vm_at_most<0>(); }
                 lds_barrier();                                              // B2 (waits for the tile reads)
             }
             if constexpr (FULL) { if (nsteps > warm) store_rows(lastc); }
