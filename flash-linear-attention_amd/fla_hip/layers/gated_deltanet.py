@@ -21,6 +21,8 @@ import warnings
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import _has_any_global_hook
+from torch.utils._device import DeviceContext
 
 from fla_hip import _lib
 from fla_hip.modules import FusedRMSNormGated, ShortConvolution
@@ -31,8 +33,25 @@ _STEP_LINEARS = ('q_proj', 'k_proj', 'v_proj', 'a_proj', 'b_proj', 'g_proj', 'o_
 _STEP_CONVS = ('q_conv1d', 'k_conv1d', 'v_conv1d')
 
 
-def _hooked(m: nn.Module) -> bool:
-    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+# The calls that the native paths stand for.  Where a caller has replaced one of them - on the class, on a module, around every
+# module - the layer runs module by module and makes it.
+_FORWARDS = {nn.Linear: nn.Linear.forward, ShortConvolution: ShortConvolution.forward, FusedRMSNormGated: FusedRMSNormGated.forward}
+_AROUND = (nn.Module.__call__, F.linear, ShortConvolution.step)
+
+
+def _own_call(m: nn.Module, cls: type) -> bool:
+    """Whether calling ``m`` is ``cls.forward`` and nothing else: no other class, no other ``forward``, no hooks, not compiled."""
+    d = m.__dict__
+    return (type(m) is cls and cls.forward is _FORWARDS[cls] and 'forward' not in d and 'step' not in d and d.get('_compiled_call_impl') is None
+            and not (d['_forward_hooks'] or d['_forward_pre_hooks'] or d['_backward_hooks'] or d['_backward_pre_hooks']))
+
+
+def _watched() -> bool:
+    """Whether something looks at, or stands in for, the calls between the layer's modules: hooks on all modules, torch's dispatch and
+    function modes (a default device is none of those), a patched ``nn.Module.__call__`` or ``F.linear``."""
+    n = torch._C._len_torch_function_stack()
+    return (_has_any_global_hook() or torch._C._len_torch_dispatch_stack() > 0 or (nn.Module.__call__, F.linear, ShortConvolution.step) != _AROUND
+            or (n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n))))
 
 
 class LayerCache:
@@ -149,20 +168,20 @@ class GatedDeltaNet(nn.Module):
 
     def _plain(self):
         """(weights of the projections, the convolutions and the norm; the convolutions; the norm) where the layer is its plain self, or
-        None: another module in a projection's place, hooks, autocast."""
-        if not (self.use_gate and self.use_short_conv) or torch.is_autocast_enabled():
+        None: another module in a projection's place or another forward in a module's, hooks, modes, autocast."""
+        if not (self.use_gate and self.use_short_conv) or torch.is_autocast_enabled() or _watched():
             return None
         mods = self._modules
         linears = [mods[n] for n in _STEP_LINEARS]
         convs = [mods[n] for n in _STEP_CONVS]
         norm = mods['o_norm']
         for m in linears:
-            if type(m) is not nn.Linear or m.bias is not None or _hooked(m):
+            if not _own_call(m, nn.Linear) or m.bias is not None:
                 return None
         for m in convs:
-            if type(m) is not ShortConvolution or m.activation is None or _hooked(m):
+            if not _own_call(m, ShortConvolution) or m.activation is None:
                 return None
-        if type(norm) is not FusedRMSNormGated or norm.activation == 'sigmoid' or _hooked(norm):
+        if not _own_call(norm, FusedRMSNormGated) or norm.activation == 'sigmoid':
             return None
         weights = [m._parameters.get('weight') for m in (*linears, *convs, norm)]
         return None if any(type(w) is not nn.Parameter for w in weights) else (weights, convs, norm)
@@ -178,7 +197,7 @@ class GatedDeltaNet(nn.Module):
 
     def _step(self, hidden_states, past_key_values):
         """One token per sequence on a filled cache through the native host path (``gdn_host.layer_step``: four launches), or None
-        where the layer is not its plain self - another module in a projection's place, hooks, autocast, a state to be converted."""
+        where the layer is not its plain self (``_plain``) or a state has to be converted."""
         if past_key_values is None or len(past_key_values) <= self.layer_idx:
             return None
         entry = past_key_values[self.layer_idx]
