@@ -16,6 +16,7 @@ In eval mode no autograd graph is built (the token recurrence of decode has no b
 from __future__ import annotations
 
 import math
+import os
 import warnings
 
 import torch
@@ -26,6 +27,7 @@ from torch.utils._device import DeviceContext
 
 from fla_hip import _lib
 from fla_hip.modules import FusedRMSNormGated, ShortConvolution
+from fla_hip.ops.backends import has_backends
 from fla_hip.ops.gated_delta_rule import chunk_gated_delta_rule, fused_recurrent_gated_delta_rule
 
 
@@ -187,12 +189,15 @@ class GatedDeltaNet(nn.Module):
         return None if any(type(w) is not nn.Parameter for w in weights) else (weights, convs, norm)
 
     def _train(self, hidden_states):
-        """Whole dense sequences without a cache through the native training path (``gdn_host.layer_train``), or None."""
+        """Whole dense sequences without a cache through the native training path (``gdn_host.layer_train``), or None (a backend is
+        registered for the operator, or a form of its scans is asked for, too)."""
+        if has_backends('gated_delta_rule') or os.environ.get('FLA_HIP_SCAN_MODE') or os.environ.get('FLA_HIP_BWD_SCAN_MODE'):
+            return None
         plain = self._plain()
         if plain is None or any(m._parameters.get('bias') is not None for m in plain[1]):
             return None
         w, _, norm = plain
-        return _lib.host().layer_train(hidden_states, *w[:7], tuple(w[7:10]), self._parameters['A_log'], self._parameters['dt_bias'], w[10], norm.eps,
+        return _lib.host().layer_train(hidden_states, *w[:7], tuple(w[7:10]), self._parameters.get('A_log'), self._parameters.get('dt_bias'), w[10], norm.eps,
                                        self.allow_neg_eigval, self.num_heads)
 
     def _step(self, hidden_states, past_key_values):
@@ -209,7 +214,7 @@ class GatedDeltaNet(nn.Module):
             return None
         weights, convs, norm = plain
         o = _lib.host().layer_step(
-            hidden_states, *weights[:7], self._parameters['A_log'], self._parameters['dt_bias'], tuple(weights[7:10]),
+            hidden_states, *weights[:7], self._parameters.get('A_log'), self._parameters.get('dt_bias'), tuple(weights[7:10]),
             tuple(m._parameters['bias'] for m in convs), tuple(conv), state, weights[10], norm.eps, self.allow_neg_eigval, self.num_heads)
         if o is not None:
             past_key_values.update(layer_idx=self.layer_idx, recurrent_state=state, conv_state=conv, offset=1)

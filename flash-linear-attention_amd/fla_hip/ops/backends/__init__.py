@@ -113,6 +113,15 @@ class BackendRegistry:
             cls._initialized.add(operation)
 
 
+def has_backends(operation: str) -> bool:
+    """Whether ``@dispatch(operation)`` has a backend to offer a call to (paths that do not go through the decorated function ask)."""
+    if _DISPATCH_DISABLED:
+        return False
+    BackendRegistry.ensure_initialized(operation)
+    registry = BackendRegistry._registries.get(operation)
+    return registry is not None and bool(registry._backends)
+
+
 def dispatch(operation: str) -> Callable[[Callable], Callable]:
     def decorator(func: Callable) -> Callable:
         if _DISPATCH_DISABLED:
@@ -151,4 +160,4 @@ def dispatch(operation: str) -> Callable[[Callable], Callable]:
     return decorator
 
 
-__all__ = ['BackendRegistry', 'BaseBackend', 'dispatch']
+__all__ = ['BackendRegistry', 'BaseBackend', 'dispatch', 'has_backends']

@@ -11,6 +11,7 @@ from torch.overrides import TorchFunctionMode
 from fla_hip import _lib
 from fla_hip.layers import GatedDeltaNet
 from fla_hip.layers.gated_deltanet import LayerCache
+from fla_hip.ops.backends import BackendRegistry, BaseBackend
 
 
 class _Host:
@@ -95,3 +96,24 @@ def test_a_replaced_call_is_made(layer, monkeypatch, change):
 def test_a_default_device_changes_nothing(layer):
     with torch.device('cpu'):
         assert paths(layer) == ('native', 'native')
+
+
+@pytest.mark.parametrize('variable', ['FLA_HIP_SCAN_MODE', 'FLA_HIP_BWD_SCAN_MODE'])
+def test_forms_of_the_scans_reach_the_operator(layer, monkeypatch, variable):
+    monkeypatch.setenv(variable, 'wide')
+    assert paths(layer) == (None, 'native')
+
+
+def test_a_backend_of_the_operator_is_asked_in_training(layer, monkeypatch):
+    monkeypatch.setattr(BackendRegistry, '_registries', dict(BackendRegistry._registries))
+    registry = BackendRegistry('gated_delta_rule')
+    registry.register(type('Other', (BaseBackend,), dict(backend_type='other'))())
+    assert paths(layer) == (None, 'native')
+
+
+def test_a_parametrised_gate_goes_through_its_modules(layer, monkeypatch):
+    torch.nn.utils.parametrize.register_parametrization(layer, 'A_log', nn.Identity())
+    seen = []
+    monkeypatch.setattr(_Host, 'layer_train', lambda self, *a: seen.append(a[9]))
+    layer._train(torch.zeros(1, 8, 64))
+    assert seen == [None]
