@@ -17,8 +17,8 @@ from fla_hip.ops.gated_delta_rule._common import (
     aligned16,
     check_operand_shapes,
     as_f32,
-    current_stream_ptr,
     dtype_code,
+    launch,
     ptr,
     require_gpu,
 )
@@ -99,11 +99,10 @@ def chunk_comba_fwd(q, k, v, p, g, beta, scale, initial_state, output_final_stat
     lib = _lib.load()
     ws_bytes = lib.gdn_chunk_kda_workspace_bytes(num_chunks, HV)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    _lib.check(lib.gdn_chunk_comba_fwd(
-        ptr(qw), ptr(kw), ptr(vw), ptr(pw), ptr(gw), ptr(bw), ptr(h0), ptr(ht), ptr(o),
+    launch(
+        lib.gdn_chunk_comba_fwd, dev, ptr(qw), ptr(kw), ptr(vw), ptr(pw), ptr(gw), ptr(bw), ptr(h0), ptr(ht), ptr(o),
         ptr(cu_seqlens), ptr(chunk_table), ptr(chunk_offsets), ptr(workspace), ws_bytes,
-        B, T, H, HV, _DIM, _DIM, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags,
-        current_stream_ptr(dev)))
+        B, T, H, HV, _DIM, _DIM, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags)
     o = o[..., :V].to(out_dtype)
     if ht is not None:
         ht = ht[..., :K, :V].contiguous()
@@ -194,12 +193,11 @@ def chunk_comba_bwd(q, k, v, p, g, beta, scale, initial_state, do, dht, cu_seqle
     lib = _lib.load()
     ws_bytes = lib.gdn_chunk_comba_bwd_qk_l2norm_workspace_bytes(num_chunks, HV, B * T) if inside else lib.gdn_chunk_bwd_workspace_bytes(num_chunks, HV, _DIM)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    _lib.check((lib.gdn_chunk_comba_bwd_qk_l2norm if inside else lib.gdn_chunk_comba_bwd)(
-        ptr(qw), ptr(kw), ptr(pw), ptr(vw), ptr(gw), ptr(bw), ptr(h0), ptr(dow), ptr(dhtw),
+    launch(
+        lib.gdn_chunk_comba_bwd_qk_l2norm if inside else lib.gdn_chunk_comba_bwd, dev, ptr(qw), ptr(kw), ptr(pw), ptr(vw), ptr(gw), ptr(bw), ptr(h0), ptr(dow), ptr(dhtw),
         ptr(dq), ptr(dk), ptr(dp), ptr(dv), ptr(dg), ptr(db), ptr(dh0),
         ptr(cu_seqlens), ptr(chunk_table), ptr(chunk_offsets), ptr(workspace), ws_bytes,
-        B, T, H, HV, _DIM, _DIM, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags,
-        current_stream_ptr(dev)))
+        B, T, H, HV, _DIM, _DIM, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags)
     dq = _finish(lib, dq, qw, q_rstd, H, K, out_dtype)
     dk = _finish(lib, dk, kw, k_rstd, H, K, out_dtype)
     dp = _finish(lib, dp, pw, p_rstd, H, K, out_dtype)

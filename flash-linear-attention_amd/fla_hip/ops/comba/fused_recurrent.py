@@ -14,9 +14,9 @@ from fla_hip.ops.gated_delta_rule._common import (
     aligned16,
     as_f32,
     check_operand_shapes,
-    current_stream_ptr,
     dtype_code,
     forward_only,
+    launch,
     ptr,
     require_gpu,
     unify_gate_beta,
@@ -65,9 +65,9 @@ def fused_recurrent_comba_fwd(q, k, p, v, g, beta, scale, initial_state, output_
         check_cu_seqlens(cu_seqlens, T)
     o = torch.empty_like(v)
     ht = torch.empty(N, HV, KP, VP, dtype=torch.float32, device=dev) if output_final_state else None
-    _lib.check(_lib.load().gdn_fused_recurrent_comba_fwd(
-        ptr(q), ptr(k), ptr(p), ptr(v), ptr(g), ptr(beta), ptr(h0), ptr(ht), ptr(o), ptr(cu_seqlens),
-        B, T, H, HV, KP, VP, N, float(scale), dtype_code(q.dtype), gb_code, flags, current_stream_ptr(dev)))
+    launch(
+        _lib.load().gdn_fused_recurrent_comba_fwd, dev, ptr(q), ptr(k), ptr(p), ptr(v), ptr(g), ptr(beta), ptr(h0), ptr(ht), ptr(o), ptr(cu_seqlens),
+        B, T, H, HV, KP, VP, N, float(scale), dtype_code(q.dtype), gb_code, flags)
     if (KP, VP) != (K, V):
         o = o[..., :V].contiguous()
         if ht is not None:

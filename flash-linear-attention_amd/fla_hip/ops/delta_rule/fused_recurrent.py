@@ -8,7 +8,7 @@ import torch
 import torch.nn.functional as F
 
 from fla_hip import _lib
-from fla_hip.ops.gated_delta_rule._common import aligned16, as_f32, current_stream_ptr, dtype_code, pad_last_two, ptr, require_gpu
+from fla_hip.ops.gated_delta_rule._common import aligned16, as_f32, dtype_code, launch, pad_last_two, ptr, require_gpu
 from fla_hip.ops.gated_delta_rule.fused_recurrent import fused_recurrent_gated_delta_rule_fwd
 from fla_hip.ops.utils.index import check_cu_seqlens, cu_bounds
 
@@ -81,10 +81,10 @@ def fused_recurrent_delta_rule_bwd(
     db = alloc(B, T, H, VP, **f32) if flags & _lib.FLAG_BETA_VECTOR else alloc(NVB, B, T, H, **f32)
     dh0 = torch.empty(N, H, KP, VP, **f32) if initial_state is not None else None
     u = torch.empty(B, T, H, VP, **f32)
-    _lib.check(lib.gdn_fused_recurrent_delta_bwd(
-        ptr(qw), ptr(kw), ptr(vw), ptr(bw), ptr(dow), ptr(h0), ptr(dhtw),
+    launch(
+        lib.gdn_fused_recurrent_delta_bwd, dev, ptr(qw), ptr(kw), ptr(vw), ptr(bw), ptr(dow), ptr(h0), ptr(dhtw),
         ptr(dq_part), ptr(dk_part), ptr(dv), ptr(db), ptr(dh0), ptr(u), ptr(cu_seqlens),
-        B, T, H, KP, VP, N, float(scale), dtype_code(work), _lib.DTYPE_F32, flags, current_stream_ptr(dev)))
+        B, T, H, KP, VP, N, float(scale), dtype_code(work), _lib.DTYPE_F32, flags)
     dq, dk = dq_part.sum(0)[..., :K], dk_part.sum(0)[..., :K]
     dbeta = None
     if beta is not None:

@@ -109,6 +109,13 @@ def current_stream_ptr(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def launch(entry, dev: torch.device, *args) -> None:
+    """``entry(*args, stream)`` of the library on ``dev``'s current stream, with ``dev`` as the current device: the default stream is
+    the current device's, whatever the tensors' is."""
+    with torch.cuda.device(dev):
+        _lib.check(entry(*args, current_stream_ptr(dev)))
+
+
 def forward_only(what: str, *activations: torch.Tensor | None) -> None:
     """Operators without a backward refuse activations that require a gradient (in grad mode) instead of returning a
     result that silently carries none.  Parameters are not looked at: inference outside ``torch.no_grad()`` is fine."""
@@ -119,5 +126,5 @@ def forward_only(what: str, *activations: torch.Tensor | None) -> None:
 def sum_rows(part: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """``part.sum(0)`` of an fp32 tensor of partial sums, in ``dtype`` (added up in fp32, in a fixed order)."""
     out = torch.empty(part.shape[1:], dtype=dtype, device=part.device)
-    _lib.check(_lib.load().gdn_sum_rows(ptr(part), ptr(out), part.shape[0], out.numel(), dtype_code(dtype), current_stream_ptr(part.device)))
+    launch(_lib.load().gdn_sum_rows, part.device, ptr(part), ptr(out), part.shape[0], out.numel(), dtype_code(dtype))
     return out

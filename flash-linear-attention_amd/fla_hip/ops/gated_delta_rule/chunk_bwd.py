@@ -12,7 +12,7 @@ import torch
 import torch.nn.functional as F
 
 from fla_hip import _lib
-from fla_hip.ops.gated_delta_rule._common import aligned16, as_f32, check_operand_shapes, current_stream_ptr, dtype_code, pad_last_two, ptr, require_gpu
+from fla_hip.ops.gated_delta_rule._common import aligned16, as_f32, check_operand_shapes, dtype_code, launch, pad_last_two, ptr, require_gpu
 from fla_hip.ops.utils.index import check_cu_seqlens, cu_bounds, prepare_chunk_indices, prepare_scan_tables
 
 _CHUNK = 64
@@ -126,12 +126,11 @@ def chunk_gated_delta_rule_bwd(
         flags |= _lib.FLAG_BETA_SIGMOID | (_lib.FLAG_NEG_EIGVAL if neg_eigval else 0)
     ws_bytes = lib.gdn_chunk_bwd_heads_workspace_bytes(num_chunks, H, HV, KD, VD, B * T, flags)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    _lib.check(lib.gdn_chunk_bwd_heads(
-        ptr(qw), ptr(kw), ptr(vw), ptr(gw), ptr(bw), ptr(A_log), ptr(dt_bias), ptr(h0), ptr(dow), ptr(dhtw),
+    launch(
+        lib.gdn_chunk_bwd_heads, dev, ptr(qw), ptr(kw), ptr(vw), ptr(gw), ptr(bw), ptr(A_log), ptr(dt_bias), ptr(h0), ptr(dow), ptr(dhtw),
         ptr(dq), ptr(dk), ptr(dv), ptr(dg), ptr(db), ptr(dh0),
         ptr(cu_seqlens), ptr(chunk_table), ptr(chunk_offsets), ptr(workspace), ws_bytes,
-        B, T, H, HV, KD, VD, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags,
-        current_stream_ptr(dev)))
+        B, T, H, HV, KD, VD, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags)
     dq = _finish(lib, dq, qw, q_rstd, H, K, out_dtype)
     dk = _finish(lib, dk, kw, k_rstd, H, K, out_dtype)
     dv = dv[..., :V].to(out_dtype)
@@ -158,10 +157,10 @@ def gate_bwd(dgate, dbeta, g, beta, A_log, dt_bias, beta_max):
     dg = torch.empty_like(g) if with_gate else None
     db = torch.empty_like(beta)
     part = torch.empty(parts, 2, HV, dtype=torch.float32, device=dev) if with_gate else None
-    _lib.check(_lib.load().gdn_gate_bwd(
-        ptr(dgate) if with_gate else None, ptr(dbeta), ptr(g) if with_gate else None, ptr(beta), ptr(A_log) if with_gate else None,
+    launch(
+        _lib.load().gdn_gate_bwd, dev, ptr(dgate) if with_gate else None, ptr(dbeta), ptr(g) if with_gate else None, ptr(beta), ptr(A_log) if with_gate else None,
         ptr(dt_bias), ptr(dg), ptr(db), ptr(part), rows, HV, parts, HV, HV, HV, HV, 0, 0,
-        dtype_code(g.dtype) if with_gate else _lib.DTYPE_F32, dtype_code(beta.dtype), beta_max, current_stream_ptr(dev)))
+        dtype_code(g.dtype) if with_gate else _lib.DTYPE_F32, dtype_code(beta.dtype), beta_max)
     return dg if with_gate else dgate, db, part
 
 
@@ -175,8 +174,8 @@ def _finish(lib, dxh: torch.Tensor, y: torch.Tensor, rstd: torch.Tensor | None, 
     if K % 8:                                       # (rows of the kernel are multiples of 8 elements)
         KP = (K + 7) // 8 * 8
         dx = torch.empty(B, T, H, KP, dtype=dxh.dtype, device=dxh.device)
-    _lib.check(lib.gdn_l2norm_bwd(ptr(dxh), ptr(y) if rstd is not None else None, ptr(rstd), ptr(dx), B * T * H, HV // H, D,
-                                  dx.shape[-1], dtype_code(dxh.dtype), current_stream_ptr(dxh.device)))
+    launch(lib.gdn_l2norm_bwd, dxh.device, ptr(dxh), ptr(y) if rstd is not None else None, ptr(rstd), ptr(dx), B * T * H, HV // H, D,
+           dx.shape[-1], dtype_code(dxh.dtype))
     return dx[..., :K].to(out_dtype)
 
 
@@ -192,8 +191,7 @@ def l2norm_fwd(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     xw = aligned16(x.to(work).contiguous())
     y = torch.empty_like(xw)
     rstd = torch.empty(*x.shape[:-1], 1, dtype=torch.float32, device=x.device)
-    _lib.check(_lib.load().gdn_l2norm_fwd(ptr(xw), ptr(y), ptr(rstd), xw.numel() // D, D, D, dtype_code(work),
-                                          current_stream_ptr(x.device)))
+    launch(_lib.load().gdn_l2norm_fwd, x.device, ptr(xw), ptr(y), ptr(rstd), xw.numel() // D, D, D, dtype_code(work))
     return y, rstd
 
 

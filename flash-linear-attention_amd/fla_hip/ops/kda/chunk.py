@@ -17,8 +17,8 @@ from fla_hip.ops.gated_delta_rule._common import (
     aligned16,
     check_operand_shapes,
     as_f32,
-    current_stream_ptr,
     dtype_code,
+    launch,
     ptr,
     require_gpu,
 )
@@ -141,12 +141,11 @@ def chunk_kda_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, st
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     hs = torch.empty(num_chunks, HV, _DIM, _DIM, dtype=work, device=dev) if return_states else None
     entry, states = (lib.gdn_chunk_kda_fwd_states, (ptr(hs),)) if return_states else (lib.gdn_chunk_kda_fwd, ())
-    _lib.check(entry(
-        ptr(qw), ptr(kw), ptr(vw), ptr(gw), ptr(bw), ptr(A_log), ptr(dt_bias),
+    launch(
+        entry, dev, ptr(qw), ptr(kw), ptr(vw), ptr(gw), ptr(bw), ptr(A_log), ptr(dt_bias),
         0.0 if lower_bound is None else float(lower_bound), gate_mode, ptr(h0), ptr(ht), ptr(o), *states,
         ptr(cu_seqlens), ptr(chunk_table), ptr(chunk_offsets), ptr(workspace), ws_bytes,
-        B, T, H, HV, _DIM, _DIM, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags,
-        current_stream_ptr(dev)))
+        B, T, H, HV, _DIM, _DIM, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags)
     o = o[..., :V].to(out_dtype)
     if ht is not None:
         ht = ht[..., :K, :V]
@@ -245,12 +244,11 @@ def chunk_kda_bwd(q, k, v, g, beta, scale, initial_state, do, dht, state_v_first
     lib = _lib.load()
     ws_bytes = lib.gdn_chunk_kda_bwd_workspace_bytes(num_chunks, HV)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    _lib.check(lib.gdn_chunk_kda_bwd(
-        ptr(qw), ptr(kw), ptr(vw), ptr(gw), ptr(bw), ptr(h0), ptr(dow), ptr(dhtw),
+    launch(
+        lib.gdn_chunk_kda_bwd, dev, ptr(qw), ptr(kw), ptr(vw), ptr(gw), ptr(bw), ptr(h0), ptr(dow), ptr(dhtw),
         ptr(dq), ptr(dk), ptr(dv), ptr(dg), ptr(db), ptr(dh0),
         ptr(cu_seqlens), ptr(chunk_table), ptr(chunk_offsets), ptr(workspace), ws_bytes,
-        B, T, H, HV, _DIM, _DIM, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags,
-        current_stream_ptr(dev)))
+        B, T, H, HV, _DIM, _DIM, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags)
     dq = _finish(lib, dq, qw, q_rstd, H, K, out_dtype)
     dk = _finish(lib, dk, kw, k_rstd, H, K, out_dtype)
     dv = dv[..., :V].to(out_dtype)
