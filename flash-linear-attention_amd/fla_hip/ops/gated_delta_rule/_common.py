@@ -125,6 +125,6 @@ def forward_only(what: str, *activations: torch.Tensor | None) -> None:
 
 def sum_rows(part: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     """``part.sum(0)`` of an fp32 tensor of partial sums, in ``dtype`` (added up in fp32, in a fixed order)."""
-    out = torch.empty(part.shape[1:], dtype=dtype, device=part.device)
-    launch(_lib.load().gdn_sum_rows, part.device, ptr(part), ptr(out), part.shape[0], out.numel(), dtype_code(dtype))
-    return out
+    out = torch.empty(part.shape[1:], dtype=dtype if dtype in _DTYPE_CODE else torch.float32, device=part.device)
+    launch(_lib.load().gdn_sum_rows, part.device, ptr(part), ptr(out), part.shape[0], out.numel(), dtype_code(out.dtype))
+    return out.to(dtype)

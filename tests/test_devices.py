@@ -45,7 +45,7 @@ def lib(monkeypatch):
 
 def _conv_bwd(q, k, v, g, beta, gk):
     x = torch.zeros(2, 70, 24)
-    convolution.causal_conv1d_bwd(x, x, None, torch.zeros(24, 4), torch.zeros(24))
+    convolution.causal_conv1d_bwd(x, x, None, torch.zeros(24, 4), torch.zeros(24, dtype=torch.float64))
 
 
 def _norm(q, k, v, g, beta, gk):
@@ -76,3 +76,7 @@ def test_launches_are_made_on_the_tensors_device(lib, call):
     v, g, gk = torch.zeros(1, 70, 2, 64), torch.zeros(1, 70, 2), torch.zeros(1, 70, 2, 64)
     CALLS[call](q, k, v, g, torch.ones(1, 70, 2), gk)
     assert lib.calls and all(inside for _, inside in lib.calls), lib.calls
+
+
+def test_sums_of_partial_rows_in_any_type(lib):
+    assert _common.sum_rows(torch.zeros(3, 8), torch.float64).dtype == torch.float64
