@@ -100,7 +100,11 @@ int code_of(at::ScalarType s) {
 
 bool plain(const Arg& a, c10::Device dev) { return !a.bad && (!a || (a->device() == dev && a->is_contiguous())); }
 bool aligned16(const void* p) { return (uintptr_t)p % 16 == 0; }
-bool truth(PyObject* o) { return PyObject_IsTrue(o) == 1; }
+bool truth(PyObject* o) {                                // (may run the caller's code: with the interpreter held, and it may raise)
+    const int is = PyObject_IsTrue(o);
+    if (is < 0) throw python_error();
+    return is;
+}
 
 // g and beta share a code, or carry one each; -1: a type the kernels do not take
 int gb_code_of(const Arg& g, const Arg& beta) {

@@ -315,10 +315,11 @@ PyObject* layer_train(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (A.dim() != 1 || dt.dim() != 1 || A.numel() != HV || dt.numel() != HV || A.scalar_type() != dt.scalar_type() || code_of(A.scalar_type()) < 0 ||
         nw.dim() != 1 || nw.numel() != V || code_of(nw.scalar_type()) < 0)
         Py_RETURN_NONE;
+    const bool neg = truth(a[13]);
     variable_list r;
     {
         const NoGil free;
-        r = LayerTrain::apply(at::TensorList(in), heads, truth(a[13]), eps);
+        r = LayerTrain::apply(at::TensorList(in), heads, neg, eps);
     }
     return THPVariable_Wrap(r[0]);
     END_HANDLE_TH_ERRORS

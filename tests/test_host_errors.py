@@ -120,3 +120,36 @@ def test_tensors_without_plain_memory_raise_on_the_gpu(op, form):
             with FakeTensorMode(allow_non_fake_inputs=True) as mode:
                 call(mode.from_tensor(q))
     assert torch.equal(call(q), want)
+
+
+class _Switch:
+    """A truth value that takes the interpreter to find out."""
+
+    def __init__(self, value):
+        self.value = value
+
+    def __bool__(self):
+        if self.value is None:
+            raise ValueError('no truth in it')
+        return sum([bool(self.value)] * 3) == 3
+
+
+def test_a_switch_without_truth_raises():
+    from fla_hip import _lib
+    with pytest.raises(ValueError, match='no truth'):
+        _lib.host().fused_recurrent(*[None] * 10, _Switch(None), *[None] * 9)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('neg', [False, True])
+def test_switches_are_read_with_the_interpreter_held(neg):
+    from fla_hip.layers import GatedDeltaNet
+    torch.manual_seed(0)
+    layer = GatedDeltaNet(hidden_size=256, head_dim=64, expand_v=1, num_heads=4, allow_neg_eigval=neg).cuda().bfloat16().train()
+    x = torch.randn(1, 130, 256, device='cuda').bfloat16()
+    want = layer._train(x)
+    layer.allow_neg_eigval = _Switch(neg)
+    assert torch.equal(layer._train(x), want)
+    layer.allow_neg_eigval = _Switch(None)
+    with pytest.raises(ValueError, match='no truth'):
+        layer._train(x)
