@@ -242,8 +242,8 @@ extern "C" int gdn_norm_gated_fwd(
     auto is_dtype = [](int d) { return d == GDN_DTYPE_BF16 || d == GDN_DTYPE_F16 || d == GDN_DTYPE_F32; };
     GDN_CHECK_ARG((x && g && y) || T == 0, GDN_ERR_INVALID, "gdn_norm_gated_fwd: x, g and y are required");
     GDN_CHECK_ARG(T >= 0 && D >= 1 && T < (1ll << 31), GDN_ERR_INVALID, "gdn_norm_gated_fwd: bad sizes T=%lld D=%lld", (long long)T, (long long)D);
-    GDN_CHECK_ARG(D <= 65536 / (x_dtype == GDN_DTYPE_F32 ? 4 : 2), GDN_ERR_UNSUPPORTED,
-                  "gdn_norm_gated_fwd: rows of 64 KB and more are not supported (D=%lld)", (long long)D);
+    GDN_CHECK_ARG(D <= GDN_NORM_MAX_ROW_BYTES / (x_dtype == GDN_DTYPE_F32 ? 4 : 2), GDN_ERR_UNSUPPORTED,
+                  "gdn_norm_gated_fwd: rows of more than 64 KB are not supported (D=%lld)", (long long)D);
     GDN_CHECK_ARG(is_dtype(x_dtype) && is_dtype(w_dtype) && is_dtype(res_dtype) && is_dtype(res_out_dtype), GDN_ERR_UNSUPPORTED,
                   "gdn_norm_gated_fwd: unknown dtype");
     GDN_CHECK_ARG(activation == GDN_ACT_SILU || activation == GDN_ACT_SIGMOID, GDN_ERR_UNSUPPORTED,

@@ -135,15 +135,15 @@ extern "C" int gdn_step_linear(const void* x, int64_t N, int64_t hidden, const g
     using namespace gdn;
     const char* who = "gdn_step_linear";
     GDN_CHECK_ARG(x && segs && nseg >= 1 && nseg <= GDN_STEP_SEGMENTS, GDN_ERR_INVALID, "%s: x and 1 to %d segments are required", who, GDN_STEP_SEGMENTS);
-    GDN_CHECK_ARG(N >= 1 && N <= 128 && hidden >= 256 && hidden % 256 == 0 && hidden < (1 << 24), GDN_ERR_UNSUPPORTED,
-                  "%s: 1 to 128 rows of a multiple of 256 elements (got %lld x %lld)", who, (long long)N, (long long)hidden);
+    GDN_CHECK_ARG(N >= 1 && N <= GDN_STEP_MAX_ROWS && hidden >= 256 && hidden % 256 == 0 && hidden <= GDN_STEP_MAX_COLS, GDN_ERR_UNSUPPORTED,
+                  "%s: 1 to %d rows of a multiple of 256 elements (got %lld x %lld)", who, GDN_STEP_MAX_ROWS, (long long)N, (long long)hidden);
     GDN_CHECK_ARG(dtype == GDN_DTYPE_BF16 || dtype == GDN_DTYPE_F16, GDN_ERR_UNSUPPORTED, "%s: bf16 or f16 only", who);
     StepLinearParams p;
     p.x = x; p.N = (int)N; p.hidden = (int)hidden; p.nseg = nseg;
     GDN_CHECK_ARG((uintptr_t)x % 16 == 0, GDN_ERR_INVALID, "%s: x must be 16-byte aligned", who);
     for (int i = 0; i < nseg; ++i) {
         const gdn_step_segment& s = segs[i];
-        GDN_CHECK_ARG(s.weight && s.out && s.cols >= 1 && s.cols < (1 << 24) && (uintptr_t)s.weight % 16 == 0, GDN_ERR_INVALID,
+        GDN_CHECK_ARG(s.weight && s.out && s.cols >= 1 && s.cols <= GDN_STEP_MAX_COLS && (uintptr_t)s.weight % 16 == 0, GDN_ERR_INVALID,
                       "%s: segment %d needs a 16-byte aligned weight and an output", who, i);
         GDN_CHECK_ARG(s.kind >= GDN_STEP_PLAIN && s.kind <= GDN_STEP_BETA2, GDN_ERR_INVALID, "%s: segment %d is of no known kind", who, i);
         GDN_CHECK_ARG(s.kind != GDN_STEP_CONV || (s.conv_weight && s.conv_state && s.conv_size >= 1 && s.conv_size <= 8 &&

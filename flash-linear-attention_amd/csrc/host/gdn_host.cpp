@@ -150,6 +150,15 @@ PyObject* pair(const at::Tensor& a, const at::Tensor& b) {
     return r;
 }
 
+// a refusal or a failed launch of the library as the exception that _lib.check raises for it
+void check_rc(int rc, const char* what) {
+    if (rc == GDN_OK) return;
+    const char* why = p_last_error ? p_last_error() : "";
+    TORCH_CHECK_VALUE(rc != GDN_ERR_INVALID, what, ": ", why);
+    TORCH_CHECK_NOT_IMPLEMENTED(rc != GDN_ERR_UNSUPPORTED, what, ": ", why);
+    TORCH_CHECK(false, what, ": libgdn_hip status ", rc, ": ", why);
+}
+
 // ---- token recurrence ----
 // (q, k, v, g, gk, beta, A_log, dt_bias, scale, initial_state, output_final_state, qk_l2norm, beta_sigmoid, neg_eigval, state_v_first,
 //  cu_seqlens, inplace_final_state, state_slots, kda_gate_mode, lower_bound); gk: the KDA operator's gate (kda_gate_mode 0 .. 2) or
@@ -312,13 +321,17 @@ PyObject* layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (t->t->scalar_type() != type || t->t->dim() != 2 || t->t->size(1) != hidden) Py_RETURN_NONE;
     if (state->scalar_type() != at::kFloat || state->dim() != 4 || state->size(0) != N) Py_RETURN_NONE;
     const int64_t HV = state->size(1), V = state->size(2), K = state->size(3), kd = H * K, vd = HV * V;
-    if (N < 1 || N > 128 || H < 1 || HV % H || K % 4 || V % 8 || K > 256 || hidden % 256 || vd % 256 || qw->size(0) != kd || kw->size(0) != kd || vw->size(0) != vd ||
+    if (N < 1 || H < 1 || HV % H || K % 4 || V % 8 || K > 256 || hidden % 256 || vd % 256 || qw->size(0) != kd || kw->size(0) != kd || vw->size(0) != vd ||
         gw->size(0) != vd || aw->size(0) != HV || bw->size(0) != HV || ow->scalar_type() != type || ow->dim() != 2 || ow->size(1) != vd ||
         A_log->numel() != HV || dt_bias->numel() != HV || A_log->scalar_type() != dt_bias->scalar_type() || norm_w->numel() != V)
         Py_RETURN_NONE;
     const int gate_code = code_of(A_log->scalar_type()), norm_code = code_of(norm_w->scalar_type());
     if (gate_code < 0 || norm_code < 0) Py_RETURN_NONE;
     const int64_t out_cols = ow->size(0);
+    // Every limit of the four launches: none may be refused once the first has moved the convolutions' states on.
+    if (N > GDN_STEP_MAX_ROWS || std::max({hidden, kd, vd, out_cols}) > GDN_STEP_MAX_COLS || out_cols < 1 || V > GDN_NORM_MAX_ROW_BYTES / 2 ||
+        (N + 8) * HV * ((V + 31) / 32) >= (1ll << 31))
+        Py_RETURN_NONE;
     gdn_step_segment seg[6] = {};
     for (int i = 10; i < 13; ++i)
         if (!PyTuple_Check(a[i]) || PyTuple_GET_SIZE(a[i]) != 3) Py_RETURN_NONE;
@@ -363,7 +376,7 @@ PyObject* layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                   GDN_DTYPE_F32, GDN_DTYPE_F32, GDN_ACT_SILU, 1, stream);
         if (rc == GDN_OK) rc = p_step_linear(base + o_y, N, vd, &last, 1, code, stream);
     }
-    if (rc != GDN_OK) { PyErr_Format(PyExc_RuntimeError, "gdn_host.layer_step: status %d", rc); return nullptr; }
+    check_rc(rc, "gdn_host.layer_step");
     return THPVariable_Wrap(out);
     END_HANDLE_TH_ERRORS
 }

@@ -5,13 +5,6 @@ using torch::autograd::AutogradContext;
 using torch::autograd::Variable;
 using torch::autograd::variable_list;
 
-void check_rc(int rc, const char* what) {
-    if (rc == GDN_OK) return;
-    const char* why = p_last_error ? p_last_error() : "";            // (types as _lib.check gives them)
-    TORCH_CHECK_VALUE(rc != GDN_ERR_INVALID, what, ": ", why);
-    TORCH_CHECK_NOT_IMPLEMENTED(rc != GDN_ERR_UNSUPPORTED, what, ": ", why);
-    TORCH_CHECK(false, what, ": libgdn_hip status ", rc, ": ", why);
-}
 template <typename T = void>
 T* ptr_of(const at::Tensor& t) { return t.defined() ? (T*)t.data_ptr() : nullptr; }
 at::Tensor to_f32(const at::Tensor& t) { return t.defined() ? t.detach().to(at::kFloat).contiguous() : t; }

@@ -115,9 +115,11 @@ int gdn_fused_recurrent_fwd(
  *                   moves one place to the left and takes y, out = silu(sum conv_state conv_weight + conv_bias)
  *   GDN_STEP_GATE   out (fp32) = -exp(A_log) softplus(y + dt_bias), A_log, dt_bias [cols] in gate_dtype (dt_bias may be NULL)
  *   GDN_STEP_BETA   out (fp32) = sigmoid(y); GDN_STEP_BETA2: twice that
- * N from 1 to 128, hidden a multiple of 256.
+ * N from 1 to GDN_STEP_MAX_ROWS, hidden a multiple of 256 and, like cols, at most GDN_STEP_MAX_COLS.
  */
 #define GDN_STEP_SEGMENTS 6
+#define GDN_STEP_MAX_ROWS 128
+#define GDN_STEP_MAX_COLS ((1 << 24) - 1)
 #define GDN_STEP_PLAIN 0
 #define GDN_STEP_CONV  1
 #define GDN_STEP_GATE  2
@@ -549,8 +551,9 @@ int gdn_causal_conv1d_update(
  *   with rstd = 1/sqrt(var + eps); is_rms_norm != 0: mean = 0 and var = mean(r^2)
  *   x, g, y [T,D] x_dtype contiguous; weight, bias [D] w_dtype or NULL; residual [T,D] res_dtype or NULL;
  *   residual_out [T,D] res_out_dtype or NULL (r is not stored); mean, rstd [T] fp32 or NULL (not stored)
- *   Requires D * sizeof(element) < 64 KB.
+ *   Requires D * sizeof(element) <= GDN_NORM_MAX_ROW_BYTES.
  */
+#define GDN_NORM_MAX_ROW_BYTES 65536
 int gdn_norm_gated_fwd(
     const void* x, const void* g, const void* weight, const void* bias, const void* residual,
     void* y, void* residual_out, float* mean, float* rstd,

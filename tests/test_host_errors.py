@@ -153,3 +153,18 @@ def test_switches_are_read_with_the_interpreter_held(neg):
     layer.allow_neg_eigval = _Switch(None)
     with pytest.raises(ValueError, match='no truth'):
         layer._train(x)
+
+
+@pytest.mark.gpu
+def test_a_refused_layer_step_leaves_the_states_alone():
+    """33024 value columns a head: more than the norm takes.  No launch may have moved the convolutions' states on by then."""
+    from fla_hip.layers import GatedDeltaNet
+    from fla_hip.layers.gated_deltanet import LayerCache
+    layer = GatedDeltaNet(hidden_size=256, head_dim=64, expand_v=516, num_heads=1, layer_idx=0).cuda().bfloat16().eval()
+    cache = LayerCache()
+    cache.update(layer_idx=0, recurrent_state=torch.randn(1, 1, 33024, 64, device='cuda'),
+                 conv_state=tuple(torch.randn(1, d, 4, device='cuda', dtype=torch.bfloat16) for d in (64, 64, 33024)))
+    states = [cache[0]['recurrent_state'], *cache[0]['conv_state']]
+    before = [s.clone() for s in states]
+    assert layer._step(torch.randn(1, 1, 256, device='cuda', dtype=torch.bfloat16), cache) is None
+    assert all(torch.equal(a, b) for a, b in zip(before, states))
