@@ -23,6 +23,7 @@ OBJ_DIR = os.path.join(HERE, 'build', 'obj')
 HOST_SRC = os.path.join(CSRC, 'host', 'gdn_host.cpp')
 HOST_HDR = os.path.join(CSRC, 'host', 'gdn_host_train.h')
 HOST_LIB = os.path.join(OUT_DIR, 'gdn_host.so')
+HOST_TORCH = os.path.join(OBJ_DIR, 'gdn_host.torch')      # the torch that HOST_LIB was built with
 
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
 FLAGS = [
@@ -52,16 +53,23 @@ def _compile(src, obj):
         sys.stderr.write(err + '\n')
 
 
+def _torch_version():
+    import torch
+    return torch.__version__
+
+
 def _compile_host():
     import torch
     root = os.path.dirname(torch.__file__)
     cmd = ['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-fvisibility=hidden', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
-           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}',
+           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}', f'-DGDN_TORCH_VERSION="{torch.__version__}"',
            *(f'-I{d}' for d in (f'{root}/include', f'{root}/include/torch/csrc/api/include', '/opt/rocm/include', sysconfig.get_paths()['include'])),
            HOST_SRC, '-o', HOST_LIB, f'-L{root}/lib', '-ltorch_python', '-ltorch', '-ltorch_cpu', '-lc10', '-lc10_hip', f'-Wl,-rpath,{root}/lib']
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f'g++ failed for {HOST_SRC}:\n{r.stderr}')
+    with open(HOST_TORCH, 'w') as f:
+        f.write(torch.__version__)
 
 
 def build(force: bool = False, verbose: bool = True) -> str:
@@ -75,7 +83,7 @@ def build(force: bool = False, verbose: bool = True) -> str:
         objs.append(o)
         if force or _newer([s, *hdrs], o):
             jobs.append((s, o))
-    host = force or _newer([HOST_SRC, HOST_HDR, hdrs[-1]], HOST_LIB)
+    host = force or _newer([HOST_SRC, HOST_HDR, hdrs[-1]], HOST_LIB) or not os.path.exists(HOST_TORCH) or open(HOST_TORCH).read() != _torch_version()
     if verbose and (jobs or host):
         print(f'[build] compiling {len(jobs)} file(s) for gfx950' + (' and the host extension' if host else ''), flush=True)
     with ThreadPoolExecutor(max_workers=min(8, max(1, len(jobs) + host))) as ex:

@@ -395,4 +395,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "gdn_host", nullptr, -1, methods, n
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_gdn_host() { return PyModule_Create(&module); }
+// (the extension holds for the torch it was built with; the binding looks)
+PyMODINIT_FUNC PyInit_gdn_host() {
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "TORCH_VERSION", GDN_TORCH_VERSION) < 0) { Py_DECREF(m); return nullptr; }
+    return m;
+}

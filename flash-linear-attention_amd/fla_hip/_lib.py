@@ -8,9 +8,18 @@ import threading
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_uint32, c_void_p
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
-LIB_PATH = os.environ.get('FLA_HIP_LIBRARY') or os.path.join(_HERE, '_C', 'libgdn_hip.so')
+_ELSEWHERE = os.environ.get('FLA_HIP_LIBRARY')
+LIB_PATH = _ELSEWHERE or os.path.join(_HERE, '_C', 'libgdn_hip.so')
 
-HOST_PATH = os.path.join(_HERE, '_C', 'gdn_host.so')
+
+def _host_path() -> str | None:
+    """The host extension that goes with the library: the one beside it, or the package's own.  None: a library that was placed elsewhere
+    without one, which then runs behind the Python host path alone."""
+    for folder in (os.path.dirname(LIB_PATH), os.path.join(_HERE, '_C')):
+        path = os.path.join(folder, 'gdn_host.so')
+        if os.path.exists(path):
+            return path
+    return None if _ELSEWHERE else path
 
 ABI_VERSION = 13
 
@@ -201,24 +210,48 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+class _PythonHost:
+    """No host extension: every call is one for the Python path, which checks its arguments and then needs the library."""
+
+    @staticmethod
+    def _leave(*args):
+        return None
+
+    fused_recurrent = chunk_fwd = chunk_train = layer_step = layer_train = _leave
+
+
 _host = None
 
 
 def host():
-    """The host path's native code (csrc/host/gdn_host.cpp), bound to the library's entry points.  Built with it and, like it,
-    without a stand-in."""
+    """The host path's native code (csrc/host/gdn_host.cpp), bound to the library's entry points.  Built with it and, where the package's
+    own library is in use, without a stand-in.  (Without the library itself the Python path is left to say what is wrong with a call, and
+    then that the library is missing.)"""
     global _host
     if _host is not None:
         return _host
+    if not os.path.exists(LIB_PATH):
+        return _PythonHost
     lib = load()
     with _lock:
         if _host is None:
-            if not os.path.exists(HOST_PATH):
-                raise GDNLibraryError(f'{HOST_PATH} is missing. Build it with `python {os.path.join(os.path.dirname(_HERE), "build.py")}`.')
-            import torch  # noqa: F401  (the extension's symbols)
-            spec = importlib.util.spec_from_file_location('gdn_host', HOST_PATH)
-            module = importlib.util.module_from_spec(spec)
-            spec.loader.exec_module(module)
+            path = _host_path()
+            if path is None:
+                _host = _PythonHost
+                return _host
+            how = f'Build it with `python {os.path.join(os.path.dirname(_HERE), "build.py")}`.'
+            if not os.path.exists(path):
+                raise GDNLibraryError(f'{path} is missing. {how}')
+            import torch
+            spec = importlib.util.spec_from_file_location('gdn_host', path)
+            try:
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+            except ImportError as exc:
+                raise GDNLibraryError(f'{path} does not load with torch {torch.__version__} ({exc}). {how}') from exc
+            built = getattr(module, 'TORCH_VERSION', 'another version')
+            if built != torch.__version__:
+                raise GDNLibraryError(f'{path} was built with torch {built}, this is {torch.__version__}. {how}')
             module.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in SIGNATURES})
             _host = module
     return _host
