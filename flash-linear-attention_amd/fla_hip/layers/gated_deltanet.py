@@ -35,24 +35,27 @@ _STEP_LINEARS = ('q_proj', 'k_proj', 'v_proj', 'a_proj', 'b_proj', 'g_proj', 'o_
 _STEP_CONVS = ('q_conv1d', 'k_conv1d', 'v_conv1d')
 
 
-# The calls that the native paths stand for.  Where a caller has replaced one of them - on the class, on a module, around every
-# module - the layer runs module by module and makes it.
-_FORWARDS = {nn.Linear: nn.Linear.forward, ShortConvolution: ShortConvolution.forward, FusedRMSNormGated: FusedRMSNormGated.forward}
-_AROUND = (nn.Module.__call__, F.linear, ShortConvolution.step)
+def _calls() -> tuple:
+    return nn.Module.__call__, F.linear, nn.Linear.forward, ShortConvolution.forward, ShortConvolution.step, FusedRMSNormGated.forward
+
+
+# The calls that the native paths stand for.  Where a caller has replaced one of them - here, on a module or around every module - the
+# layer runs module by module and makes it.
+_CALLS = _calls()
 
 
 def _own_call(m: nn.Module, cls: type) -> bool:
-    """Whether calling ``m`` is ``cls.forward`` and nothing else: no other class, no other ``forward``, no hooks, not compiled."""
+    """Whether calling ``m`` is ``cls.forward`` and nothing else: no other class, no hooks, no ``forward`` of its own, not compiled."""
     d = m.__dict__
-    return (type(m) is cls and cls.forward is _FORWARDS[cls] and 'forward' not in d and 'step' not in d and d.get('_compiled_call_impl') is None
-            and not (d['_forward_hooks'] or d['_forward_pre_hooks'] or d['_backward_hooks'] or d['_backward_pre_hooks']))
+    return type(m) is cls and not (d['_forward_hooks'] or d['_forward_pre_hooks'] or d['_backward_hooks'] or d['_backward_pre_hooks']
+                                   or 'forward' in d or 'step' in d or '_compiled_call_impl' in d)
 
 
 def _watched() -> bool:
-    """Whether something looks at, or stands in for, the calls between the layer's modules: hooks on all modules, torch's dispatch and
-    function modes (a default device is none of those), a patched ``nn.Module.__call__`` or ``F.linear``."""
+    """Whether something looks at, or stands in for, the calls between all modules: hooks on every module, torch's dispatch and
+    function modes (a default device is none of those), one of ``_CALLS`` patched."""
     n = torch._C._len_torch_function_stack()
-    return (_has_any_global_hook() or torch._C._len_torch_dispatch_stack() > 0 or (nn.Module.__call__, F.linear, ShortConvolution.step) != _AROUND
+    return (_has_any_global_hook() or torch._C._len_torch_dispatch_stack() > 0 or _calls() != _CALLS
             or (n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n))))
 
 
