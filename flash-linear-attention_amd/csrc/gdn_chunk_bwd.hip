@@ -109,7 +109,43 @@ struct BwdParams {
     int nseg, seg_chunks, warm_cap;
     int64_t tokens;                      // rows of q and k per head
     int parts;                           // dq and dk leave as this many partial rows per token and q/k head (a divisor of HV / H)
+    // Partial rows that are added up here (BwdParts) leave in fp32 to these places instead of dq and dk (NULL: they do not), and where
+    // the parts cut a value head's blocks of columns, `split` > 1 parts to a head, so do the partial sums of dg and dbeta.
+    float* dq_part; float* dk_part; float* dg_part; float* db_part;
+    int split;
 };
+
+// How a q/k head's value heads (their blocks of columns, `nb` each) are dealt out to the workgroups of gdn_bwd_unit_kernel: all to one
+// where (chunk, q/k head) pairs fill the chip, in equal parts where they do not.  In units of what a block takes (9 us at 64 and 128 key
+// features, 20 us at 256), a workgroup spends 0.3 on its rows of q and k, and the pass over the parts costs a half.  It is a launch more
+// too, which a call of a few chunks waits for on the host.  Training step, one part -> the number chosen:
+//   1024 tokens, 2 q/k and 16 value heads of 128   202 -> 137 us (8 parts)     2 and 8 heads of 256        322 -> 218 us (8)
+//   2048 tokens, 4 and 32 heads of 128             270 -> 238 us (2; 4: 245)   2 and 16 heads of 64        177 -> 112 us (8)
+//   2048 tokens, 8 and 32 heads of 128 (256 pairs)       231 us (2: 245)       512 tokens, 16 and 32 heads 106 -> 103 us (2)
+//   256 tokens, 16 and 32 heads of 128              89.6 us (2: 93)            layer, 1000 tokens: the kernel 87 -> 56 + 9 us (2)
+struct BwdParts {
+    int parts = 1, split = 1;
+    size_t row_bytes = 0, head_bytes = 0;        // of dq_part (dk_part), of dg_part (db_part); 0: none
+    size_t bytes() const { return 2 * ws_align(row_bytes) + 2 * ws_align(head_bytes); }
+};
+inline BwdParts bwd_parts(int64_t num_chunks, int64_t tokens, int64_t H, int64_t HV, int64_t nb, int64_t KD) {
+    const int64_t slots = KD == 64 ? 512 : 256, items = num_chunks * H, heads = HV / H * nb;
+    BwdParts x;
+    if (items >= slots) return x;
+    double best = 1e30;
+    for (int64_t n = 1; n <= heads && items * n <= 2 * slots; ++n) {
+        // whole value heads, or an equal share of one's blocks
+        if (heads % n || !((heads / n) % nb == 0 || nb % (heads / n) == 0)) continue;
+        const double cost = (double)((items * n + slots - 1) / slots) * ((double)(heads / n) + 0.3) + (n == 1 ? 0.0 : num_chunks < 8 ? 1.2 : 0.5);
+        if (cost < best) { best = cost; x.parts = (int)n; }
+    }
+    if (x.parts > 1) {
+        x.split = (int)std::max<int64_t>(1, nb / (heads / x.parts));
+        x.row_bytes = (size_t)(tokens * H * x.parts) * KD * 4;
+        if (x.split > 1) x.head_bytes = (size_t)(tokens * HV * x.split) * 4;
+    }
+    return x;
+}
 
 // The mirror image of warm_chunks() for the scan that runs backwards: how many chunks AFTER chunk it1 - 1 a run must start from a
 // zero state so that at it1 - 1 it has forgotten the difference to the true state.  When the end of the sequence comes first the
@@ -959,6 +995,34 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
 
 #include "gdn_chunk_bwd_unit.h"
 
+// The partial rows of dq and dk (and, where parts cut a value head, the partial sums of dg and dbeta) added up in fp32, in a fixed order:
+// eight rows of a chunk and q/k head per workgroup.
+template <typename T, int KD>
+__global__ __launch_bounds__(256) void gdn_bwd_add_parts_kernel(BwdParams p, int64_t) {
+    typedef typename Mma<T>::V4 V4;
+    const uint32_t unit = blockIdx.x >> 3, ch = unit / (uint32_t)p.H, hq = unit - ch * p.H;
+    const ChunkAt c = chunk_at(p, ch);
+    const int row0 = 8 * (blockIdx.x & 7), rows = min(8, c.valid - row0);        // (none: the loops below have nothing to do)
+    constexpr int PIECES = KD / 4;
+    for (int i = threadIdx.x; i < 2 * PIECES * rows; i += 256) {
+        const int piece = i % PIECES, r = i / PIECES, isk = r >= rows;
+        const int64_t row = (c.tok0 + row0 + (isk ? r - rows : r)) * p.H + hq;
+        const f32x4* part = (const f32x4*)(isk ? p.dk_part : p.dq_part) + row * p.parts * PIECES + piece;
+        f32x4 sum = part[0];
+        for (int n = 1; n < p.parts; ++n) sum += part[(int64_t)n * PIECES];
+        *(V4*)((T*)(isk ? p.dk : p.dq) + row * KD + 4 * piece) = pack4<T>(sum);
+    }
+    if (p.split > 1) {
+        const int HVg = p.HV / p.nb, group = HVg / p.H;
+        for (int i = threadIdx.x; i < group * rows; i += 256) {
+            const int64_t at = (c.tok0 + row0 + i / group) * HVg + hq * group + i % group;
+            float dg = 0.f, db = 0.f;
+            for (int n = 0; n < p.split; ++n) { dg += p.dg_part[at * p.split + n]; db += p.db_part[at * p.split + n]; }
+            p.dg[at] = dg; p.dbeta[at] = db;
+        }
+    }
+}
+
 struct BwdLaunch { const void* f; size_t smem; const char* name; unsigned grid, threads; int64_t arg; };
 static int launch_all(const BwdParams& p, const BwdLaunch* ks, int n, hipStream_t stream) {
     for (int i = 0; i < n; ++i) {
@@ -1014,7 +1078,7 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
             p.warm_cap = std::min(WARM_CAP_MAX, p.seg_chunks + p.seg_chunks / 4 + 6);
         }
     }
-    BwdLaunch ks[4] = {};
+    BwdLaunch ks[5] = {};
     const unsigned pgrid = (units + BP_WAVES - 1) / BP_WAVES;
     if constexpr (KD <= BD) ks[0] = {l2 ? (const void*)gdn_bwd_prepare_kernel<T, KD, true> : (const void*)gdn_bwd_prepare_kernel<T, KD, false>, 0, "gdn_bwd_prepare_kernel", pgrid, 64 * BP_WAVES, units};
     else ks[0] = {(const void*)gdn_bwd_prepare_kernel<T, KD, false>, 0, "gdn_bwd_prepare_kernel", pgrid, 64 * BP_WAVES, units};
@@ -1038,7 +1102,8 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
     const int64_t items = num_chunks * p.H * p.parts;
     ks[3] = {l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, true> : (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, false>,
              bwd_unit_smem<KD, VD, NW>(), "gdn_bwd_unit_kernel", (unsigned)std::min<int64_t>(items, NW == 4 ? 512 : 256), 64 * NW, items};
-    return launch_all(p, ks, 4, stream);
+    if (p.dq_part) ks[4] = {(const void*)gdn_bwd_add_parts_kernel<T, KD>, 0, "gdn_bwd_add_parts_kernel", (unsigned)(num_chunks * p.H * 8), 256, 0};
+    return launch_all(p, ks, 5, stream);
 }
 
 template <typename T>
@@ -1102,6 +1167,9 @@ static int chunk_bwd_entry(
     const size_t rows_bytes = ws_align((size_t)(B * T * H) * K * 2), factors_bytes = ws_align((size_t)(B * T * H) * 4);
     const size_t l2_at = need;
     if (l2) need += (comba ? 3 : 2) * (rows_bytes + factors_bytes);
+    const size_t parts_at = need;
+    BwdParts parts;
+    if (per_head && !comba) { parts = bwd_parts(num_chunks, B * T, H, HV, nb, K); need += parts.bytes(); }
     GDN_CHECK_ARG(workspace && workspace_bytes >= need, GDN_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who,
                   need, workspace_bytes);
     if (l2) {
@@ -1122,7 +1190,13 @@ static int chunk_bwd_entry(
     p.T = T; p.H = (int)H; p.HV = (int)(HV * nb); p.nb = (int)nb; p.N = N; p.NT = (T + CH - 1) / CH; p.tokens = B * T;
     p.scale = scale; p.gb_dtype = gb_dtype & 255; p.beta_dtype = beta_dtype_of(gb_dtype); p.flags = flags;
     p.nseg = 1; p.seg_chunks = (int)p.NT; p.warm_cap = 0;
-    p.parts = per_head ? 1 : (int)(HV / H);
+    p.parts = per_head ? parts.parts : (int)(HV / H);
+    p.split = parts.split;
+    if (parts.row_bytes) {
+        WsTake take{(char*)workspace + parts_at};
+        p.dq_part = (float*)take(parts.row_bytes); p.dk_part = (float*)take(parts.row_bytes);
+        if (parts.split > 1) { p.dg_part = (float*)take(parts.head_bytes); p.db_part = (float*)take(parts.head_bytes); }
+    }
     const bool b16 = qkv_dtype == GDN_DTYPE_BF16;
     if (comba) return b16 ? launch_bwd_comba<bf16_t>(p, num_chunks, s) : launch_bwd_comba<f16_t>(p, num_chunks, s);
     if (K == 64) return b16 ? launch_bwd<bf16_t, 64, 64>(p, num_chunks, s) : launch_bwd<f16_t, 64, 64>(p, num_chunks, s);
@@ -1148,7 +1222,7 @@ extern "C" size_t gdn_chunk_bwd_heads_workspace_bytes(int64_t num_chunks, int64_
     const int64_t VD = K == 64 ? 64 : BD;
     size_t need = bwd_ws_layout(num_chunks, HV, V / VD, K, VD, nullptr, nullptr);
     if (flags & GDN_FLAG_QK_L2NORM) need += 2 * ws_align((size_t)(tokens * H) * K * 2) + 2 * ws_align((size_t)(tokens * H) * 4);
-    return need;
+    return need + (HV % H == 0 ? bwd_parts(num_chunks, tokens, H, HV, V / VD, K).bytes() : 0);
 }
 
 extern "C" int gdn_chunk_bwd_heads(

@@ -6,7 +6,7 @@
 //   Y = dA A^T, dL = -stril(A^T Y), E = diag(beta) dL o D;   dk += E k + E^T k;   dbeta, dgam from every factor, dg = the reverse
 //   cumulative sum of dgam inside the chunk.
 //
-// One workgroup takes the value heads of a q/k head (or an even share of them, `parts`; with more value columns than VD their blocks
+// One workgroup takes the value heads of a q/k head (or an equal share of them, BwdParts; with more value columns than VD their blocks
 // count as heads) of one chunk in turn, with k and q in LDS and
 // dq, dk in fp32 registers over all of them.  What used to be two kernels moved 312 KB per chunk and value head at 128 x 128 (dw, the
 // first half of dk, dv_new, k twice, per-head dq and dk); this one moves 168 KB + 96 KB per q/k head.  Eight waves, one workgroup per
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
     TileRegs<KD, NTH> rK, rQ;
     V8 sf[SV], df[SV];
     float rGam = 0.f, rBeta = 0.f, rRq = 0.f, rRk = 0.f;
-    const int HVg = p.HV / p.nb;
+    const int HVg = p.HV / p.nb, nbp = min(p.nb, heads);        // (blocks of a value head that this item takes)
     auto fetch_state = [&](const Item& at, int hv, int a, int w, int lane) {     // feature tile a of this wave
         const int64_t u = at.ch * p.HV + hv;
         const int64_t off = u * KD * VD + (16 * (NA * w + a) + (lane & 15)) * VD + 8 * (lane >> 4);
@@ -399,11 +399,12 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
                     if (lane + off < 64) x += y;
                 }
                 // (the blocks of a value head one after the other: their sums leave together)
-                const int blk = hv % p.nb;
+                const int blk = hv % nbp;
                 dg_sum = blk ? dg_sum + x : x; db_sum = blk ? db_sum + b : b;
-                if (blk == p.nb - 1 && lane < at.c.valid) {
-                    p.dg[(at.c.tok0 + lane) * HVg + hv / p.nb] = dg_sum;
-                    p.dbeta[(at.c.tok0 + lane) * HVg + hv / p.nb] = db_sum;
+                if (blk == nbp - 1 && lane < at.c.valid) {
+                    const int64_t to = (at.c.tok0 + lane) * (p.HV / nbp) + hv / nbp;
+                    (p.split > 1 ? p.dg_part : p.dg)[to] = dg_sum;
+                    (p.split > 1 ? p.db_part : p.dbeta)[to] = db_sum;
                 }
             }
             lds_barrier();
@@ -451,8 +452,13 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
 #pragma unroll
                             for (int r = 0; r < 4; ++r) { q_[r] = (q_[r] - (float)q4[r] * qd) * rq; k_[r] = (k_[r] - (float)k4[r] * kd) * rk; }
                         }
-                        *(V4*)((T*)p.dq + row * KD + n16) = pack4<T>(q_);
-                        *(V4*)((T*)p.dk + row * KD + n16) = pack4<T>(k_);
+                        if (p.dq_part) {                        // (one of several parts of this row: gdn_bwd_add_parts_kernel)
+                            *(f32x4*)(p.dq_part + row * KD + n16) = q_;
+                            *(f32x4*)(p.dk_part + row * KD + n16) = k_;
+                        } else {
+                            *(V4*)((T*)p.dq + row * KD + n16) = pack4<T>(q_);
+                            *(V4*)((T*)p.dk + row * KD + n16) = pack4<T>(k_);
+                        }
                     }
                 }
             }
