@@ -68,12 +68,14 @@ struct NoGil {
 
 // ---- arguments ----
 // Strided memory behind it: not the tensors of tracing, vmap and the other transforms, of subclasses with a dispatch of their own, and
-// none that is sparse, nested or to be negated when it is read (the Python path says what becomes of those).
-bool has_memory(const at::Tensor& t) {
-    return t.layout() == at::kStrided && !t.is_neg() && !t.is_nested() && t.has_storage() &&
-           !t.key_set().has_any(c10::DispatchKeySet{c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
-                                                    c10::DispatchKey::Functionalize, c10::DispatchKey::ZeroTensor});
-}
+// none that is sparse, nested or to be negated when it is read (the Python path says what becomes of those).  One load
+// and one test of a tensor's keys: every call asks this of every tensor.
+const uint64_t KEYS_WITHOUT_MEMORY =
+    c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::Negative, c10::DispatchKey::Conjugate, c10::DispatchKey::ZeroTensor,
+                         c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize,
+                         c10::DispatchKey::Sparse, c10::DispatchKey::SparseCsr, c10::DispatchKey::NestedTensor, c10::DispatchKey::MkldnnCPU})
+        .raw_repr() & ~c10::full_backend_mask;
+inline bool has_memory(const at::Tensor& t) { return (t.unsafeGetTensorImpl()->key_set().raw_repr() & KEYS_WITHOUT_MEMORY) == 0; }
 
 // A tensor argument: absent (None), present, or something else.
 struct Arg {
