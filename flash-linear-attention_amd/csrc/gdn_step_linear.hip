@@ -7,7 +7,8 @@
 //
 // A step reads every weight once and little else, so it is bound by how much of the weights is in flight: a workgroup takes 16 (32)
 // output columns, its eight waves an eighth of the contraction each, all operand fragments straight from memory (a lane: 16 bytes of
-// one row; x comes from the L2), the partial sums through LDS.  16 rows x (9228 + 2048) columns of the default layer: DESIGN table.
+// one row; x comes from the L2), the partial sums through LDS.  More than 128 rows are taken 128 at a time by workgroups of their own
+// (a workgroup's tiles of rows share its registers with the weights' fragments); the weights then come from the L2 and the cache behind it.
 #include "gdn_chunk_common.h"
 
 namespace gdn {
@@ -19,7 +20,7 @@ struct StepLinearParams {
     int first[GDN_STEP_SEGMENTS + 1];            // a segment's first workgroup
 };
 
-// NT: tiles of 16 rows, CT: tiles of 16 columns per workgroup
+// NT: tiles of 16 rows, CT: tiles of 16 columns per workgroup; blockIdx.y: 16 NT rows each
 template <typename T, int NT, int CT>
 __global__ __launch_bounds__(512) void gdn_step_linear_kernel(StepLinearParams p) {
     typedef typename Mma<T>::V8 V8;
@@ -30,7 +31,7 @@ __global__ __launch_bounds__(512) void gdn_step_linear_kernel(StepLinearParams p
     while (si + 1 < p.nseg && (int)blockIdx.x >= p.first[si + 1]) ++si;
     const gdn_step_segment s = p.seg[si];
     const int col0 = ((int)blockIdx.x - p.first[si]) * 16 * CT, cols = (int)s.cols;
-    const int hidden = p.hidden, kw = hidden / WAVES;
+    const int hidden = p.hidden, kw = hidden / WAVES, row0 = (int)blockIdx.y * 16 * NT;
 
     f32x4 acc[CT][NT];
 #pragma unroll
@@ -42,7 +43,7 @@ __global__ __launch_bounds__(512) void gdn_step_linear_kernel(StepLinearParams p
 #pragma unroll
     for (int c = 0; c < CT; ++c) wr[c] = (const T*)s.weight + (int64_t)min(col0 + 16 * c + c16, cols - 1) * hidden + w * kw + 8 * g;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) xr[t] = (const T*)p.x + (int64_t)min(16 * t + c16, p.N - 1) * hidden + w * kw + 8 * g;
+    for (int t = 0; t < NT; ++t) xr[t] = (const T*)p.x + (int64_t)min(row0 + 16 * t + c16, p.N - 1) * hidden + w * kw + 8 * g;
     constexpr int U = NT >= 8 ? 2 : 4;           // steps of 32 requested together
     for (int k = 0; k < kw; k += 32 * U) {
         V8 fw[CT][U], fx[NT][U];
@@ -75,11 +76,11 @@ __global__ __launch_bounds__(512) void gdn_step_linear_kernel(StepLinearParams p
         for (int t = 0; t < NT; ++t) *(f32x4*)&part[w][16 * t + c16][4 * g] = acc[c][t];
         __syncthreads();
         for (int i = tid; i < NT * 256; i += 512) {
-            const int n = i >> 4, j = i & 15, d = col0 + 16 * c + j;
+            const int r = i >> 4, n = row0 + r, j = i & 15, d = col0 + 16 * c + j;
             if (n >= p.N || d >= cols) continue;
             float sum = 0.f;
 #pragma unroll
-            for (int x = 0; x < WAVES; ++x) sum += part[x][n][j];
+            for (int x = 0; x < WAVES; ++x) sum += part[x][r][j];
             const T yt = from_f32<T>(sum);
             const float y = to_f32(yt);
             if (s.kind == GDN_STEP_PLAIN) {
@@ -115,18 +116,18 @@ __global__ __launch_bounds__(512) void gdn_step_linear_kernel(StepLinearParams p
 
 template <typename T>
 static int launch_step_linear(StepLinearParams& p, hipStream_t stream) {
-    auto go = [&](auto kern, int ct) {
+    auto go = [&](auto kern, int ct, int nt) {
         int at = 0;
         for (int i = 0; i < p.nseg; ++i) { p.first[i] = at; at += (int)((p.seg[i].cols + 16 * ct - 1) / (16 * ct)); }
         p.first[p.nseg] = at;
-        hipLaunchKernelGGL(kern, dim3((unsigned)at), dim3(512), 0, stream, p);
+        hipLaunchKernelGGL(kern, dim3((unsigned)at, (unsigned)((p.N + 16 * nt - 1) / (16 * nt))), dim3(512), 0, stream, p);
         return check_launch("gdn_step_linear_kernel");
     };
-    if (p.N <= 16) return go(gdn_step_linear_kernel<T, 1, 1>, 1);
-    if (p.N <= 32) return go(gdn_step_linear_kernel<T, 2, 1>, 1);
+    if (p.N <= 16) return go(gdn_step_linear_kernel<T, 1, 1>, 1, 1);
+    if (p.N <= 32) return go(gdn_step_linear_kernel<T, 2, 1>, 1, 2);
     // (more rows: 32 columns, so that the rows of x are read half as often)
-    if (p.N <= 64) return go(gdn_step_linear_kernel<T, 4, 2>, 2);
-    return go(gdn_step_linear_kernel<T, 8, 2>, 2);
+    if (p.N <= 64) return go(gdn_step_linear_kernel<T, 4, 2>, 2, 4);
+    return go(gdn_step_linear_kernel<T, 8, 2>, 2, 8);
 }
 
 }  // namespace gdn

@@ -330,6 +330,10 @@ PyObject* layer_step(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int gate_code = code_of(A_log->scalar_type()), norm_code = code_of(norm_w->scalar_type());
     if (gate_code < 0 || norm_code < 0) Py_RETURN_NONE;
     const int64_t out_cols = ow->size(0);
+    // Many sequences of a large layer leave the host time behind and are products of a library's size: there the modules are faster.
+    // Native and by modules, us a step: 6 heads of 256 x 512 at 2048 (25.2 M weights), 129 sequences 219 and 335, 192 296 and 334, 256 376
+    // and 369, 512 701 and 666; 8 heads of 128 at 1024 (5.3 M weights), 129 sequences 61 and 325, 512 147 and 325, 1024 260 and 327.
+    if (N > 128 && N * ((2 * kd + 2 * vd + 2 * HV) * hidden + vd * out_cols) > 5600000000ll) Py_RETURN_NONE;
     // Every limit of the four launches: none may be refused once the first has moved the convolutions' states on.
     if (N > GDN_STEP_MAX_ROWS || std::max({hidden, kd, vd, out_cols}) > GDN_STEP_MAX_COLS || out_cols < 1 || V > GDN_NORM_MAX_ROW_BYTES / 2 ||
         (N + 8) * HV * ((V + 31) / 32) >= (1ll << 31))

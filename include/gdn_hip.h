@@ -118,7 +118,7 @@ int gdn_fused_recurrent_fwd(
  * N from 1 to GDN_STEP_MAX_ROWS, hidden a multiple of 256 and, like cols, at most GDN_STEP_MAX_COLS.
  */
 #define GDN_STEP_SEGMENTS 6
-#define GDN_STEP_MAX_ROWS 128
+#define GDN_STEP_MAX_ROWS 4096
 #define GDN_STEP_MAX_COLS ((1 << 24) - 1)
 #define GDN_STEP_PLAIN 0
 #define GDN_STEP_CONV  1

@@ -71,3 +71,20 @@ def test_layer_step_in_four_launches(N, hidden, heads, v_heads, D, expand, conv,
         assert O.get_err_ratio(caches[1][0]['recurrent_state'], caches[0][0]['recurrent_state']) < 2e-3
         for a, b in zip(caches[1][0]['conv_state'], caches[0][0]['conv_state']):
             assert O.get_err_ratio(a.float(), b.float()) < 2e-3
+
+
+@pytest.mark.parametrize('N', [128, 129, 255, 257])
+def test_layer_step_beyond_one_tile_of_rows(N, monkeypatch):
+    test_layer_step_in_four_launches(N, 512, 2, 4, 64, 1, 4, False, monkeypatch)
+
+
+def test_layer_step_leaves_many_sequences_of_a_large_layer_to_its_modules():
+    from fla_hip.layers import GatedDeltaNet
+    from fla_hip.layers.gated_deltanet import LayerCache
+    layer = GatedDeltaNet(hidden_size=2048, layer_idx=0).cuda().bfloat16().eval()
+    for N, native in ((192, True), (256, False)):
+        cache = LayerCache()
+        cache.update(layer_idx=0, recurrent_state=torch.zeros(N, 6, 512, 256, device='cuda'),
+                     conv_state=tuple(torch.zeros(N, d, 4, device='cuda', dtype=torch.bfloat16) for d in (1536, 1536, 3072)))
+        x = torch.randn(N, 1, 2048, device='cuda', dtype=torch.bfloat16)
+        assert (layer._step(x, cache) is not None) == native
