@@ -14,6 +14,14 @@ at::Tensor sum_rows(const at::Tensor& part, at::ScalarType type, at::IntArrayRef
     return out;
 }
 
+// A saved tensor as the kernels read it.  Saved-tensor hooks (offloading, checkpointing, compression) may hand back another layout,
+// place or type than they were given.
+at::Tensor saved(const at::Tensor& t, at::ScalarType type, c10::Device dev) {
+    if (!t.defined() || (t.scalar_type() == type && t.device() == dev && t.is_contiguous() && aligned16(t.data_ptr()))) return t;
+    const at::Tensor r = t.to(at::TensorOptions().dtype(type).device(dev)).contiguous();
+    return aligned16(r.data_ptr()) ? r : r.clone();
+}
+
 // What a call of the operator is made of besides its tensors.
 struct ChunkCall {
     int64_t B, T, H, HV, K, V, N, num_chunks;
@@ -80,6 +88,8 @@ struct ChunkTrain : torch::autograd::Function<ChunkTrain> {
         ctx->save_for_backward({q, k, v, g, beta, h0, A_log, dt_bias, cu, table, offsets});
         ctx->saved_data["dims"] = std::vector<int64_t>{c.B, c.T, c.H, c.HV, c.K, c.V, c.N, c.num_chunks, (int64_t)c.flags, c.out_final, c.vfirst, c.whole};
         ctx->saved_data["scale"] = c.scale;
+        ctx->saved_data["types"] = std::vector<int64_t>{(int64_t)q.scalar_type(), (int64_t)(g.defined() ? g : beta).scalar_type(), (int64_t)beta.scalar_type()};
+        ctx->saved_data["device"] = q.device();
         ctx->set_materialize_grads(false);
         if (!c.out_final) return {o};
         return {o, ht};
@@ -89,12 +99,17 @@ struct ChunkTrain : torch::autograd::Function<ChunkTrain> {
         return cb == cg ? cg : GDN_GB_DTYPES(cg, cb);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
-        const auto s = ctx->get_saved_variables();
+        const c10::Device dev = ctx->saved_data["device"].toDevice();
+        const c10::DeviceGuard guard(dev);
+        const std::vector<int64_t> types = ctx->saved_data["types"].toIntVector();
+        auto s = ctx->get_saved_variables();
+        for (int i = 0; i < 5; ++i) s[i] = saved(s[i], (at::ScalarType)types[std::max(0, i - 2)], dev);
+        for (int i = 5; i < (int)s.size(); ++i)
+            if (s[i].defined()) s[i] = saved(s[i], i == 5 ? at::kFloat : s[i].scalar_type(), dev);
         const at::Tensor &q = s[0], &k = s[1], &v = s[2], &g = s[3], &beta = s[4], &h0 = s[5], &A_log = s[6], &dt_bias = s[7];
         const std::vector<int64_t> n = ctx->saved_data["dims"].toIntVector();
         const ChunkCall c{n[0], n[1], n[2], n[3], n[4], n[5], n[6], n[7], ctx->saved_data["scale"].toDouble(), (uint32_t)n[8], n[9] != 0, n[10] != 0, n[11] != 0};
-        const c10::DeviceGuard guard(q.device());
-        void* stream = stream_of(q.device());
+        void* stream = stream_of(dev);
         at::Tensor dout = grads[0].defined() ? grads[0].to(v.scalar_type()).contiguous() : at::zeros_like(v);
         if (!aligned16(dout.data_ptr())) dout = dout.clone();
         const at::Tensor A = to_f32(A_log), dt = to_f32(dt_bias);
@@ -198,6 +213,8 @@ struct LayerTrain : torch::autograd::Function<LayerTrain> {
         for (const at::Tensor& t : {w, p, gate, qkv[0], qkv[1], qkv[2], graw, braw, o, y, rstd}) keep.push_back(t);
         ctx->save_for_backward(keep);
         ctx->saved_data["heads"] = heads;
+        ctx->saved_data["type"] = (int64_t)type;
+        ctx->saved_data["device"] = dev;
         ctx->saved_data["neg"] = neg;
         return {out};
     }
@@ -206,12 +223,14 @@ struct LayerTrain : torch::autograd::Function<LayerTrain> {
                          GDN_FLAG_QK_L2NORM | GDN_FLAG_BETA_SIGMOID | GDN_FLAG_STATE_V_FIRST | (neg ? GDN_FLAG_NEG_EIGVAL : 0u), false, true};
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
-        const auto s = ctx->get_saved_variables();
+        const c10::Device dev = ctx->saved_data["device"].toDevice();
+        const c10::DeviceGuard guard(dev);
+        const at::ScalarType type = (at::ScalarType)ctx->saved_data["type"].toInt();
+        auto s = ctx->get_saved_variables();
+        for (int i = 0; i < (int)s.size(); ++i)
+            s[i] = saved(s[i], i >= A_LOG && i <= NW ? s[i].scalar_type() : i == INPUTS + 10 ? at::kFloat : type, dev);
         const at::Tensor &w = s[INPUTS], &p = s[INPUTS + 1], &gate = s[INPUTS + 2], *qkv = &s[INPUTS + 3], &graw = s[INPUTS + 6], &braw = s[INPUTS + 7],
                          &o = s[INPUTS + 8], &y = s[INPUTS + 9], &rstd = s[INPUTS + 10], &x = s[X];
-        const c10::Device dev = x.device();
-        const c10::DeviceGuard guard(dev);
-        const at::ScalarType type = x.scalar_type();
         void* stream = stream_of(dev);
         const int code = code_of(type);
         const int64_t heads = ctx->saved_data["heads"].toInt();

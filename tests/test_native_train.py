@@ -1,6 +1,8 @@
 """The native training path against the Python path behind it: the operator (same kernels, same bits), the layer (one product for the
 projections instead of six: same numbers up to rounding), and the kernels of its backward - the gate's, the sums of partial rows, runs
 of the convolution that end inside a sequence."""
+import contextlib
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -77,3 +79,38 @@ def test_gate_backward(rows, HV, beta_max):
     sums = out[2].double().sum(0).cpu()
     for r, o, bar in ((ref[0], out[0], 1e-5), (ref[1], out[1], 4e-3), (ref[2], sums[0], 1e-4), (ref[3], sums[1], 1e-4)):
         assert O.get_err_ratio(r, o.double().cpu()) < bar
+
+
+@pytest.mark.parametrize('what', ['operator', 'layer'])
+def test_saved_tensors_may_come_back_in_another_layout_and_place(what):
+    """Saved-tensor hooks: every tensor goes to the host and comes back strided, in fp32 where it was of 16 bits."""
+    from fla_hip.layers import GatedDeltaNet
+    from fla_hip.ops.gated_delta_rule import chunk_gated_delta_rule
+    gen = torch.Generator(device='cuda').manual_seed(2)
+    rn = lambda *s: torch.randn(*s, generator=gen, device='cuda')
+    if what == 'operator':
+        leaves = [rn(1, 130, 2, 128).bfloat16(), rn(1, 130, 2, 128).bfloat16(), rn(1, 130, 4, 128).bfloat16(), rn(1, 130, 4), rn(1, 130, 4).bfloat16(),
+                  rn(2, 4, 128, 128), rn(4), rn(4)]
+        leaves = [x.requires_grad_() for x in leaves]
+        cu = torch.tensor([0, 60, 130], device='cuda')
+        call = lambda: chunk_gated_delta_rule(*leaves[:5], initial_state=leaves[5], cu_seqlens=cu, use_qk_l2norm_in_kernel=True, use_gate_in_kernel=True,
+                                              A_log=leaves[6], dt_bias=leaves[7], use_beta_sigmoid_in_kernel=True)[0]
+    else:
+        torch.manual_seed(3)
+        layer = GatedDeltaNet(hidden_size=256, head_dim=64, expand_v=1, num_heads=4).cuda().bfloat16().train()
+        x = rn(1, 130, 256).bfloat16().requires_grad_()
+        leaves = [x, *layer.parameters()]
+        call = lambda: layer(x)[0]
+
+    def unpack(x):
+        x = x.cuda()
+        if x.dtype == torch.bfloat16:
+            x = x.float()
+        return torch.stack([x, torch.zeros_like(x)], -1)[..., 0]
+
+    def grads(*hooks):
+        with torch.autograd.graph.saved_tensors_hooks(*hooks) if hooks else contextlib.nullcontext():
+            o = call()
+        return torch.autograd.grad(o, leaves, torch.ones_like(o))
+    for i, (a, b) in enumerate(zip(grads(), grads(lambda x: x.cpu(), unpack))):
+        assert a.dtype == b.dtype and O.get_err_ratio(a.float(), b.float()) < 1e-3, f'gradient {i}'
