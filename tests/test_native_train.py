@@ -8,6 +8,7 @@ import torch
 import torch.nn.functional as F
 
 from oracle import gdn_oracle as O
+from oracle import modules_oracle as M
 
 pytestmark = pytest.mark.gpu
 
@@ -114,3 +115,49 @@ def test_saved_tensors_may_come_back_in_another_layout_and_place(what):
         return torch.autograd.grad(o, leaves, torch.ones_like(o))
     for i, (a, b) in enumerate(zip(grads(), grads(lambda x: x.cpu(), unpack))):
         assert a.dtype == b.dtype and O.get_err_ratio(a.float(), b.float()) < 1e-3, f'gradient {i}'
+
+
+def _layer_in_float64(layer, x, dy):
+    """The layer's output and gradients by the oracle, from its (16-bit) weights and input in 64 bits."""
+    p = {n: t.detach().double().cpu().requires_grad_(True) for n, t in layer.named_parameters()}
+    xd = x.detach().double().cpu().requires_grad_(True)
+    B, T, _ = xd.shape
+    heads = dict(q=layer.num_heads, k=layer.num_heads, v=layer.num_v_heads)
+    q, k, v = (M.causal_conv1d(xd @ p[f'{n}_proj.weight'].t(), p[f'{n}_conv1d.weight'].squeeze(1), activation='silu', dtype=torch.float64)[0]
+               .view(B, T, h, -1) for n, h in heads.items())
+    o, _ = O.recurrent_gated_delta_rule(q, k, v, xd @ p['a_proj.weight'].t(), xd @ p['b_proj.weight'].t(), use_qk_l2norm_in_kernel=True,
+                                        use_gate_in_kernel=True, A_log=p['A_log'], dt_bias=p['dt_bias'], use_beta_sigmoid_in_kernel=True,
+                                        allow_neg_eigval=layer.allow_neg_eigval, dtype=torch.float64)
+    gate = (xd @ p['g_proj.weight'].t()).view(o.shape)
+    y = M.norm_gated(o.reshape(-1, o.shape[-1]), gate.reshape(-1, o.shape[-1]), p['o_norm.weight'], eps=layer.o_norm.eps, is_rms_norm=True,
+                     dtype=torch.float64)[0]
+    out = y.view(B, T, -1) @ p['o_proj.weight'].t()
+    return (out.detach(), *torch.autograd.grad(out, [xd, *p.values()], dy.double().cpu()))
+
+
+@pytest.mark.parametrize('B,T,hidden,heads,D,expand,HV,neg', [(2, 130, 256, 2, 64, 1, 2, False), (1, 65, 1024, 2, 256, 2, 4, True), (1, 300, 256, 3, 128, 1, 3, False)])
+def test_layer_against_float64(B, T, hidden, heads, D, expand, HV, neg):
+    """Output and gradients of the native step, and of the same step module by module, against 64 bits."""
+    from fla_hip.layers import GatedDeltaNet
+    torch.manual_seed(1)
+    layer = GatedDeltaNet(hidden_size=hidden, expand_v=expand, head_dim=D, num_heads=heads, num_v_heads=HV, allow_neg_eigval=neg).cuda().bfloat16().train()
+    x = torch.randn(B, T, hidden, device='cuda').bfloat16().requires_grad_(True)
+    dy = torch.randn(B, T, hidden, device='cuda').bfloat16()
+    names, params = zip(*layer.named_parameters())
+
+    def step():
+        o = layer(x)[0]
+        return [t.double().cpu() for t in (o, *torch.autograd.grad(o, [x, *params], dy))]
+    ref = _layer_in_float64(layer, x, dy)
+    assert layer._train(x) is not None
+    native = step()
+    hook = layer.q_proj.register_forward_hook(lambda *a: None)
+    parts = step()
+    hook.remove()
+    for name, r, a, b in zip(('o', 'dx', *names), ref, native, parts):
+        # A value rounded to bf16 is off by 2^-9 / sqrt(3) = 1.1e-3 on average, and a gradient passes through some twenty such roundings
+        # in a row (the layer's eight stages and the chunked operator's operands): 5e-3, twice that allowed.  The gradients of A_log and
+        # dt_bias are sums over all tokens of terms of both signs: twice that again.
+        native_err, parts_err = O.get_err_ratio(r, a), O.get_err_ratio(r, b)
+        assert native_err < (2e-2 if name in ('A_log', 'dt_bias') else 1e-2), f'{name}: {native_err:.2e}'
+        assert native_err < 1.05 * parts_err, f'{name}: {native_err:.2e}, module by module {parts_err:.2e}'
