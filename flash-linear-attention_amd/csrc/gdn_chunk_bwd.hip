@@ -1100,8 +1100,10 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
     }
     constexpr int NW = KD == 64 ? 4 : 8;
     const int64_t items = num_chunks * p.H * p.parts;
-    ks[3] = {l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, true> : (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, false>,
-             bwd_unit_smem<KD, VD, NW>(), "gdn_bwd_unit_kernel", (unsigned)std::min<int64_t>(items, NW == 4 ? 512 : 256), 64 * NW, items};
+    constexpr bool APART = KD <= BD;
+    const void* unit = APART && p.dq_part ? (l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, true, APART> : (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, false, APART>)
+                                          : (l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, true, false> : (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, false, false>);
+    ks[3] = {unit, bwd_unit_smem<KD, VD, NW>(), "gdn_bwd_unit_kernel", (unsigned)std::min<int64_t>(items, NW == 4 ? 512 : 256), 64 * NW, items};
     if (p.dq_part) ks[4] = {(const void*)gdn_bwd_add_parts_kernel<T, KD>, 0, "gdn_bwd_add_parts_kernel", (unsigned)(num_chunks * p.H * 8), 256, 0};
     return launch_all(p, ks, 5, stream);
 }

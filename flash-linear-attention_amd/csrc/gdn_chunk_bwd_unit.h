@@ -28,7 +28,9 @@ template <int KD, int VD, int NW> constexpr size_t bwd_unit_smem() {
 // Computed here and not where it is used (the compiler would sink a sum to its use and keep all its terms in registers until then).
 __device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
 
-template <typename T, int KD, int VD, int NW, bool L2>
+// PARTS: rows and sums leave in fp32 to be added up (BwdParts).  At 128 key features the kernel loses 3 % to a choice of its own (16000
+// packed tokens, 32 heads: the step 1084 -> 1097 us), at 256 it makes one (3855 us with two kernels, 3824 us; 8 x 2048 tokens, 32 heads).
+template <typename T, int KD, int VD, int NW, bool L2, bool PARTS>
 __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, int64_t items) {
     typedef typename Mma<T>::V8 V8;
     typedef typename Mma<T>::V4 V4;
@@ -55,7 +57,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
     TileRegs<KD, NTH> rK, rQ;
     V8 sf[SV], df[SV];
     float rGam = 0.f, rBeta = 0.f, rRq = 0.f, rRk = 0.f;
-    const int HVg = p.HV / p.nb, nbp = min(p.nb, heads);        // (blocks of a value head that this item takes)
+    const int HVg = p.HV / p.nb;
+    const bool parts_out = LEAN ? p.dq_part != nullptr : PARTS;
     auto fetch_state = [&](const Item& at, int hv, int a, int w, int lane) {     // feature tile a of this wave
         const int64_t u = at.ch * p.HV + hv;
         const int64_t off = u * KD * VD + (16 * (NA * w + a) + (lane & 15)) * VD + 8 * (lane >> 4);
@@ -399,12 +402,13 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
                     if (lane + off < 64) x += y;
                 }
                 // (the blocks of a value head one after the other: their sums leave together)
+                const int nbp = parts_out ? min(p.nb, heads) : p.nb;     // (blocks of a value head that this item takes)
                 const int blk = hv % nbp;
                 dg_sum = blk ? dg_sum + x : x; db_sum = blk ? db_sum + b : b;
                 if (blk == nbp - 1 && lane < at.c.valid) {
-                    const int64_t to = (at.c.tok0 + lane) * (p.HV / nbp) + hv / nbp;
-                    (p.split > 1 ? p.dg_part : p.dg)[to] = dg_sum;
-                    (p.split > 1 ? p.db_part : p.dbeta)[to] = db_sum;
+                    const int64_t to = (at.c.tok0 + lane) * (parts_out ? p.HV / nbp : HVg) + hv / nbp;
+                    (parts_out && p.split > 1 ? p.dg_part : p.dg)[to] = dg_sum;
+                    (parts_out && p.split > 1 ? p.db_part : p.dbeta)[to] = db_sum;
                 }
             }
             lds_barrier();
@@ -452,7 +456,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
 #pragma unroll
                             for (int r = 0; r < 4; ++r) { q_[r] = (q_[r] - (float)q4[r] * qd) * rq; k_[r] = (k_[r] - (float)k4[r] * kd) * rk; }
                         }
-                        if (p.dq_part) {                        // (one of several parts of this row: gdn_bwd_add_parts_kernel)
+                        if (parts_out) {                  // (one of several parts of this row: gdn_bwd_add_parts_kernel)
                             *(f32x4*)(p.dq_part + row * KD + n16) = q_;
                             *(f32x4*)(p.dk_part + row * KD + n16) = k_;
                         } else {
