@@ -36,6 +36,7 @@ def lib(monkeypatch):
     lib = Library()
     monkeypatch.setattr(_lib, 'load', lambda: lib)
     monkeypatch.setattr(torch.cuda, 'device', lib.device)
+    monkeypatch.setattr(_common, 'current_device', lambda: 7)
     for m in (_common, convolution, fused_norm_gate):
         monkeypatch.setattr(m, 'current_stream_ptr', lambda dev: 0)
     for m in (_common, chunk_bwd, convolution, fused_norm_gate, kda_chunk, comba_chunk, comba_recurrent, delta_recurrent):
@@ -76,6 +77,12 @@ def test_launches_are_made_on_the_tensors_device(lib, call):
     v, g, gk = torch.zeros(1, 70, 2, 64), torch.zeros(1, 70, 2), torch.zeros(1, 70, 2, 64)
     CALLS[call](q, k, v, g, torch.ones(1, 70, 2), gk)
     assert lib.calls and all(inside for _, inside in lib.calls), lib.calls
+
+
+def test_no_guard_where_the_device_is_current(lib, monkeypatch):
+    monkeypatch.setattr(_common, 'current_device', lambda: None)         # (the index of the CPU device the tensors are on)
+    _common.sum_rows(torch.zeros(3, 8), torch.bfloat16)
+    assert lib.calls == [('gdn_sum_rows', False)]
 
 
 def test_sums_of_partial_rows_in_any_type(lib):
