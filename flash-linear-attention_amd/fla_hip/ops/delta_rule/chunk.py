@@ -3,7 +3,7 @@ validation and error types of fla/ops/delta_rule/chunk.py:223-349.  It is the ga
 g = 0 (the reference runs the same state and output kernels with ``g=None``,
 fla/ops/delta_rule/chunk.py:39-62), so it runs on the same HIP kernels: the library takes
 ``g = NULL`` and skips nothing but the gate load.  Differentiable like the gated operator (backward through
-``gdn_chunk_bwd`` with ``g = NULL``; the reference's own backward is fla/ops/delta_rule/chunk.py:65-140)."""
+``gdn_chunk_bwd_heads`` with ``g = NULL``; the reference's own backward is fla/ops/delta_rule/chunk.py:65-140)."""
 from __future__ import annotations
 
 import torch

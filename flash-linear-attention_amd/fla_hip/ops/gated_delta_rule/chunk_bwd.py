@@ -1,9 +1,9 @@
 """Backward of ``chunk_gated_delta_rule``: ``chunk_gated_delta_rule_bwd`` with the argument meaning of
 fla/ops/gated_delta_rule/chunk.py:125-257 and the autograd function around forward and backward
-(chunk.py:260-395).  One call into libgdn_hip.so (``gdn_chunk_bwd``) replaces the reference's seven launches;
-nothing is kept from the forward call but its inputs (A, w, u, the per-chunk states and v_new are computed
-again).  The activations the forward kernels apply themselves (l2 norm of q and k, gate, beta sigmoid) and
-their derivatives are elementwise work around that call, as in the reference (chunk.py:278-288, 385-393)."""
+(chunk.py:260-395) for calls that the native one (csrc/host/gdn_host_train.h) leaves.  One call into libgdn_hip.so
+(``gdn_chunk_bwd_heads``) replaces the reference's seven launches and, with the in-kernel l2 norm, the four around them
+(chunk.py:278-288, 385-393); nothing is kept from the forward call but its inputs (A, P, the per-chunk states and v_new are computed
+again).  The derivatives of the gate and of beta's sigmoid are one more kernel (``gate_bwd``)."""
 from __future__ import annotations
 
 import os
@@ -196,7 +196,7 @@ def l2norm_fwd(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
 
 
 class ChunkGatedDeltaRuleFunction(torch.autograd.Function):
-    """Forward through the fused inference kernels, backward through ``gdn_chunk_bwd``."""
+    """Forward through the fused inference kernels, backward through ``gdn_chunk_bwd_heads``."""
 
     @staticmethod
     def forward(ctx, q, k, v, g, beta, scale, initial_state, output_final_state, state_v_first, cu_seqlens,

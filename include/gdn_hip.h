@@ -277,7 +277,7 @@ int gdn_chunk_fwd_scan(
  * recompute_w_u_fwd (fla/ops/gated_delta_rule/wy_fast.py:236-296), chunk_gated_delta_rule_fwd_h and
  * chunk_gated_delta_rule_bwd_dhu (fla/ops/common/chunk_delta_h.py:563-744, 747-828), chunk_bwd_dv_local and
  * chunk_bwd_dqkwg (fla/ops/common/chunk_o.py:647-697, 700-779), prepare_wy_repr_bwd (wy_fast.py:298-351) and the
- * reverse chunk_local_cumsum of dg (fla/ops/utils/cumsum.py).  Nothing is kept from the forward call: A, w, u, the
+ * reverse chunk_local_cumsum of dg (fla/ops/utils/cumsum.py).  Nothing is kept from the forward call: A, P, the
  * per-chunk states and v_new are computed again, into the workspace.
  *   q, k [B,T,H,K]; v, dout [B,T,HV,V] (qkv_dtype: bf16 or f16); g (log decay, may be NULL), beta [B,T,HV] (gb_dtype),
  *   both as the recurrence uses them: the activations of the forward call (l2 norm, gate, sigmoid) and their
@@ -334,6 +334,7 @@ int gdn_chunk_bwd_qk_l2norm(
  *   flags: also GDN_FLAG_QK_L2NORM (dq, dk: gradients of the rows before normalisation), GDN_FLAG_BETA_SIGMOID, GDN_FLAG_NEG_EIGVAL,
  *   GDN_FLAG_SEQ_ORDER; gb_dtype may be GDN_GB_DTYPES(g, beta)
  *   workspace: at least gdn_chunk_bwd_heads_workspace_bytes(num_chunks, H, HV, K, V, B * T, flags) bytes (0: unsupported K, V)
+ *   (calls of few chunks and q/k heads reserve fp32 parts of dq and dk there, at most 64 MB)
  */
 size_t gdn_chunk_bwd_heads_workspace_bytes(int64_t num_chunks, int64_t H, int64_t HV, int64_t K, int64_t V, int64_t tokens, uint32_t flags);
 int gdn_chunk_bwd_heads(
