@@ -1171,7 +1171,9 @@ static int chunk_bwd_entry(
     if (l2) need += (comba ? 3 : 2) * (rows_bytes + factors_bytes);
     const size_t parts_at = need;
     BwdParts parts;
-    if (per_head && !comba) { parts = bwd_parts(num_chunks, B * T, H, HV, nb, K); need += parts.bytes(); }
+    if (per_head && !comba) parts = bwd_parts(num_chunks, B * T, H, HV, nb, K);
+    if (workspace_bytes < need + parts.bytes()) parts = BwdParts();      // (a caller's workspace without room for them: one part)
+    need += parts.bytes();
     GDN_CHECK_ARG(workspace && workspace_bytes >= need, GDN_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who,
                   need, workspace_bytes);
     if (l2) {

@@ -334,7 +334,7 @@ int gdn_chunk_bwd_qk_l2norm(
  *   flags: also GDN_FLAG_QK_L2NORM (dq, dk: gradients of the rows before normalisation), GDN_FLAG_BETA_SIGMOID, GDN_FLAG_NEG_EIGVAL,
  *   GDN_FLAG_SEQ_ORDER; gb_dtype may be GDN_GB_DTYPES(g, beta)
  *   workspace: at least gdn_chunk_bwd_heads_workspace_bytes(num_chunks, H, HV, K, V, B * T, flags) bytes (0: unsupported K, V)
- *   (calls of few chunks and q/k heads reserve fp32 parts of dq and dk there, at most 64 MB)
+ *   (calls of few chunks and q/k heads reserve fp32 parts of dq and dk there, at most 64 MB; without that room they run slower)
  */
 size_t gdn_chunk_bwd_heads_workspace_bytes(int64_t num_chunks, int64_t H, int64_t HV, int64_t K, int64_t V, int64_t tokens, uint32_t flags);
 int gdn_chunk_bwd_heads(

@@ -68,3 +68,32 @@ def test_parts_against_the_oracle(B, T, H, HV, K, V, cu, dtype, l2):
         at = (lambda x: x) if n == 'dh0' else lambda x: x[:, inside]
         err = O.get_err_ratio(at(ref[n]), at(got.float().cpu()))
         assert err <= bar, f'{n}: rel-rmse {err:.3e}'
+
+
+@pytest.mark.gpu
+def test_a_workspace_without_room_for_parts_is_enough():
+    """The C entry with the workspace of the call's other arrays alone: all heads of a group in one workgroup, the same gradients."""
+    from fla_hip import _lib
+    lib = _lib.load()
+    B, T, H, HV, D = 1, 300, 2, 8, 128
+    nc = 5
+    gen = torch.Generator(device='cuda').manual_seed(7)
+    rn = lambda *s: torch.randn(*s, generator=gen, device='cuda')
+    q, k = (F.normalize(rn(B, T, H, D), dim=-1).bfloat16() for _ in range(2))
+    v, do = rn(B, T, HV, D).bfloat16(), rn(B, T, HV, D).bfloat16()
+    g, beta = F.logsigmoid(rn(B, T, HV)), rn(B, T, HV).sigmoid()
+    full, least = (lib.gdn_chunk_bwd_heads_workspace_bytes(nc, h, HV, D, D, B * T, 0) for h in (H, HV))
+    assert full > least
+    out = []
+    for size, status in ((full, 0), (least, 0), (least - 256, _lib.GDN_ERR_WORKSPACE)):
+        ws = torch.empty(size, dtype=torch.uint8, device='cuda')
+        grads = [torch.zeros_like(q), torch.zeros_like(k), torch.zeros_like(v), torch.zeros_like(g), torch.zeros_like(beta)]
+        rc = lib.gdn_chunk_bwd_heads(
+            *(x.data_ptr() for x in (q, k, v, g, beta)), None, None, None, do.data_ptr(), None, *(x.data_ptr() for x in grads), None,
+            None, None, None, ws.data_ptr(), size, B, T, H, HV, D, D, B, nc, D ** -0.5, _lib.DTYPE_BF16, _lib.DTYPE_F32, 0,
+            torch.cuda.current_stream().cuda_stream)
+        assert rc == status
+        out.append(grads)
+    # (dq and dk: the same fp32 sums in another order, each rounded to bf16 once; the rest: the same bits)
+    for a, b, bar in zip(out[0], out[1], (1e-3, 1e-3, 0, 0, 0)):
+        assert (torch.equal(a, b) if bar == 0 else O.get_err_ratio(b.float(), a.float()) < bar)
