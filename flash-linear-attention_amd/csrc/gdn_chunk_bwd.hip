@@ -118,7 +118,8 @@ struct BwdParams {
 // How a q/k head's value heads (their blocks of columns, `nb` each) are dealt out to the workgroups of gdn_bwd_unit_kernel: all to one
 // where (chunk, q/k head) pairs fill the chip, in equal parts where they do not.  In units of what a block takes (9 us at 64 and 128 key
 // features, 20 us at 256), a workgroup spends 0.3 on its rows of q and k, and the pass over the parts costs a half.  It is a launch more
-// too, which a call of a few chunks waits for on the host.  Training step, one part -> the number chosen:
+// too, which a call waits for on the host where its sequences are short (fewer than 8 chunks on average, of `num_seqs`): not for one
+// block saved.  (The workspace is sized as for one sequence: never smaller.)  Training step, one part -> the number chosen:
 //   1024 tokens, 2 q/k and 16 value heads of 128   202 -> 137 us (8 parts)     2 and 8 heads of 256        322 -> 218 us (8)
 //   2048 tokens, 4 and 32 heads of 128             270 -> 238 us (2; 4: 245)   2 and 16 heads of 64        177 -> 112 us (8)
 //   2048 tokens, 8 and 32 heads of 128 (256 pairs)       231 us (2: 245)       512 tokens, 16 and 32 heads 106 -> 103 us (2)
@@ -128,7 +129,7 @@ struct BwdParts {
     size_t row_bytes = 0, head_bytes = 0;        // of dq_part (dk_part), of dg_part (db_part); 0: none
     size_t bytes() const { return 2 * ws_align(row_bytes) + 2 * ws_align(head_bytes); }
 };
-inline BwdParts bwd_parts(int64_t num_chunks, int64_t tokens, int64_t H, int64_t HV, int64_t nb, int64_t KD) {
+inline BwdParts bwd_parts(int64_t num_chunks, int64_t num_seqs, int64_t tokens, int64_t H, int64_t HV, int64_t nb, int64_t KD) {
     const int64_t slots = KD == 64 ? 512 : 256, items = num_chunks * H, heads = HV / H * nb;
     BwdParts x;
     if (items >= slots) return x;
@@ -136,7 +137,7 @@ inline BwdParts bwd_parts(int64_t num_chunks, int64_t tokens, int64_t H, int64_t
     for (int64_t n = 1; n <= heads && items * n <= 2 * slots; ++n) {
         // whole value heads, or an equal share of one's blocks
         if (heads % n || !((heads / n) % nb == 0 || nb % (heads / n) == 0)) continue;
-        const double cost = (double)((items * n + slots - 1) / slots) * ((double)(heads / n) + 0.3) + (n == 1 ? 0.0 : num_chunks < 8 ? 1.2 : 0.5);
+        const double cost = (double)((items * n + slots - 1) / slots) * ((double)(heads / n) + 0.3) + (n == 1 ? 0.0 : num_chunks < 8 * num_seqs ? 1.2 : 0.5);
         if (cost < best) { best = cost; x.parts = (int)n; }
     }
     if (x.parts > 1) {
@@ -1171,7 +1172,7 @@ static int chunk_bwd_entry(
     if (l2) need += (comba ? 3 : 2) * (rows_bytes + factors_bytes);
     const size_t parts_at = need;
     BwdParts parts;
-    if (per_head && !comba) parts = bwd_parts(num_chunks, B * T, H, HV, nb, K);
+    if (per_head && !comba) parts = bwd_parts(num_chunks, N, B * T, H, HV, nb, K);
     if (workspace_bytes < need + parts.bytes()) parts = BwdParts();      // (a caller's workspace without room for them: one part)
     need += parts.bytes();
     GDN_CHECK_ARG(workspace && workspace_bytes >= need, GDN_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who,
@@ -1226,7 +1227,7 @@ extern "C" size_t gdn_chunk_bwd_heads_workspace_bytes(int64_t num_chunks, int64_
     const int64_t VD = K == 64 ? 64 : BD;
     size_t need = bwd_ws_layout(num_chunks, HV, V / VD, K, VD, nullptr, nullptr);
     if (flags & GDN_FLAG_QK_L2NORM) need += 2 * ws_align((size_t)(tokens * H) * K * 2) + 2 * ws_align((size_t)(tokens * H) * 4);
-    return need + (HV % H == 0 ? bwd_parts(num_chunks, tokens, H, HV, V / VD, K).bytes() : 0);
+    return need + (HV % H == 0 ? bwd_parts(num_chunks, 1, tokens, H, HV, V / VD, K).bytes() : 0);
 }
 
 extern "C" int gdn_chunk_bwd_heads(
