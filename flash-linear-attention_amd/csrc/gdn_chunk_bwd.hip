@@ -35,12 +35,11 @@ namespace gdn {
 // Comba adds gam0 and dgam [64] fp32 (dgam partial, between the last two kernels), P^T in P's place, w, dw [64][128], u [64][128].
 // The KDA operator (a decay per key feature) has instead: Gk, the running sums of the log decays [64][128] fp32; QG = scale q e^Gk,
 // KG = k e^(Gk_last - Gk) [64][128] and P [64][64] in the operand type, EGL = e^Gk_last [128] fp32 (all four as the forward's
-// chunk-parallel kernel writes them); dPs = scale tril(do v_new^T) [64][64]; dGk [64][128] fp32 (partial, between the last two kernels);
-// u and v_new share their place.
+// chunk-parallel kernel writes them); w, u; u and v_new share their place.
 struct BwdWs {
     float* Gam; float* Bet; float* Dgam; float* Gam0;
     void* Am; void* PT; void* Wm; void* Vn; void* Hs; void* dHs; void* dVn; void* dWm;
-    float* Gk; void* QG; void* KG; void* Pm; float* EGL; void* dPs; float* dGk;
+    float* Gk; void* QG; void* KG; void* Pm; float* EGL;
     void* Um; float* Bound;
 };
 struct WsTake {
@@ -75,12 +74,12 @@ inline size_t kda_bwd_ws_layout(int64_t units, char* base, BwdWs* ws) {
     WsTake take{base};
     const size_t u = (size_t)units;
     BwdWs x{};
-    x.Am = take(u * 64 * 64 * 2); x.Pm = take(u * 64 * 64 * 2); x.dPs = take(u * 64 * 64 * 2);
+    x.Am = take(u * 64 * 64 * 2); x.Pm = take(u * 64 * 64 * 2);
     x.Wm = take(u * 64 * BD * 2); x.Um = x.Vn = take(u * 64 * BD * 2);
     x.QG = take(u * 64 * BD * 2); x.KG = take(u * 64 * BD * 2);
     x.Hs = take(u * BD * BD * 2); x.dHs = take(u * BD * BD * 2);
-    x.dVn = take(u * 64 * BD * 2); x.dWm = take(u * 64 * BD * 2);
-    x.Gk = (float*)take(u * 64 * BD * 4); x.dGk = (float*)take(u * 64 * BD * 4); x.EGL = (float*)take(u * BD * 4);
+    x.dVn = take(u * 64 * BD * 2);
+    x.Gk = (float*)take(u * 64 * BD * 4); x.EGL = (float*)take(u * BD * 4);
     if (ws) *ws = x;
     return take.off;
 }
@@ -1338,7 +1337,8 @@ extern "C" size_t gdn_chunk_kda_bwd_workspace_bytes(int64_t num_chunks, int64_t 
     return gdn::kda_bwd_ws_layout(num_chunks * HV, nullptr, nullptr);
 }
 
-extern "C" int gdn_chunk_kda_bwd(
+static int kda_bwd_entry(
+    const char* who, bool l2,
     const void* q, const void* k, const void* v, const float* g, const void* beta,
     const float* h0, const void* dout, const float* dht,
     void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0,
@@ -1348,9 +1348,9 @@ extern "C" int gdn_chunk_kda_bwd(
     int64_t N, int64_t num_chunks,
     float scale, int qkv_dtype, int gb_dtype, uint32_t flags, void* stream) {
     using namespace gdn;
-    const char* who = "gdn_chunk_kda_bwd";
     GDN_CHECK_ARG(B >= 1 && T >= 0 && H >= 1 && HV >= 1 && N >= 1 && num_chunks >= 0, GDN_ERR_INVALID, "%s: bad dimension", who);
     GDN_CHECK_ARG(HV % H == 0, GDN_ERR_INVALID, "%s: HV=%lld not divisible by H=%lld", who, (long long)HV, (long long)H);
+    GDN_CHECK_ARG(!l2 || H == HV, GDN_ERR_UNSUPPORTED, "%s: the l2 normalisation is taken in here for H == HV only", who);
     GDN_CHECK_ARG(K == BD && V == BD, GDN_ERR_UNSUPPORTED, "%s: K = V = 128 only (got K=%lld V=%lld); pad smaller head dims with zeros",
                   who, (long long)K, (long long)V);
     GDN_CHECK_ARG(qkv_dtype == GDN_DTYPE_BF16 || qkv_dtype == GDN_DTYPE_F16, GDN_ERR_UNSUPPORTED, "%s: q/k/v/do must be bf16 or f16", who);
@@ -1394,6 +1394,32 @@ extern "C" int gdn_chunk_kda_bwd(
     kp.cu_seqlens = cu_seqlens; kp.chunk_table = chunk_table; kp.chunk_offsets = chunk_offsets;
     kp.ws = KdaWs{p.ws.Wm, p.ws.Vn, p.ws.QG, p.ws.KG, p.ws.Pm, p.ws.EGL, p.ws.Am, p.ws.Gk};
     kp.T = T; kp.H = (int)H; kp.HV = (int)HV; kp.N = N; kp.NT = p.NT;
-    kp.scale = scale; kp.gb_dtype = gb_dtype; kp.flags = flags;
+    kp.scale = scale; kp.gb_dtype = gb_dtype; kp.flags = flags | (l2 ? GDN_FLAG_QK_L2NORM : 0);
     return qkv_dtype == GDN_DTYPE_BF16 ? launch_bwd_kda<bf16_t>(p, kp, num_chunks, qkv_dtype, s) : launch_bwd_kda<f16_t>(p, kp, num_chunks, qkv_dtype, s);
+}
+
+extern "C" int gdn_chunk_kda_bwd(
+    const void* q, const void* k, const void* v, const float* g, const void* beta,
+    const float* h0, const void* dout, const float* dht,
+    void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0,
+    const void* cu_seqlens, const void* chunk_table, const void* chunk_offsets,
+    void* workspace, size_t workspace_bytes,
+    int64_t B, int64_t T, int64_t H, int64_t HV, int64_t K, int64_t V,
+    int64_t N, int64_t num_chunks,
+    float scale, int qkv_dtype, int gb_dtype, uint32_t flags, void* stream) {
+    return kda_bwd_entry("gdn_chunk_kda_bwd", false, q, k, v, g, beta, h0, dout, dht, dq, dk, dv, dg, dbeta, dh0, cu_seqlens, chunk_table, chunk_offsets,
+                         workspace, workspace_bytes, B, T, H, HV, K, V, N, num_chunks, scale, qkv_dtype, gb_dtype, flags, stream);
+}
+
+extern "C" int gdn_chunk_kda_bwd_qk_l2norm(
+    const void* q, const void* k, const void* v, const float* g, const void* beta,
+    const float* h0, const void* dout, const float* dht,
+    void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0,
+    const void* cu_seqlens, const void* chunk_table, const void* chunk_offsets,
+    void* workspace, size_t workspace_bytes,
+    int64_t B, int64_t T, int64_t H, int64_t HV, int64_t K, int64_t V,
+    int64_t N, int64_t num_chunks,
+    float scale, int qkv_dtype, int gb_dtype, uint32_t flags, void* stream) {
+    return kda_bwd_entry("gdn_chunk_kda_bwd_qk_l2norm", true, q, k, v, g, beta, h0, dout, dht, dq, dk, dv, dg, dbeta, dh0, cu_seqlens, chunk_table, chunk_offsets,
+                         workspace, workspace_bytes, B, T, H, HV, K, V, N, num_chunks, scale, qkv_dtype, gb_dtype, flags, stream);
 }

@@ -132,6 +132,7 @@ SIGNATURES['gdn_chunk_comba_bwd_qk_l2norm_workspace_bytes'] = (c_size_t, [c_int6
 SIGNATURES['gdn_chunk_comba_bwd_qk_l2norm'] = SIGNATURES['gdn_chunk_comba_bwd']      # (q, k, p before their l2 normalisation)
 SIGNATURES['gdn_chunk_kda_bwd_workspace_bytes'] = (c_size_t, [c_int64, c_int64])
 SIGNATURES['gdn_chunk_kda_bwd'] = SIGNATURES['gdn_chunk_bwd']        # (g: [B,T,HV,K] fp32, dg likewise)
+SIGNATURES['gdn_chunk_kda_bwd_qk_l2norm'] = SIGNATURES['gdn_chunk_kda_bwd']      # (q, k before their l2 normalisation)
 SIGNATURES['gdn_l2norm_fwd'] = (c_int, [c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int, c_void_p])
 SIGNATURES['gdn_l2norm_bwd'] = (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int, c_void_p])
 SIGNATURES['gdn_fused_recurrent_delta_bwd_value_block'] = (c_int64, [c_int64])

@@ -158,11 +158,13 @@ def chunk_kda_fwd(q, k, v, g, beta, scale, initial_state, output_final_state, st
 
 
 def chunk_kda_bwd(q, k, v, g, beta, scale, initial_state, do, dht, state_v_first=False, cu_seqlens=None, cu_seqlens_cpu=None,
-                  q_rstd=None, k_rstd=None):
+                  q_rstd=None, k_rstd=None, qk_l2norm=False):
     """q, k ``[B,T,H,K]``, v, do ``[B,T,HV,V]``, g ``[B,T,HV,K]`` (log decays), beta ``[B,T,HV]`` as the recurrence uses them.
     Returns ``(dq, dk, dv, dbeta, dg, dh0)``: dq, dk, dv in q's dtype, dbeta ``[B,T,HV]`` and dg ``[B,T,HV,K]`` fp32, dh0 fp32
     (None without ``initial_state``).  With ``q_rstd``, ``k_rstd`` (what ``l2norm_fwd`` returns next to the normalised rows
-    passed as q and k) dq and dk are the gradients of the rows before normalisation."""
+    passed as q and k) dq and dk are the gradients of the rows before normalisation.  With ``qk_l2norm`` q and k are the rows
+    BEFORE their l2 normalisation and dq, dk the gradients of those: one C call (``gdn_chunk_kda_bwd_qk_l2norm``) where every value
+    head has a q/k head of its own, ``l2norm_fwd`` and the route above otherwise."""
     dev = require_gpu(q, k, v, g, beta, do)
     check_operand_shapes(q, k, v, beta=beta, gk=g)
     if do.shape != v.shape:
@@ -173,6 +175,10 @@ def chunk_kda_bwd(q, k, v, g, beta, scale, initial_state, do, dht, state_v_first
         raise NotImplementedError(f'the chunked KDA kernels cover key head dims up to {_DIM} (got K={K})')
     N = B if cu_seqlens is None else len(cu_seqlens) - 1
     nb = (V + _DIM - 1) // _DIM
+    inside = qk_l2norm and H == HV and nb == 1
+    if qk_l2norm and not inside:
+        (q, q_rstd), (k, k_rstd) = l2norm_fwd(q), l2norm_fwd(k)
+        q, k = q[..., :K], k[..., :K]                       # (l2norm_fwd pads rows to a multiple of 8)
     if nb > 1:
         # value columns are independent: a head with V > 128 is nb heads of 128 columns that share q, k, g, beta
         def split(s):       # [N, HV, K, V] -> [N, HV*nb, K, 128]  (V-first: [N, HV, V, K] -> [N, HV*nb, 128, K])
@@ -245,7 +251,7 @@ def chunk_kda_bwd(q, k, v, g, beta, scale, initial_state, do, dht, state_v_first
     ws_bytes = lib.gdn_chunk_kda_bwd_workspace_bytes(num_chunks, HV)
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
     launch(
-        lib.gdn_chunk_kda_bwd, dev, ptr(qw), ptr(kw), ptr(vw), ptr(gw), ptr(bw), ptr(h0), ptr(dow), ptr(dhtw),
+        lib.gdn_chunk_kda_bwd_qk_l2norm if inside else lib.gdn_chunk_kda_bwd, dev, ptr(qw), ptr(kw), ptr(vw), ptr(gw), ptr(bw), ptr(h0), ptr(dow), ptr(dhtw),
         ptr(dq), ptr(dk), ptr(dv), ptr(dg), ptr(db), ptr(dh0),
         ptr(cu_seqlens), ptr(chunk_table), ptr(chunk_offsets), ptr(workspace), ws_bytes,
         B, T, H, HV, _DIM, _DIM, N, num_chunks, float(scale), dtype_code(work), _lib.DTYPE_F32, flags)
@@ -289,19 +295,14 @@ class ChunkKDAFunction(torch.autograd.Function):
     def backward(ctx, do, dht):
         q, k, v, g_in, beta_raw, A_log, dt_bias, h0, cu_seqlens, cu_seqlens_cpu = ctx.saved_tensors
         scale, l2, gate_mode, bsig, neg, state_v_first, lower_bound = ctx.opts
-        q_rstd = k_rstd = None
-        qn, kn = q, k
-        if l2:
-            (qn, q_rstd), (kn, k_rstd) = l2norm_fwd(q), l2norm_fwd(k)
-            qn, kn = qn[..., :q.shape[-1]], kn[..., :k.shape[-1]]       # (l2norm_fwd pads rows to a multiple of 8)
         beta = beta_raw
         if bsig:
             beta = torch.sigmoid(beta_raw.float()) * (2.0 if neg else 1.0)
         g = g_in
         if gate_mode:
             g, x, a = _kda_gate(g_in, A_log, dt_bias, lower_bound if gate_mode == 2 else None)
-        dq, dk, dv, db, dg, dh0 = chunk_kda_bwd(qn, kn, v, g, beta, scale, h0, do.contiguous(), dht, state_v_first,
-                                                cu_seqlens, cu_seqlens_cpu, q_rstd, k_rstd)
+        dq, dk, dv, db, dg, dh0 = chunk_kda_bwd(q, k, v, g, beta, scale, h0, do.contiguous(), dht, state_v_first,
+                                                cu_seqlens, cu_seqlens_cpu, qk_l2norm=l2)
         if bsig:
             s = torch.sigmoid(beta_raw.float())
             db = db * s * (1 - s) * (2.0 if neg else 1.0)

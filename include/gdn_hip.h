@@ -391,9 +391,9 @@ int gdn_chunk_comba_bwd_qk_l2norm(
 /*
  * Backward pass of the chunked KDA operator.  Replaces chunk_kda_bwd (fla/ops/kda/chunk_bwd.py, called from
  * ChunkKDAFunction.backward, fla/ops/kda/chunk.py:124-175): the forward's intermediates are computed again (the
- * chunk-parallel kernel of gdn_chunk_kda_fwd, then the state scan), then the reverse scan, dq / dk / dw and the way back
- * through w, u and the two matrices with a decay per pair of rows and key feature (the reference's
- * chunk_kda_bwd_intra / chunk_kda_bwd_wy_dqkg_fused), and the reverse chunk-local cumulative sum of dg.
+ * chunk-parallel kernel of gdn_chunk_kda_fwd, then the state scan), then the reverse scan, and in one kernel dq / dk / dw, the way
+ * back through w, u and the two matrices with a decay per pair of rows and key feature (the reference's
+ * chunk_kda_bwd_intra / chunk_kda_bwd_wy_dqkg_fused) and the reverse chunk-local cumulative sum of dg.
  * Arguments as for gdn_chunk_bwd, except:
  *   g [B,T,HV,K] fp32: the log decay per key feature as the recurrence uses it (after the gate activation, whose
  *   derivative is the caller's, like those of the l2 norm and of the beta sigmoid); must not be NULL
@@ -403,6 +403,22 @@ int gdn_chunk_comba_bwd_qk_l2norm(
  */
 size_t gdn_chunk_kda_bwd_workspace_bytes(int64_t num_chunks, int64_t HV);
 int gdn_chunk_kda_bwd(
+    const void* q, const void* k, const void* v, const float* g, const void* beta,
+    const float* h0, const void* dout, const float* dht,
+    void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0,
+    const void* cu_seqlens, const void* chunk_table, const void* chunk_offsets,
+    void* workspace, size_t workspace_bytes,
+    int64_t B, int64_t T, int64_t H, int64_t HV, int64_t K, int64_t V,
+    int64_t N, int64_t num_chunks,
+    float scale, int qkv_dtype, int gb_dtype, uint32_t flags, void* stream);
+
+/*
+ * gdn_chunk_kda_bwd with the l2 normalisation of q and k taken inside, as gdn_chunk_comba_bwd_qk_l2norm does it: q and k are the rows
+ * as the caller has them, dq and dk the gradients of those rows.  Replaces the two l2norm_fwd and two l2norm_bwd launches around
+ * chunk_kda_bwd in ChunkKDAFunction.backward (fla/ops/kda/chunk.py:124-175).  H == HV only (GDN_ERR_UNSUPPORTED otherwise);
+ * everything else as for gdn_chunk_kda_bwd, whose workspace size it shares.
+ */
+int gdn_chunk_kda_bwd_qk_l2norm(
     const void* q, const void* k, const void* v, const float* g, const void* beta,
     const float* h0, const void* dout, const float* dht,
     void* dq, void* dk, void* dv, float* dg, float* dbeta, float* dh0,

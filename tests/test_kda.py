@@ -586,6 +586,26 @@ def test_chunk_kda_backward(B, T, H, HV, D, scale, gate_div, mask_p, l2, gate_in
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('l2', [False, True])
+@pytest.mark.parametrize('T,dtype', [(1, torch.bfloat16), (17, torch.float16), (64, torch.bfloat16), (65, torch.bfloat16), (150, torch.float16)])
+def test_chunk_kda_backward_strong_decay_in_some_features(T, dtype, l2):
+    """The backward's last kernel decides per block of 16 rows whether the decay inside a diagonal block fits the operand type: blocks on
+    both sides of that line next to each other, the decay strong in a few features only."""
+    q, k, v, g, beta, h0, _, _ = _chunk_inputs(1, T, 2, 2, 128, 4.0, 0, False, False, dtype)
+    g = g.clone()
+    g[:, :, 0, 32:48] *= 80                 # every block of one head,
+    g[:, 20:40, 1, 127] *= 60               # two blocks of the other
+    if not l2:
+        q, k = F.normalize(q.float(), p=2, dim=-1).to(dtype), F.normalize(k.float(), p=2, dim=-1).to(dtype)
+    gen = torch.Generator().manual_seed(43)
+    do, dht = torch.randn(1, T, 2, 128, generator=gen).to(dtype), torch.randn(1, 2, 128, 128, generator=gen)
+    kw = dict(scale=0.1, use_qk_l2norm_in_kernel=l2)
+    ref = O.kda_grads(q, k, v, g, beta, do, dht, initial_state=h0, dtype=torch.float64, **kw)
+    _, _, got = _kda_grads_gpu(q, k, v, g, beta, h0, None, None, do, dht, **kw)
+    _compare_grads(ref, got)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('H,D,mask_p,cu,gate_in_kernel,safe_gate,idx_dtype', [
     (4, 60, 0.1, [0, 15], True, False, torch.int32),
     (4, 64, 0.9, [0, 256, 500, 1000], True, False, torch.int64),
