@@ -33,7 +33,7 @@ namespace gdn {
 // In separate arrays, per (chunk, v-head): gam, beta [64] fp32, A, P [64][64], Bound (one float, see gdn_chunk_common.h, WARM_LOG2); and per
 // (chunk, v-head, block of VD value columns): v_new, dv_new [64][VD], S, dS [KD][VD] ([K][V]), all in the operand type.
 // Comba adds gam0 and dgam [64] fp32 (dgam partial, between the last two kernels), P^T in P's place, w, dw [64][128], u [64][128].
-// The KDA operator (a decay per key feature) has instead: Gk, the running sums of the log decays [64][128] fp32; QG = scale q e^Gk,
+// The KDA operator (a decay per key feature) has instead: Gk, the running sums of the log decays, divided by ln 2, [64][128] fp32; QG = scale q e^Gk,
 // KG = k e^(Gk_last - Gk) [64][128] and P [64][64] in the operand type, EGL = e^Gk_last [128] fp32 (all four as the forward's
 // chunk-parallel kernel writes them); w, u; u and v_new share their place.
 struct BwdWs {

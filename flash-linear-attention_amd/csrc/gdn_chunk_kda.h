@@ -7,8 +7,23 @@ namespace gdn {
 
 constexpr int PG = BD + 4;           // pitch of the fp32 gate tile
 
+// The decay across a block of 16 rows (in log2 units) down to which the block's own pairs of rows go through the matrix cores: their factors
+// e^(R - Gk_j) >= 1 then stay within what the operand type holds.
+template <typename T> struct SpanOk { static constexpr float value = -80.f * RCP_LN2_F; };
+template <> struct SpanOk<f16_t> { static constexpr float value = -8.f * RCP_LN2_F; };
+
+__device__ __forceinline__ float min_over_wave(float x) {
+    auto dpp = [](float y, auto ctrl) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, y), decltype(ctrl)::value, 0xF, 0xF, true)); };
+    x = fminf(x, dpp(x, std::integral_constant<int, 0xB1>{}));   // (over sixteen lanes as in sum_over_c16)
+    x = fminf(x, dpp(x, std::integral_constant<int, 0x4E>{}));
+    x = fminf(x, dpp(x, std::integral_constant<int, 0x141>{}));
+    x = fminf(x, dpp(x, std::integral_constant<int, 0x140>{}));
+    auto lane = [](float y, int n) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, y), n)); };
+    return fminf(fminf(lane(x, 0), lane(x, 16)), fminf(lane(x, 32), lane(x, 48)));
+}
+
 // Am, Gk: for the backward pass (NULL otherwise): A = (I + diag(beta) M)^-1 [64][64] in the operand type and the
-// running sums of the log decays [64][128] fp32, per unit
+// running sums of the log decays, divided by ln 2, [64][128] fp32, per unit
 struct KdaWs { void* Wm; void* Um; void* QG; void* KG; void* Pm; float* EGL; void* Am; float* Gk; };
 inline size_t kda_ws_layout(int64_t units, char* base, KdaWs* ws) {
     size_t off = 0;

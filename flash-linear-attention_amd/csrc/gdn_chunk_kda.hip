@@ -26,10 +26,20 @@ namespace gdn {
 // ---------------------------------------------------------------------------------------------
 // prepare
 // ---------------------------------------------------------------------------------------------
-// Two workgroups share a CU (80 KB of LDS each; a workgroup's phases are chains of dependent steps - the substitution above all -
-// that leave most of a CU idle): only k is kept as a tile; a wave reads nothing of q but its own 16 rows, which stay in
-// registers as operand fragments from the load to the store of qg; v arrives late, in the place of the matrix L.
-static_assert(64 * PL * 4 == 64 * P128 * 2, "the rows of v take the place of the matrix L");
+// Two workgroups share a CU (80 KB of LDS each; a workgroup's phases are chains of dependent steps that leave most of a CU idle).
+// Wave w owns the rows 16w .. of the chunk: q and k are matrix-core operand fragments (row 16w + c16, features 32s + 8g ..) from the load on,
+// and every decay of a row is a product of two per element,
+//     f = e^(Gam_i - R) (R: the row in front of the block)   and   h = e^(E - Gam_i) (E: the block's last row),
+// with factors per feature between the ends of the blocks (seven rows of 128, once per unit): k f and q f meet k h of the earlier blocks,
+// k / f of their own; e^Gam_i = f e^R, e^(Gam_last - Gam_i) = h e^(Gam_last - E).  The blocks 2 and 3 meet the rows 0 .. 31 with the
+// decay to row 31 on them, which is block 2's reference; only block 3 needs k f and q f a second time.  All exponents but that of 1 / f are <= 0, so
+// that a factor that underflows stands for a product that does.  What leaves does so as whole rows: through rows of LDS that only the
+// wave itself uses by then.
+// Bound by the rate at which two waves per SIMD issue vector instructions: with exponentials for every pair of blocks and every use, six to
+// eight per element, 592 us at 8192 tokens, 96 heads; with these two 446 us (1.9 GB, 4.2 TB/s), in the backward pass, where A and Gam
+// leave as well, 490 us (2.4 GB, 4.8 TB/s).
+static_assert(64 * PL * 4 == 64 * P128 * 2, "the rows of v, and on their way out qg and kg, take the place of the matrix L, row by row");
+static_assert(10 * BD * 4 <= 64 * P64 * 2, "the factors per feature lie where A will");
 constexpr size_t KDA_PREP_SMEM = (2 * 64 * P128 + 64 * P64) * 2 + (64 * PG + 64) * 4;
 
 template <typename T>
@@ -39,150 +49,205 @@ __global__ __launch_bounds__(256, 2) void gdn_kda_prepare_kernel(KdaParams p, in
     extern __shared__ __align__(16) char smem[];
     T* sK = (T*)smem; T* sV = sK + 64 * P128; T* sA = sV + 64 * P128;
     float* sL = (float*)sV;
-    float* sG = (float*)(sA + 64 * P64); float* sBeta = sG + 64 * PG;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c16 = lane & 15, g = lane >> 4;
+    float* sF = (float*)sA;                                     // ones, e^R of blocks 1 .. 3, e^(Gam_last - E) of blocks 0 .. 2, the decays across blocks 1 and 2, zeros
+    float* sG = (float*)(sA + 64 * P64); float* sBeta = sG + 64 * PG;      // (Gam / ln 2: every decay is one exp2)
+    // (the later row blocks meet more of the earlier ones: of the two workgroups of a CU one takes the blocks in reverse, so that every
+    // SIMD gets as much)
+    const bool flip = blockIdx.x >= 256;
 
-    // A workgroup walks over the units; the next unit's rows and gates are fetched into registers meanwhile.
-    TileRegs<BD> rK, rV;
-    V8 rQ[4];                                                   // q: row 16w + c16, features 32s + 8g .. + 7
+    // A workgroup walks over the units; the next unit's rows are fetched into registers meanwhile.
+    TileRegs<BD> rV;
+    V8 rK[4], rQ[4];                                            // row 16w + c16, features 32s + 8g .. + 7
     float rG[32];                                               // gates: a thread per key feature and half of the chunk's rows
     uint32_t rB = 0;                                            // (raw bits: converted when the unit's turn comes)
     // (the lane number is an argument: inside the loop over the units it is the opaque copy, see there)
+    auto block_of = [&](int tid) { const int w = __builtin_amdgcn_readfirstlane(tid >> 6); return flip ? 3 - w : w; };
     auto fetch_v = [&](int64_t u, int tid) {
-        const ChunkAt c = chunk_at(p, u / p.HV);
-        fetch_tile<BD>(rV, (const T*)p.v + (c.tok0 * p.HV + (int)(u % p.HV)) * BD, (int64_t)p.HV * BD, c.valid, tid);
+        const UnitAt at = unit_at(p, u);
+        fetch_tile<BD>(rV, (const T*)p.v + (at.c.tok0 * p.HV + at.hv) * BD, (int64_t)p.HV * BD, at.c.valid, tid);
     };
     auto fetch = [&](int64_t u, int tid) {
-        const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = lane & 15, g = lane >> 4;
-        const int hv = (int)(u % p.HV), hq = hv / (p.HV / p.H);
-        const ChunkAt c = chunk_at(p, u / p.HV);
-        fetch_tile<BD>(rK, (const T*)p.k + (c.tok0 * p.H + hq) * BD, (int64_t)p.H * BD, c.valid, tid);
+        const int lane = tid & 63, row = 16 * block_of(tid) + (lane & 15), g = lane >> 4;
+        const UnitAt at = unit_at(p, u);
+        const int64_t off = ((at.c.tok0 + row) * p.H + at.hq) * BD + 8 * g;
+        if (at.c.valid == CH) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
+            for (int s = 0; s < 4; ++s) { rK[s] = *(const V8*)((const T*)p.k + off + 32 * s); rQ[s] = *(const V8*)((const T*)p.q + off + 32 * s); }
+        } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) rQ[s][e] = (T)0.f;
-            if (16 * w + c16 < c.valid) rQ[s] = *(const V8*)((const T*)p.q + ((c.tok0 + 16 * w + c16) * p.H + hq) * BD + 32 * s + 8 * g);
+            for (int s = 0; s < 4; ++s) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) rK[s][e] = rQ[s][e] = (T)0.f;
+                if (row < at.c.valid) { rK[s] = *(const V8*)((const T*)p.k + off + 32 * s); rQ[s] = *(const V8*)((const T*)p.q + off + 32 * s); }
+            }
         }
-        rB = (tid < 64 && tid < c.valid) ? load_scalar_bits(p.beta, (c.tok0 + tid) * p.HV + hv, p.gb_dtype) : 0;
+        rB = (tid < 64 && tid < at.c.valid) ? load_scalar_bits(p.beta, (at.c.tok0 + tid) * p.HV + at.hv, p.gb_dtype) : 0;
     };
     auto fetch_g = [&](int64_t u, int tid) {
-        const int hv = (int)(u % p.HV);
-        const ChunkAt c = chunk_at(p, u / p.HV);
+        const UnitAt at = unit_at(p, u);
         const int col = tid & 127, half = tid >> 7;
+        const float* gp = p.g + ((at.c.tok0 + 32 * half) * p.HV + at.hv) * BD + col;
 #pragma unroll
-        for (int r = 0; r < 32; ++r) {
-            const int row = 32 * half + r;
-            rG[r] = row < c.valid ? p.g[((c.tok0 + row) * p.HV + hv) * BD + col] : 0.f;
-        }
+        for (int r = 0; r < 32; ++r) rG[r] = 32 * half + r < at.c.valid ? gp[(int64_t)r * p.HV * BD] : 0.f;
     };
-    fetch(blockIdx.x, tid);
-    const int tid_outer = tid;
+    fetch(blockIdx.x, threadIdx.x);
     for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
     // (everything derived from the lane number is derived again per unit from a copy the compiler cannot see through: hoisted out
     // of this loop, the addresses of its fully unrolled body would fill the register file before the loop starts, and spill)
-    int tid_opaque = tid_outer;
+    int tid_opaque = threadIdx.x;
     asm volatile("" : "+v"(tid_opaque));
-    const int tid = tid_opaque, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = lane & 15, g = lane >> 4;
-    const int hv = (int)(u % p.HV);
-    const ChunkAt c = chunk_at(p, u / p.HV);
-    fetch_g(u, tid);                                                 // (the gates are not fetched ahead: no 32 registers to carry them round the loop)
-    put_tile<BD>(sK, P128, rK, tid);
-    V8 qx[4];
+    const int tid = tid_opaque, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
+    const int w = block_of(tid);
+    const UnitAt at = unit_at(p, u);
+    const int hv = at.hv;
+    const ChunkAt c = at.c;
+    const int i = 16 * w + c16;                                 // the row this lane's operand fragments belong to
+    fetch_g(u, tid);                                            // (the gates are not fetched ahead: no 32 registers to carry them round the loop)
+    V8 kx[4], qx[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) qx[s] = rQ[s];
-    {
-        // running sums of the gates inside each half of the rows first
-        const int col = tid & 127, half = tid >> 7;
-        const float a_k = p.gk_act ? (p.A_log ? __expf(p.A_log[hv]) : (p.gk_act == 2 ? 1.f : __expf(1.f))) : 0.f;
-        const float bias = (p.gk_act && p.gk_bias) ? p.gk_bias[hv * BD + col] : 0.f;
-        float run = 0.f;
-#pragma unroll
-        for (int r = 0; r < 32; ++r) {
-            const int row = 32 * half + r;
-            float gt = rG[r];
-            if (p.gk_act && row < c.valid) {
-                gt += bias;
-                gt = p.gk_act == 2 ? p.gk_lower * sigmoid_f(a_k * gt) : -a_k * softplus_f(gt);
-            }
-            run += gt;
-            sG[row * PG + col] = run;
-            __builtin_amdgcn_sched_barrier(0);                  // (one row at a time: 32 activations in flight at once cost 100 registers)
-        }
-    }
+    for (int s = 0; s < 4; ++s) { kx[s] = rK[s]; qx[s] = rQ[s]; }
     if (tid < 64) {
         float b = scalar_of_bits(rB, p.gb_dtype);
         if ((p.flags & GDN_FLAG_BETA_SIGMOID) && tid < c.valid) b = sigmoid_f(b) * ((p.flags & GDN_FLAG_NEG_EIGVAL) ? 2.f : 1.f);
         sBeta[tid] = b;
     }
-    lds_barrier();
-    fetch_v(u, tid);
-    {
-        // second half of the rows: add the first half's total
-        const int col = tid & 127, half = tid >> 7;
-        if (half == 1) {
-            const float tot = sG[31 * PG + col];
+    if (p.flags & GDN_FLAG_QK_L2NORM) {
+        // rows of q and k divided by sqrt(sum x^2 + 1e-6): the four lanes that share c16 hold a row
+        float sk = 0.f, sq = 0.f;
 #pragma unroll
-            for (int r = 0; r < 32; ++r) sG[(32 + r) * PG + col] += tot;
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { sk += (float)kx[s][e] * (float)kx[s][e]; sq += (float)qx[s][e] * (float)qx[s][e]; }
+        const float rk = rsqrtf(sum_over_g(sk) + 1e-6f), rq = rsqrtf(sum_over_g(sq) + 1e-6f);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { kx[s][e] = (T)((float)kx[s][e] * rk); qx[s][e] = (T)((float)qx[s][e] * rq); }
+    }
+    {
+        // running sums of the gates inside each half of the rows first
+        const int col = tid & 127, half = tid >> 7;
+        const float a_k = p.gk_act ? (p.A_log ? __expf(p.A_log[hv]) : (p.gk_act == 2 ? 1.f : __expf(1.f))) : 0.f;
+        const float bias = (p.gk_act && p.gk_bias) ? p.gk_bias[hv * BD + col] : 0.f;
+        if (p.gk_act) {
+#pragma unroll
+            for (int r = 0; r < 32; ++r) {
+                if (32 * half + r >= c.valid) break;
+                const float gt = rG[r] + bias;
+                rG[r] = p.gk_act == 2 ? p.gk_lower * sigmoid_f(a_k * gt) : -a_k * softplus_f(gt);
+                __builtin_amdgcn_sched_barrier(0);              // (one row at a time: 32 activations in flight at once cost 100 registers)
+            }
+        }
+        float run = 0.f;
+#pragma unroll
+        for (int r = 0; r < 32; ++r) {
+            run += rG[r];
+            sG[(32 * half + r) * PG + col] = run * RCP_LN2_F;
         }
     }
-    if (p.flags & GDN_FLAG_QK_L2NORM) {
-        // rows of q and k divided by sqrt(sum x^2 + 1e-6).  k: 16 consecutive lanes hold the 16 pieces of a row
+    lds_barrier();
+    if (tid >> 7) {
+        // second half of the rows: add the first half's total; and the factors between the ends of the blocks
+        const int col = tid & 127;
+        float* gc = sG + col;
+        const float G15 = gc[15 * PG], G31 = gc[31 * PG];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = (tid >> 4) + 16 * i, pc = tid & 15;
-            T* at = sK + row * P128 + pc * 8;
-            V8 x = *(V8*)at;
-            float ss = 0.f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) ss += (float)x[e] * (float)x[e];
-            const float r = rsqrtf(sum_over_c16(ss) + 1e-6f);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = (T)((float)x[e] * r);
-            *(V8*)at = x;
-        }
-        // q: the four lanes that share c16 hold a row
-        float ss = 0.f;
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) ss += (float)qx[s][e] * (float)qx[s][e];
-        const float r = rsqrtf(sum_over_g(ss) + 1e-6f);
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) qx[s][e] = (T)((float)qx[s][e] * r);
+        for (int r = 0; r < 32; ++r) gc[(32 + r) * PG] += G31;
+        const float G47 = gc[47 * PG], G63 = gc[63 * PG];
+        sF[0 * BD + col] = 1.f;
+        sF[1 * BD + col] = fast_exp2(G15); sF[2 * BD + col] = fast_exp2(G31); sF[3 * BD + col] = fast_exp2(G47);
+        sF[4 * BD + col] = fast_exp2(G63 - G15); sF[5 * BD + col] = fast_exp2(G63 - G31); sF[6 * BD + col] = fast_exp2(G63 - G47);
+        sF[7 * BD + col] = fast_exp2(G31 - G15); sF[8 * BD + col] = fast_exp2(G47 - G31);
+        sF[9 * BD + col] = 0.f;
+        p.ws.EGL[u * BD + col] = fast_exp2(G63);
     }
     lds_barrier();
 
+    // ---- every row's factors; qg and kg leave, k h goes to LDS for the later blocks ----
+    const float bi = sBeta[i];
+    float f[4][8];
+    V8 kw[4];                                                   // beta k e^Gam, the factor of w
+    V8 kd[4], qd[4];                                            // k f, q f
+    // 16 rows of 128 through this wave's own rows of LDS
+    auto rows_out = [&](T* rows) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        u32x4 x[4];
+#pragma unroll
+        for (int n = 0; n < 4; ++n) x[n] = *(const u32x4*)(sV + (16 * w + (lane >> 4) + 4 * n) * P128 + (lane & 15) * 8);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) *(u32x4*)(rows + (16 * w + (lane >> 4) + 4 * n) * BD + (lane & 15) * 8) = x[n];
+        asm volatile("" ::: "memory");
+    };
+    {
+        const float* gi = sG + i * PG + 8 * g;
+        const float* gr = (w > 0 ? sG + (16 * w - 1) * PG : sF + 9 * BD) + 8 * g;
+        const float* ge = sG + (16 * w + 15) * PG + 8 * g;
+        const float* t2 = sF + w * BD + 8 * g;                  // e^R
+        const float* t1 = sF + (w < 3 ? 4 + w : 0) * BD + 8 * g;       // e^(Gam_last - E)
+        const float* t0 = sF + (w == 0 ? 7 : 0) * BD + 8 * g;   // from the block's end to row 31, or to its end
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            __builtin_amdgcn_sched_barrier(0);
+            V8 kn, kg, k1;
+#pragma unroll
+            for (int h4 = 0; h4 < 2; ++h4) {
+                const int o = 32 * s + 4 * h4;
+                const f32x4 G = *(const f32x4*)(gi + o), R = *(const f32x4*)(gr + o), E = *(const f32x4*)(ge + o);
+                const f32x4 eR = *(const f32x4*)(t2 + o), eL = *(const f32x4*)(t1 + o), e1 = *(const f32x4*)(t0 + o);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int e = 4 * h4 + r;
+                    f[s][e] = fast_exp2(G[r] - R[r]);
+                    const float k = (float)kx[s][e], kh = k * fast_exp2(E[r] - G[r]), kf = k * f[s][e];
+                    kd[s][e] = (T)kf;
+                    qd[s][e] = (T)((float)qx[s][e] * f[s][e]);
+                    kn[e] = (T)(kh * e1[r]);
+                    k1[e] = (T)kh;
+                    kg[e] = (T)(kh * eL[r]);
+                    kw[s][e] = (T)(kf * (bi * eR[r]));
+                }
+            }
+            // (with the decay to row 31 on block 0; to its own end, for block 1, in the rows of block 3, which no later block meets)
+            if (w < 3) *(V8*)(sK + i * P128 + 32 * s + 8 * g) = kn;
+            if (w == 0) *(V8*)(sK + (48 + i) * P128 + 32 * s + 8 * g) = k1;
+            *(V8*)(sV + i * P128 + 32 * s + 8 * g) = kg;
+        }
+        rows_out((T*)p.ws.KG + u * 64 * BD);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            V8 qg;
+#pragma unroll
+            for (int h4 = 0; h4 < 2; ++h4) {
+                const f32x4 eR = *(const f32x4*)(t2 + 32 * s + 4 * h4);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) { const int e = 4 * h4 + r; qg[e] = (T)((float)qx[s][e] * f[s][e] * (p.scale * eR[r])); }
+            }
+            *(V8*)(sV + i * P128 + 32 * s + 8 * g) = qg;
+        }
+        rows_out((T*)p.ws.QG + u * 64 * BD);
+    }
+    lds_barrier();
+
+    // (the rows anew for every use that follows: converted once they would take 64 registers)
+    auto anew = [&] {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            u32x4 a = __builtin_bit_cast(u32x4, kx[s]), b = __builtin_bit_cast(u32x4, qx[s]);
+            asm volatile("" : "+v"(a), "+v"(b));
+            kx[s] = __builtin_bit_cast(V8, a); qx[s] = __builtin_bit_cast(V8, b);
+        }
+    };
+    anew();
     // ---- M (as L = diag(beta) M, for the substitution) and P, this wave's 16 rows ----
     {
         T* Pu = (T*)p.ws.Pm + u * 64 * 64;
-        const int i = 16 * w + c16;                             // the row this lane's operand fragments belong to
-        // rows of this block against rows of earlier blocks: reference = the row in front of the block (zeros for block 0)
-        V8 kd[4], qd[4];
-        const float* gref = sG + (16 * w - 1) * PG + 8 * g;         // the reference row, read where it is used (w > 0)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const float* gi = sG + i * PG + 32 * s + 8 * g;
-            const float* gr = sG + (16 * w - 1) * PG + 32 * s + 8 * g;
-            const V8 kx = frag_rows(sK, P128, 16 * w, 32 * s, lane);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float f = __expf(gi[e] - (w > 0 ? gr[e] : 0.f));
-                kd[s][e] = (T)((float)kx[e] * f);
-                qd[s][e] = (T)((float)qx[s][e] * f);
-            }
-        }
-#pragma unroll
-        for (int tj = 0; tj < 3; ++tj) {
-            if (tj >= w) break;
+        // rows of this block against rows of an earlier block (at `at` in sK)
+        auto pair = [&](int tj, int at) {
+            __builtin_amdgcn_sched_barrier(0);
             f32x4 m = ZERO4, pt = ZERO4;
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                const float* gj = sG + (16 * tj + c16) * PG + 32 * s + 8 * g;
-                V8 kn = frag_rows(sK, P128, 16 * tj, 32 * s, lane);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) kn[e] = (T)((float)kn[e] * __expf(gref[32 * s + e] - gj[e]));        // (tj < w: w > 0)
+                const V8 kn = frag_rows(sK, P128, at, 32 * s, lane);
                 m = Mma<T>::run(kd[s], kn, m);                 // lane: column j = 16tj + c16, rows i = 16w + 4g + r
                 pt = Mma<T>::run(kn, qd[s], pt);               // lane: column i = 16w + c16, rows j = 16tj + 4g + r
             }
@@ -193,13 +258,16 @@ __global__ __launch_bounds__(256, 2) void gdn_kda_prepare_kernel(KdaParams p, in
                 sL[ir * PL + (j & 3) * 16 + (j >> 2)] = sBeta[ir] * m[r];
             }
             *(V4*)(Pu + i * 64 + 16 * tj + 4 * g) = pack4<T>(pt * p.scale);
-        }
+        };
+        if (w == 1) pair(0, 48);
+        else if (w == 2) { pair(0, 0); pair(1, 16); }
+        else if (w == 3) pair(2, 32);
         // blocks to the right of the diagonal: zeros
 #pragma unroll
         for (int tj = 1; tj < 4; ++tj)
             if (tj > w) *(V4*)(Pu + i * 64 + 16 * tj + 4 * g) = pack4<T>(ZERO4);
         // The diagonal block.  Where the decay across the block stays within what the operand type can hold as a factor
-        // e^(ref - Gam_j) >= 1 (the usual case), the same reference serves and the block is one more tile on the matrix
+        // e^(R - Gam_j) >= 1 (the usual case), the same reference serves and the block is one more tile on the matrix
         // cores; otherwise every pair of rows gets its own exponentials.
         float span = 0.f;
 #pragma unroll
@@ -207,17 +275,14 @@ __global__ __launch_bounds__(256, 2) void gdn_kda_prepare_kernel(KdaParams p, in
             const int col = lane + 64 * h;
             span = fminf(span, sG[(16 * w + 15) * PG + col] - (w > 0 ? sG[(16 * w - 1) * PG + col] : 0.f));
         }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) span = fminf(span, __shfl_xor(span, off, 64));
-        constexpr float SPAN_OK = std::is_same<T, bf16_t>::value ? -80.f : -8.f;
-        if (span >= SPAN_OK) {
+        anew();
+        if (min_over_wave(span) >= SpanOk<T>::value) {
             f32x4 m = ZERO4, pt = ZERO4;
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                const float* gj = sG + i * PG + 32 * s + 8 * g;
-                V8 kn = frag_rows(sK, P128, 16 * w, 32 * s, lane);
+                V8 kn;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) kn[e] = (T)((float)kn[e] * __expf((w > 0 ? gref[32 * s + e] : 0.f) - gj[e]));
+                for (int e = 0; e < 8; ++e) kn[e] = (T)((float)kx[s][e] * __builtin_amdgcn_rcpf(f[s][e]));
                 m = Mma<T>::run(kd[s], kn, m);                 // lane: column j = 16w + c16, rows i = 16w + 4g + r
                 pt = Mma<T>::run(kn, qd[s], pt);               // lane: column i = 16w + c16, rows j = 16w + 4g + r
             }
@@ -230,24 +295,31 @@ __global__ __launch_bounds__(256, 2) void gdn_kda_prepare_kernel(KdaParams p, in
             }
             *(V4*)(Pu + i * 64 + 16 * w + 4 * g) = pack4<T>(pt);
         } else
-        // (lane (c16, g) takes row i against every row j of the block over the features of its own fragments; the four lanes that
-        // share a row add up)
+        // (lane (c16, g) takes row i against every row j of the block over the features of its own fragments, row j's from the lane
+        // that holds them; the four lanes that share a row add up)
         {
 #pragma unroll 1
             for (int jl = 0; jl < 16; ++jl) {
                 const int rj = 16 * w + jl;
                 float mj = 0.f, pj = 0.f;
-                if (jl <= c16) {
 #pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const V8 ki = frag_rows(sK, P128, 16 * w, 32 * s, lane), kj = *(const V8*)(sK + rj * P128 + 32 * s + 8 * g);
-                        const float* gi = sG + i * PG + 32 * s + 8 * g;
-                        const float* gj = sG + rj * PG + 32 * s + 8 * g;
+                for (int s = 0; s < 4; ++s) {
+                    // (the rows and their place anew every time: converted once they would take the registers of the whole kernel)
+                    u32x4 bits = __builtin_bit_cast(u32x4, kx[s]), qbits = __builtin_bit_cast(u32x4, qx[s]);
+                    int row = i;
+                    asm volatile("" : "+v"(bits), "+v"(qbits), "+v"(row));
+                    const V8 ki = __builtin_bit_cast(V8, bits), qi = __builtin_bit_cast(V8, qbits);
+#pragma unroll
+                    for (int n = 0; n < 4; ++n) bits[n] = (uint32_t)__shfl((int)bits[n], (lane & 48) + jl, 64);
+                    const V8 kj = __builtin_bit_cast(V8, bits);
+                    const float* gi = sG + row * PG + 32 * s + 8 * g;
+                    const float* gj = sG + rj * PG + 32 * s + 8 * g;
+                    if (jl <= c16) {
 #pragma unroll
                         for (int e = 0; e < 8; ++e) {
-                            const float kk = (float)kj[e] * __expf(gi[e] - gj[e]);
+                            const float kk = (float)kj[e] * fast_exp2(gi[e] - gj[e]);
                             mj += (float)ki[e] * kk;
-                            pj += (float)qx[s][e] * kk;
+                            pj += (float)qi[e] * kk;
                         }
                     }
                 }
@@ -258,85 +330,91 @@ __global__ __launch_bounds__(256, 2) void gdn_kda_prepare_kernel(KdaParams p, in
                 }
             }
         }
+        if (w == 3) {
+            // the rows 0 .. 31: the decay across block 2 lies between
+            anew();
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int h4 = 0; h4 < 2; ++h4) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    const f32x4 F = *(const f32x4*)(sF + 8 * BD + 32 * s + 8 * g + 4 * h4);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int e = 4 * h4 + r;
+                        const float x = f[s][e] * F[r];
+                        kd[s][e] = (T)((float)kx[s][e] * x);
+                        qd[s][e] = (T)((float)qx[s][e] * x);
+                    }
+                }
+            pair(0, 0); pair(1, 16);
+        }
     }
     lds_barrier();
+    fetch_v(u, tid);
     solve_unit_lower_blocks<T>(sL, (float*)sA, sA, w, lane);
     lds_barrier();
-    if (p.ws.Am) {                                              // (for the backward pass)
+    if (p.ws.Am) {                                              // (for the backward pass; A: this wave's own rows)
         T* Au = (T*)p.ws.Am + u * 64 * 64;
         float* Gu = p.ws.Gk + u * 64 * BD;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int idx = tid + 256 * i, row = idx >> 3, pc = idx & 7;
+        for (int n = 0; n < 2; ++n) {
+            const int row = 16 * w + 8 * n + (lane >> 3), pc = lane & 7;
             *(u32x4*)(Au + row * 64 + pc * 8) = *(const u32x4*)(sA + row * P64 + pc * 8);
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int idx = tid + 256 * i, row = idx >> 5, pc = idx & 31;
+        for (int n = 0; n < 8; ++n) {
+            const int idx = tid + 256 * n, row = idx >> 5, pc = idx & 31;
             *(f32x4*)(Gu + row * BD + pc * 4) = *(const f32x4*)(sG + row * PG + pc * 4);
         }
     }
-    {
-        // what the scan needs of q and k, and k, v as the factors of w, u
-        T* QGu = (T*)p.ws.QG + u * 64 * BD;
-        T* KGu = (T*)p.ws.KG + u * 64 * BD;
+    // the factors of w and u (that of u in the place of L: the substitution is over); beta goes onto them and not onto A, whose
+    // rounded entries the backward pass takes as they are: with other ones the parts of dGk would not cancel
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {                        // (the pieces of v: those this thread fetched)
-            const int idx = tid + 256 * it, row = idx >> 4, pc = idx & 15;
-            const float* gi = sG + row * PG + pc * 8;
-            const float* gl = sG + 63 * PG + pc * 8;
-            V8 kx = *(V8*)(sK + row * P128 + pc * 8), vx = __builtin_bit_cast(V8, rV.x[it]);
-            V8 kg;
-            const float b = sBeta[row];
+    for (int s = 0; s < 4; ++s) *(V8*)(sK + i * P128 + 32 * s + 8 * g) = kw[s];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float eg = __expf(gi[e]);
-                kg[e] = (T)((float)kx[e] * __expf(gl[e] - gi[e]));
-                kx[e] = (T)((float)kx[e] * (b * eg));
-                vx[e] = (T)((float)vx[e] * b);
-            }
-            *(V8*)(KGu + row * BD + pc * 8) = kg;
-            *(V8*)(sK + row * P128 + pc * 8) = kx;
-            *(V8*)(sV + row * P128 + pc * 8) = vx;                                  // (in the place of L: the substitution is over)
-        }
-        {
-            const int i = 16 * w + c16;
+    for (int n = 0; n < 4; ++n) {
+        const float b = sBeta[(tid >> 4) + 16 * n];
+        V8 vx = __builtin_bit_cast(V8, rV.x[n]);
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const float* gi = sG + i * PG + 32 * s + 8 * g;
-                V8 qg;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) qg[e] = (T)((float)qx[s][e] * (p.scale * __expf(gi[e])));
-                *(V8*)(QGu + i * BD + 32 * s + 8 * g) = qg;
-            }
-        }
-        if (tid < BD) p.ws.EGL[u * BD + tid] = __expf(sG[63 * PG + tid]);
+        for (int e = 0; e < 8; ++e) vx[e] = (T)((float)vx[e] * b);
+        rV.x[n] = __builtin_bit_cast(u32x4, vx);
     }
+    put_tile<BD>(sV, P128, rV, tid);
+    // (the next unit's rows: requested this late because the phases above have no registers to spare under the cap that lets two
+    // workgroups share a CU; the other workgroup covers the wait)
+    fetch(u + gridDim.x < units ? u + gridDim.x : u, tid);
     lds_barrier();
     {
-        // w^T and u^T tiles: features on the rows, this wave's 16 tokens on the columns
-        T* Wu = (T*)p.ws.Wm + u * 64 * BD;
-        T* Uu = (T*)p.ws.Um + u * 64 * BD;
-        const int i = 16 * w + c16;
+        // w^T and u^T tiles: features on the rows, this wave's 16 tokens on the columns; 64 features at a time they leave through this
+        // wave's own rows of A, which it has read
         V8 fa[2];
 #pragma unroll
         for (int s = 0; s < 2; ++s) fa[s] = frag_rows(sA, P64, 16 * w, 32 * s, lane);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-        for (int n = 0; n < 8; ++n) {
-            f32x4 aw = ZERO4, au = ZERO4;
+        for (int q4 = 0; q4 < 4; ++q4) {
+            const T* rows = q4 < 2 ? sK : sV;
+            T* out = (T*)(q4 < 2 ? p.ws.Wm : p.ws.Um) + u * 64 * BD + 64 * (q4 & 1);
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                if (2 * s > w) continue;                        // A is lower triangular
-                aw = Mma<T>::run(frag_cols(sK, P128, 32 * s, 16 * n, lane), fa[s], aw);
-                au = Mma<T>::run(frag_cols(sV, P128, 32 * s, 16 * n, lane), fa[s], au);
+            for (int n = 0; n < 4; ++n) {
+                f32x4 acc = ZERO4;
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    if (2 * s > w) continue;                    // A is lower triangular
+                    acc = Mma<T>::run(frag_cols(rows, P128, 32 * s, 64 * (q4 & 1) + 16 * n, lane), fa[s], acc);
+                }
+                *(V4*)(sA + i * P64 + 16 * n + 4 * g) = pack4<T>(acc);
             }
-            *(V4*)(Wu + i * BD + 16 * n + 4 * g) = pack4<T>(aw);
-            *(V4*)(Uu + i * BD + 16 * n + 4 * g) = pack4<T>(au);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+                const int row = 16 * w + 8 * n + (lane >> 3), pc = lane & 7;
+                *(u32x4*)(out + row * BD + pc * 8) = *(const u32x4*)(sA + row * P64 + pc * 8);
+            }
+            asm volatile("" ::: "memory");
         }
     }
-    // (the next unit's rows: requested this late because the phases above have no registers to spare under the cap that lets two
-    // workgroups share a CU; the other workgroup covers the wait)
-    if (u + gridDim.x < units) fetch(u + gridDim.x, tid);
     lds_barrier();
     }
 }

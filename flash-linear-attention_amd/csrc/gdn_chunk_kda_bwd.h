@@ -2,7 +2,7 @@
 // to 128 by the host).  Included by gdn_chunk_bwd.hip inside namespace gdn, after its types and its two scans, which serve this
 // pass in their KDA form.  Replaces
 // chunk_kda_bwd (fla/ops/kda/chunk_bwd.py): the forward's chunk-parallel kernel runs again (A, w, u, qg, kg, P and the
-// running sums Gk of the log decays), then
+// running sums Gk of the log decays, in log2 units), then
 //
 //   state, dstate   as for the gated delta rule, with kg / qg in place of k / q and a decay per key feature
 //   unit            per (chunk, v-head), from S, dS, v_new, dv_new to dq, dk, dv, dg, dbeta:
@@ -24,16 +24,6 @@
 // operand k e^(R - Gk) for the row side, and for the column side one 32-deep step whose contraction index runs over the
 // block's 16 rows twice (dPs^T against q e^(Gk - R), dL^T against beta k e^(Gk - R)).
 
-template <typename T> struct SpanOk { static constexpr float value = -8.f * RCP_LN2_F; };       // f16: factors up to e^8 (log2 units)
-template <> struct SpanOk<bf16_t> { static constexpr float value = -80.f * RCP_LN2_F; };
-
-__device__ __forceinline__ float min_over_c16(float x) {         // over the sixteen lanes that share g
-    auto other = [](float y, auto ctrl) { return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, y), decltype(ctrl)::value, 0xF, 0xF, true)); };
-    x = fminf(x, other(x, std::integral_constant<int, 0xB1>{}));
-    x = fminf(x, other(x, std::integral_constant<int, 0x4E>{}));
-    x = fminf(x, other(x, std::integral_constant<int, 0x141>{}));
-    return fminf(x, other(x, std::integral_constant<int, 0x140>{}));
-}
 // x of this lane and of the lanes behind it in its row of sixteen, added up
 template <int N> __device__ __forceinline__ float add_behind(float x) {
     return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x100 + N, 0xF, 0xF, true));     // row_shl: N lanes on, zero past the row
@@ -139,7 +129,7 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int idx = tid + NTH * i;
-            *(f32x4*)(sG + (idx >> 5) * PG + (idx & 31) * 4) = rG[i] * RCP_LN2_F;
+            *(f32x4*)(sG + (idx >> 5) * PG + (idx & 31) * 4) = rG[i];
         }
         if (tid < 64) sBeta[tid] = scalar_of_bits(rBeta, p.gb_dtype);
         lds_barrier();
@@ -264,9 +254,7 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
                 const float* col = sG + lane + 64 * h;
                 span = fminf(span, col[(16 * w + 15) * PG] - (w > 0 ? col[(16 * w - 1) * PG] : 0.f));
             }
-            span = min_over_c16(span);
-#pragma unroll
-            for (int off = 16; off < 64; off <<= 1) span = fminf(span, __shfl_xor(span, off, 64));
+            span = min_over_wave(span);
             if (lane == 0) sSpan[w] = span;
         }
         {                                                       // (the zero tiles of dA and dL, in v_new's place)
