@@ -78,6 +78,14 @@ def test_layer_step_beyond_one_tile_of_rows(N, monkeypatch):
     test_layer_step_in_four_launches(N, 512, 2, 4, 64, 1, 4, False, monkeypatch)
 
 
+@pytest.mark.parametrize('N,hidden,heads,v_heads,D,expand', [
+    (1, 4096, 4, 4, 64, 1), (16, 768, 3, 6, 64, 2), (7, 256, 8, 8, 32, 1), (15, 512, 3, 3, 256, 4), (2, 256, 8, 8, 256, 2), (16, 256, 1, 32, 64, 0.625)])
+def test_layer_step_of_few_sequences(N, hidden, heads, v_heads, D, expand, monkeypatch):
+    """The projections' kernel for up to 16 rows: fewer steps than waves, more than it requests at once, hidden sizes that are no power of two,
+    columns in each number of tiles a workgroup takes, segments of a few columns."""
+    test_layer_step_in_four_launches(N, hidden, heads, v_heads, D, expand, 4, False, monkeypatch)
+
+
 def test_layer_step_leaves_many_sequences_of_a_large_layer_to_its_modules():
     from fla_hip.layers import GatedDeltaNet
     from fla_hip.layers.gated_deltanet import LayerCache
