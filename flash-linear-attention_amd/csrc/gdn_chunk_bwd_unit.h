@@ -15,7 +15,9 @@
 // (always, the last time for nothing: behind a condition the registers of the last request stay alive through the whole head).
 // 16000 packed tokens, 16 q/k and 32 value heads of 128: 650 us as two kernels, 490 us; with the heads of a group added up and the l2
 // normalisation taken back in here 500 us, and 132 us of passes around it gone.  8 x 2048 tokens, 32 heads of 256 x 256: 2230 us with
-// those passes, 1830 us (state fragments requested a head ahead there: 1920 us, for want of registers).
+// those passes, 1830 us (state fragments requested a head ahead there: 1920 us, for want of registers), now 1570 us: the first feature tile's
+// fragments are requested in front of the dP phase, and the products with the state follow one another (1642 us with the three of them
+// side by side, whose accumulators spilled; at 128 key features they stay side by side: 475 us against 487 us).
 
 // lower triangle of 4 x 4 tiles, row by row
 __device__ __forceinline__ int tri_row(int idx) { return idx < 1 ? 0 : idx < 3 ? 1 : idx < 6 ? 2 : 3; }
@@ -143,6 +145,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
             const bool last = hi + 1 == heads;
             const Item& to = last ? nx : at;
             const int to_hv = last ? nx.hv0 : hv + 1;
+            if constexpr (LEAN) fetch_state(at, hv, 0, w, lane);
             lds_barrier();
             if constexpr (!LEAN) fetch_out(to, to_hv, tid);
 
@@ -172,50 +175,114 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
             float dglast = 0.f, dgx[4] = {0.f, 0.f, 0.f, 0.f}, dbx[4] = {0.f, 0.f, 0.f, 0.f};    // this lane's share of dgam, dbeta of token 16t + c16
             f32x4 sd = ZERO4;                                    // diagonal: <S, dS> of this wave's rows
             V4 dw[NA][4];
+            if constexpr (LEAN) {
 #pragma unroll
-            for (int a = 0; a < NA; ++a) {
-                if constexpr (LEAN) {                           // (the lane number anew: one tile's fragments at a time)
-                    int lane_a = lane;
-                    asm volatile("" : "+v"(lane_a));
-                    fetch_state(at, hv, a, w, lane_a);
-                }
-                f32x4 G1[4], dKS[4], dWt[4];
+                for (int a = 0; a < NA; ++a) {
+                    const int n16 = feat(a);
+                    // one product with the state at a time: sixteen accumulator registers instead of forty-eight, and the next tile's fragments
+                    // on their way during the last of the tile's own work
+                    f32x4 acc[4];
+                    auto product = [&](const V8 (&f)[SV], const T* rows) {
 #pragma unroll
-                for (int t = 0; t < 4; ++t) G1[t] = dKS[t] = dWt[t] = ZERO4;
+                        for (int t = 0; t < 4; ++t) acc[t] = ZERO4;
 #pragma unroll
-                for (int s = 0; s < SV; ++s) {
+                        for (int s = 0; s < SV; ++s) {
+                            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                            for (int t = 0; t < 4; ++t) acc[t] = Mma<T>::run(f[s], frag_rows(rows, PV, 16 * t, 32 * s, lane), acc[t]);
+                        }
+                    };
+                    product(sf, sDO);
+                    {
+                        V8 fk[2];
+#pragma unroll
+                        for (int s = 0; s < 2; ++s) fk[s] = frag_cols(sK, PK, 32 * s, n16, lane);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) {
+                            __builtin_amdgcn_sched_barrier(0);
+                            const int x = 16 * t + c16;
+                            f32x4 q_ = acc[t] * (p.scale * sEg[x]);
+                            const V4 q4 = *(const V4*)(sQ + x * PK + n16 + 4 * g);
+#pragma unroll
+                            for (int s = 0; s < 2; ++s)
+                                if (32 * s <= 16 * t + 15) q_ = Mma<T>::run(fk[s], frag_rows(sM1, P64, 16 * t, 32 * s, lane), q_);     // dP[i][j] = 0 for j > i
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) dgx[t] += (float)q4[r] * q_[r];
+                            pin(dgx[t]);
+                            dq[a][t] += q_;
+                        }
+                    }
+                    product(sf, sDvn);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) dw[a][t] = pack4<T>(-acc[t]);
+#pragma unroll
+                    for (int s = 0; s < SV; ++s) sd = Mma<T>::run(sf[s], df[s], sd);
+                    product(df, sVn);
                     __builtin_amdgcn_sched_barrier(0);
-                    sd = Mma<T>::run(sf[s], df[s], sd);
+                    if (a + 1 < NA) fetch_state(at, hv, a + 1, w, lane);
+                    {
+                        V8 fq[2];
+#pragma unroll
+                        for (int s = 0; s < 2; ++s) fq[s] = frag_cols(sQ, PK, 32 * s, n16, lane);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) {
+                            __builtin_amdgcn_sched_barrier(0);
+                            const int x = 16 * t + c16;
+                            f32x4 k_ = acc[t] * sEl[x];
+                            const V4 k4 = *(const V4*)(sK + x * PK + n16 + 4 * g);
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) dglast += (float)k4[r] * k_[r];
+#pragma unroll
+                            for (int s = 0; s < 2; ++s)
+                                if (32 * s + 31 >= 16 * t) k_ = Mma<T>::run(fq[s], frag_cols(sM1, P64, 32 * s, 16 * t, lane), k_);     // ... and for i < j
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) dgx[t] -= (float)k4[r] * k_[r];
+                            pin(dgx[t]);
+                            dk[a][t] += k_;
+                        }
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int a = 0; a < NA; ++a) {
+                    f32x4 G1[4], dKS[4], dWt[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) G1[t] = dKS[t] = dWt[t] = ZERO4;
+#pragma unroll
+                    for (int s = 0; s < SV; ++s) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        sd = Mma<T>::run(sf[s], df[s], sd);
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) {
+                            G1[t] = Mma<T>::run(sf[s], frag_rows(sDO, PV, 16 * t, 32 * s, lane), G1[t]);
+                            dWt[t] = Mma<T>::run(sf[s], frag_rows(sDvn, PV, 16 * t, 32 * s, lane), dWt[t]);
+                            dKS[t] = Mma<T>::run(df[s], frag_rows(sVn, PV, 16 * t, 32 * s, lane), dKS[t]);
+                        }
+                    }
+                    const int n16 = feat(a);
+                    V8 fk[2], fq[2];
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) { fk[s] = frag_cols(sK, PK, 32 * s, n16, lane); fq[s] = frag_cols(sQ, PK, 32 * s, n16, lane); }
 #pragma unroll
                     for (int t = 0; t < 4; ++t) {
-                        G1[t] = Mma<T>::run(sf[s], frag_rows(sDO, PV, 16 * t, 32 * s, lane), G1[t]);
-                        dWt[t] = Mma<T>::run(sf[s], frag_rows(sDvn, PV, 16 * t, 32 * s, lane), dWt[t]);
-                        dKS[t] = Mma<T>::run(df[s], frag_rows(sVn, PV, 16 * t, 32 * s, lane), dKS[t]);
+                        __builtin_amdgcn_sched_barrier(0);
+                        dw[a][t] = pack4<T>(-dWt[t]);
+                        const int x = 16 * t + c16;
+                        f32x4 q_ = G1[t] * (p.scale * sEg[x]), k_ = dKS[t] * sEl[x];
+                        const V4 q4 = *(const V4*)(sQ + x * PK + n16 + 4 * g), k4 = *(const V4*)(sK + x * PK + n16 + 4 * g);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) dglast += (float)k4[r] * k_[r];
+#pragma unroll
+                        for (int s = 0; s < 2; ++s) {
+                            if (32 * s <= 16 * t + 15) q_ = Mma<T>::run(fk[s], frag_rows(sM1, P64, 16 * t, 32 * s, lane), q_);     // dP[i][j] = 0 for j > i
+                            if (32 * s + 31 >= 16 * t) k_ = Mma<T>::run(fq[s], frag_cols(sM1, P64, 32 * s, 16 * t, lane), k_);     // ... and for i < j
+                        }
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) dgx[t] += (float)q4[r] * q_[r] - (float)k4[r] * k_[r];
+                        pin(dgx[t]);
+                        dq[a][t] += q_;
+                        dk[a][t] += k_;
                     }
-                }
-                const int n16 = feat(a);
-                V8 fk[2], fq[2];
-#pragma unroll
-                for (int s = 0; s < 2; ++s) { fk[s] = frag_cols(sK, PK, 32 * s, n16, lane); fq[s] = frag_cols(sQ, PK, 32 * s, n16, lane); }
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    dw[a][t] = pack4<T>(-dWt[t]);
-                    const int x = 16 * t + c16;
-                    f32x4 q_ = G1[t] * (p.scale * sEg[x]), k_ = dKS[t] * sEl[x];
-                    const V4 q4 = *(const V4*)(sQ + x * PK + n16 + 4 * g), k4 = *(const V4*)(sK + x * PK + n16 + 4 * g);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) dglast += (float)k4[r] * k_[r];
-#pragma unroll
-                    for (int s = 0; s < 2; ++s) {
-                        if (32 * s <= 16 * t + 15) q_ = Mma<T>::run(fk[s], frag_rows(sM1, P64, 16 * t, 32 * s, lane), q_);     // dP[i][j] = 0 for j > i
-                        if (32 * s + 31 >= 16 * t) k_ = Mma<T>::run(fq[s], frag_cols(sM1, P64, 32 * s, 16 * t, lane), k_);     // ... and for i < j
-                    }
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) dgx[t] += (float)q4[r] * q_[r] - (float)k4[r] * k_[r];
-                    pin(dgx[t]);
-                    dq[a][t] += q_;
-                    dk[a][t] += k_;
                 }
             }
 #pragma unroll
