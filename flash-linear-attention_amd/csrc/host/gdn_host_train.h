@@ -72,7 +72,7 @@ ChunkGrads chunk_backward(const ChunkCall& c, const at::Tensor& q, const at::Ten
     return r;
 }
 
-int64_t gate_parts(int64_t rows, int64_t HV) { return std::max<int64_t>(1, std::min<int64_t>(256, rows * HV / 2048)); }
+int64_t gate_parts(int64_t rows, int64_t HV) { return std::max<int64_t>(1, std::min<int64_t>(256, rows * HV / 256)); }
 
 // ---- the operator ----
 struct ChunkTrain : torch::autograd::Function<ChunkTrain> {

@@ -153,7 +153,7 @@ def gate_bwd(dgate, dbeta, g, beta, A_log, dt_bias, beta_max):
         g = g.contiguous()
     beta = beta if beta.dtype in (torch.bfloat16, torch.float16, torch.float32) else beta.float()
     beta = beta.contiguous()
-    parts = max(1, min(256, rows * HV // 2048))
+    parts = max(1, min(256, rows * HV // 256))
     dg = torch.empty_like(g) if with_gate else None
     db = torch.empty_like(beta)
     part = torch.empty(parts, 2, HV, dtype=torch.float32, device=dev) if with_gate else None

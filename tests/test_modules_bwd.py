@@ -367,3 +367,16 @@ def test_modules_backward_without_tokens():
     out = mods.rms_norm_gated(xn, xn.detach(), wn, None)
     out.sum().backward()
     assert xn.grad.shape == xn.shape and not wn.grad.any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('rows,n', [(1, 1), (31, 33), (32, 32), (33, 31), (256, 5), (257, 64), (1024, 512), (1030, 12)])
+def test_sum_rows_edges(rows, n):
+    """Rows that are no multiple of the 256 a pass takes, columns that are no multiple of a workgroup's 32: fp32 sums of `rows` terms
+    are within rows * 2^-24 of the sum of the magnitudes."""
+    from fla_hip.ops.gated_delta_rule._common import sum_rows
+    part = torch.randn(rows, n, device='cuda', generator=torch.Generator('cuda').manual_seed(rows))
+    got = sum_rows(part, torch.float32)
+    bound = part.double().abs().sum(0) * max(rows, 2) * 2.0 ** -24
+    assert ((got.double() - part.double().sum(0)).abs() <= bound).all()
+    assert torch.equal(got, sum_rows(part, torch.float32))
