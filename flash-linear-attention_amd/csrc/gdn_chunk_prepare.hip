@@ -276,8 +276,242 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
     }
 }
 
+// The same with four waves to a unit, for calls of so few units that the waves of a CU have nobody to wait for but themselves (launch_prepare):
+// what bounds them is one unit's chain of steps.  Wave w takes the tiles (a, w), a <= w, of K K^T and of k q^T - loads, products, gates,
+// P and X of token tile w are its own -, the diagonal block w of the inverse, and after that the block column w of T from the bottom up,
+//     T_aw = -T_aa sum_{a < m <= w} U_am T_mw,
+// left factors U_am and T_aa from LDS, right factors the blocks it has just computed.  Two barriers: one for the gates and the norms, which wave 0
+// and the diagonal tiles' owners supply, one for the left factors.
+// 333 tokens, 32 heads (192 units): 27.5 -> 22.3 us a call; 1000 tokens, 16 heads: 42.7 -> 37.7; 1000 tokens, 8 heads of 256: 77.4 -> 69.7.
+// Up to three workgroups a CU, one round of the chip: at 704 units still 54.8 -> 52.5 us, at 792 already 49.8 -> 51.4, at 1008 122.5 -> 124.4.
+constexpr int TEAM_TILE = 16 * TP;
+constexpr int64_t TEAM_UNITS = 3 * 256;
+template <typename T, bool WANT_P>
+__global__ __launch_bounds__(256, 2) void gdn_chunk_prepare_team_kernel(ChunkParams p) {
+    typedef typename Mma<T>::V8 V8;
+    __shared__ __align__(16) float smem[10 * TEAM_TILE + 4 * 256 + 4 * 64];
+    auto tile = [&](int n) { return smem + n * TEAM_TILE; };
+    auto pair = [](int a, int m) { return 4 + m * (m - 1) / 2 + a; };        // U_am, a < m, behind the four T_aa
+    float* sG = smem + 10 * TEAM_TILE + 4 * 256; float* sBeta = sG + 64; float* sK2 = sBeta + 64; float* sNQ = sK2 + 64;
+    const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float* sLd = smem + 10 * TEAM_TILE + w * 256;                            // the diagonal block of L, by rows
+    const int64_t u = blockIdx.x;
+    const int H = p.H, HV = p.HV, G = HV / H, K = p.K;
+    const int64_t ci = u / HV;
+    const int hv = (int)(u % HV), h = hv / G;
+    const bool cu32 = p.flags & GDN_FLAG_CU_INT32;
+    int64_t tok0;
+    int valid;
+    if (p.cu_seqlens) {
+        const int64_t n = load_index(p.chunk_table, 2 * ci, cu32), it = load_index(p.chunk_table, 2 * ci + 1, cu32);
+        const int64_t bos = load_index(p.cu_seqlens, n, cu32), eos = load_index(p.cu_seqlens, n + 1, cu32);
+        tok0 = bos + it * CH;
+        valid = (int)min((int64_t)CH, eos - tok0);
+    } else {
+        const int64_t b = ci / p.NT, it = ci % p.NT;
+        tok0 = b * p.T + it * CH;
+        valid = (int)min((int64_t)CH, p.T - it * CH);
+    }
+    const bool l2 = p.flags & GDN_FLAG_QK_L2NORM, q_norms_here = l2 && !(p.flags & FLAG_Q_NORM_IN_SCAN), want_q = WANT_P || q_norms_here;
+    char* rec = p.ws.Rec + (ci * HV + hv) * REC_BYTES;
+
+    uint32_t rg = 0, rb = 0;
+    if (w == 0 && lane < valid) {
+        rg = p.g ? load_scalar_bits(p.g, (tok0 + lane) * HV + hv, p.gb_dtype) : 0;
+        rb = load_scalar_bits(p.beta, (tok0 + lane) * HV + hv, p.beta_dtype);
+    }
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 U[4], QK[4], QQ = zero;                            // tiles (a, w): rows keys of tile a, columns tokens of tile w
+#pragma unroll
+    for (int a = 0; a < 4; ++a) U[a] = QK[a] = zero;
+    {
+        const T* kg = (const T*)p.k + (tok0 * H + h) * K;
+        const T* qg = (const T*)p.q + (tok0 * H + h) * K;
+        const u32x4 z = {0u, 0u, 0u, 0u};
+        const uint32_t lane_off = ((uint32_t)c16 * (uint32_t)(H * K) + 8u * g) * (uint32_t)sizeof(T);
+        auto fragment = [&](const T* rows, int t, int col0) {
+            const char* bp = (const char*)(rows + (int64_t)(16 * t) * H * K + col0);
+            if (valid == CH && col0 + 32 <= K) return *(const u32x4*)(bp + lane_off);
+            return (16 * t + c16 < valid && col0 + 8 * g < K) ? *(const u32x4*)(bp + lane_off) : z;
+        };
+        for (int k0 = 0; k0 < K; k0 += 128) {
+            u32x4 fo[4], fk[4][4], fq[4];                    // (fo: the wave's own tile)
+#pragma unroll
+            for (int s4 = 0; s4 < 4; ++s4) fo[s4] = fragment(kg, w, k0 + 32 * s4);
+#pragma unroll
+            for (int s4 = 0; s4 < 4; ++s4) fq[s4] = want_q ? fragment(qg, w, k0 + 32 * s4) : z;
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                if (a < w) {
+#pragma unroll
+                    for (int s4 = 0; s4 < 4; ++s4) fk[a][s4] = fragment(kg, a, k0 + 32 * s4);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s4 = 0; s4 < 4; ++s4) {
+                const V8 o8 = __builtin_bit_cast(V8, fo[s4]), q8 = __builtin_bit_cast(V8, fq[s4]);
+                U[3] = Mma<T>::run(o8, o8, U[3]);            // (the diagonal tile lies at 3 until it is moved to its place below)
+                if constexpr (WANT_P) QK[3] = Mma<T>::run(o8, q8, QK[3]);
+                if (want_q) QQ = Mma<T>::run(q8, q8, QQ);
+            }
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                if (a < w) {
+#pragma unroll
+                    for (int s4 = 0; s4 < 4; ++s4) {
+                        const V8 k8 = __builtin_bit_cast(V8, fk[a][s4]);
+                        U[a] = Mma<T>::run(k8, __builtin_bit_cast(V8, fo[s4]), U[a]);
+                        if constexpr (WANT_P) QK[a] = Mma<T>::run(k8, __builtin_bit_cast(V8, fq[s4]), QK[a]);
+                    }
+                }
+        }
+    }
+    const f32x4 Ud = U[3], QKd = QK[3];
+    // |k_t|^2 and |q_t|^2 are the diagonals of the diagonal tiles
+    {
+        float dk = 0.f, dq = 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (r == (c16 & 3)) { dk = Ud[r]; dq = QQ[r]; }
+        if ((c16 >> 2) == g) { sK2[16 * w + c16] = dk; sNQ[16 * w + c16] = l2 && want_q ? rsqrtf(dq + 1e-6f) : 1.f; }
+    }
+    float x = 0.f, b = 0.f;                                  // (wave 0: the running sum of the gates and beta of token `lane`)
+    if (w == 0) {
+        x = scalar_of_bits(rg, p.gb_dtype); b = scalar_of_bits(rb, p.beta_dtype);
+        if (lane < valid) {
+            if (p.A_log && p.g) x = -__expf(p.A_log[hv]) * softplus_f(x + (p.dt_bias ? p.dt_bias[hv] : 0.f));
+            if (p.flags & GDN_FLAG_BETA_SIGMOID) b = sigmoid_f(b) * ((p.flags & GDN_FLAG_NEG_EIGVAL) ? 2.f : 1.f);
+        }
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const float y = __shfl_up(x, off, 64);
+            if (lane >= off) x += y;
+        }
+        x *= RCP_LN2_F;
+        sG[lane] = x;
+        sBeta[lane] = b;
+    }
+    __syncthreads();
+
+    auto norm_of = [&](float k2) { return l2 ? rsqrtf(k2 + 1e-6f) : 1.f; };
+    const int i = 16 * w + c16;                              // this lane's column: token i
+    const float gi = sG[i], nki = norm_of(sK2[i]), bni = sBeta[i] * nki, st = p.scale * sNQ[i];
+    V8 pf[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pf[s][e] = from_f32<T>(0.f);
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        if (a > w) continue;
+        const f32x4 gj = *(const f32x4*)(sG + 16 * a + 4 * g), kj = *(const f32x4*)(sK2 + 16 * a + 4 * g);
+        const f32x4 Ua = a == w ? Ud : U[a < 3 ? a : 0], Qa = a == w ? QKd : QK[a < 3 ? a : 0];
+        f32x4 val;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            // select, never multiply by a mask: 2^(G_i-G_j) may overflow for i < j
+            const float d = a < w || c16 >= 4 * g + r ? fast_exp2(gi - gj[r]) * norm_of(kj[r]) : 0.f;
+            val[r] = a < w || c16 > 4 * g + r ? bni * Ua[r] * d : 0.f;
+            if constexpr (WANT_P) pf[a >> 1][4 * (a & 1) + r] = from_f32<T>(st * Qa[r] * d);
+        }
+        if (a == w) *(f32x4*)(sLd + c16 * 16 + 4 * g) = val;           // L[i = c16][j = 4g + r]
+        else {
+            float* t = tile(pair(a, w));
+#pragma unroll
+            for (int r = 0; r < 4; ++r) t[(4 * g + r) * TP + c16] = val[r];
+        }
+    }
+    if constexpr (WANT_P) {
+        store_frag<T>(rec + REC_P, w, 0, lane, pf[0]);
+        if (w >= 2) store_frag<T>(rec + REC_P, w, 1, lane, pf[1]);     // (identically zero for the first two tiles, not stored)
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (LDS operations of a wave execute in order)
+    // ---- the diagonal block: X (I + L) = I by rows, from the right; lane c16 owns row c16 (every lane group the same) ----
+    {
+        float xr[16], acc[16];
+#pragma unroll
+        for (int n = 0; n < 16; ++n) acc[n] = 0.f;
+#pragma unroll
+        for (int n = 15; n >= 0; --n) {
+            xr[n] = ((n == c16) ? 1.f : 0.f) - acc[n];
+            float row[16];
+#pragma unroll
+            for (int q4 = 0; q4 < (n + 3) / 4; ++q4) *(f32x4*)(row + 4 * q4) = *(const f32x4*)(sLd + n * 16 + 4 * q4);
+#pragma unroll
+            for (int j = 0; j < n; ++j) acc[j] += row[j] * xr[n];
+        }
+        if (g == 0) {                                        // T(w,w) = X^T as a left factor: [row j][column c16]
+            float* t = tile(w);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) t[j * TP + c16] = xr[j];
+        }
+    }
+    if (w == 0) {
+        // the tables and the bound on the chunk's transition (as in gdn_chunk_prepare_kernel)
+        const float xl = __shfl(x, 63, 64), ex = fast_exp2(x);
+        const float k2 = sK2[lane], nk = norm_of(k2), nq = q_norms_here ? sNQ[lane] : 1.f;
+        float* tab = (float*)(rec + REC_TAB);
+        tab[TAB_DEC + lane] = fast_exp2(xl - x) * nk;
+        tab[TAB_SG + lane] = p.scale * ex * nq;
+        tab[TAB_EG + lane] = ex * nk;
+        if (lane == 63) tab[TAB_GLAST] = x;
+        float* tab2 = (float*)(rec + REC_TAB2);
+        tab2[TAB2_G + lane] = x;
+        tab2[TAB2_NQS + lane] = p.scale * nq;
+        tab2[TAB2_NK + lane] = nk;
+        float lb = fabsf(1.f - b * k2 * nk * nk);
+        lb = lb > 1.f ? __log2f(lb) : 0.f;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) lb += __shfl_xor(lb, off, 64);
+        if (lane == 63) p.ws.Bound[ci * HV + hv] = x + lb;
+    }
+    __syncthreads();
+
+    // ---- block column w of T ----
+    auto mul = [&](int n, f32x4 B, f32x4 acc) {              // acc + A B: A a tile of LDS by rows, B in accumulator layout
+        const f32x4 A = *(const f32x4*)(tile(n) + c16 * TP + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(A[e], B[e], acc, 0, 0, 0);
+        return acc;
+    };
+    f32x4 X[4];
+#pragma unroll
+    for (int a = 3; a >= 0; --a) {
+        X[a] = zero;
+        if (a > w) continue;
+        if (a == w) {
+            const float* t = tile(a);
+            X[a] = f32x4{t[(4 * g) * TP + c16], t[(4 * g + 1) * TP + c16], t[(4 * g + 2) * TP + c16], t[(4 * g + 3) * TP + c16]};
+            continue;
+        }
+        f32x4 t = zero;
+#pragma unroll
+        for (int m = a + 1; m < 4; ++m)
+            if (m <= w) t = mul(pair(a, m), X[m], t);
+        X[a] = -mul(a, t, zero);
+    }
+    // ---- Xb = X diag(beta) of token tile w as operand fragments: columns {32sp + 4g + e} and {32sp + 16 + 4g + e} ----
+#pragma unroll
+    for (int sp = 0; sp < 2; ++sp) {
+        if (2 * sp > w) continue;
+        const f32x4 blo = *(const f32x4*)(sBeta + 32 * sp + 4 * g), bhi = *(const f32x4*)(sBeta + 32 * sp + 16 + 4 * g);
+        V8 frag;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            frag[e] = from_f32<T>(X[2 * sp][e] * blo[e]);
+            frag[4 + e] = from_f32<T>(X[2 * sp + 1][e] * bhi[e]);
+        }
+        store_frag<T>(rec + REC_X, w, sp, lane, frag);
+    }
+}
+
 template <typename T, bool WANT_P>
 static int launch_prepare_as(const ChunkParams& p, int64_t units, hipStream_t stream) {
+    if (units <= TEAM_UNITS) {
+        hipLaunchKernelGGL((gdn_chunk_prepare_team_kernel<T, WANT_P>), dim3((unsigned)units), dim3(256), 0, stream, p);
+        return check_launch("gdn_chunk_prepare_team_kernel");
+    }
     auto kern = gdn_chunk_prepare_kernel<T, WANT_P>;
     static SmemAttrDone attr_done;       // per instantiation
     if (int rc = ensure_dynamic_smem((const void*)kern, PREP_SMEM, attr_done, "hipFuncSetAttribute(prepare)")) return rc;

@@ -605,3 +605,27 @@ def test_reference_whole_operator_backend_matrix_packed(H, D, cu):
     o, ht = _run(q, k, v, g, beta, h0, cu, scale=D ** -0.5, use_qk_l2norm_in_kernel=True)
     _check('o', ref_o, o, ratio=0.008)
     _check('ht', ref_ht, ht, ratio=0.008)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('l2norm', [False, True])
+@pytest.mark.parametrize('T,K,V,dtype', [(1, 128, 128, torch.bfloat16), (17, 64, 64, torch.bfloat16), (64, 128, 128, torch.float16), (100, 200, 128, torch.bfloat16),
+                                         (63, 40, 64, torch.bfloat16)])
+def test_prepare_by_four_waves_or_one(T, K, V, dtype, l2norm):
+    """Few (chunk, head) pairs are prepared by four waves each, many by one: the same sequence alone and in a batch on the other side of the
+    line gives the same results but for the last bit of an operand, and both hold to the oracle."""
+    from fla_hip.ops.gated_delta_rule import chunk_gated_delta_rule
+    q, k, v, g, beta, h0 = O.make_inputs(1, T, 1, 2, K, V, seed=T, gate_div=2.0, h0_std=0.3, N=1)
+    if not l2norm:
+        q, k = F.normalize(q, dim=-1), F.normalize(k, dim=-1)
+    q, k, v = (x.to(dtype) for x in (q, k, v))
+    ref_o, ref_ht = O.recurrent_gated_delta_rule(q, k, v, g, beta, initial_state=h0, output_final_state=True, use_qk_l2norm_in_kernel=l2norm)
+    out = []
+    for B in (1, 384 // ((T + 63) // 64) + 1):
+        args = [x.cuda().expand(B, *x.shape[1:]).contiguous() for x in (q, k, v, g, beta)]
+        o, ht = chunk_gated_delta_rule(*args, initial_state=h0.cuda().expand(B, *h0.shape[1:]).contiguous(), output_final_state=True,
+                                       use_qk_l2norm_in_kernel=l2norm)
+        assert torch.equal(o, o[:1].expand_as(o)) and torch.equal(ht, ht[:1].expand_as(ht))
+        out.append((o[:1].float().cpu(), ht[:1].cpu()))
+        assert O.get_err_ratio(ref_o, out[-1][0]) < 5e-3 and O.get_err_ratio(ref_ht, out[-1][1]) < 5e-3
+    assert O.get_err_ratio(out[0][0], out[1][0]) < 3e-3 and O.get_err_ratio(out[0][1], out[1][1]) < 3e-3
