@@ -149,8 +149,12 @@ inline size_t ws_align(size_t x) { return (x + 255) & ~(size_t)255; }
 // chip: a step of half a run takes 1.6 us, one of a whole run 2.7 - 3.2.  Not where the caller asks for one form of the scan.  Up to 36
 // chunks they also beat time segments, whose steps are those of whole runs, with a warm-up of some 8 of them and two more launches, or
 // the exact path's twice as many (1 x 2048 tokens, 32 heads, 4 segments: 98 us with heads that forget slowly).
+// 64 x 64: the same kernel's form for these, a workgroup a run (a step 1.2 us against 2.0): 500 tokens, 8 heads 25.1 -> 19.6 us, 8 x 1024 tokens,
+// 8 heads 44.5 -> 36.9, 20000 tokens of 32 heads in 4 sequences 343 -> 304; with more runs the chip is full, and P costs the prepare kernel
+// more than it saves the scan (256 runs of 40 chunks: 160 -> 172 us).  Time segments are as good from where they begin, 32 chunks (heads that
+// forget within one: 44.1 us, whole 47.8; that forget slowly: 70.5, whole 51.4), and keep these.
 inline bool halves_fit(int64_t NH, int64_t K, int64_t V, uint32_t flags) {
-    return K == 128 && V == 128 && NH <= 128 && !(flags & (GDN_FLAG_SCAN_WIDE | GDN_FLAG_SCAN_SEGMENTS | GDN_FLAG_SCAN_PAIR | GDN_FLAG_RECORD_P));
+    return ((K == 128 && V == 128) || (K == 64 && V == 64)) && NH <= 128 && !(flags & (GDN_FLAG_SCAN_WIDE | GDN_FLAG_SCAN_SEGMENTS | GDN_FLAG_SCAN_PAIR | GDN_FLAG_RECORD_P));
 }
 
 // Number of time segments the sequential stage cuts every sequence into (0: whole sequences, one
@@ -164,7 +168,7 @@ inline bool halves_fit(int64_t NH, int64_t K, int64_t V, uint32_t flags) {
 inline int plan_segments(int64_t N, int64_t HV, int64_t NT, int64_t num_chunks, bool dense, uint32_t flags, int64_t K, int64_t V) {
     const int64_t NH = N * HV;
     int nseg = 0;
-    if (halves_fit(NH, K, V, flags) && NT <= 36) return 0;
+    if (halves_fit(NH, K, V, flags) && NT <= (K == 128 ? 36 : 31)) return 0;
     if (dense && NH > 0) {
         // (GDN_FLAG_SCAN_SEGMENTS asks for segments wherever they are possible at all: segments of 4 chunks)
         nseg = (int)std::min<int64_t>(256 / NH, NT / ((flags & GDN_FLAG_SCAN_SEGMENTS) ? 4 : 8));

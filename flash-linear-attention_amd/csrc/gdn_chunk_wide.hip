@@ -61,9 +61,14 @@ constexpr int WIDE_THREADS = (CW + 4) * 64;
 // HALF: three buffers (chunk % 3) for k, q and the 64 columns of v, so that everything is requested two steps ahead (a step of half the
 // length leaves no time for a copy issued one ahead), two for the records (Xb, P, the first table), a narrower output tile.  v: blocks
 // of 4 rows x 8 pieces, laid out like the first half of the blocks above, two to a copy.
-constexpr int HALF_Q = 3 * 16384, HALF_V = 6 * 16384, HALF_V_BYTES = 8192, HALF_REC = HALF_V + 3 * HALF_V_BYTES;
-constexpr int HALF_NREC = REC_PIECES_X + REC_PIECES_P + 1, HALF_OT = HALF_REC + 2 * HALF_NREC * 1024, HALF_OT_PITCH = 144;
-constexpr size_t HALF_SMEM = HALF_OT + 64 * HALF_OT_PITCH;
+// The 64 x 64 form (SMALL with HALF: a whole run, its tiles of k and q laid out like that of v) has the same in half the room.
+constexpr int HALF_V_BYTES = 8192, HALF_NREC = REC_PIECES_X + REC_PIECES_P + 1, HALF_OT_PITCH = 144;
+constexpr int half_k_bytes(bool small) { return small ? 8192 : 16384; }
+constexpr int half_q(bool small) { return 3 * half_k_bytes(small); }
+constexpr int half_v(bool small) { return 6 * half_k_bytes(small); }
+constexpr int half_rec(bool small) { return half_v(small) + 3 * HALF_V_BYTES; }
+constexpr int half_ot(bool small) { return half_rec(small) + 2 * HALF_NREC * 1024; }
+constexpr size_t half_smem(bool small) { return half_ot(small) + 64 * HALF_OT_PITCH; }
 
 template <typename T, bool FULL, bool DIMS128, bool SMALL, bool HALF = false>
 __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParams p, SegmentPlan sp) {
@@ -77,8 +82,12 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
     // forming P would then be the longest part of a step: P comes with the records (the prepare kernel forms it for all chunks at once),
     // and the output wave copies them.  A step takes 3900 cycles alone on its CU (6000 for a whole run), 2300 of them the LDS' share:
     // every wave reads all of k and q.  1500 tokens, 32 heads: 87 -> 57 us a call; 333 tokens: 33.5 -> 28 us.
-    static_assert(!HALF || (DIMS128 && FULL), "whole runs of 128 x 128");
-    const int K = DIMS128 ? 128 : p.K, V = DIMS128 ? 128 : p.V;
+    // SMALL with HALF (K = V = 64): a workgroup a run - four compute waves of 16 columns are all of them -, everything else as above: what
+    // bounds a step of the 64 x 64 form otherwise are copies issued one step ahead and P (2.0 us a step, 1.2 us here; halves_fit).
+    constexpr bool HALF64 = HALF && SMALL;
+    static_assert(!HALF || (DIMS128 != SMALL && FULL), "whole runs of 128 x 128 or 64 x 64");
+    const int K = DIMS128 ? 128 : HALF64 ? 64 : p.K, V = DIMS128 ? 128 : HALF64 ? 64 : p.V;
+    constexpr int HALF_K_BYTES = half_k_bytes(SMALL), HALF_Q = half_q(SMALL), HALF_V = half_v(SMALL), HALF_REC = half_rec(SMALL), HALF_OT = half_ot(SMALL);
     constexpr int KS = SMALL ? 2 : 4;                 // pairs of 16-row key tiles (32 key features each)
     typedef typename Mma<T>::V8 V8;
     typedef typename Mma<T>::V4 V4;
@@ -107,7 +116,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
     const float* src = nullptr;
     float* dst = nullptr;
     if (sp.kind == WIDE_WHOLE) {
-        const int64_t member = HALF ? slot >> 1 : slot, group = (member / G) * 8 + xcd;                 // (sequence, q/k head)
+        const int64_t member = HALF && !SMALL ? slot >> 1 : slot, group = (member / G) * 8 + xcd;                 // (sequence, q/k head)
         if (group >= p.N * H) return;
         int64_t nseq = group / H;
         if (p.flags & GDN_FLAG_SEQ_ORDER) nseq = load_index(p.chunk_offsets, p.N + 1 + nseq, cu32);     // longest sequences start first
@@ -156,7 +165,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         }
         if (seg == sp.nseg - 1 && p.ht) { dst = p.ht + inh * (int64_t)(K * V); dst_user = true; }
     }
-    const int col0 = HALF ? 64 * (int)(slot & 1) : 0;       // first value column of this workgroup
+    const int col0 = HALF && !SMALL ? 64 * (int)(slot & 1) : 0;       // first value column of this workgroup
     const int64_t n = inh / HV;
     const int hv = (int)(inh % HV);
     const int h = hv / (HV / H);
@@ -193,7 +202,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
     // chunk it+1 must have landed at B2.  Loads complete in issue order, so "at most
     // N operations outstanding" proves that all but the N newest have landed.
     // =====================================================================================
-    if (K < 128 && nsteps > 0) {
+    if (!HALF && K < 128 && nsteps > 0) {
         // key features past K: clear the q and k tiles once; the copies never touch those pieces
         const u32x4 z = {0u, 0u, 0u, 0u};
         for (int i = tid; i < (2 * 16384) / 16; i += WIDE_THREADS) {
@@ -319,7 +328,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         // The records of a full run: copied by the output wave, or, where REC_Q, by q's.  In the 64 x 64 form a step is short and the
         // output wave, with its share of P and the stores, has no room left for them: 8 x 1024 tokens, 8 heads 46.2 us there, 42.9 us on
         // q's wave; 20000 packed tokens, 32 heads 154.0 and 149.9 us.
-        constexpr bool REC_Q = FULL && SMALL;
+        constexpr bool REC_Q = FULL && SMALL && !HALF;
         auto copy_records = [&](int64_t it, uint32_t st) {
             copy_rec(it, 0, REC_PIECES_X, st);
             copy_rec(it, REC_PIECE_TAB, REC_PIECE_TAB + 1, st);
@@ -340,21 +349,25 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
                     lds_barrier();                                          // B2
                 }
             };
-            if (w == CW) walk([&](int64_t i) { gather_blocks((const T*)p.k, min(it0 + i, lastc), 0, 16, lds0 + (int)(i % 3) * 16384); }, std::integral_constant<int, 16>{});
-            else if (w == CW + 1) walk([&](int64_t i) { gather_blocks((const T*)p.q, min(it0 + i, lastc), 0, 16, lds0 + HALF_Q + (int)(i % 3) * 16384); }, std::integral_constant<int, 16>{});
-            else if (w == CW + 2) {
-                const int s5 = lane & 31;                                   // slot inside a block of 4 rows x 8 pieces
-                walk([&](int64_t i) {
-                    const int64_t it = min(it0 + i, lastc);
-                    const int valid = (int)min((int64_t)CH, len - it * CH);
-                    const char* base = (const char*)((const T*)p.v + ((bos + it * CH) * HV + hv) * V);
+            // a tile of 64 rows of 128 bytes: two blocks of 4 rows x 8 pieces to a copy
+            auto gather_rows64 = [&](const T* tensor, int64_t i, uint32_t lds_tile) {
+                const int s5 = lane & 31;                                   // slot inside a block
+                const int64_t it = min(it0 + i, lastc);
+                const int valid = (int)min((int64_t)CH, len - it * CH);
+                const char* base = (const char*)(tensor + ((bos + it * CH) * heads + head) * dim);
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const int b = 2 * j + (lane >> 5), row = min(4 * b + ((s5 & 15) >> 2), valid - 1), c = 4 * (s5 >> 4) + ((s5 - b) & 3);
-                        gather_1k_to_lds(base, (uint32_t)row * row_bytes + 16 * c + 2 * col0, lds0 + HALF_V + (int)(i % 3) * HALF_V_BYTES + j * 1024);
-                    }
-                }, std::integral_constant<int, 8>{});
-            }
+                for (int j = 0; j < 8; ++j) {
+                    const int b = 2 * j + (lane >> 5), row = min(4 * b + ((s5 & 15) >> 2), valid - 1), c = 4 * (s5 >> 4) + ((s5 - b) & 3);
+                    gather_1k_to_lds(base, (uint32_t)row * row_bytes + 16 * c + (is_v ? 2 * col0 : 0), lds_tile + j * 1024);
+                }
+            };
+            if constexpr (SMALL) {
+                const T* tensor = (const T*)(w == CW ? p.k : w == CW + 1 ? p.q : p.v);
+                const int at = w == CW ? 0 : w == CW + 1 ? HALF_Q : HALF_V;
+                walk([&](int64_t i) { gather_rows64(tensor, i, lds0 + at + (int)(i % 3) * 8192); }, std::integral_constant<int, 8>{});
+            } else if (w == CW) walk([&](int64_t i) { gather_blocks((const T*)p.k, min(it0 + i, lastc), 0, 16, lds0 + (int)(i % 3) * 16384); }, std::integral_constant<int, 16>{});
+            else if (w == CW + 1) walk([&](int64_t i) { gather_blocks((const T*)p.q, min(it0 + i, lastc), 0, 16, lds0 + HALF_Q + (int)(i % 3) * 16384); }, std::integral_constant<int, 16>{});
+            else walk([&](int64_t i) { gather_rows64((const T*)p.v, i, lds0 + HALF_V + (int)(i % 3) * HALF_V_BYTES); }, std::integral_constant<int, 8>{});
         } else if (w == CW) {
             // ---- k: the copy of chunk i+2 is issued at the start of step i (its buffer was last read
             // in step i-1) and awaited at the end of step i+1 ----
@@ -508,8 +521,9 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
     // four 4-element runs addressed by lanes j, j+4, j+8, j+12 of its 16-lane group: this lane
     // addresses row i = c16/4 of the 4-row run and column group j = c16%4.
     const int tr_i = c16 >> 2, tr_j = c16 & 3;
-    const int a_off = (c16 >> 2) * 64 + 4 * (c16 & 3) + ((g + (c16 >> 2)) & 3);  // operand piece 4s + g of row c16 of a t-tile: + tt*256 + 16*s  (16-byte units)
-    const int k_tr = (g * 64 + 4 * tr_i + ((tr_j + g) & 3)) * 8;                 // row 4g+i of a 16-row group, piece 4*(m/2) + j: + (32*sp2 + 16*half)*128 + 128*(m/2) + 4*(m&1)  (elements)
+    constexpr int BLK = HALF64 ? 32 : 64;                                         // slots of a block of 4 rows of k and q
+    const int a_off = (c16 >> 2) * BLK + 4 * (c16 & 3) + ((g + (c16 >> 2)) & 3);  // operand piece 4s + g of row c16 of a t-tile: + tt*4*BLK + 16*s  (16-byte units)
+    const int k_tr = (g * BLK + 4 * tr_i + ((tr_j + g) & 3)) * 8;                 // row 4g+i of a 16-row group, piece 4*(m/2) + j: + (32*sp2 + 16*half)*128 + 128*(m/2) + 4*(m&1)  (elements)
     int v_tr[NN];                                                                 // row 4g+i, piece = 8-column group of tile nn: + tt*2048
 #pragma unroll
     for (int nn = 0; nn < NN; ++nn) {
@@ -534,14 +548,14 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         auto fence = [] { if constexpr (!HALF) __builtin_amdgcn_sched_barrier(0); };      // (HALF: the compiler's own order is 1 % faster)
 
         // fragment f = (t-tile f/4, key tiles (2s, 2s+1) with s = f%4) of k and q, in a ring of RING register sets
-        constexpr int RING = HALF ? 6 : WIDE_RING;
+        constexpr int RING = HALF64 ? 9 : HALF ? 6 : WIDE_RING;           // (HALF64: all eight)
         V8 ak[RING], aq[RING];
         // (HALF: the t-tiles of a pair take turns, so that neighbouring matrix instructions do not wait for each other's sums)
-        auto tile_of = [](int f) { return HALF ? 2 * (f >> 3) + (f & 1) : f / KS; };
-        auto pair_of = [](int f) { return HALF ? (f & 7) >> 1 : f % KS; };
+        auto tile_of = [](int f) { return HALF ? 2 * (f / (2 * KS)) + (f & 1) : f / KS; };
+        auto pair_of = [](int f) { return HALF ? f % (2 * KS) >> 1 : f % KS; };
         auto F = [&](int f) {
-            ak[f % RING] = sK[tile_of(f) * 256 + 16 * pair_of(f) + a_off];
-            if constexpr (FULL) aq[f % RING] = sQ[tile_of(f) * 256 + 16 * pair_of(f) + a_off];
+            ak[f % RING] = sK[tile_of(f) * (4 * BLK) + 16 * pair_of(f) + a_off];
+            if constexpr (FULL) aq[f % RING] = sQ[tile_of(f) * (4 * BLK) + 16 * pair_of(f) + a_off];
         };
         f32x4 ks[4][NN], ao[4][NN];
         V8 Sb[KS][NN];
@@ -571,8 +585,8 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         };
         V8 kt[2][2 * KS];                       // k^T rows of key tile m over t-tile pair sp2
         auto FK = [&](int sp2, int m) {
-            const T* a = sKt + sp2 * 4096 + 128 * (m >> 1) + 4 * (m & 1) + k_tr;
-            kt[sp2][m] = join<V8>(Mma<T>::tr_read(a), Mma<T>::tr_read(a + 2048));
+            const T* a = sKt + sp2 * (64 * BLK) + 128 * (m >> 1) + 4 * (m & 1) + k_tr;
+            kt[sp2][m] = join<V8>(Mma<T>::tr_read(a), Mma<T>::tr_read(a + 32 * BLK));
         };
         float gamma, vscale;
         V8 Db[2][NN], Vn[2][NN], Vg[2][NN];
@@ -666,7 +680,24 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
             }
             lg = lazy ? lg_try : 0.f;
         };
-        if constexpr (SMALL) {
+        if constexpr (HALF64) {
+            FV(0); FV(1); FX(0); FX(1);
+            M(0); M(1); M(2); M(3);
+            FV(2); FV(3); FX(2); FX(3);
+            M(4); M(5); M(6); M(7);
+            TD(0); TD(1); FK(0, 0); FK(0, 1); FK(0, 2); FK(0, 3);
+            TXa(0); TXa(1); FK(1, 0); FK(1, 1); FK(1, 2); FK(1, 3);
+            TXb(0); TXb(1);
+            fold();
+            TD(2); TD(3); U(0, 0); U(0, 1); U(0, 2); U(0, 3);
+            TXa(2); TXa(3); FP(0); FP(1); FP(2); FP(3);
+            TXb(2); TXb(3); TPa(0); TPa(1);
+            U(1, 0); U(1, 1); TPb(0); TPb(1); TPa(2); TPa(3);
+            TPb(2); TPb(3);
+            lds_barrier();                                          // B1
+            U(1, 2); U(1, 3);
+            lds_barrier();                                          // B2
+        } else if constexpr (SMALL) {
             // ---- eight fragments (two per t-tile), four state tiles per wave.  The chain that the next step waits for
             // is M(7) -> D, v_new of t-tiles 2, 3 -> their state update; the tail of tiles 0, 1 and everything of the
             // output fill its gaps ----
@@ -734,7 +765,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         for (int64_t i = 0; i < nsteps; ++i) {
             const char* st = smem + (i & 1) * STG_BYTES;
             const int b3 = (int)(i % 3);
-            if constexpr (HALF) step(smem + b3 * 16384, smem + HALF_Q + b3 * 16384, smem + HALF_V + b3 * HALF_V_BYTES, smem + HALF_REC + (int)(i & 1) * (HALF_NREC * 1024), 0);
+            if constexpr (HALF) step(smem + b3 * HALF_K_BYTES, smem + HALF_Q + b3 * HALF_K_BYTES, smem + HALF_V + b3 * HALF_V_BYTES, smem + HALF_REC + (int)(i & 1) * (HALF_NREC * 1024), 0);
             else step(smem + KBUF + b3 * 16384, st + STG_Q, st + STG_V, st + STG_REC, 4 * ((int)i + 1));
         }
     }
@@ -850,9 +881,10 @@ template <typename T, bool FULL, bool DIMS128, bool SMALL, bool HALF = false>
 static int launch_wide_dims(const ChunkParams& p, const SegmentPlan& sp, int64_t blocks, hipStream_t stream) {
     auto kern = gdn_chunk_wide_kernel<T, FULL, DIMS128, SMALL, HALF>;
     static SmemAttrDone attr_done;       // per instantiation
-    if (int rc = ensure_dynamic_smem((const void*)kern, HALF ? HALF_SMEM : WIDE_SMEM, attr_done, "hipFuncSetAttribute(wide)")) return rc;
+    constexpr size_t smem = HALF ? half_smem(SMALL) : WIDE_SMEM;
+    if (int rc = ensure_dynamic_smem((const void*)kern, smem, attr_done, "hipFuncSetAttribute(wide)")) return rc;
     if (blocks <= 0) return GDN_OK;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(WIDE_THREADS), HALF ? HALF_SMEM : WIDE_SMEM, stream, p, sp);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(WIDE_THREADS), smem, stream, p, sp);
     return check_launch("gdn_chunk_wide_kernel");
 }
 
@@ -872,6 +904,7 @@ int launch_wide(const ChunkParams& p, SegmentPlan sp, hipStream_t stream) {
     if (sp.kind == WIDE_WHOLE) {
         sp.nseg = 1;
         sp.seg_chunks = 1 << 30;
+        if (p.halves && p.K == 64) return launch_wide_dims<T, true, false, true, true>(p, sp, (p.N * p.H + 7) / 8 * 8 * G, stream);
         if (p.halves) return launch_wide_dims<T, true, true, false, true>(p, sp, (p.N * p.H + 7) / 8 * 8 * G * 2, stream);
         return launch_wide_kind<T, true>(p, sp, (p.N * p.H + 7) / 8 * 8 * G, stream);
     }

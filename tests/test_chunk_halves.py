@@ -1,5 +1,5 @@
-"""The scan in halves of 64 value columns (whole sequences, up to 128 runs of 128 x 128): one chunk and less, remainders, the last run
-count that takes it and the first that does not, packed sequences with an empty one, states in both layouts."""
+"""The scan in halves of 64 value columns (whole sequences, up to 128 runs of 128 x 128) and its form for whole runs of 64 x 64: one chunk and
+less, remainders, the last run count that takes it and the first that does not, packed sequences with an empty one, states in both layouts."""
 import pytest
 import torch
 
@@ -13,10 +13,10 @@ pytestmark = pytest.mark.gpu
     (8, 65, 16, 16, None, torch.bfloat16, False, True), (3, 129, 43, 43, None, torch.bfloat16, False, True), (1, 449, 2, 4, None, torch.bfloat16, False, True),
     (1, 700, 2, 4, [0, 1, 65, 65, 193, 700], torch.bfloat16, False, True), (1, 2304, 1, 2, None, torch.bfloat16, True, False),
     (1, 2305, 1, 2, None, torch.bfloat16, True, True)])
-def test_halves(B, T, H, HV, cu, dtype, vfirst, l2):
+def test_halves(B, T, H, HV, cu, dtype, vfirst, l2, D=128):
     from fla_hip.ops.gated_delta_rule import chunk_gated_delta_rule
     N = B if cu is None else len(cu) - 1
-    q, k, v, g, beta, h0 = O.make_inputs(B, T, H, HV, 128, 128, seed=T, gate_div=4.0, h0_std=0.3, N=N, dtype=dtype)
+    q, k, v, g, beta, h0 = O.make_inputs(B, T, H, HV, D, D, seed=T, gate_div=4.0, h0_std=0.3, N=N, dtype=dtype)
     qr, kr = (O.l2norm(q), O.l2norm(k)) if l2 else (q, k)
     ref_o, ref_h = O.chunk_gated_delta_rule(qr, kr, v, g, beta, None, h0, True, cu_seqlens=cu)
     h = h0.transpose(-1, -2).contiguous() if vfirst else h0
@@ -25,3 +25,12 @@ def test_halves(B, T, H, HV, cu, dtype, vfirst, l2):
     ht = ht.transpose(-1, -2) if vfirst else ht
     assert O.get_err_ratio(ref_o.float(), o.float().cpu()) < 5e-3
     assert O.get_err_ratio(ref_h, ht.cpu()) < 5e-3
+
+
+@pytest.mark.parametrize('B,T,H,HV,cu,dtype,vfirst,l2', [
+    (1, 1, 1, 1, None, torch.bfloat16, False, False), (1, 63, 2, 6, None, torch.float16, True, True), (2, 64, 4, 4, None, torch.bfloat16, True, True),
+    (8, 65, 16, 16, None, torch.bfloat16, False, True), (3, 129, 43, 43, None, torch.bfloat16, False, True), (1, 449, 2, 4, None, torch.float16, False, False),
+    (1, 700, 2, 4, [0, 1, 65, 65, 193, 700], torch.bfloat16, False, True), (1, 1984, 1, 2, None, torch.bfloat16, True, False),
+    (1, 1985, 1, 2, None, torch.bfloat16, True, True)])
+def test_whole_runs_of_64(B, T, H, HV, cu, dtype, vfirst, l2):
+    test_halves(B, T, H, HV, cu, dtype, vfirst, l2, D=64)
