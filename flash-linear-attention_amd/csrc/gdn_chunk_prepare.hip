@@ -75,12 +75,14 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
 #pragma unroll
         for (int b = a; b < 4; ++b) U[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
     float sq[4] = {0.f, 0.f, 0.f, 0.f};
-    f32x4 QK[4][4];                              // (WANT_P) raw k q^T tiles, like U
+    f32x4 QK[4][4], QQ[4];                       // (WANT_P) raw k q^T tiles, like U; the diagonal tiles of q q^T
     if constexpr (WANT_P) {
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
+        for (int a = 0; a < 4; ++a) {
+            QQ[a] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int b = a; b < 4; ++b) QK[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
     }
     {
         const T* kg = (const T*)p.k + (tok0 * H + h) * K;
@@ -98,11 +100,17 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
         // 128 features at a time: all 16 fragments of a round are requested before the first product; the q rows (for
         // their norms only) follow into the same registers once the products have been issued
         for (int k0 = 0; k0 < K; k0 += 128) {
-            u32x4 fk[4][4];
+            u32x4 fk[4][4], fq[WANT_P ? 4 : 1][4];
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
                 for (int s4 = 0; s4 < 4; ++s4) fk[t][s4] = fragment(kg, t, k0 + 32 * s4);
+            if constexpr (WANT_P) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int s4 = 0; s4 < 4; ++s4) fq[t][s4] = fragment(qg, t, k0 + 32 * s4);
+            }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int a = 0; a < 4; ++a)
@@ -113,11 +121,6 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
                         U[a][b] = Mma<T>::run(__builtin_bit_cast(V8, fk[a][s4]), __builtin_bit_cast(V8, fk[b][s4]), U[a][b]);
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (WANT_P) {
-                u32x4 fq[4][4];
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int s4 = 0; s4 < 4; ++s4) fq[t][s4] = fragment(qg, t, k0 + 32 * s4);
 #pragma unroll
                 for (int a = 0; a < 4; ++a)
 #pragma unroll
@@ -130,8 +133,7 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
 #pragma unroll
                     for (int s4 = 0; s4 < 4; ++s4) {
                         const V8 q8 = __builtin_bit_cast(V8, fq[t][s4]);
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) { const float x = to_f32(q8[e]); sq[t] += x * x; }
+                        QQ[t] = Mma<T>::run(q8, q8, QQ[t]);
                     }
             } else if (q_norms_here) {                       // the q rows into the registers that held k
 #pragma unroll
@@ -150,15 +152,18 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
             }
         }
     }
-    // |k_t|^2 is the diagonal of K K^T; |q_t|^2 (for P only) is summed over the four lanes that share a row
+    // |k_t|^2 is the diagonal of K K^T; |q_t|^2 that of q q^T, or summed over the four lanes that share a row
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        float d = 0.f;
+        float d = 0.f, dq = 0.f;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            if (r == (c16 & 3)) d = U[t][t][r];
-        if ((c16 >> 2) == g) sK2[16 * t + c16] = d;
-        if (WANT_P || q_norms_here) {
+            if (r == (c16 & 3)) { d = U[t][t][r]; if constexpr (WANT_P) dq = QQ[t][r]; }
+        if ((c16 >> 2) == g) {
+            sK2[16 * t + c16] = d;
+            if constexpr (WANT_P) sNQ[16 * t + c16] = l2 ? rsqrtf(dq + 1e-6f) : 1.f;
+        }
+        if (!WANT_P && q_norms_here) {
             float a = sq[t];
             a += __shfl_xor(a, 16, 64);
             a += __shfl_xor(a, 32, 64);
