@@ -1044,7 +1044,7 @@ template <typename T, int FORM>
 static BwdLaunch scans_128(const BwdParams& p) {
     const int64_t runs = p.N * p.HV;
     auto apart = [&](const void* f, size_t smem, int v) {
-        return BwdLaunch{f, smem, "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, BD, v), v == BD ? 512u : 256u, (int64_t)scan_grid(p, BD, v)};
+        return BwdLaunch{f, smem, "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, BD, v), v >= 64 ? 512u : 256u, (int64_t)scan_grid(p, BD, v)};
     };
     if (runs <= 32) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, BD, BD, FORM>, bwd_scans_apart_smem<32, 32, BD, FORM>(), 32);
     if (runs <= 64) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, BD, BD, FORM>, bwd_scans_apart_smem<64, 64, BD, FORM>(), 64);
@@ -1092,10 +1092,10 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
     } else {
         // 256 key features: the reverse scan's tiles leave room for 64 columns at most
         if (runs <= 32) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
-        else if (runs <= 128) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 64), 256, (int64_t)scan_grid(p, VD, 64)};
+        else if (runs <= 128) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 64), 512, (int64_t)scan_grid(p, VD, 64)};
         else {
             ks[1] = {(const void*)gdn_bwd_state_kernel<T, 128, KD, VD>, bwd_state_smem<128, KD, FORM_GATED>(), "gdn_bwd_state_kernel", scan_grid(p, VD, 128), 512, 0};
-            ks[2] = {(const void*)gdn_bwd_dstate_kernel<T, 64, KD, VD>, bwd_dstate_smem<64, KD, FORM_GATED>(), "gdn_bwd_dstate_kernel", scan_grid(p, VD, 64), 256, 0};
+            ks[2] = {(const void*)gdn_bwd_dstate_kernel<T, 64, KD, VD>, bwd_dstate_smem<64, KD, FORM_GATED>(), "gdn_bwd_dstate_kernel", scan_grid(p, VD, 64), 512, 0};
         }
     }
     constexpr int NW = KD == 64 ? 4 : 8;
