@@ -1086,9 +1086,11 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
         if (p.nseg > 1)                                         // both scans side by side in a workgroup: every CU has one already
             ks[1] = {(const void*)gdn_bwd_scans_kernel<T, 32, KD, VD>, bwd_scans_smem<32, KD>(), "gdn_bwd_scans_kernel", scan_grid(p, VD, 32) * p.nseg, 512, 0};
         else if constexpr (VD == BD) ks[1] = scans_128<T, FORM_GATED>(p);
-        // (64 x 64: two workgroups fit a CU, so that 32-column slices pay up to twice as many runs)
-        else if (runs <= 128) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
-        else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 64), 256, (int64_t)scan_grid(p, VD, 64)};
+        // (64 x 64: two workgroups fit a CU, so that 32-column slices pay up to twice as many runs.  They read every tile twice, which
+        // costs once the tiles outgrow the caches: 80 heads, step with 32 / 64 columns at 1500 tokens 192.5 / 194.0 us, 2500 tokens
+        // 333 / 322, 5000 tokens 625 / 596; 96 heads at 2000 tokens 331.7 / 333.6; 128 at 1000 tokens 177.0 / 175.9, 2000 tokens 371 / 351)
+        else if (runs <= 64 || (runs < 128 && units <= 3072)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
+        else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 64), 512, (int64_t)scan_grid(p, VD, 64)};
     } else {
         // 256 key features: the reverse scan's tiles leave room for 64 columns at most
         if (runs <= 32) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};

@@ -14,7 +14,7 @@
 constexpr int FORM_GATED = 0, FORM_COMBA = 1, FORM_KDA = 2;
 // (64 or 128 value columns: eight waves, two per SIMD, share one set of tiles.  64 columns with four waves: 8 x 2048 tokens, 32 heads of 256 features, the
 // step 3765 us, with eight 3588; 8000 tokens in 4 sequences, 16 heads of 128: 486 and 458 us)
-template <int VBT, int KD> constexpr int scan_waves() { return VBT == BD || (KD >= BD && VBT == 64) ? 8 : 4; }
+template <int VBT> constexpr int scan_waves() { return VBT >= 64 ? 8 : 4; }
 
 // (the forward scan keeps v_new twice where a CU's LDS has the room: as the operand of the state update, with the decay to the end
 // of the chunk on it, and as it is stored, so that it can leave as whole rows)
@@ -413,21 +413,21 @@ template <int VBT, int VBR, int KD, int FORM> constexpr size_t bwd_scans_apart_s
     return bwd_state_smem<VBT, KD, FORM>() > bwd_dstate_smem<VBR, KD, FORM>() ? bwd_state_smem<VBT, KD, FORM>() : bwd_dstate_smem<VBR, KD, FORM>();
 }
 template <typename T, int VBT, int VBR, int KD, int VD, int FORM>
-__global__ __launch_bounds__((64 * scan_waves<VBT, KD>())) void gdn_bwd_scans_apart_kernel(BwdParams p, int64_t nrev) {
+__global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_scans_apart_kernel(BwdParams p, int64_t nrev) {
     extern __shared__ __align__(16) char smem[];
-    static_assert(scan_waves<VBT, KD>() == scan_waves<VBR, KD>(), "workgroups of one size");
-    if (blockIdx.x < nrev) bwd_dstate_body<T, VBR, KD, VD, FORM, scan_waves<VBR, KD>()>(p, smem, threadIdx.x, blockIdx.x, (unsigned)nrev);
-    else bwd_state_body<T, VBT, KD, VD, FORM, scan_waves<VBT, KD>()>(p, smem, threadIdx.x, blockIdx.x - (unsigned)nrev, gridDim.x - (unsigned)nrev);
+    static_assert(scan_waves<VBT>() == scan_waves<VBR>(), "workgroups of one size");
+    if (blockIdx.x < nrev) bwd_dstate_body<T, VBR, KD, VD, FORM, scan_waves<VBR>()>(p, smem, threadIdx.x, blockIdx.x, (unsigned)nrev);
+    else bwd_state_body<T, VBT, KD, VD, FORM, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x - (unsigned)nrev, gridDim.x - (unsigned)nrev);
 }
 // ... and in a launch of their own each, where the two want workgroups of different sizes.
 template <typename T, int VBT, int KD, int VD>
-__global__ __launch_bounds__((64 * scan_waves<VBT, KD>())) void gdn_bwd_state_kernel(BwdParams p, int64_t) {
+__global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_state_kernel(BwdParams p, int64_t) {
     extern __shared__ __align__(16) char smem[];
-    bwd_state_body<T, VBT, KD, VD, FORM_GATED, scan_waves<VBT, KD>()>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
+    bwd_state_body<T, VBT, KD, VD, FORM_GATED, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
 }
 template <typename T, int VBT, int KD, int VD>
-__global__ __launch_bounds__((64 * scan_waves<VBT, KD>())) void gdn_bwd_dstate_kernel(BwdParams p, int64_t) {
+__global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_dstate_kernel(BwdParams p, int64_t) {
     extern __shared__ __align__(16) char smem[];
-    bwd_dstate_body<T, VBT, KD, VD, FORM_GATED, scan_waves<VBT, KD>()>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
+    bwd_dstate_body<T, VBT, KD, VD, FORM_GATED, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
 }
 

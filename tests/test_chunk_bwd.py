@@ -537,3 +537,25 @@ def test_chunk_backward_time_segments(B, T, H, HV, gate_div, h0_std, forced, mon
         if a[n] is not None:
             assert O.get_err_ratio(b[n].float().cpu(), a[n].float().cpu()) < 2e-3, n
 
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('B,T,H,HV,l2', [(2, 70, 32, 64, True), (2, 2435, 20, 40, False), (3, 1, 44, 44, True)])
+def test_chunk_backward_64_columns_of_64_features(B, T, H, HV, l2, monkeypatch):
+    """64 x 64 heads, 128 runs or more, or more than 3072 pairs of a chunk and a head on more than 64 runs: the scans hold all 64 value
+    columns in eight waves.  A sequence by itself has fewer runs and takes slices of 32 columns; the sums over features and tokens
+    are the same ones in the same order, so that every gradient has the same bits."""
+    monkeypatch.setenv('FLA_HIP_BWD_SCAN_MODE', 'wide')
+    D = 64
+    q, k, v, g, beta, h0 = O.make_inputs(B, T, HV, HV, D, D, seed=T, gate_div=4.0, h0_std=0.5)
+    q, k, v = q[:, :, :H].bfloat16(), k[:, :, :H].bfloat16(), v.bfloat16()
+    gen = torch.Generator().manual_seed(T + 1)
+    do = torch.randn(B, T, HV, D, generator=gen).bfloat16()
+    dht = torch.randn(B, HV, D, D, generator=gen)
+    _, _, got = _grads_gpu(q, k, v, g, beta, h0, do, dht, use_qk_l2norm_in_kernel=l2)
+    for b in range(B):
+        s = slice(b, b + 1)
+        _, _, alone = _grads_gpu(q[s], k[s], v[s], g[s], beta[s], h0[s], do[s], dht[s], use_qk_l2norm_in_kernel=l2)
+        for n in got:
+            if got[n] is not None:
+                assert torch.equal(got[n][s], alone[n]), (n, b, O.get_err_ratio(alone[n].float().cpu(), got[n][s].float().cpu()))
