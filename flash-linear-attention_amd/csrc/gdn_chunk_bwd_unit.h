@@ -15,9 +15,10 @@
 // (always, the last time for nothing: behind a condition the registers of the last request stay alive through the whole head).
 // 16000 packed tokens, 16 q/k and 32 value heads of 128: 650 us as two kernels, 490 us; with the heads of a group added up and the l2
 // normalisation taken back in here 500 us, and 132 us of passes around it gone.  8 x 2048 tokens, 32 heads of 256 x 256: 2230 us with
-// those passes, 1830 us (state fragments requested a head ahead there: 1920 us, for want of registers), now 1570 us: the first feature tile's
+// those passes, 1830 us (state fragments requested a head ahead there: 1920 us, for want of registers), now 1370 us: the first feature tile's
 // fragments are requested in front of the dP phase, and the products with the state follow one another (1642 us with the three of them
-// side by side, whose accumulators spilled; at 128 key features they stay side by side: 475 us against 487 us).
+// side by side, whose accumulators spilled; at 128 key features they stay side by side: 475 us against 487 us); no sum's terms wait in
+// registers (1570 us with those of dglast kept to the end of the products: 116 B of scratch a thread, 0.6 GB of 1.4 GB written).
 
 // lower triangle of 4 x 4 tiles, row by row
 __device__ __forceinline__ int tri_row(int idx) { return idx < 1 ? 0 : idx < 3 ? 1 : idx < 6 ? 2 : 3; }
@@ -232,6 +233,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
                             const V4 k4 = *(const V4*)(sK + x * PK + n16 + 4 * g);
 #pragma unroll
                             for (int r = 0; r < 4; ++r) dglast += (float)k4[r] * k_[r];
+                            pin(dglast);
 #pragma unroll
                             for (int s = 0; s < 2; ++s)
                                 if (32 * s + 31 >= 16 * t) k_ = Mma<T>::run(fq[s], frag_cols(sM1, P64, 32 * s, 16 * t, lane), k_);     // ... and for i < j
