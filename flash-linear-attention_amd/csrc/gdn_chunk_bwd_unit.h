@@ -15,10 +15,11 @@
 // (always, the last time for nothing: behind a condition the registers of the last request stay alive through the whole head).
 // 16000 packed tokens, 16 q/k and 32 value heads of 128: 650 us as two kernels, 490 us; with the heads of a group added up and the l2
 // normalisation taken back in here 500 us, and 132 us of passes around it gone.  8 x 2048 tokens, 32 heads of 256 x 256: 2230 us with
-// those passes, 1830 us (state fragments requested a head ahead there: 1920 us, for want of registers), now 1370 us: the first feature tile's
+// those passes, 1830 us (state fragments requested a head ahead there: 1920 us, for want of registers), now 1330 us: the first feature tile's
 // fragments are requested in front of the dP phase, and the products with the state follow one another (1642 us with the three of them
 // side by side, whose accumulators spilled; at 128 key features they stay side by side: 475 us against 487 us); no sum's terms wait in
-// registers (1570 us with those of dglast kept to the end of the products: 116 B of scratch a thread, 0.6 GB of 1.4 GB written).
+// registers (1570 us with those of dglast kept to the end of the products: 116 B of scratch a thread, 0.6 GB of 1.4 GB written), and the
+// next head's tiles are requested in three places, the last of them late (all at once behind the products 1400 us).
 
 // lower triangle of 4 x 4 tiles, row by row
 __device__ __forceinline__ int tri_row(int idx) { return idx < 1 ? 0 : idx < 3 ? 1 : idx < 6 ? 2 : 3; }
@@ -62,11 +63,14 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
     float rGam = 0.f, rBeta = 0.f, rRq = 0.f, rRk = 0.f;
     const int HVg = p.HV / p.nb;
     const bool parts_out = LEAN ? p.dq_part != nullptr : PARTS;
-    auto fetch_state = [&](const Item& at, int hv, int a, int w, int lane) {     // feature tile a of this wave
+    auto fetch_state = [&](const Item& at, int hv, int a, int w, int lane, bool S = true, bool dS = true) {     // feature tile a of this wave
         const int64_t u = at.ch * p.HV + hv;
         const int64_t off = u * KD * VD + (16 * (NA * w + a) + (lane & 15)) * VD + 8 * (lane >> 4);
 #pragma unroll
-        for (int s = 0; s < SV; ++s) { sf[s] = *(const V8*)((const T*)p.ws.Hs + off + 32 * s); df[s] = *(const V8*)((const T*)p.ws.dHs + off + 32 * s); }
+        for (int s = 0; s < SV; ++s) {
+            if (S) sf[s] = *(const V8*)((const T*)p.ws.Hs + off + 32 * s);
+            if (dS) df[s] = *(const V8*)((const T*)p.ws.dHs + off + 32 * s);
+        }
     };
     auto fetch_out = [&](const Item& at, int hv, int tid) {
         const int64_t u = at.ch * p.HV + hv;
@@ -181,7 +185,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
                 for (int a = 0; a < NA; ++a) {
                     const int n16 = feat(a);
                     // one product with the state at a time: sixteen accumulator registers instead of forty-eight, and the next tile's fragments
-                    // on their way during the last of the tile's own work
+                    // on their way from where this tile has used its own for the last time
                     f32x4 acc[4];
                     auto product = [&](const V8 (&f)[SV], const T* rows) {
 #pragma unroll
@@ -218,9 +222,11 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
                     for (int t = 0; t < 4; ++t) dw[a][t] = pack4<T>(-acc[t]);
 #pragma unroll
                     for (int s = 0; s < SV; ++s) sd = Mma<T>::run(sf[s], df[s], sd);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (a + 1 < NA) fetch_state(at, hv, a + 1, w, lane, true, false);
                     product(df, sVn);
                     __builtin_amdgcn_sched_barrier(0);
-                    if (a + 1 < NA) fetch_state(at, hv, a + 1, w, lane);
+                    if (a + 1 < NA) fetch_state(at, hv, a + 1, w, lane, false, true);
                     {
                         V8 fq[2];
 #pragma unroll
@@ -333,8 +339,8 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
 #pragma unroll
                 for (int t = 0; t < 4; ++t) *(V4*)(sDW + (16 * t + c16) * PK + feat(a) + 4 * g) = dw[a][t];
             lds_barrier();
-            if constexpr (LEAN) { fetch_out(to, to_hv, tid); fetch_in(to, to_hv, tid); }
-            fetch_rest(to, to_hv, tid);
+            if constexpr (LEAN) fetch_out(to, to_hv, tid);
+            if constexpr (!LEAN) fetch_rest(to, to_hv, tid);
             if constexpr (!LEAN) fetch_state(to, to_hv, 0, w, lane);
             // dX's second term dw (e^gam k)^T, dA = stril(dX diag(beta)), k k^T of the same tiles
             f32x4 kk[NTRI];
@@ -397,6 +403,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
             }
             lds_barrier();
             if (!LEAN && last && more) fetch_qk(nx, tid);
+            if constexpr (LEAN) fetch_in(to, to_hv, tid);
             // Y = dA A^T (in dv_new's place)
 #pragma unroll
             for (int n = 0; n < 16 / NW; ++n) {
@@ -446,6 +453,7 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
             }
             lds_barrier();
             // dk += E k + E^T k
+            if constexpr (LEAN) fetch_rest(to, to_hv, tid);
 #pragma unroll
             for (int a = 0; a < NA; ++a) {
                 V8 fk[2];
