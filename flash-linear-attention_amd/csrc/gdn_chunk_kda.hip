@@ -609,22 +609,27 @@ __global__ __launch_bounds__(256, 2) void gdn_comba_prepare_kernel(KdaParams p, 
 // ---------------------------------------------------------------------------------------------
 // scan: the state slice [128][VBT] lives in registers as transposed tiles (wave w: key rows 32w .. 32w+31 as two tiles a2,
 // lane (c16, g): key 16(2w+a2) + c16, value columns 16b + 4g .. +3); the next chunk's tiles are fetched into registers
-// while the current chunk is computed.
+// while the current chunk is computed.  64 and 128 columns: eight waves, two per SIMD, waves w and w + 4 the same rows of either
+// half of the columns (with four, nothing covers a step's chains and barriers: 8192 tokens,
+// 96 heads 345 -> 313 us; 4 x 2000 tokens, 64 heads, 128 columns 164 -> 153.  At 64 runs 32 columns stay the better ones: the step 1141 against 1158 us).
 // ---------------------------------------------------------------------------------------------
 // (u comes in, and o leaves, as whole rows through LDS tiles of their own: the lanes that hold them as matrix-instruction operands
 // and results would move 8-byte pieces of 16 rows per instruction)
 template <int VBT> constexpr size_t kda_scan_smem() { return (3 * 64 * P128 + 64 * P64 + BD * (VBT + 8) + 3 * 64 * (VBT + 8)) * 2 + (BD + 64) * 4; }
 
+template <int VBT> constexpr int kda_scan_waves() { return VBT >= 64 ? 8 : 4; }
+
 template <typename T, int VBT>
-__global__ __launch_bounds__(256) void gdn_kda_scan_kernel(KdaParams p) {
+__global__ __launch_bounds__(64 * kda_scan_waves<VBT>()) void gdn_kda_scan_kernel(KdaParams p) {
     typedef typename Mma<T>::V8 V8;
     typedef typename Mma<T>::V4 V4;
-    constexpr int PV = VBT + 8, NB = VBT / 16, NVS = BD / VBT;
+    constexpr int NTH = 64 * kda_scan_waves<VBT>(), PV = VBT + 8, NVS = BD / VBT, NB = VBT / 16 / (NTH / 256);      // (16-column blocks of a wave)
     extern __shared__ __align__(16) char smem[];
     T* sW = (T*)smem; T* sKG = sW + 64 * P128; T* sQG = sKG + 64 * P128; T* sP = sQG + 64 * P128;
     T* sS = sP + 64 * P64; T* sVn = sS + BD * PV; T* sU = sVn + 64 * PV; T* sO = sU + 64 * PV;
     float* sE = (float*)(sO + 64 * PV);
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c16 = lane & 15, g = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, w = (tid >> 6) & 3, c16 = lane & 15, g = lane >> 4;
+    const int wcol = 16 * NB * (tid >> 8);                       // first value column of this wave in the slice
     const int64_t run = (int64_t)(blockIdx.x / (8 * NVS)) * 8 + blockIdx.x % 8;       // (slices of one head on one XCD)
     if (run >= p.N * p.HV) return;
     const int vs = (blockIdx.x / 8) % NVS, hv = (int)(run % p.HV);
@@ -638,38 +643,38 @@ __global__ __launch_bounds__(256) void gdn_kda_scan_kernel(KdaParams p) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             const int kk = 16 * (2 * w + a2) + c16;
-            S[a2][b] = p.h0 ? *(const f32x4*)(p.h0 + ((n * p.HV + hv) * BD + kk) * BD + vcol0 + 16 * b + 4 * g) : ZERO4;
+            S[a2][b] = p.h0 ? *(const f32x4*)(p.h0 + ((n * p.HV + hv) * BD + kk) * BD + vcol0 + wcol + 16 * b + 4 * g) : ZERO4;
         }
-    TileRegs<BD> rW, rKG, rQG;
-    TileRegs<CH> rP;
-    TileRegs<VBT> rU;
+    TileRegs<BD, NTH> rW, rKG, rQG;
+    TileRegs<CH, NTH> rP;
+    TileRegs<VBT, NTH> rU;
     float rE = 0.f;
     auto fetch = [&](int64_t ic) {
         const int64_t u = (sq.cbase + ic) * p.HV + hv;
-        fetch_tile<BD>(rW, (const T*)p.ws.Wm + u * 64 * BD, BD, 64, tid);
-        fetch_tile<BD>(rKG, (const T*)p.ws.KG + u * 64 * BD, BD, 64, tid);
-        fetch_tile<BD>(rQG, (const T*)p.ws.QG + u * 64 * BD, BD, 64, tid);
-        fetch_tile<CH>(rP, (const T*)p.ws.Pm + u * 64 * 64, 64, 64, tid);
+        fetch_tile<BD, NTH>(rW, (const T*)p.ws.Wm + u * 64 * BD, BD, 64, tid);
+        fetch_tile<BD, NTH>(rKG, (const T*)p.ws.KG + u * 64 * BD, BD, 64, tid);
+        fetch_tile<BD, NTH>(rQG, (const T*)p.ws.QG + u * 64 * BD, BD, 64, tid);
+        fetch_tile<CH, NTH>(rP, (const T*)p.ws.Pm + u * 64 * 64, 64, 64, tid);
         if (tid < BD) rE = p.ws.EGL[u * BD + tid];
-        fetch_tile<VBT>(rU, (const T*)p.ws.Um + u * 64 * BD + vcol0, BD, 64, tid);
+        fetch_tile<VBT, NTH>(rU, (const T*)p.ws.Um + u * 64 * BD + vcol0, BD, 64, tid);
     };
     if (sq.nc > 0) fetch(0);
     for (int64_t ic = 0; ic < sq.nc; ++ic) {
         const int64_t tok0 = sq.bos + ic * CH;
         const int valid = (int)min((int64_t)CH, sq.len - ic * CH);
-        put_tile<BD>(sW, P128, rW, tid);
-        put_tile<BD>(sKG, P128, rKG, tid);
-        put_tile<BD>(sQG, P128, rQG, tid);
-        put_tile<CH>(sP, P64, rP, tid);
-        put_tile<VBT>(sU, PV, rU, tid);
+        put_tile<BD, NTH>(sW, P128, rW, tid);
+        put_tile<BD, NTH>(sKG, P128, rKG, tid);
+        put_tile<BD, NTH>(sQG, P128, rQG, tid);
+        put_tile<CH, NTH>(sP, P64, rP, tid);
+        put_tile<VBT, NTH>(sU, PV, rU, tid);
         if (tid < BD) sE[tid] = rE;
 #pragma unroll
         for (int a2 = 0; a2 < 2; ++a2)
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 const V4 s4 = pack4<T>(S[a2][b]);
-                *(V4*)(sS + (16 * (2 * w + a2) + c16) * PV + 16 * b + 4 * g) = s4;
-                if (p.hs) *(V4*)((T*)p.hs + (((sq.cbase + ic) * p.HV + hv) * BD + 16 * (2 * w + a2) + c16) * BD + vcol0 + 16 * b + 4 * g) = s4;
+                *(V4*)(sS + (16 * (2 * w + a2) + c16) * PV + wcol + 16 * b + 4 * g) = s4;
+                if (p.hs) *(V4*)((T*)p.hs + (((sq.cbase + ic) * p.HV + hv) * BD + 16 * (2 * w + a2) + c16) * BD + vcol0 + wcol + 16 * b + 4 * g) = s4;
             }
         lds_barrier();
         if (ic + 1 < sq.nc) fetch(ic + 1);
@@ -686,15 +691,15 @@ __global__ __launch_bounds__(256) void gdn_kda_scan_kernel(KdaParams p) {
                 oacc[b] = ZERO4;
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    const V8 fs = frag_cols(sS, PV, 32 * s, 16 * b, lane);
+                    const V8 fs = frag_cols(sS, PV, 32 * s, wcol + 16 * b, lane);
                     acc = Mma<T>::run(fs, wf[s], acc);
                     oacc[b] = Mma<T>::run(fs, qf[s], oacc[b]);
                 }
-                const V4 u4 = *(const V4*)(sU + i * PV + 16 * b + 4 * g);
+                const V4 u4 = *(const V4*)(sU + i * PV + wcol + 16 * b + 4 * g);
                 f32x4 vn;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) vn[r] = (float)u4[r] - acc[r];
-                *(V4*)(sVn + i * PV + 16 * b + 4 * g) = pack4<T>(vn);
+                *(V4*)(sVn + i * PV + wcol + 16 * b + 4 * g) = pack4<T>(vn);
             }
         }
         lds_barrier();
@@ -718,16 +723,16 @@ __global__ __launch_bounds__(256) void gdn_kda_scan_kernel(KdaParams p) {
             for (int b = 0; b < NB; ++b) {
 #pragma unroll
                 for (int s = 0; s < 2; ++s) {
-                    const V8 fv = frag_cols(sVn, PV, 32 * s, 16 * b, lane);
+                    const V8 fv = frag_cols(sVn, PV, 32 * s, wcol + 16 * b, lane);
                     if (32 * s <= 16 * w + 15) oacc[b] = Mma<T>::run(fv, pf[s], oacc[b]);      // P[i][j] = 0 for j > i
 #pragma unroll
                     for (int a2 = 0; a2 < 2; ++a2) S[a2][b] = Mma<T>::run(fv, kf[a2][s], S[a2][b]);
                 }
-                *(V4*)(sO + i * PV + 16 * b + 4 * g) = pack4<T>(oacc[b]);
+                *(V4*)(sO + i * PV + wcol + 16 * b + 4 * g) = pack4<T>(oacc[b]);
             }
         }
         lds_barrier();
-        copy_rows_out<64, VBT, 256>((T*)p.o + (tok0 * p.HV + hv) * BD + vcol0, (int64_t)p.HV * BD, sO, PV, tid, valid);
+        copy_rows_out<64, VBT, NTH>((T*)p.o + (tok0 * p.HV + hv) * BD + vcol0, (int64_t)p.HV * BD, sO, PV, tid, valid);
     }
     if (p.ht) {
 #pragma unroll
@@ -735,7 +740,7 @@ __global__ __launch_bounds__(256) void gdn_kda_scan_kernel(KdaParams p) {
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 const int kk = 16 * (2 * w + a2) + c16;
-                *(f32x4*)(p.ht + ((n * p.HV + hv) * BD + kk) * BD + vcol0 + 16 * b + 4 * g) = S[a2][b];
+                *(f32x4*)(p.ht + ((n * p.HV + hv) * BD + kk) * BD + vcol0 + wcol + 16 * b + 4 * g) = S[a2][b];
             }
     }
 }
@@ -745,19 +750,19 @@ static int launch_kda(const KdaParams& p, int64_t num_chunks, hipStream_t stream
     const int64_t runs1 = p.N * p.HV;
     const int vbt = runs1 <= 64 ? 32 : runs1 <= 128 ? 64 : 128;
     const unsigned units = (unsigned)(num_chunks * p.HV), runs = (unsigned)((runs1 + 7) / 8 * 8 * (BD / vbt));
-    struct K { const void* f; size_t smem; const char* name; unsigned grid; };
+    struct K { const void* f; size_t smem; const char* name; unsigned grid, threads; };
     K scan;
-    if (vbt == 32) scan = {(const void*)gdn_kda_scan_kernel<T, 32>, kda_scan_smem<32>(), "gdn_kda_scan_kernel", runs};
-    else if (vbt == 64) scan = {(const void*)gdn_kda_scan_kernel<T, 64>, kda_scan_smem<64>(), "gdn_kda_scan_kernel", runs};
-    else scan = {(const void*)gdn_kda_scan_kernel<T, 128>, kda_scan_smem<128>(), "gdn_kda_scan_kernel", runs};
-    const K prep = comba ? K{(const void*)gdn_comba_prepare_kernel<T>, COMBA_PREP_SMEM, "gdn_comba_prepare_kernel", units < 512u ? units : 512u}
-                         : K{(const void*)gdn_kda_prepare_kernel<T>, KDA_PREP_SMEM, "gdn_kda_prepare_kernel", units < 512u ? units : 512u};
+    if (vbt == 32) scan = {(const void*)gdn_kda_scan_kernel<T, 32>, kda_scan_smem<32>(), "gdn_kda_scan_kernel", runs, 64u * kda_scan_waves<32>()};
+    else if (vbt == 64) scan = {(const void*)gdn_kda_scan_kernel<T, 64>, kda_scan_smem<64>(), "gdn_kda_scan_kernel", runs, 64u * kda_scan_waves<64>()};
+    else scan = {(const void*)gdn_kda_scan_kernel<T, 128>, kda_scan_smem<128>(), "gdn_kda_scan_kernel", runs, 64u * kda_scan_waves<128>()};
+    const K prep = comba ? K{(const void*)gdn_comba_prepare_kernel<T>, COMBA_PREP_SMEM, "gdn_comba_prepare_kernel", units < 512u ? units : 512u, 256}
+                         : K{(const void*)gdn_kda_prepare_kernel<T>, KDA_PREP_SMEM, "gdn_kda_prepare_kernel", units < 512u ? units : 512u, 256};
     const K ks[2] = {prep, scan};
     for (int i = 0; i < 2; ++i) {
         if (int rc = ensure_dynamic_smem_for(ks[i].f, ks[i].smem, ks[i].name)) return rc;
         int64_t nunits = units;
         void* args[] = {(void*)&p, (void*)&nunits};             // (the prepare kernel walks over the units and takes their number)
-        if (hipLaunchKernel(ks[i].f, dim3(ks[i].grid), dim3(256), args, ks[i].smem, stream) != hipSuccess) return check_launch(ks[i].name);
+        if (hipLaunchKernel(ks[i].f, dim3(ks[i].grid), dim3(ks[i].threads), args, ks[i].smem, stream) != hipSuccess) return check_launch(ks[i].name);
         if (int rc = check_launch(ks[i].name)) return rc;
     }
     return GDN_OK;

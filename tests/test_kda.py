@@ -446,6 +446,21 @@ def test_chunk_kda_wide_keys_forward(B, T, H, HV, D, V, l2, gate_in_kernel, safe
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('B,T,H', [(2, 130, 33), (2, 65, 64), (3, 70, 43), (3, 1, 44)])
+def test_chunk_kda_scan_columns(B, T, H):
+    """The forward scan with 64 (65 to 128 runs) and 128 value columns (more) to a workgroup of eight waves, against its sequences one by
+    one, which take 32 columns and four waves: the same sums in the same order, hence the same bits."""
+    from fla_hip.ops.kda import chunk_kda
+    q, k, v, g, beta, h0, _, _ = _chunk_inputs(B, T, H, H, 128, 1.0, 0, False, False, torch.bfloat16)
+    args = [x.cuda() for x in (q, k, v, g, beta, h0)]
+    call = lambda xs: chunk_kda(*xs[:5], initial_state=xs[5], output_final_state=True, use_qk_l2norm_in_kernel=True)
+    o, ht = call(args)
+    for b in range(B):
+        o1, ht1 = call([x[b:b + 1] for x in args])
+        assert torch.equal(o[b:b + 1], o1) and torch.equal(ht[b:b + 1], ht1), b
+
+
+@pytest.mark.gpu
 def test_chunk_kda_validation():
     from fla_hip.ops.kda import chunk_kda
     x = torch.zeros(1, 64, 2, 64, dtype=torch.bfloat16, device='cuda')
