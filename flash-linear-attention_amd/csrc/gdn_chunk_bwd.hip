@@ -1043,12 +1043,17 @@ static unsigned scan_grid(const BwdParams& p, int VD, int v) { return (unsigned)
 template <typename T, int FORM>
 static BwdLaunch scans_128(const BwdParams& p) {
     const int64_t runs = p.N * p.HV;
-    auto apart = [&](const void* f, size_t smem, int v) {
-        return BwdLaunch{f, smem, "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, BD, v), v >= 64 ? 512u : 256u, (int64_t)scan_grid(p, BD, v)};
+    auto apart = [&](const void* f, size_t smem, int v, int vr) {         // columns forwards, backwards
+        const unsigned nrev = scan_grid(p, BD, vr);
+        return BwdLaunch{f, smem, "gdn_bwd_scans_apart_kernel", nrev + scan_grid(p, BD, v), v >= 64 ? 512u : 256u, (int64_t)nrev};
     };
-    if (runs <= 32) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, BD, BD, FORM>, bwd_scans_apart_smem<32, 32, BD, FORM>(), 32);
-    if (runs <= 64) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, BD, BD, FORM>, bwd_scans_apart_smem<64, 64, BD, FORM>(), 64);
-    return apart((const void*)gdn_bwd_scans_apart_kernel<T, 128, 128, BD, BD, FORM>, bwd_scans_apart_smem<128, 128, BD, FORM>(), 128);
+    if (runs <= 32) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, BD, BD, FORM>, bwd_scans_apart_smem<32, 32, BD, FORM>(), 32, 32);
+    if (runs <= 64) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, BD, BD, FORM>, bwd_scans_apart_smem<64, 64, BD, FORM>(), 64, 64);
+    // (65 to 80 runs: the longer, backward scan halves its columns where a workgroup each still has a CU to itself: 80 runs of 1500 tokens
+    // 353 -> 325 us a step, 80 packed ones of 1600 456 -> 400, KDA, 72 runs of 4000 tokens, 1161 -> 1109)
+    if (scan_grid(p, BD, 128) + scan_grid(p, BD, 64) <= 256)
+        return apart((const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, BD, BD, FORM>, bwd_scans_apart_smem<128, 64, BD, FORM>(), 128, 64);
+    return apart((const void*)gdn_bwd_scans_apart_kernel<T, 128, 128, BD, BD, FORM>, bwd_scans_apart_smem<128, 128, BD, FORM>(), 128, 128);
 }
 
 template <typename T, int KD, int VD>
@@ -1092,13 +1097,14 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
         else if (runs <= 64 || (runs < 128 && units <= 3072)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
         else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 64), 512, (int64_t)scan_grid(p, VD, 64)};
     } else {
-        // 256 key features: the reverse scan's tiles leave room for 64 columns at most
+        // 256 key features: the reverse scan's tiles leave room for 64 columns at most.  The forward scan takes 128 where a workgroup each
+        // still has a CU to itself (72 runs, step with 64 / 128 columns: 477 / 462 us), and beyond 128 runs, where rounds follow one another anyway
+        // and its workgroups fill up the last one of the reverse scan (in a launch of its own behind it / in one launch: 160 runs 1011 / 901 us, 256
+        // runs 875 / 857, 336 packed runs 2661 / 2621, 512 runs equal); in between, 96 packed runs 820 / 838, 128 runs 660 / 699.
+        const unsigned half = scan_grid(p, VD, 64), whole = scan_grid(p, VD, 128);
         if (runs <= 32) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
-        else if (runs <= 128) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 64), 512, (int64_t)scan_grid(p, VD, 64)};
-        else {
-            ks[1] = {(const void*)gdn_bwd_state_kernel<T, 128, KD, VD>, bwd_state_smem<128, KD, FORM_GATED>(), "gdn_bwd_state_kernel", scan_grid(p, VD, 128), 512, 0};
-            ks[2] = {(const void*)gdn_bwd_dstate_kernel<T, 64, KD, VD>, bwd_dstate_smem<64, KD, FORM_GATED>(), "gdn_bwd_dstate_kernel", scan_grid(p, VD, 64), 512, 0};
-        }
+        else if (runs > 128 || (runs > 64 && half + whole <= 256)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<128, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", half + whole, 512, (int64_t)half};
+        else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * half, 512, (int64_t)half};
     }
     constexpr int NW = KD == 64 ? 4 : 8;
     const int64_t items = num_chunks * p.H * p.parts;

@@ -419,15 +419,3 @@ __global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_scans_apart_ke
     if (blockIdx.x < nrev) bwd_dstate_body<T, VBR, KD, VD, FORM, scan_waves<VBR>()>(p, smem, threadIdx.x, blockIdx.x, (unsigned)nrev);
     else bwd_state_body<T, VBT, KD, VD, FORM, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x - (unsigned)nrev, gridDim.x - (unsigned)nrev);
 }
-// ... and in a launch of their own each, where the two want workgroups of different sizes.
-template <typename T, int VBT, int KD, int VD>
-__global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_state_kernel(BwdParams p, int64_t) {
-    extern __shared__ __align__(16) char smem[];
-    bwd_state_body<T, VBT, KD, VD, FORM_GATED, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
-}
-template <typename T, int VBT, int KD, int VD>
-__global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_dstate_kernel(BwdParams p, int64_t) {
-    extern __shared__ __align__(16) char smem[];
-    bwd_dstate_body<T, VBT, KD, VD, FORM_GATED, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
-}
-

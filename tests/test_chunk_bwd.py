@@ -225,8 +225,8 @@ def test_chunk_backward_packed_tokens_outside_every_sequence_get_zero_gradients(
     (1, 300, 1, 2, 192, 128, True, None),
     (1, 257, 2, 2, 256, 512, True, None),                  # the reference layer's default head shape (head_dim 256, expand_v 2)
     (1, 0, 2, 4, 160, 64, False, [0, 100, 101, 300]),
-    (3, 100, 12, 24, 256, 128, True, None),                 # 72 runs: the forward scan takes 64 columns per workgroup
-    (2, 130, 16, 32, 256, 256, False, None),                # 128 runs: the reverse scan takes 64 columns, P^T straight from memory
+    (3, 100, 12, 24, 256, 128, True, None),                 # 72 runs: 128 columns per workgroup forwards, 64 backwards
+    (2, 130, 16, 32, 256, 256, False, None),                # 128 runs: both scans take 64 columns, P^T straight from memory
     (1, 70, 136, 136, 200, 64, True, None),                 # 136 runs, a ragged chunk
 ])
 def test_chunk_backward_wide_keys(B, T, H, HV, K, V, l2, cu):
@@ -559,3 +559,23 @@ def test_chunk_backward_64_columns_of_64_features(B, T, H, HV, l2, monkeypatch):
         for n in got:
             if got[n] is not None:
                 assert torch.equal(got[n][s], alone[n]), (n, b, O.get_err_ratio(alone[n].float().cpu(), got[n][s].float().cpu()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('B,T,H,K,l2', [(2, 70, 33, 128, True), (2, 130, 40, 128, False), (2, 65, 40, 256, True), (5, 70, 33, 256, True)])
+def test_chunk_backward_scans_of_different_columns(B, T, H, K, l2, monkeypatch):
+    """65 to 80 runs (256 key features: and from 129 on): the scan forwards takes 128 value columns to a workgroup, the one backwards 64.
+    A sequence by itself has fewer runs and takes 64 or 32 columns in both: the same sums in the same order, hence the same bits."""
+    monkeypatch.setenv('FLA_HIP_BWD_SCAN_MODE', 'wide')
+    q, k, v, g, beta, h0 = O.make_inputs(B, T, H, H, K, 128, seed=T, gate_div=4.0, h0_std=0.5)
+    q, k, v = q.bfloat16(), k.bfloat16(), v.bfloat16()
+    gen = torch.Generator().manual_seed(T + 1)
+    do = torch.randn(B, T, H, 128, generator=gen).bfloat16()
+    dht = torch.randn(B, H, K, 128, generator=gen)
+    _, _, got = _grads_gpu(q, k, v, g, beta, h0, do, dht, use_qk_l2norm_in_kernel=l2)
+    for b in range(B):
+        s = slice(b, b + 1)
+        _, _, alone = _grads_gpu(q[s], k[s], v[s], g[s], beta[s], h0[s], do[s], dht[s], use_qk_l2norm_in_kernel=l2)
+        for n in got:
+            if got[n] is not None:
+                assert torch.equal(got[n][s], alone[n]), (n, b)

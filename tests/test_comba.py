@@ -433,3 +433,17 @@ def test_chunk_comba_backward_l2norm_inside_the_kernels(B, T, H, K, cu):
     assert rc == _lib.GDN_ERR_UNSUPPORTED and 'H == HV' in _lib.last_error()
     assert lib.gdn_chunk_comba_bwd_qk_l2norm(x.data_ptr(), x.data_ptr(), x.data_ptr(), *tail, *dims(2)) == _lib.GDN_OK
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+def test_comba_backward_scans_of_different_columns():
+    """65 to 80 runs: 128 value columns to a workgroup forwards, 64 backwards, against the sequences one by one (64 in both): the same bits."""
+    q, k, v, p, g, beta, h0 = _inputs(2, 70, 33, 33, 128, torch.bfloat16)
+    gen = torch.Generator().manual_seed(45)
+    do, dht = torch.randn(2, 70, 33, 128, generator=gen).bfloat16(), torch.randn(2, 33, 128, 128, generator=gen)
+    _, _, got = _comba_grads_gpu(q, k, v, p, g, beta, h0, do, dht, 0.1)
+    for b in range(2):
+        s = slice(b, b + 1)
+        _, _, alone = _comba_grads_gpu(q[s], k[s], v[s], p[s], g[s], beta[s], h0[s], do[s], dht[s], 0.1)
+        for n in got:
+            assert torch.equal(got[n][s], alone[n]), (n, b)

@@ -621,6 +621,22 @@ def test_chunk_kda_backward_strong_decay_in_some_features(T, dtype, l2):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('T,H', [(70, 33), (65, 40)])
+def test_chunk_kda_backward_scans_of_different_columns(T, H):
+    """65 to 80 runs: 128 value columns to a workgroup forwards, 64 backwards, against the sequences one by one (64 in both): the same bits."""
+    q, k, v, g, beta, h0, _, _ = _chunk_inputs(2, T, H, H, 128, 1.0, 0, False, False, torch.bfloat16)
+    gen = torch.Generator().manual_seed(45)
+    do, dht = torch.randn(2, T, H, 128, generator=gen).bfloat16(), torch.randn(2, H, 128, 128, generator=gen)
+    kw = dict(use_qk_l2norm_in_kernel=True)
+    _, _, got = _kda_grads_gpu(q, k, v, g, beta, h0, None, None, do, dht, **kw)
+    for b in range(2):
+        s = slice(b, b + 1)
+        _, _, alone = _kda_grads_gpu(q[s], k[s], v[s], g[s], beta[s], h0[s], None, None, do[s], dht[s], **kw)
+        for n in ('dq', 'dk', 'dv', 'dg', 'dbeta', 'dh0'):
+            assert torch.equal(got[n][s], alone[n]), (n, b)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('H,D,mask_p,cu,gate_in_kernel,safe_gate,idx_dtype', [
     (4, 60, 0.1, [0, 15], True, False, torch.int32),
     (4, 64, 0.9, [0, 256, 500, 1000], True, False, torch.int64),
