@@ -197,12 +197,12 @@ __global__ __launch_bounds__(512) void gdn_step_linear_kernel(StepLinearParams p
 
 template <typename T>
 static int launch_step_linear(StepLinearParams& p, hipStream_t stream) {
-    auto go = [&](auto kern, int threads, int columns, int rows) {
+    auto go = [&](auto kern, const char* name, int threads, int columns, int rows) {
         int at = 0;
         for (int i = 0; i < p.nseg; ++i) { p.first[i] = at; at += (int)((p.seg[i].cols + columns - 1) / columns); }
         p.first[p.nseg] = at;
         hipLaunchKernelGGL(kern, dim3((unsigned)at, (unsigned)((p.N + rows - 1) / rows)), dim3((unsigned)threads), 0, stream, p);
-        return check_launch("gdn_step_linear_kernel");
+        return check_launch(name);
     };
     if (p.N <= 16) {
         // rounds of the chip's CUs times the bytes of a workgroup, in columns of weights
@@ -217,15 +217,17 @@ static int launch_step_linear(StepLinearParams& p, hipStream_t stream) {
             if (x < cost) { cost = x; best = c; }
         }
         p.columns = (int)best;
+        const char* name = "gdn_step_linear_few_kernel";
         if (p.hidden <= 1024 && best <= 32)
-            return best <= 16 ? go(gdn_step_linear_few_kernel<T, 1, 8>, 512, (int)best, 16) : go(gdn_step_linear_few_kernel<T, 2, 8>, 512, (int)best, 16);
-        return best <= 16 ? go(gdn_step_linear_few_kernel<T, 1, 16>, 1024, (int)best, 16) : best <= 32 ? go(gdn_step_linear_few_kernel<T, 2, 16>, 1024, (int)best, 16)
-                                                                                                       : go(gdn_step_linear_few_kernel<T, 3, 16>, 1024, (int)best, 16);
+            return best <= 16 ? go(gdn_step_linear_few_kernel<T, 1, 8>, name, 512, (int)best, 16) : go(gdn_step_linear_few_kernel<T, 2, 8>, name, 512, (int)best, 16);
+        return best <= 16 ? go(gdn_step_linear_few_kernel<T, 1, 16>, name, 1024, (int)best, 16) : best <= 32 ? go(gdn_step_linear_few_kernel<T, 2, 16>, name, 1024, (int)best, 16)
+                                                                                                             : go(gdn_step_linear_few_kernel<T, 3, 16>, name, 1024, (int)best, 16);
     }
-    if (p.N <= 32) return go(gdn_step_linear_kernel<T, 2, 1>, 512, 16, 32);
+    const char* name = "gdn_step_linear_kernel";
+    if (p.N <= 32) return go(gdn_step_linear_kernel<T, 2, 1>, name, 512, 16, 32);
     // (more rows: 32 columns, so that the rows of x are read half as often)
-    if (p.N <= 64) return go(gdn_step_linear_kernel<T, 4, 2>, 512, 32, 64);
-    return go(gdn_step_linear_kernel<T, 8, 2>, 512, 32, 128);
+    if (p.N <= 64) return go(gdn_step_linear_kernel<T, 4, 2>, name, 512, 32, 64);
+    return go(gdn_step_linear_kernel<T, 8, 2>, name, 512, 32, 128);
 }
 
 }  // namespace gdn

@@ -93,3 +93,25 @@ def test_another_torch_rebuilds_the_extension(monkeypatch):
     monkeypatch.setattr(build, '_torch_version', lambda: '1.0')
     build.build(verbose=False)
     assert built == [1]
+
+
+@needs_build
+@pytest.mark.skipif(os.path.exists('/dev/kfd') or torch.cuda.is_available(), reason='a launch that fails by itself: only where there is no GPU')
+@pytest.mark.parametrize('N,hidden,kernel', [(1, 2048, 'gdn_step_linear_few_kernel'), (16, 256, 'gdn_step_linear_few_kernel'), (17, 256, 'gdn_step_linear_kernel'),
+                                             (129, 256, 'gdn_step_linear_kernel')])
+def test_a_failed_launch_of_the_step_projections_names_its_kernel(N, hidden, kernel):
+    import ctypes
+
+    from fla_hip import _lib
+
+    class Segment(ctypes.Structure):
+        _fields_ = [('weight', ctypes.c_void_p), ('cols', ctypes.c_int64), ('out', ctypes.c_void_p), ('conv_weight', ctypes.c_void_p),
+                    ('conv_bias', ctypes.c_void_p), ('conv_state', ctypes.c_void_p), ('A_log', ctypes.c_void_p), ('dt_bias', ctypes.c_void_p),
+                    ('kind', ctypes.c_int), ('conv_size', ctypes.c_int), ('gate_dtype', ctypes.c_int), ('reserved', ctypes.c_int)]
+
+    x, w, out = (torch.zeros(n, hidden, dtype=torch.bfloat16) for n in (N, 32, N))
+    assert x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+    seg = Segment(weight=w.data_ptr(), cols=32, out=out.data_ptr())              # (kind 0: the map alone)
+    status = _lib.load().gdn_step_linear(x.data_ptr(), N, hidden, ctypes.addressof(seg), 1, _lib.DTYPE_BF16, None)
+    assert status == _lib.GDN_ERR_LAUNCH
+    assert _lib.last_error().startswith(kernel + ':'), _lib.last_error()
