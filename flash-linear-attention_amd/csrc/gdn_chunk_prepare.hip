@@ -287,12 +287,14 @@ __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void g
 //     T_aw = -T_aa sum_{a < m <= w} U_am T_mw,
 // left factors U_am and T_aa from LDS, right factors the blocks it has just computed.  Two barriers: one for the gates and the norms, which wave 0
 // and the diagonal tiles' owners supply, one for the left factors.
-// 333 tokens, 32 heads (192 units): 27.5 -> 22.3 us a call; 1000 tokens, 16 heads: 42.7 -> 37.7; 1000 tokens, 8 heads of 256: 77.4 -> 69.7.
-// Up to three workgroups a CU, one round of the chip: at 704 units still 54.8 -> 52.5 us, at 792 already 49.8 -> 51.4, at 1008 122.5 -> 124.4.
+// A call with four waves to a unit instead of one, on inputs in the caches and out of them: 333 tokens, 32 heads (192 units) 27.0 -> 22.0 us and
+// 28.1 -> 23.0; 1000 tokens, 16 heads 42.3 -> 37.1 and 43.3 -> 38.9; 1000 tokens, 8 heads of 256 77.5 -> 69.9 and 84.3 -> 76.3.
+// Up to three workgroups a CU, one round of the chip: 32 heads, at 704 and 768 units still 54.6 -> 52.8 and 57.7 -> 56.0 us, at 800 already 59.1 -> 61.2.
+// The results are not those of the other kernel bit by bit (sums in another order), so a sequence's last bits depend on how many units its call has.
 constexpr int TEAM_TILE = 16 * TP;
 constexpr int64_t TEAM_UNITS = 3 * 256;
 template <typename T, bool WANT_P>
-__global__ __launch_bounds__(256, 2) void gdn_chunk_prepare_team_kernel(ChunkParams p) {
+__global__ __launch_bounds__(256, 2) void gdn_chunk_prepare_team_kernel(ChunkParams p, uint32_t units, uint32_t share_log2, uint32_t G) {
     typedef typename Mma<T>::V8 V8;
     __shared__ __align__(16) float smem[10 * TEAM_TILE + 4 * 256 + 4 * 64];
     auto tile = [&](int n) { return smem + n * TEAM_TILE; };
@@ -301,10 +303,13 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk_prepare_team_kernel(ChunkPar
     const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     float* sLd = smem + 10 * TEAM_TILE + w * 256;                            // the diagonal block of L, by rows
-    const int64_t u = blockIdx.x;
-    const int H = p.H, HV = p.HV, G = HV / H, K = p.K;
-    const int64_t ci = u / HV;
-    const int hv = (int)(u % HV), h = hv / G;
+    // (chunk, value head), heads fastest; 2^share_log2 in a row on one XCD (see launch_prepare_as)
+    const uint32_t slot = blockIdx.x >> 3, run = (slot >> share_log2) * 8 + (blockIdx.x & 7);
+    const uint32_t u = (run << share_log2) + (slot & ((1u << share_log2) - 1));
+    if (u >= units) return;
+    const int H = p.H, HV = p.HV, K = p.K;
+    const int64_t ci = u / (uint32_t)HV;
+    const int hv = (int)(u % (uint32_t)HV), h = (int)((uint32_t)hv / G);
     const bool cu32 = p.flags & GDN_FLAG_CU_INT32;
     int64_t tok0;
     int valid;
@@ -514,7 +519,14 @@ __global__ __launch_bounds__(256, 2) void gdn_chunk_prepare_team_kernel(ChunkPar
 template <typename T, bool WANT_P>
 static int launch_prepare_as(const ChunkParams& p, int64_t units, hipStream_t stream) {
     if (units <= TEAM_UNITS) {
-        hipLaunchKernelGGL((gdn_chunk_prepare_team_kernel<T, WANT_P>), dim3((unsigned)units), dim3(256), 0, stream, p);
+        // The value heads of a q/k head read the same rows: they go to one XCD (workgroups are dealt to the 8 of them in turn), and where the
+        // q/k heads are a multiple of 8 to that of the scan's workgroups, so that the rows come from memory once: 333 tokens, 16 q/k and 32 value
+        // heads 6.4 -> 3.7 MB read, the call 22.5 -> 22.0 us, on inputs out of the caches 23.4 -> 23.0; 700 tokens 33.2 -> 31.9 and 34.2 -> 33.2.
+        // As many of a group as a power of two counts, and no more than an XCD's 32 CUs: 32 value heads to a q/k head 31.1 -> 29.8 us (190 tokens,
+        // 3 q/k heads), 64 to one 32.0 -> 33.1, 128 to one 52.3 -> 59.5 (64 tokens).
+        const uint32_t G = (uint32_t)(p.HV / p.H), share = G <= 32 ? G & (0u - G) : 1, n = (uint32_t)units;
+        hipLaunchKernelGGL((gdn_chunk_prepare_team_kernel<T, WANT_P>), dim3((n / share + 7) / 8 * 8 * share), dim3(256), 0, stream, p, n,
+                           (uint32_t)__builtin_ctz(share), G);
         return check_launch("gdn_chunk_prepare_team_kernel");
     }
     auto kern = gdn_chunk_prepare_kernel<T, WANT_P>;

@@ -51,10 +51,31 @@ def _records(call, num_chunks, HV):
     (1, 128, 1, 2, 32, torch.bfloat16, 2.0, 'long'),           # keys of length 1.7: beta |k|^2 > 2 stretches the state
 ])
 def test_prepare_stage_against_closed_forms(B, T, H, HV, K, dtype, gate_div, l2, monkeypatch):
-    from fla_hip.ops.gated_delta_rule.chunk import ChunkLaunch
     # the scan kernels form P themselves; the chunk-parallel stage leaves it in its records only on request
     monkeypatch.setenv('FLA_HIP_SCAN_MODE', 'record-p')
-    has_P = True
+    _compare(B, T, H, HV, K, K, dtype, gate_div, l2, has_P=True)
+
+
+# Up to 768 units (one chunk of one value head): four waves to each, the value heads of a q/k head on one XCD.  Of many units a few are
+# compared: the first, the last and some between.
+@pytest.mark.parametrize('P', [True, False])
+@pytest.mark.parametrize('B,T,H,HV,K,dtype,gate_div,l2', [
+    (1, 190, 3, 6, 128, torch.bfloat16, 4.0, True),            # four waves: 9 (chunk, q/k head) pairs on 8 XCDs
+    (2, 100, 1, 33, 64, torch.bfloat16, 4.0, False),           # more value heads to a q/k head than an XCD has CUs
+    (1, 64, 1, 32, 128, torch.float16, 4.0, True),             # as many
+    (3, 130, 5, 10, 256, torch.bfloat16, 4.0, True),
+    (1, 64 * 192, 2, 4, 128, torch.bfloat16, 16.0, True),      # 768 units: the most
+])
+def test_prepare_stage_of_few_units_against_closed_forms(B, T, H, HV, K, dtype, gate_div, l2, P, monkeypatch):
+    monkeypatch.setenv('FLA_HIP_SCAN_MODE', 'record-p' if P else 'wide')          # (with and without P: two instances of each kernel)
+    units = B * ((T + 63) // 64) * HV
+    some = None if units <= 150 else {0, units - 1, *torch.randint(units, (14,), generator=torch.Generator().manual_seed(units)).tolist()}
+    _compare(B, T, H, HV, K, 8, dtype, gate_div, l2, has_P=P, some=some)
+
+
+def _compare(B, T, H, HV, K, V, dtype, gate_div, l2, has_P, some=None):
+    """Records against closed forms; `some`: the numbers of the units that are compared (chunk by chunk, value heads fastest; None: all)."""
+    from fla_hip.ops.gated_delta_rule.chunk import ChunkLaunch
     gen = torch.Generator().manual_seed(7)
     q = torch.randn(B, T, H, K, generator=gen)
     k = torch.randn(B, T, H, K, generator=gen)
@@ -64,7 +85,7 @@ def test_prepare_stage_against_closed_forms(B, T, H, HV, K, dtype, gate_div, l2,
     if long_keys:
         k = 1.7 * k
     q, k = q.to(dtype), k.to(dtype)
-    v = torch.randn(B, T, HV, K, generator=gen).to(dtype)
+    v = torch.randn(B, T, HV, V, generator=gen).to(dtype)
     g = F.logsigmoid(torch.randn(B, T, HV, generator=gen)) / gate_div
     beta = torch.sigmoid(torch.randn(B, T, HV, generator=gen))
     scale = K ** -0.5
@@ -84,6 +105,8 @@ def test_prepare_stage_against_closed_forms(B, T, H, HV, K, dtype, gate_div, l2,
             n = min(64, T - 64 * it)
             sl = slice(64 * it, 64 * it + n)
             for hv in range(HV):
+                if some is not None and (b * NT + it) * HV + hv not in some:
+                    continue
                 rec = recs[b * NT + it, hv]
                 gc = torch.cumsum(g[b, sl, hv].double(), 0) / math.log(2)            # chunk-local, log2 units
                 bt = beta[b, sl, hv].double()
