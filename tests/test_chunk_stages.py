@@ -56,8 +56,8 @@ def test_prepare_stage_against_closed_forms(B, T, H, HV, K, dtype, gate_div, l2,
     _compare(B, T, H, HV, K, K, dtype, gate_div, l2, has_P=True)
 
 
-# Up to 768 units (one chunk of one value head): four waves to each, the value heads of a q/k head on one XCD.  Of many units a few are
-# compared: the first, the last and some between.
+# What prepares a unit (one chunk of one value head) depends on how many there are: up to 768 four waves each, more one wave each.  Of many
+# units a few are compared: the first, the last and some between.
 @pytest.mark.parametrize('P', [True, False])
 @pytest.mark.parametrize('B,T,H,HV,K,dtype,gate_div,l2', [
     (1, 190, 3, 6, 128, torch.bfloat16, 4.0, True),            # four waves: 9 (chunk, q/k head) pairs on 8 XCDs
@@ -65,8 +65,15 @@ def test_prepare_stage_against_closed_forms(B, T, H, HV, K, dtype, gate_div, l2,
     (1, 64, 1, 32, 128, torch.float16, 4.0, True),             # as many
     (3, 130, 5, 10, 256, torch.bfloat16, 4.0, True),
     (1, 64 * 192, 2, 4, 128, torch.bfloat16, 16.0, True),      # 768 units: the most
+    (1, 64 * 192 + 1, 2, 4, 128, torch.bfloat16, 16.0, True),  # 772: one wave each, a chunk of one token
+    (4, 3200, 2, 4, 64, torch.bfloat16, 4.0, False),
+    (1, 25603, 1, 2, 40, torch.float16, 4.0, True),            # features that fill no fragment
+    (2, 6363, 2, 8, 128, torch.bfloat16, 16.0, True),          # 1600 units, ragged
+    (1, 12799, 3, 6, 128, torch.float16, 1.0, False),
+    (1, 12799, 3, 6, 256, torch.bfloat16, 16.0, True),
+    (1, 44795, 2, 6, 256, torch.float16, 16.0, True),          # 4200 units of wide keys: q's norms are the scan's
 ])
-def test_prepare_stage_of_few_units_against_closed_forms(B, T, H, HV, K, dtype, gate_div, l2, P, monkeypatch):
+def test_prepare_stage_of_few_and_many_units_against_closed_forms(B, T, H, HV, K, dtype, gate_div, l2, P, monkeypatch):
     monkeypatch.setenv('FLA_HIP_SCAN_MODE', 'record-p' if P else 'wide')          # (with and without P: two instances of each kernel)
     units = B * ((T + 63) // 64) * HV
     some = None if units <= 150 else {0, units - 1, *torch.randint(units, (14,), generator=torch.Generator().manual_seed(units)).tolist()}
