@@ -879,7 +879,7 @@ extern "C" int gdn_sum_rows(const float* part, void* out, int64_t rows, int64_t 
     GDN_CHECK_ARG(rows >= 0 && n >= 0 && n < (1ll << 36) && known_dtype(out_dtype), GDN_ERR_INVALID, "%s: bad sizes or dtype", who);
     if (n == 0) return GDN_OK;
     GDN_CHECK_ARG(out && (part || rows == 0), GDN_ERR_INVALID, "%s: NULL tensor", who);
-    const dim3 grid((unsigned)std::min<int64_t>((n + 31) / 32, 1 << 24));
+    const dim3 grid((unsigned)std::min<int64_t>((n + 31) / 32, 1 << 21));       // (a launch holds less than 2^32 threads; the kernel walks over the rest)
     hipStream_t s = (hipStream_t)stream;
     if (out_dtype == GDN_DTYPE_BF16) hipLaunchKernelGGL(sum_rows_kernel<bf16_t>, grid, dim3(1024), 0, s, part, (bf16_t*)out, rows, n);
     else if (out_dtype == GDN_DTYPE_F16) hipLaunchKernelGGL(sum_rows_kernel<f16_t>, grid, dim3(1024), 0, s, part, (f16_t*)out, rows, n);

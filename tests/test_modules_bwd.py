@@ -380,3 +380,12 @@ def test_sum_rows_edges(rows, n):
     bound = part.double().abs().sum(0) * max(rows, 2) * 2.0 ** -24
     assert ((got.double() - part.double().sum(0)).abs() <= bound).all()
     assert torch.equal(got, sum_rows(part, torch.float32))
+
+
+@pytest.mark.gpu
+def test_sum_rows_of_more_columns_than_one_launch_holds():
+    """32 threads a column: from 2^27 columns on these are more threads than a launch takes."""
+    from fla_hip.ops.gated_delta_rule._common import sum_rows
+    n = (1 << 27) + 40
+    part = torch.randint(-8, 8, (2, n), dtype=torch.int8, device='cuda').float()
+    assert torch.equal(sum_rows(part, torch.float32), part[0] + part[1])
