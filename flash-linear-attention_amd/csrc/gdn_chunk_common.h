@@ -61,15 +61,16 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // lower triangular: the fragments (tt, sp) = (0,1), (1,1) are identically zero and are not
 // stored, and of (0,0), (2,1) only the first half (4 values per lane) is.
 //   Xb   T    5 KB        (I+L)^-1 diag(beta)
-//   P    T    5 KB        scale * tril(q k^T 2^(G_t-G_t')): room only.  Every scan kernel forms P itself, from its q and k
-//                         tiles and the second table, into this place of its LDS copy; the prepare kernel writes it to
-//                         memory on request (GDN_FLAG_RECORD_P), for callers that look at the records
+//   P    T    5 KB        scale * tril(q k^T 2^(G_t-G_t')).  Written by the prepare kernel for the scan in halves (halves_fit)
+//                         and on request (GDN_FLAG_RECORD_P), for callers that look at the records; otherwise room only: the
+//                         scan kernels form P themselves, from their q and k tiles and the second table, into this place of
+//                         their LDS copy
 //   tab  fp32 [256]       [0..63] 2^(G_last-G_t), [64..127] scale*2^G_t, [128..191] 2^G_t, [192] G_last (log2 units),
 //                         the first and the third times the row factor 1/|k_t| of the l2 normalisation
 //   tab2 fp32 [256]       [0..63] G_t (log2 units), [64..127] scale, [128..191] 1/|k_t|: what P needs
-// The row factors 1/|q_t| of the l2 normalisation are not in the records: the prepare kernel does not read q.  The scan
+// The row factors 1/|q_t| of the l2 normalisation are not in the records where the prepare kernel does not read q.  The scan
 // kernels take them from the q tiles in LDS where they form P (row_rnorm below), scale P with them and multiply them
-// into [64..127] of their LDS copy of `tab` before anything reads it.  (Not always: see FLAG_Q_NORM_IN_SCAN; without it the
+// into [64..127] of their LDS copy of `tab` before anything reads it.  (Not in halves, nor always else: see FLAG_Q_NORM_IN_SCAN; without it the
 // prepare kernel reads q for its norms and both tables carry 1/|q_t|, scale/|q_t|.)
 constexpr int REC_X = 0, REC_P = 5120, REC_TAB = 10240, REC_TAB2 = 11264;
 constexpr int64_t REC_BYTES = 12288;
@@ -105,9 +106,9 @@ __device__ __forceinline__ float row_rnorm(const typename Mma<T>::V8 (&qb)[N], i
 // dropped part to reach the rounding of the fp32 state (2^-24 of its own size), and 2^24 times its size to reach the
 // operator's error bar (5e-3, set by the 16-bit operands).  So a time segment may start from a ZERO state that many
 // chunks early instead of from the exact state that a first pass and a merge would have to compute.  (Measured against
-// -48: warm-ups a third shorter, config 3 0.317 instead of 0.32 ms; with wide keys, where a head that cannot start warm is
+// -48: warm-ups a third shorter, 32768 tokens of 32 heads 0.317 instead of 0.32 ms; with wide keys, where a head that cannot start warm is
 // evaluated whole, more heads qualify: the forward of the layer's default shape with a random A_log 0.5 instead of 1.95 ms.
-// -24 would take config 3 to 0.304 ms and leave no margin over the fp32 rounding.)
+// -24 would take the first to 0.304 ms and leave no margin over the fp32 rounding.)
 constexpr float WARM_LOG2 = -32.f;
 constexpr int WARM_CAP_MAX = 64;
 __host__ __device__ constexpr int p_slot(int tt, int sp) { return tt < 2 ? tt : 2 + 2 * (tt - 2) + sp; }

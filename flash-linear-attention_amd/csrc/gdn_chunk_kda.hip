@@ -36,8 +36,8 @@ namespace gdn {
 // that a factor that underflows stands for a product that does.  What leaves does so as whole rows: through rows of LDS that only the
 // wave itself uses by then.
 // Bound by the rate at which two waves per SIMD issue vector instructions: with exponentials for every pair of blocks and every use, six to
-// eight per element, 592 us at 8192 tokens, 96 heads; with these two 446 us (1.9 GB, 4.2 TB/s), in the backward pass, where A and Gam
-// leave as well, 490 us (2.4 GB, 4.8 TB/s).
+// eight per element, 592 us at 8192 tokens, 96 heads; with these two 446 us (1.96 GB, 4.4 TB/s), in the backward pass, where A and Gam
+// leave as well, 490 us (2.47 GB, 5.0 TB/s).
 static_assert(64 * PL * 4 == 64 * P128 * 2, "the rows of v, and on their way out qg and kg, take the place of the matrix L, row by row");
 static_assert(10 * BD * 4 <= 64 * P64 * 2, "the factors per feature lie where A will");
 constexpr size_t KDA_PREP_SMEM = (2 * 64 * P128 + 64 * P64) * 2 + (64 * PG + 64) * 4;

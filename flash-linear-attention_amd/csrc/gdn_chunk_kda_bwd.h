@@ -36,7 +36,7 @@ __device__ __forceinline__ float suffix_sum_c16(float x) { return add_behind<8>(
 // L2: q and k are the rows before their l2 normalisation and dq, dk the gradients of those.
 // As two kernels of four waves this moved 530 KB per unit (dw, dPs, the first parts of dq, dk and dGk through memory, k, q and Gk twice) where
 // it now moves 280 KB, and the l2 normalisation was four passes over q and k around it.  8192 tokens, 96 heads: 1834 us + 320 us of passes ->
-// 1006 us (3.4 TB/s; bound by its chain of phases with two waves per SIMD, the longest of 3100 instructions and no barrier), the step
+// 1006 us (3.63 GB, 3.6 TB/s; bound by its chain of phases with two waves per SIMD, the longest of 3100 instructions and no barrier), the step
 // 4250 -> 3093 us.  The next unit's tiles are requested in the order of their use, the state's fragments last: earlier there
 // are no registers for them (112 bytes of scratch).
 constexpr size_t BWD_UNIT_KDA_SMEM = (6 * 64 * P128 + 2 * 64 * P64) * 2 + (64 * PG + 3 * 64 + 8 * 64 + 4) * 4;

@@ -1,17 +1,20 @@
-// Chunk-parallel stage of the chunked prefill: one WAVE per (chunk, value head) computes what does not depend on the
+// Chunk-parallel stage of the chunked prefill: one WAVE per (chunk, value head) - four where there are few - computes what does not depend on the
 // running state and is not a plain copy of the inputs:
 //   G = cumsum(g)/ln2,  L = beta*(K K^T)*2^(G_i-G_j) (i>j),  X = (I+L)^-1 in fp32,  Xb = X diag(beta),
-//   the per-token gate tables, a bound on the chunk's transition, and on request P = scale*tril(q k^T * 2^(G_i-G_j)).
+//   the per-token gate tables, a bound on the chunk's transition, and for the scan in halves or on request
+//   P = scale*tril(q k^T * 2^(G_i-G_j)).
 // Optional prologues of the reference are folded in: the gate and beta activations, and the l2 normalisation of k as
 // per-row factors 1/|k_t| on L and the tables (so the sequential stage reads q and k exactly as the caller gave them;
-// q is read here only for P, its row factors 1/|q_t| are applied by the scan where it has q in LDS anyway).  Xb and P are written in the exact register order ("fragments") in which the scan kernel feeds
-// them to the matrix cores; the scan forms v_new = Xb (v - 2^G (k S)) itself from the raw k and v, so neither
+// q is read here only for P and, where the scan does not apply them - it has q in LDS anyway -, for its row factors
+// 1/|q_t|).  Xb and P are written in the exact register order ("fragments") in which the scan kernel feeds them to the
+// matrix cores; the scan forms v_new = Xb (v - 2^G (k S)) itself from the raw k and v, so neither
 // w = Xb 2^G k nor u = Xb v is ever materialised.
 //
 // A wave shares nothing with the other waves of its workgroup, so there is no workgroup barrier:
 //   * The k rows are loaded straight into matrix-core operand registers (the operand layout of A and of B is the same:
 //     lane (c16, g) holds 8 features of token row c16), so K K^T needs no LDS; the value heads of a q/k head sit in
-//     neighbouring waves and read the same lines.
+//     neighbouring waves and read the same lines, which come from memory once (32768 tokens, 16 q/k and 32 value heads: 1.58 M requests of
+//     128 bytes, 1.05 M of them k; the others are the gates, a token's line of which the workgroups of 4 value heads each read on all XCDs).
 //   * Everything is kept TRANSPOSED: the raw tile (a, b), a <= b, holds (k_j . k_i) for rows j of t-tile a and columns i
 //     of t-tile b, gated it is U = L^T, and T = X^T = (I + U)^-1 is upper triangular (gdn_chunk_inverse.h).  The transposed X in
 //     accumulator layout is also exactly the order of the Xb operand fragments (row c16, columns 4g + e): results go from
@@ -25,8 +28,8 @@ namespace gdn {
 constexpr int PW_WAVES = 4;                                  // waves per workgroup: small workgroups keep the CU's wave slots filled
 constexpr size_t PREP_SMEM = (size_t)PW_WAVES * PW_FLOATS * 4;
 
-// WANT_P: also the records' P (for callers that look at the records; the scan kernels form P themselves): keeps the q
-// rows in registers beside the k rows, so half as many waves fit.
+// WANT_P: also the records' P (for the scan in halves, and for callers that look at the records; the other scan kernels form P
+// themselves): keeps the q rows in registers beside the k rows, so half as many waves fit.
 template <typename T, bool WANT_P>
 __global__ __launch_bounds__(64 * PW_WAVES, (WANT_P ? 8 : 16) / PW_WAVES) void gdn_chunk_prepare_kernel(ChunkParams p, int64_t units) {
     typedef typename Mma<T>::V8 V8;

@@ -62,6 +62,7 @@ __device__ __forceinline__ void step_result(const gdn_step_segment& s, int cols,
 // (9228 columns of 2048: 40 columns to a workgroup): 14.3 us with 16 columns and eight waves, half of the loads at a time, 11.4 us (37.8 MB);
 // its output projection (2048 columns of 3072: 8) 7.2 -> 6.8 us, the layer's step 45.1 -> 40.8 us.  The gated norm inside the output projection -
 // every workgroup would bring all rows of x through it - made that 16.6 us, against 7.2 + 4.6 in a launch of its own.
+// The line at 16 rows is one matrix tile of them, not a measured one: this form has not been tried with more tiles.
 template <typename T, int CT, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void gdn_step_linear_few_kernel(StepLinearParams p) {
     typedef typename Mma<T>::V8 V8;
