@@ -138,10 +138,13 @@ __global__ __launch_bounds__(256, 2) void gdn_kda_prepare_kernel(KdaParams p, in
                 __builtin_amdgcn_sched_barrier(0);              // (one row at a time: 32 activations in flight at once cost 100 registers)
             }
         }
+        // (after a mask of the type's lowest value the sums must stay numbers whose differences are numbers, also divided by ln 2: e to this is 0 as
+        // well.  `maximum`, not fmaxf: a NaN stays one)
+        constexpr float LOWEST = -1e36f;
         float run = 0.f;
 #pragma unroll
         for (int r = 0; r < 32; ++r) {
-            run += rG[r];
+            run = __builtin_elementwise_maximum(run + rG[r], LOWEST);
             sG[(32 * half + r) * PG + col] = run * RCP_LN2_F;
         }
     }

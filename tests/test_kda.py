@@ -621,6 +621,33 @@ def test_chunk_kda_backward_strong_decay_in_some_features(T, dtype, l2):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('lowest', [float('-inf'), torch.finfo(torch.float32).min, torch.finfo(torch.bfloat16).min, -1e30])
+def test_chunk_kda_gates_of_the_type_s_lowest_value(lowest, dtype):
+    """A mask of the type's lowest value as the log decay wipes the state (or features of it) in front of its token: outputs, final state and
+    gradients are finite and those of the recurrence, in the rows and blocks of a chunk on either side of it."""
+    T = 150
+    q, k, v, g, beta, h0, _, _ = _chunk_inputs(1, T, 2, 2, 128, 4.0, 0, False, False, dtype)
+    g = g.clone()
+    # (the running sum of a chunk swallows the gates behind a mask: they are zeros here)
+    for token, head, features in ((62, 0, slice(0, 4)), (63, 0, slice(0, 128)), (64, 0, slice(7, 8)), (30, 1, slice(5, 9)), (45, 1, slice(6, 8)), (T - 1, 1, slice(0, 64))):
+        g[:, token, head, features] = lowest
+        g[:, token + 1:(token // 64 + 1) * 64, head, features] = 0
+    gen = torch.Generator().manual_seed(47)
+    do, dht = torch.randn(1, T, 2, 128, generator=gen).to(dtype), torch.randn(1, 2, 128, 128, generator=gen)
+    kw = dict(scale=0.1, use_qk_l2norm_in_kernel=True)
+    ref_o, ref_ht = O.recurrent_kda(q, k, v, g, beta, 0.1, h0, True, use_qk_l2norm_in_kernel=True)
+    ref = O.kda_grads(q, k, v, g, beta, do, dht, initial_state=h0, dtype=torch.float64, **kw)
+    o, ht, got = _kda_grads_gpu(q, k, v, g, beta, h0, None, None, do, dht, **kw)
+    assert O.get_err_ratio(ref_o, o.float().cpu()) < 0.005 and O.get_err_ratio(ref_ht, ht.cpu()) < 0.005
+    _compare_grads(ref, got)
+    g[:, 10, 1, 3] = float('nan')                              # (and what is no number stays none, in its own head)
+    o, ht, got = _kda_grads_gpu(q, k, v, g, beta, h0, None, None, do, dht, **kw)
+    for x in (o.transpose(1, 2), ht, got['dh0']):
+        assert x[:, 1].isnan().any() and not x[:, 0].isnan().any()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('T,H', [(70, 33), (65, 40)])
 def test_chunk_kda_backward_scans_of_different_columns(T, H):
     """65 to 80 runs: 128 value columns to a workgroup forwards, 64 backwards, against the sequences one by one (64 in both): the same bits."""
