@@ -34,3 +34,10 @@ def test_halves(B, T, H, HV, cu, dtype, vfirst, l2, D=128):
     (1, 1985, 1, 2, None, torch.bfloat16, True, True)])
 def test_whole_runs_of_64(B, T, H, HV, cu, dtype, vfirst, l2):
     test_halves(B, T, H, HV, cu, dtype, vfirst, l2, D=64)
+
+
+@pytest.mark.parametrize('l2', [False, True])
+@pytest.mark.parametrize('D,dtype', [(128, torch.bfloat16), (128, torch.float16), (64, torch.bfloat16), (64, torch.float16)])
+def test_records_of_many_units(D, dtype, l2):
+    """64 runs of 13 chunks: 832 units, which the kernel with one wave to a unit prepares, P with them."""
+    test_halves(4, 829, 8, 16, None, dtype, False, l2, D=D)

@@ -46,21 +46,21 @@ def test_native_path_gives_the_general_path_s_bits(cu):
 @pytest.mark.parametrize('N,hidden,heads,v_heads,D,expand,conv,neg', [
     (1, 256, 2, 2, 128, 1, 4, False), (3, 512, 2, 4, 128, 2, 3, True), (16, 2048, 6, 6, 256, 2, 4, False), (17, 1024, 4, 4, 256, 1, 4, False),
     (33, 1024, 8, 8, 128, 1, 4, True), (65, 512, 4, 4, 64, 1, 4, False), (128, 512, 4, 4, 128, 1, 2, False)])
-def test_layer_step_in_four_launches(N, hidden, heads, v_heads, D, expand, conv, neg, monkeypatch):
+def test_layer_step_in_four_launches(N, hidden, heads, v_heads, D, expand, conv, neg, monkeypatch, dtype=torch.bfloat16):
     """The native decode step of the layer against the same step module by module: output and every state, two steps in a row."""
     from fla_hip.layers import GatedDeltaNet
     from fla_hip.layers.gated_deltanet import LayerCache
     torch.manual_seed(N)
     layer = GatedDeltaNet(hidden_size=hidden, expand_v=expand, head_dim=D, num_heads=heads, num_v_heads=v_heads, conv_size=conv, conv_bias=neg,
-                          allow_neg_eigval=neg, layer_idx=0).cuda().bfloat16().eval()
+                          allow_neg_eigval=neg, layer_idx=0).cuda().to(dtype).eval()
     caches = []
     state = 0.1 * torch.randn(N, v_heads, layer.head_v_dim, D, device='cuda')
-    convs = [torch.randn(N, d, conv, device='cuda', dtype=torch.bfloat16) for d in (layer.key_dim, layer.key_dim, layer.value_dim)]
+    convs = [torch.randn(N, d, conv, device='cuda', dtype=dtype) for d in (layer.key_dim, layer.key_dim, layer.value_dim)]
     for _ in range(2):
         caches.append(LayerCache())
         caches[-1].update(layer_idx=0, recurrent_state=state.clone(), conv_state=tuple(c.clone() for c in convs))
     for step in range(2):
-        x = torch.randn(N, 1, hidden, device='cuda', dtype=torch.bfloat16)
+        x = torch.randn(N, 1, hidden, device='cuda', dtype=dtype)
         assert layer._step(x, None) is None
         got = layer._step(x, caches[0])
         assert got is not None
@@ -82,8 +82,15 @@ def test_layer_step_beyond_one_tile_of_rows(N, monkeypatch):
     (1, 4096, 4, 4, 64, 1), (16, 768, 3, 6, 64, 2), (7, 256, 8, 8, 32, 1), (15, 512, 3, 3, 256, 4), (2, 256, 8, 8, 256, 2), (16, 256, 1, 32, 64, 0.625)])
 def test_layer_step_of_few_sequences(N, hidden, heads, v_heads, D, expand, monkeypatch):
     """The projections' kernel for up to 16 rows: fewer steps than waves, more than it requests at once, hidden sizes that are no power of two,
-    columns in each number of tiles a workgroup takes, segments of a few columns."""
+    one to three tiles of columns to a workgroup, segments of a few columns."""
     test_layer_step_in_four_launches(N, hidden, heads, v_heads, D, expand, 4, False, monkeypatch)
+
+
+@pytest.mark.parametrize('N,heads,v_heads,expand,dtype', [(16, 3, 6, 1, torch.bfloat16), (5, 4, 4, 2, torch.bfloat16), (13, 4, 4, 2, torch.float16),
+                                                          (3, 3, 6, 1, torch.float16)])
+def test_layer_step_of_few_sequences_in_two_tiles_of_columns(N, heads, v_heads, expand, dtype, monkeypatch):
+    """Two tiles in sixteen waves (a contraction of more than 1024): projections of 4620 columns, 24 to a workgroup, and of 6152, 32 to one."""
+    test_layer_step_in_four_launches(N, 2048, heads, v_heads, 256, expand, 4, False, monkeypatch, dtype)
 
 
 def test_layer_step_leaves_many_sequences_of_a_large_layer_to_its_modules():
