@@ -135,6 +135,16 @@ __device__ __forceinline__ void store_frag(char* m, int tt, int sp, int lane, ty
     else *(typename Mma<T>::V8*)(m + frag_off(tt, sp) + lane * 16) = f;
 }
 
+// Where the 16-byte piece c of row 4j + r of a tile lies: tiles are blocks of 4 rows (j), 16 slots of a block hold four pieces of its rows,
+// piece c of row r in slot 4r + piece_slot(c, j).  Four consecutive lanes of a copy fetch 64 contiguous bytes of one row (neighbouring lanes on
+// different rows would go through the memory pipeline one lane at a time).  A 16-byte read of the LDS serves the lanes 0-3, 12-15, 20-27 of a half wave in
+// one cycle and the others in the next, so an operand read (lane (c16, g): piece 4s + g of row c16) meets blocks 0 and 3 with g and blocks 1
+// and 2 with g + 1: flipping bit 1 in odd blocks puts those sixteen on sixteen slots, and the two blocks that a transpose read of a
+// pair of pieces (32 lanes a cycle) meets on different pairs.  With (c + j) & 3 instead both were two-way conflicts (8.1 and 4.2 cycles
+// an instruction, now 4.2 and 2.5): 333 tokens, 32 heads 21.8 -> 21.3 us a call, 32768 tokens 310 -> 303, 65536 packed tokens 551 -> 546, 8 x 2048
+// tokens, 32 heads of 256 forwards and backwards 3290 -> 3261.
+__host__ __device__ constexpr int piece_slot(int c, int j) { return (c & 3) ^ (2 * (j & 1)); }
+
 struct ChunkWs {
     float* Seg;          // 3 * seg_slots 128x128 fp32 matrices for the segment-parallel scan
     float* Bound;        // [NC][HV] log2 bound on the norm of every chunk's transition

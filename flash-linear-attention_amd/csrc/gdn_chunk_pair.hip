@@ -148,9 +148,7 @@ __global__ __launch_bounds__(PAIR_THREADS) void gdn_chunk_pair_kernel(ChunkParam
     const uint32_t rowB_qk = (uint32_t)H * K * 2, rowB_v = (uint32_t)HV * V * 2;
     const int k_pieces = K >> 3, v_pieces = V >> 3;
     // k and q tiles in LDS: 64 token rows x 256 B as 16 blocks of 4 rows (1 KB, one copy each).  In block j
-    // the 16-byte piece c of row 4j + r sits in slot 16*(c/4) + 4r + ((c + j) & 3): four consecutive lanes
-    // fetch 64 contiguous bytes of one row, and both the operand reads (16 rows x one piece) and the
-    // transpose reads (4 rows x 4 pieces) of a 16-lane group touch 16 different slots modulo 16.
+    // the 16-byte piece c of row 4j + r sits in slot 16*(c/4) + 4r + piece_slot(c, j) (gdn_chunk_common.h).
     // This wave copies blocks 2w and 2w+1: lane -> (row, byte offset of its piece)
     int kq_row[2];
     uint32_t kq_cb[2];
@@ -158,7 +156,7 @@ __global__ __launch_bounds__(PAIR_THREADS) void gdn_chunk_pair_kernel(ChunkParam
     for (int e = 0; e < 2; ++e) {
         const int j = 2 * w + e;
         kq_row[e] = 4 * j + (c16 >> 2);
-        kq_cb[e] = 16 * (4 * g + ((c16 - j) & 3));
+        kq_cb[e] = 16 * (4 * g + piece_slot(c16, j));
     }
     uint64_t kq_mask[2];
 #pragma unroll
@@ -265,8 +263,8 @@ __global__ __launch_bounds__(PAIR_THREADS) void gdn_chunk_pair_kernel(ChunkParam
     float lg = 0.f;
 
     const int tr_i = c16 >> 2, tr_j = c16 & 3;
-    const int a_off = (c16 >> 2) * 64 + 4 * (c16 & 3) + ((g + (c16 >> 2)) & 3);     // operand piece 4s + g of row c16 of a t-tile: + tt*256 + 16*s  (16-byte units)
-    const int k_tr = (g * 64 + 4 * tr_i + ((tr_j + g) & 3)) * 8;                    // row 4g+i of a 16-row group, piece 4*(m/2) + j: + (32*sp2 + 16*half)*128 + 128*(m/2) + 4*(m&1)  (elements)
+    const int a_off = (c16 >> 2) * 64 + 4 * (c16 & 3) + piece_slot(g, c16 >> 2);     // operand piece 4s + g of row c16 of a t-tile: + tt*256 + 16*s  (16-byte units)
+    const int k_tr = (g * 64 + 4 * tr_i + piece_slot(tr_j, g)) * 8;                    // row 4g+i of a 16-row group, piece 4*(m/2) + j: + (32*sp2 + 16*half)*128 + 128*(m/2) + 4*(m&1)  (elements)
     const int v_tr = (4 * (4 * g + tr_i) + tr_j) * 8;                     // private v area: row 4g + i of a block, piece j: + 4*nn + tt*512  (elements)
     // Output: a lane of the transposed tile holds token row c16, 8 value columns (piece g of the wave's
     // 64 bytes of that row).  Stored like that, neighbouring lanes would write to different rows, which

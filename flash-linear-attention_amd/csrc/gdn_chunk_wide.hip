@@ -36,11 +36,7 @@ namespace gdn {
 
 // LDS stage of one chunk.  q, k, v tiles: 64 token rows x 256 B as 16 blocks of 4 rows (1 KB, one
 // asynchronous copy each: 4 whole rows is the access shape the memory pipeline moves fastest).
-// Inside block j the 16-byte piece c of row 4j + r sits in slot 16*(c/4) + 4r + ((c + j) & 3): four consecutive
-// lanes of a copy fetch 64 contiguous bytes of one row (neighbouring lanes on different rows would go through
-// the memory pipeline one lane at a time), and the rotation makes both the 16-byte operand reads (16 rows x
-// one piece) and the LDS transpose reads (4 rows x 4 pieces) of a 16-lane group touch 16 different slots
-// modulo 16, i.e. all banks.
+// Inside block j the 16-byte piece c of row 4j + r sits in slot 16*(c/4) + 4r + piece_slot(c, j) (gdn_chunk_common.h).
 // q, v and the record are double-buffered (stage = chunk % 2); k, the one operand that is read until the
 // very end of a step, has three buffers (chunk % 3) so that its copy can be issued two steps ahead.
 constexpr int STG_Q = 0, STG_V = 16384, STG_REC = 32768;
@@ -226,7 +222,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
                 const V8* sK = (const V8*)kbuf;
                 const V8* sQ = (const V8*)(st + STG_Q);
                 const float* t2 = (const float*)(st + STG_TAB2);
-                const int a_off = (c16 >> 2) * 64 + 4 * (c16 & 3) + ((g + (c16 >> 2)) & 3);
+                const int a_off = (c16 >> 2) * 64 + 4 * (c16 & 3) + piece_slot(g, c16 >> 2);
                 auto frag = [&](int tt, int sp) {
                     V8 qb[KS];
 #pragma unroll
@@ -280,16 +276,16 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
         // A copy wave moves one tensor: k (wave CW), q (CW+1) or v (CW+2), whose rows hold `dim` = K or V elements
         // (a multiple of 8, <= 128).  Pieces of q and k past K stay zero in LDS (the tiles were cleared once and those
         // lanes copy nothing); pieces of v past V re-read valid ones: value columns never mix, and the padded ones
-        // are never stored.  What a lane fetches depends on the block only through j % 4: prepared once.
+        // are never stored.  What a lane fetches depends on the block only through j % 2: prepared once.
         const bool is_v = (w == CW + 2);
         const int dim = is_v ? V : K, pieces = dim >> 3;
         const int heads = is_v ? HV : H, head = is_v ? hv : h;
         const uint32_t row_bytes = (uint32_t)(heads * dim * 2);
-        uint32_t piece_off[4];
-        uint64_t piece_mask[4];
+        uint32_t piece_off[2];
+        uint64_t piece_mask[2];
 #pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-            const int c = 4 * g + ((c16 - jj) & 3);                         // this lane's slot holds piece c of row 4j + r
+        for (int jj = 0; jj < 2; ++jj) {
+            const int c = 4 * g + piece_slot(c16, jj);                      // this lane's slot holds piece c of row 4j + r
             piece_off[jj] = 16 * (is_v ? c % pieces : c);
             piece_mask[jj] = __builtin_amdgcn_ballot_w64(is_v || c < pieces);
         }
@@ -305,12 +301,12 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
             for (int j = 0; j < 16; ++j) {
                 if (j < j0 || j >= j1) continue;
                 const int row = min(4 * j + (c16 >> 2), valid - 1);
-                const uint32_t voff = (uint32_t)row * row_bytes + piece_off[j & 3];
+                const uint32_t voff = (uint32_t)row * row_bytes + piece_off[j & 1];
                 if constexpr (DIMS128) {
                     if (FULL && warm > 0) gather_1k_to_lds_masked(base, voff, lds_tile + j * 1024, keep);
                     else gather_1k_to_lds(base, voff, lds_tile + j * 1024);
                 } else {
-                    gather_1k_to_lds_masked(base, voff, lds_tile + j * 1024, piece_mask[j & 3] & keep);
+                    gather_1k_to_lds_masked(base, voff, lds_tile + j * 1024, piece_mask[j & 1] & keep);
                 }
             }
         };
@@ -357,7 +353,7 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
                 const char* base = (const char*)(tensor + ((bos + it * CH) * heads + head) * dim);
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const int b = 2 * j + (lane >> 5), row = min(4 * b + ((s5 & 15) >> 2), valid - 1), c = 4 * (s5 >> 4) + ((s5 - b) & 3);
+                    const int b = 2 * j + (lane >> 5), row = min(4 * b + ((s5 & 15) >> 2), valid - 1), c = 4 * (s5 >> 4) + piece_slot(s5, b);
                     gather_1k_to_lds(base, (uint32_t)row * row_bytes + 16 * c + (is_v ? 2 * col0 : 0), lds_tile + j * 1024);
                 }
             };
@@ -522,13 +518,13 @@ __global__ __launch_bounds__(WIDE_THREADS) void gdn_chunk_wide_kernel(ChunkParam
     // addresses row i = c16/4 of the 4-row run and column group j = c16%4.
     const int tr_i = c16 >> 2, tr_j = c16 & 3;
     constexpr int BLK = HALF64 ? 32 : 64;                                         // slots of a block of 4 rows of k and q
-    const int a_off = (c16 >> 2) * BLK + 4 * (c16 & 3) + ((g + (c16 >> 2)) & 3);  // operand piece 4s + g of row c16 of a t-tile: + tt*4*BLK + 16*s  (16-byte units)
-    const int k_tr = (g * BLK + 4 * tr_i + ((tr_j + g) & 3)) * 8;                 // row 4g+i of a 16-row group, piece 4*(m/2) + j: + (32*sp2 + 16*half)*128 + 128*(m/2) + 4*(m&1)  (elements)
+    const int a_off = (c16 >> 2) * BLK + 4 * (c16 & 3) + piece_slot(g, c16 >> 2);  // operand piece 4s + g of row c16 of a t-tile: + tt*4*BLK + 16*s  (16-byte units)
+    const int k_tr = (g * BLK + 4 * tr_i + piece_slot(tr_j, g)) * 8;                 // row 4g+i of a 16-row group, piece 4*(m/2) + j: + (32*sp2 + 16*half)*128 + 128*(m/2) + 4*(m&1)  (elements)
     int v_tr[NN];                                                                 // row 4g+i, piece = 8-column group of tile nn: + tt*2048
 #pragma unroll
     for (int nn = 0; nn < NN; ++nn) {
         const int c = 2 * (NN * w + nn) + (tr_j >> 1);
-        v_tr[nn] = (g * (HALF ? 32 : 64) + 16 * (c >> 2) + 4 * tr_i + ((c + g) & 3)) * 8 + 4 * (tr_j & 1);
+        v_tr[nn] = (g * (HALF ? 32 : 64) + 16 * (c >> 2) + 4 * tr_i + piece_slot(c, g)) * 8 + 4 * (tr_j & 1);
     }
 
     // One step, written as a fixed sequence of small scheduling regions (the compiler may reorder

@@ -129,7 +129,7 @@ __global__ __launch_bounds__(W2_THREADS) void gdn_chunk_wide256_kernel(ChunkPara
     }
     lds_barrier();
 
-    const int a_off = (c16 >> 2) * 64 + 4 * (c16 & 3) + ((g + (c16 >> 2)) & 3);   // operand piece 4s + g of row c16 of a t-tile (16-byte units)
+    const int a_off = (c16 >> 2) * 64 + 4 * (c16 & 3) + piece_slot(g, c16 >> 2);   // operand piece 4s + g of row c16 of a t-tile (16-byte units)
 
     // =====================================================================================
     // Copy waves.  Step i reads stage i & 1 of k, v and the record; barrier B1 ends the reads of q, v, the record and
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(W2_THREADS) void gdn_chunk_wide256_kernel(ChunkPara
             __builtin_amdgcn_s_setprio(0);
         };
         // Rows 4j .. 4j+3 of a [token][head][K] tensor, 128 features of them (`half`), into block j of a 16 KB tile:
-        // lane (g, c16) holds piece c = 4g + ((c16 - j) & 3) of row 4j + c16 / 4.  Rows past the end of the sequence
+        // lane (g, c16) holds piece c = 4g + piece_slot(c16, j) of row 4j + c16 / 4.  Rows past the end of the sequence
         // re-read its last row (finite, and multiplied by zeros everywhere).
         auto gather_qk = [&](const T* tensor, int64_t it, uint32_t lds_tile) {
             const int valid = (int)min((int64_t)CH, len - it * CH);
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(W2_THREADS) void gdn_chunk_wide256_kernel(ChunkPara
             for (int half = 0; half < 2; ++half)
 #pragma unroll
                 for (int j = 0; j < 16; ++j) {
-                    const int c = 4 * g + ((c16 - j) & 3);
+                    const int c = 4 * g + piece_slot(c16, j);
                     const uint64_t mask = __builtin_amdgcn_ballot_w64(128 * half + 8 * c < K);
                     const int row = min(4 * j + (c16 >> 2), valid - 1);
                     gather_1k_to_lds_masked(base, (uint32_t)row * row_bytes + 256 * half + 16 * c, lds_tile + half * 16384 + j * 1024, mask);
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(W2_THREADS) void gdn_chunk_wide256_kernel(ChunkPara
                 const uint32_t row_bytes = (uint32_t)(HV * V * 2);
 #pragma unroll
                 for (int j = 0; j < 16; ++j) {
-                    const int c = 4 * g + ((c16 - j) & 3);
+                    const int c = 4 * g + piece_slot(c16, j);
                     const uint64_t mask = __builtin_amdgcn_ballot_w64(c < 8 && v0 + 8 * c < V);
                     const int row = min(4 * j + (c16 >> 2), valid - 1);
                     gather_1k_to_lds_masked(base, (uint32_t)row * row_bytes + 16 * c, lds_tile + j * 1024, mask);
@@ -327,11 +327,11 @@ __global__ __launch_bounds__(W2_THREADS) void gdn_chunk_wide256_kernel(ChunkPara
     float lg = 0.f;
 
     const int tr_i = c16 >> 2, tr_j = c16 & 3;
-    const int k_tr = (g * 64 + 4 * tr_i + ((tr_j + g) & 3)) * 8;
+    const int k_tr = (g * 64 + 4 * tr_i + piece_slot(tr_j, g)) * 8;
     int v_tr;
     {
         const int c = 2 * w + (tr_j >> 1);
-        v_tr = (g * 64 + 16 * (c >> 2) + 4 * tr_i + ((c + g) & 3)) * 8 + 4 * (tr_j & 1);
+        v_tr = (g * 64 + 16 * (c >> 2) + 4 * tr_i + piece_slot(c, g)) * 8 + 4 * (tr_j & 1);
     }
 
     auto step = [&](const char* kbuf, const char* vbuf, const char* rec, int istep) {
