@@ -31,7 +31,7 @@
 namespace gdn {
 
 // In separate arrays, per (chunk, v-head): gam, beta [64] fp32, A, P [64][64], Bound (one float, see gdn_chunk_common.h, WARM_LOG2); and per
-// (chunk, v-head, block of VD value columns): v_new, dv_new [64][VD], S, dS [KD][VD] ([K][V]), all in the operand type.
+// (chunk, v-head, block of VD value columns): v_new, dv_new [64][VD], S, dS [KD][VD] as operand fragments (state_frag), all in the operand type.
 // Comba adds gam0 and dgam [64] fp32 (dgam partial, between the last two kernels), P^T in P's place, w, dw [64][128], u [64][128].
 // The KDA operator (a decay per key feature) has instead: Gk, the running sums of the log decays, divided by ln 2, [64][128] fp32; QG = scale q e^Gk,
 // KG = k e^(Gk_last - Gk) [64][128] and P [64][64] in the operand type, EGL = e^Gk_last [128] fp32 (all four as the forward's
@@ -430,9 +430,8 @@ __global__ __launch_bounds__(256, 1) void gdn_bwd_dqkw_kernel(BwdParams p, int64
             for (int a2 = 0; a2 < 2; ++a2)
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    const int kk = 16 * (2 * w + a2) + c16;
-                    rS[a2][s] = *(const V8*)(Hu + kk * BD + 32 * s + 8 * g);
-                    rdS[a2][s] = *(const V8*)(dHu + kk * BD + 32 * s + 8 * g);
+                    rS[a2][s] = *(const V8*)(Hu + state_frag<BD>(2 * w + a2, s, lane));
+                    rdS[a2][s] = *(const V8*)(dHu + state_frag<BD>(2 * w + a2, s, lane));
                 }
         }
         fetch_tile<KD>(rK, (const T*)p.k + (c.tok0 * p.H + hq) * KD, (int64_t)p.H * KD, c.valid, tid);

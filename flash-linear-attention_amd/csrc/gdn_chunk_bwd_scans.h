@@ -133,7 +133,7 @@ __device__ __forceinline__ void bwd_state_body(const BwdParams& p, char* smem, c
                 *(V4*)(sS + kk * PV + vq0 + 16 * b + 4 * g) = pack4<T>(S[a2][b]);
             }
         lds_barrier();
-        if (keep) copy_rows_out<KD, VBT, NTH>(Hu + vcol0, VD, sS, PV, tid);     // (whole rows of the tile: 16 bytes a lane)
+        if (keep) copy_state_out<KD, VBT, VD, NTH>(Hu, vcol0 / 32, sS, PV, tid);
         if (ic + 1 < c_end) fetch(ic + 1);
         const float glast = sGam[63];
         // transposed tiles: value columns on the rows, this wave's 16 tokens on the columns
@@ -302,7 +302,7 @@ __device__ __forceinline__ void bwd_dstate_body(const BwdParams& p, char* smem, 
                 *(V4*)(sDS + kk * PV + vq0 + 16 * b + 4 * g) = pack4<T>(dS[a2][b]);
             }
         lds_barrier();
-        if (keep) copy_rows_out<KD, VBT, NTH>(dHu + vcol0, VD, sDS, PV, tid);
+        if (keep) copy_state_out<KD, VBT, VD, NTH>(dHu, at.vcol0 / 32, sDS, PV, tid);
         if (ic >= c_lo + 1) fetch(ic - 1);
         const float glast = sGam[63];
         const int j = 16 * w + c16;

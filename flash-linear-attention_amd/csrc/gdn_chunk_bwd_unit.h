@@ -77,11 +77,11 @@ __global__ __launch_bounds__(64 * NW, 2) void gdn_bwd_unit_kernel(BwdParams p, i
     const bool parts_out = LEAN ? p.dq_part != nullptr : PARTS;
     auto fetch_state = [&](const Item& at, int hv, int a, int w, int lane, bool S = true, bool dS = true) {     // feature tile a of this wave
         const int64_t u = at.ch * p.HV + hv;
-        const int64_t off = u * KD * VD + (16 * (NA * w + a) + (lane & 15)) * VD + 8 * (lane >> 4);
+        const int64_t off = u * KD * VD + state_frag<VD>(NA * w + a, 0, lane);
 #pragma unroll
         for (int s = 0; s < SV; ++s) {
-            if (S) sf[s] = *(const V8*)((const T*)p.ws.Hs + off + 32 * s);
-            if (dS) df[s] = *(const V8*)((const T*)p.ws.dHs + off + 32 * s);
+            if (S) sf[s] = *(const V8*)((const T*)p.ws.Hs + off + 512 * s);
+            if (dS) df[s] = *(const V8*)((const T*)p.ws.dHs + off + 512 * s);
         }
     };
     auto fetch_out = [&](const Item& at, int hv, int tid) {

@@ -69,9 +69,9 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
         fetch_tile<BD, NTH>(rV, (const T*)p.v + (at.c.tok0 * p.HV + at.hv) * BD, (int64_t)p.HV * BD, at.c.valid, tid);
     };
     auto fetch_state = [&](const UnitAt& at, int64_t u, int tid) {
-        const int64_t off = u * BD * BD + (16 * (tid >> 6) + (tid & 15)) * BD + 8 * ((tid & 63) >> 4);
+        const int64_t off = u * BD * BD + state_frag<BD>(tid >> 6, 0, tid & 63);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) { sf[s] = *(const V8*)((const T*)p.ws.Hs + off + 32 * s); df[s] = *(const V8*)((const T*)p.ws.dHs + off + 32 * s); }
+        for (int s = 0; s < 4; ++s) { sf[s] = *(const V8*)((const T*)p.ws.Hs + off + 512 * s); df[s] = *(const V8*)((const T*)p.ws.dHs + off + 512 * s); }
         fetch_tile<CH, NTH>(rA, (const T*)p.ws.Am + u * 64 * 64, 64, 64, tid);
         if (tid < 64) rBeta = tid < at.c.valid ? load_scalar_bits(p.beta, (at.c.tok0 + tid) * p.HV + at.hv, p.gb_dtype) : 0;
     };

@@ -124,6 +124,29 @@ __device__ __forceinline__ void copy_rows_out(T* g, int64_t stride, const T* s, 
         if (idx / PPR < valid) *(u32x4*)(g + (int64_t)(idx / PPR) * stride + (idx % PPR) * 8) = x[i];
     }
 }
+// A state in the workspace lies as the operand fragments that its readers take from it: 16 key features (tile a) x 32 of VD value columns (step s) after one
+// another, in them 16 bytes a lane - key 16a + c16, value columns 32s + 8g .. +7.  A wave's load is 1 KB in a row (from rows of VD elements its lanes would go
+// to sixteen rows, which the memory pipeline takes one lane at a time).  Step of 8 x 2048 tokens, 32 heads of 256: 3255 -> 3225 us; 16000 packed tokens, 32 heads
+// of 128: 1081 -> 1074; 8 x 1024 tokens, 8 heads of 64: 120.8 -> 119.5.
+template <int VD> __device__ __forceinline__ int state_frag(int a, int s, int lane) { return ((a * (VD / 32) + s) * 64 + lane) * 8; }
+// ... and out of a row-major LDS tile of KD rows of NCOLS of the value columns, from step s0 on
+template <int KD, int NCOLS, int VD, int NTH, typename T>
+__device__ __forceinline__ void copy_state_out(T* g, int s0, const T* t, int pitch, int tid) {
+    constexpr int SN = NCOLS / 32, N = KD * NCOLS / 8 / NTH;
+    static_assert(N * NTH * 8 == KD * NCOLS, "whole rounds of the workgroup's threads");
+    const int lane = tid & 63, w = tid >> 6;
+    u32x4 x[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int f = w + NTH / 64 * i;
+        x[i] = *(const u32x4*)(t + (16 * (f / SN) + (lane & 15)) * pitch + 32 * (f % SN) + 8 * (lane >> 4));
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int f = w + NTH / 64 * i;
+        *(u32x4*)(g + state_frag<VD>(f / SN, s0 + f % SN, lane)) = x[i];
+    }
+}
 // operand fragment whose contraction runs along a row: index r0 + c16, contraction c0 + 8g + e
 template <typename T>
 __device__ __forceinline__ typename Mma<T>::V8 frag_rows(const T* s, int pitch, int r0, int c0, int lane) {
