@@ -993,6 +993,7 @@ __global__ __launch_bounds__(256, 2) void gdn_bwd_wy2_kernel(BwdParams p, int64_
 }
 
 #include "gdn_chunk_bwd_unit.h"
+#include "gdn_chunk_bwd_unit256.h"
 
 // The partial rows of dq and dk (and, where parts cut a value head, the partial sums of dg and dbeta) added up in fp32, in a fixed order:
 // eight rows of a chunk and q/k head per workgroup.
@@ -1105,12 +1106,15 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
         else if (runs > 128 || (runs > 64 && half + whole <= 256)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<128, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", half + whole, 512, (int64_t)half};
         else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * half, 512, (int64_t)half};
     }
-    constexpr int NW = KD == 64 ? 4 : 8;
     const int64_t items = num_chunks * p.H * p.parts;
-    constexpr bool APART = KD <= BD;
-    const void* unit = APART && p.dq_part ? (l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, true, APART> : (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, false, APART>)
-                                          : (l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, true, false> : (const void*)gdn_bwd_unit_kernel<T, KD, VD, NW, false, false>);
-    ks[3] = {unit, bwd_unit_smem<KD, VD, NW>(), "gdn_bwd_unit_kernel", (unsigned)std::min<int64_t>(items, NW == 4 ? 512 : 256), 64 * NW, items};
+    if constexpr (KD <= BD) {
+        const void* unit = p.dq_part ? (l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, VD, true, true> : (const void*)gdn_bwd_unit_kernel<T, KD, VD, false, true>)
+                                     : (l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, VD, true, false> : (const void*)gdn_bwd_unit_kernel<T, KD, VD, false, false>);
+        ks[3] = {unit, bwd_unit_smem<KD>(), "gdn_bwd_unit_kernel", (unsigned)std::min<int64_t>(items, KD == 64 ? 512 : 256), 64 * bwd_unit_waves<KD>(), items};
+    } else {
+        const void* unit = l2 ? (const void*)gdn_bwd_unit256_kernel<T, true> : (const void*)gdn_bwd_unit256_kernel<T, false>;
+        ks[3] = {unit, BWD_UNIT256_SMEM, "gdn_bwd_unit256_kernel", (unsigned)std::min<int64_t>(items, 256), 64 * UNIT256_NW, items};
+    }
     if (p.dq_part) ks[4] = {(const void*)gdn_bwd_add_parts_kernel<T, KD>, 0, "gdn_bwd_add_parts_kernel", (unsigned)(num_chunks * p.H * 8), 256, 0};
     return launch_all(p, ks, 5, stream);
 }

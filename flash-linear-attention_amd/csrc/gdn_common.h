@@ -95,9 +95,11 @@ __device__ __forceinline__ int64_t load_index(const void* p, int64_t i, bool is_
 // The same for an index that is the same in every lane, from a table no kernel in flight writes: scalar loads, which do not stand in
 // the queue of the vector loads (a wave that walks over units would wait for its whole prefetch before it knew the next unit).
 __device__ __forceinline__ int64_t load_index_uniform(const void* p, int64_t i, bool is_i32) {
-    typedef const __attribute__((address_space(4))) int32_t* c32;
-    typedef const __attribute__((address_space(4))) int64_t* c64;
-    return is_i32 ? (int64_t)((c32)(uintptr_t)p)[i] : ((c64)(uintptr_t)p)[i];
+    // (both halves by loads of their own, without a branch: two indices in a row are in flight together)
+    typedef const __attribute__((address_space(4))) uint32_t* c32;
+    const c32 at = (c32)((uintptr_t)p + ((uint64_t)i << (is_i32 ? 2 : 3)));
+    const uint32_t lo = at[0], hi = at[is_i32 ? 0 : 1];
+    return is_i32 ? (int64_t)(int32_t)lo : (int64_t)((uint64_t)hi << 32 | lo);
 }
 
 __device__ __forceinline__ float softplus_f(float x) {

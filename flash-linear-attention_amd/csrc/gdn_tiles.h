@@ -159,6 +159,80 @@ __device__ __forceinline__ typename Mma<T>::V8 frag_cols(const T* s, int pitch, 
     const T* at = s + (r0 + 8 * (lane >> 4) + (a >> 2)) * pitch + c0 + 4 * (a & 3);
     return join<typename Mma<T>::V8>(Mma<T>::tr_read(at), Mma<T>::tr_read(at + 4 * pitch));
 }
+// ---- tiles in blocks -----------------------------------------------------------------------
+// 64 rows of COLS elements without padding: blocks of four rows, in a block groups of sixteen 16-byte slots, group n the pieces (8 elements) 4n .. 4n+3 of its
+// rows; piece c of row 4j + r in slot 4r + ((c & 3) ^ block_flip(j)) of its group.  A CU's LDS serves 256 bytes a cycle: of a 16-byte read the lanes {0-3, 12-15,
+// 20-27} and {4-11, 16-19, 28-31} of each half wave together, of an 8-byte read (transposing or not) a half wave, of a store sixteen lanes.  block_flip puts
+// what each of them meets on different banks: block_rows, block_cols and 8-byte accesses to (16t + c16, 4g).  (Rows padded by 16 bytes, as in the tiles above,
+// put two rows of an operand read on a bank: 8.1 cycles an instruction, here 4.2; block_cols 2.5 each, there 4.2.)  Unlike pieces that trade places
+// over a whole row, tiles and steps of a product are constants in the address.
+__device__ __forceinline__ constexpr int block_flip(int j) { return (4 - j) & 3; }
+// The address of an access is the tile, constants (or scalars) for where in it, and a lane's share in bytes that is the same for all tiles of a width: the caller
+// computes it once and keeps it (`opaque`: the compiler would take it apart and add it up again at every access).  Odd 16-column tiles lie 32 bytes apart: the share ^ 32.
+__device__ __forceinline__ int opaque(int x) { asm volatile("" : "+v"(x)); return x; }
+template <int COLS> __device__ __forceinline__ constexpr int block_off(int r0, int c0) { return (r0 * COLS + (c0 >> 5) * 128) * 2; }      // r0, c0: multiples of 16
+// element (r, c) of a 16 x 16 tile
+template <int COLS> __device__ __forceinline__ constexpr int block_lane(int r, int c) {
+    return ((r & ~3) * COLS + 32 * (r & 3) + (((c >> 3) ^ block_flip((r >> 2) & 3)) << 3) + (c & 7)) * 2;
+}
+// as frag_rows and frag_cols: the shares of lane (c16, g), then the reads
+template <int COLS> __device__ __forceinline__ int block_rows_lane(int lane) {
+    return ((lane & 12) * COLS + 32 * (lane & 3) + 8 * ((lane >> 4) ^ block_flip((lane >> 2) & 3))) * 2;
+}
+template <int COLS, typename T>
+__device__ __forceinline__ typename Mma<T>::V8 block_rows(const T* s, int r0, int c0, int share) {
+    return *(const typename Mma<T>::V8*)((const char*)s + block_off<COLS>(r0, c0) + share);
+}
+struct ColsLane { int a, b; };                                  // of the two transposing reads (of an even 16-column tile)
+template <int COLS> __device__ __forceinline__ ColsLane block_cols_lane(int lane) {
+    const int a = lane & 15, g = lane >> 4, x = ((a >> 1) & 1) ^ (2 * (g & 1)), at = 8 * g * COLS + 32 * (a >> 2) + 4 * (a & 1);
+    return ColsLane{(at + 8 * x) * 2, (at + 4 * COLS + 8 * (x ^ 3)) * 2};
+}
+template <int COLS, typename T>
+__device__ __forceinline__ typename Mma<T>::V8 block_cols(const T* s, int r0, int c0, ColsLane share) {
+    const char* at = (const char*)s + block_off<COLS>(r0, c0);
+    return join<typename Mma<T>::V8>(Mma<T>::tr_read((const T*)(at + share.a)), Mma<T>::tr_read((const T*)(at + share.b)));
+}
+__device__ __forceinline__ ColsLane odd_tile(ColsLane x) { return ColsLane{x.a ^ 32, x.b ^ 32}; }
+// as fetch_tile and put_tile: a thread's pieces are those of the slots tid, tid + NTH, ..., four lanes on 64 bytes of a row
+// (rows from `valid` on are fetched from the last valid one, and zeros by the time they are put)
+template <int NCOLS, int NTH, typename T>
+__device__ __forceinline__ void fetch_blocks(TileRegs<NCOLS, NTH>& r, const T* g, int64_t stride, int valid, int tid) {
+    constexpr int SLOTS = NCOLS / 2, N = 64 * NCOLS / 8 / NTH, RPI = NTH / SLOTS * 4;      // a thread's pieces lie RPI rows apart
+    static_assert(N >= 1 && N * NTH * 8 == 64 * NCOLS && RPI % 16 == 0, "whole rounds of the workgroup's threads");
+    const int row0 = 4 * (tid / SLOTS) + ((tid >> 2) & 3), pc = 4 * ((tid % SLOTS) >> 4) + ((tid & 3) ^ block_flip((tid / SLOTS) & 3));
+#pragma unroll
+    for (int i = 0; i < N; ++i) r.x[i] = *(const u32x4*)((const char*)g + ((uint32_t)min(row0 + RPI * i, valid - 1) * (uint32_t)(stride * sizeof(T)) + (uint32_t)(pc * 16)));
+}
+template <int NCOLS, int NTH, typename T>
+__device__ __forceinline__ void put_blocks(T* s, const TileRegs<NCOLS, NTH>& r, int valid, int tid) {
+    constexpr int SLOTS = NCOLS / 2, N = 64 * NCOLS / 8 / NTH, RPI = NTH / SLOTS * 4;
+    const int row0 = 4 * (tid / SLOTS) + ((tid >> 2) & 3);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        u32x4 x = r.x[i];
+        if (valid < 64) { if (row0 + RPI * i >= valid) x = u32x4{0u, 0u, 0u, 0u}; }
+        *(u32x4*)(s + (tid + NTH * i) * 8) = x;
+    }
+}
+// The same straight into the LDS, without registers: issued here, landed when the issuing waves have waited for their vector-memory operations
+// (wait_vm_at_most) and met at a barrier.  Rows from `valid` on are zeros.  Nobody may still read the tile.
+template <int NCOLS, int NW, typename T>
+__device__ __forceinline__ void copy_blocks(T* s, const T* g, int64_t stride, int valid, int w, int lane) {
+    constexpr int SLOTS = NCOLS / 2, N = NCOLS / 8 / NW;
+    static_assert(N * NW * 8 == NCOLS && SLOTS <= 64, "whole rounds of the workgroup's waves, a block or two each");
+    const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)s;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int k = w + NW * i, b = k * (64 / SLOTS) + lane / SLOTS, row = 4 * b + ((lane >> 2) & 3), pc = 4 * ((lane % SLOTS) >> 4) + ((lane & 3) ^ block_flip(b & 3));
+        const uint32_t voff = (uint32_t)row * (uint32_t)(stride * sizeof(T)) + 16 * pc;
+        if (valid >= 64) gather_1k_to_lds((const char*)g, voff, lds + k * 1024);
+        else {
+            gather_1k_to_lds_masked((const char*)g, voff, lds + k * 1024, __builtin_amdgcn_ballot_w64(row < valid));
+            if (row >= valid) *(u32x4*)(s + (k * 64 + lane) * 8) = u32x4{0u, 0u, 0u, 0u};
+        }
+    }
+}
 template <typename T>
 __device__ __forceinline__ typename Mma<T>::V4 pack4(f32x4 x) {
     return typename Mma<T>::V4{(T)x[0], (T)x[1], (T)x[2], (T)x[3]};
