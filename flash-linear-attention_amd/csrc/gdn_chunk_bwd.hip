@@ -1062,14 +1062,6 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
     const int64_t runs = p.N * p.HV;
     const unsigned units = (unsigned)(num_chunks * (p.HV / p.nb));
     const bool l2 = p.q_raw != nullptr;
-    if constexpr (KD > BD) {
-        // (rows of two rounds do not wait in registers for their factors: normalised in passes of their own)
-        if (l2) {
-            const int dtype = std::is_same<T, bf16_t>::value ? GDN_DTYPE_BF16 : GDN_DTYPE_F16;
-            if (int rc = gdn_l2norm_fwd(p.q_raw, (void*)p.q, (float*)p.q_rstd, p.tokens * p.H, KD, KD, dtype, stream)) return rc;
-            if (int rc = gdn_l2norm_fwd(p.k_raw, (void*)p.k, (float*)p.k_rstd, p.tokens * p.H, KD, KD, dtype, stream)) return rc;
-        }
-    }
     // Time segments for the two scans (up to 128 key features, dense input): long sequences on few heads leave CUs without a
     // workgroup; never more workgroups than CUs, segments of 8 chunks or more, and at least 24 steps saved per workgroup
     // (a warm-up of typical length must pay).  GDN_FLAG_SCAN_WIDE asks for whole sequences, GDN_FLAG_SCAN_SEGMENTS for segments of 4.
@@ -1085,8 +1077,7 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
     }
     BwdLaunch ks[5] = {};
     const unsigned pgrid = (units + BP_WAVES - 1) / BP_WAVES;
-    if constexpr (KD <= BD) ks[0] = {l2 ? (const void*)gdn_bwd_prepare_kernel<T, KD, true> : (const void*)gdn_bwd_prepare_kernel<T, KD, false>, 0, "gdn_bwd_prepare_kernel", pgrid, 64 * BP_WAVES, units};
-    else ks[0] = {(const void*)gdn_bwd_prepare_kernel<T, KD, false>, 0, "gdn_bwd_prepare_kernel", pgrid, 64 * BP_WAVES, units};
+    ks[0] = {l2 ? (const void*)gdn_bwd_prepare_kernel<T, KD, true> : (const void*)gdn_bwd_prepare_kernel<T, KD, false>, 0, "gdn_bwd_prepare_kernel", pgrid, 64 * BP_WAVES, units};
     if constexpr (KD <= BD) {
         if (p.nseg > 1)                                         // both scans side by side in a workgroup: every CU has one already
             ks[1] = {(const void*)gdn_bwd_scans_kernel<T, 32, KD, VD>, bwd_scans_smem<32, KD>(), "gdn_bwd_scans_kernel", scan_grid(p, VD, 32) * p.nseg, 512, 0};

@@ -6,18 +6,22 @@
 // both [64][64] row-major in the operand type; gam and beta as the scans and the last kernel want them (after their activations); a
 // bound on the chunk's transition; and with the l2 normalisation of q and k taken in here (L2) the normalised rows and their factors,
 // left by the first of the value heads that share them.  The rows are loaded straight into matrix-core operand registers and serve as
-// both factors of k k^T; results go from registers to memory, four columns of a row per lane.  Two waves per SIMD (k and q rows and
-// both products: some 200 registers).
-// 16000 packed tokens, 16 q/k and 32 value heads of 128, normalisation inside: 128 us; as four waves per unit with row-major LDS tiles, which also formed
+// both factors of k k^T; results go from registers to memory, four columns of a row per lane.  P is formed a column of tiles at a time and
+// on its way to memory before k k^T is begun, so that the rows of k stay in registers also at 256 features (128 registers, and two of q's
+// four row tiles, 64) and need no normalising pass before: memory bounds the kernel, 1.2 GB at 4.9 TB/s there.  Two waves per SIMD: three,
+// which 164 registers would let in at 128 features, only push one another's rows out of the caches (122 -> 136 us).
+// 16000 packed tokens, 16 q/k and 32 value heads of 128, normalisation inside: 122 us; as four waves per unit with row-major LDS tiles, which also formed
 // w = A (beta e^gam k) and u = A (beta v) - 32 KB per unit that the scans now do without - 264 us.
+// 8 x 2048 tokens, 32 heads of 256, normalisation inside: 240 us; in two passes over q and k of their own before, whose rows were then
+// read 128 features of k and q at a time: 320 us.
 constexpr int BP_WAVES = 4;
 
 template <typename T, int KD, bool L2>
-__global__ __launch_bounds__(64 * BP_WAVES, 2) void gdn_bwd_prepare_kernel(BwdParams p, int64_t units) {
+__global__ __launch_bounds__(64 * BP_WAVES) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_bwd_prepare_kernel(BwdParams p, int64_t units) {
     typedef typename Mma<T>::V8 V8;
     typedef typename Mma<T>::V4 V4;
-    constexpr int ROUND = KD < 128 ? KD : 128, NS = ROUND / 32;       // key features of a round, 32 at a time
-    static_assert(!L2 || KD == ROUND, "the rows wait for their factors in the registers of one round");
+    constexpr int NS = KD / 32;                                      // operands of 32 features per row tile
+    constexpr int QT = KD <= 128 ? 4 : 2;                            // q's row tiles in registers at a time
     __shared__ __align__(16) float smem[BP_WAVES * PW_FLOATS];
     const int tid = threadIdx.x, lane = tid & 63, c16 = lane & 15, g = lane >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -36,11 +40,6 @@ __global__ __launch_bounds__(64 * BP_WAVES, 2) void gdn_bwd_prepare_kernel(BwdPa
         rg = p.g ? load_scalar_bits(p.g, (c.tok0 + lane) * HVg + hv, p.gb_dtype) : 0;
         rb = load_scalar_bits(p.beta, (c.tok0 + lane) * HVg + hv, p.beta_dtype);
     }
-    f32x4 U[4][4], QK[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = a; b < 4; ++b) U[a][b] = QK[a][b] = ZERO4;
     const int64_t row0 = (c.tok0 * p.H + hq) * KD;
     const T* kg = (const T*)(L2 ? p.k_raw : p.k) + row0;
     const T* qg = (const T*)(L2 ? p.q_raw : p.q) + row0;
@@ -63,6 +62,7 @@ __global__ __launch_bounds__(64 * BP_WAVES, 2) void gdn_bwd_prepare_kernel(BwdPa
         const float r = rsqrtf(sum_over_g(ss) + 1e-6f);
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
+            if constexpr (std::is_same<T, f16_t>::value) asm volatile("" : "+v"(f[s]));      // (or the sum's 32-bit values are kept till here)
             V8 x = __builtin_bit_cast(V8, f[s]);
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[e] = (T)((float)x[e] * r);
@@ -70,52 +70,91 @@ __global__ __launch_bounds__(64 * BP_WAVES, 2) void gdn_bwd_prepare_kernel(BwdPa
         }
         return r;
     };
-    u32x4 fk[4][NS], fq[4][NS];
-#pragma unroll 1
-    for (int k0 = 0; k0 < KD; k0 += ROUND) {
+    // row tile t normalised; the first of the value heads that share the rows leaves them, with their factors
+    auto normalise = [&](u32x4 (&f)[NS], int t, const void* rows, const float* factors) {
+        const float n = unit_rows(f);
+        if (hq * G == hv && 16 * t + c16 < c.valid) {
+            char* bp = (char*)((T*)rows + row0 + (int64_t)(16 * t) * p.H * KD);
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int s = 0; s < NS; ++s) fk[t][s] = fragment(kg, t, k0 + 32 * s);
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int s = 0; s < NS; ++s) fq[t][s] = fragment(qg, t, k0 + 32 * s);
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (L2) {
-            const bool leave = hq * G == hv;                         // (the first of the value heads that share the rows leaves them)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const float nk = unit_rows(fk[t]), nq = unit_rows(fq[t]);
-                if (leave && 16 * t + c16 < c.valid) {
-#pragma unroll
-                    for (int s = 0; s < NS; ++s) {
-                        const int64_t at = row0 + (int64_t)(16 * t + c16) * p.H * KD + 32 * s + 8 * g;
-                        *(u32x4*)((T*)p.k + at) = fk[t][s];
-                        *(u32x4*)((T*)p.q + at) = fq[t][s];
-                    }
-                    if (g == 0) {
-                        ((float*)p.k_rstd)[(c.tok0 + 16 * t + c16) * p.H + hq] = nk;
-                        ((float*)p.q_rstd)[(c.tok0 + 16 * t + c16) * p.H + hq] = nq;
-                    }
-                }
-            }
+            for (int s = 0; s < NS; ++s) *(u32x4*)(bp + lane_off + 64 * s) = f[s];
+            if (g == 0) ((float*)factors)[(c.tok0 + 16 * t + c16) * p.H + hq] = n;
         }
+        __builtin_amdgcn_sched_barrier(0);                               // (one tile's values in 32 bits at a time)
+    };
+    u32x4 fk[4][NS], fq[QT][NS];
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int a = 0; a <= b; ++a)
+        for (int s = 0; s < NS; ++s) fk[t][s] = fragment(kg, t, 32 * s);
 #pragma unroll
-                for (int s = 0; s < NS; ++s) U[a][b] = Mma<T>::run(__builtin_bit_cast(V8, fk[a][s]), __builtin_bit_cast(V8, fk[b][s]), U[a][b]);
+    for (int t = 0; t < QT; ++t)
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int s = 0; s < NS; ++s) {
-                const V8 q8 = __builtin_bit_cast(V8, fq[b][s]);
-#pragma unroll
-                for (int a = 0; a <= b; ++a) QK[a][b] = Mma<T>::run(__builtin_bit_cast(V8, fk[a][s]), q8, QK[a][b]);      // rows: keys j, column: query i
-            }
+        for (int s = 0; s < NS; ++s) fq[t][s] = fragment(qg, t, 32 * s);
+    __builtin_amdgcn_sched_barrier(0);
+    float x = scalar_of_bits(rg, p.gb_dtype), beta = scalar_of_bits(rb, p.beta_dtype);
+    if (lane < c.valid) {
+        if (p.A_log && p.g) x = -__expf(p.A_log[hv]) * softplus_f(x + (p.dt_bias ? p.dt_bias[hv] : 0.f));
+        if (p.flags & GDN_FLAG_BETA_SIGMOID) beta = sigmoid_f(beta) * ((p.flags & GDN_FLAG_NEG_EIGVAL) ? 2.f : 1.f);
     }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const float y = __shfl_up(x, off, 64);
+        if (lane >= off) x += y;
+    }
+    sG[lane] = x * RCP_LN2_F;
+    sBeta[lane] = beta;
+    p.ws.Gam[u * 64 + lane] = x;
+    p.ws.Bet[u * 64 + lane] = beta;
+    lds_sync();
+    if constexpr (L2) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) normalise(fk[t], t, p.k, p.k_rstd);
+    }
+    // P, then L: transposed tiles (rows: key tokens j, column: token i).  P's first, a column of tiles at a time, and on its way to memory
+    // before L's are begun: either alone leaves room for the rows.
+    // (select, never multiply by a mask: e^(gam_i - gam_j) may overflow for i < j)
+    auto decay = [&](int a, int b, int r, int first, float gi, const f32x4& gj) {
+        return a < b || c16 >= 4 * g + r + first ? fast_exp2(gi - gj[r]) : 0.f;
+    };
+    T* Pu = (T*)p.ws.Pm + u * 64 * 64;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        if constexpr (L2) normalise(fq[b % QT], b, p.q, p.q_rstd);
+        f32x4 QK[4];
+#pragma unroll
+        for (int a = 0; a < 4; ++a) QK[a] = ZERO4;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const V8 q8 = __builtin_bit_cast(V8, fq[b % QT][s]);
+#pragma unroll
+            for (int a = 0; a <= b; ++a) QK[a] = Mma<T>::run(__builtin_bit_cast(V8, fk[a][s]), q8, QK[a]);
+        }
+        if (b + QT < 4) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) fq[b % QT][s] = fragment(qg, b + QT, 32 * s);
+        }
+        const int i = 16 * b + c16;
+        const float gi = sG[i];
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            f32x4 pt = ZERO4;
+            if (a <= b) {
+                const f32x4 gj = *(const f32x4*)(sG + 16 * a + 4 * g);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) pt[r] = p.scale * QK[a][r] * decay(a, b, r, 0, gi, gj);
+            }
+            *(V4*)(Pu + i * 64 + 16 * a + 4 * g) = pack4<T>(pt);
+        }
+    }
+    f32x4 U[4][4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int a = 0; a <= b; ++a) {
+            U[a][b] = ZERO4;
+#pragma unroll
+            for (int s = 0; s < NS; ++s) U[a][b] = Mma<T>::run(__builtin_bit_cast(V8, fk[a][s]), __builtin_bit_cast(V8, fk[b][s]), U[a][b]);
+        }
     // |k_t|^2 is the diagonal of k k^T
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -127,51 +166,24 @@ __global__ __launch_bounds__(64 * BP_WAVES, 2) void gdn_bwd_prepare_kernel(BwdPa
     }
     lds_sync();
     {
-        float x = scalar_of_bits(rg, p.gb_dtype), b = scalar_of_bits(rb, p.beta_dtype);
-        if (lane < c.valid) {
-            if (p.A_log && p.g) x = -__expf(p.A_log[hv]) * softplus_f(x + (p.dt_bias ? p.dt_bias[hv] : 0.f));
-            if (p.flags & GDN_FLAG_BETA_SIGMOID) b = sigmoid_f(b) * ((p.flags & GDN_FLAG_NEG_EIGVAL) ? 2.f : 1.f);
-        }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const float y = __shfl_up(x, off, 64);
-            if (lane >= off) x += y;
-        }
-        sG[lane] = x * RCP_LN2_F;
-        sBeta[lane] = b;
-        p.ws.Gam[u * 64 + lane] = x;
-        p.ws.Bet[u * 64 + lane] = b;
         // how much this chunk's transition can stretch a state, in log2 units: every token's factor gamma_t (I - beta_t k_t k_t^T)
-        float lb = fabsf(1.f - b * sK2[lane]);
+        float lb = fabsf(1.f - beta * sK2[lane]);
         lb = lb > 1.f ? __log2f(lb) : 0.f;
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) lb += __shfl_xor(lb, off, 64);
         if (lane == 63) p.ws.Bound[u] = x * RCP_LN2_F + lb;
     }
-    lds_sync();
-    // P and, in the same places, L: transposed tiles (rows: key tokens j, column: token i)
-    T* Pu = (T*)p.ws.Pm + u * 64 * 64;
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-        const int i = 16 * b + c16;
-        const float gi = sG[i], bi = sBeta[i];
+        const float gi = sG[16 * b + c16], bi = sBeta[16 * b + c16];
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            f32x4 pt = ZERO4;
-            if (a <= b) {
-                const f32x4 gj = *(const f32x4*)(sG + 16 * a + 4 * g);
-                f32x4 val;
+        for (int a = 0; a <= b; ++a) {
+            const f32x4 gj = *(const f32x4*)(sG + 16 * a + 4 * g);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    // select, never multiply by a mask: e^(gam_i - gam_j) may overflow for i < j
-                    const int j = 4 * g + r;
-                    const float d = a < b || c16 >= j ? fast_exp2(gi - gj[r]) : 0.f;
-                    pt[r] = p.scale * QK[a][b][r] * d;
-                    val[r] = a < b || c16 > j ? bi * U[a][b][r] * d : 0.f;
-                }
-                U[a][b] = val;
+            for (int r = 0; r < 4; ++r) {
+                const float d = decay(a, b, r, 1, gi, gj);
+                U[a][b][r] = a < b || c16 > 4 * g + r ? bi * U[a][b][r] * d : 0.f;
             }
-            *(V4*)(Pu + i * 64 + 16 * a + 4 * g) = pack4<T>(pt);
         }
     }
 #pragma unroll

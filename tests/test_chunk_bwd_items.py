@@ -14,6 +14,8 @@ from oracle import gdn_oracle as O
     (1, 300, 70, 70, 128, [0, 1, 65, 65, 190, 290], torch.bfloat16),        # packed, 1 .. 64 tokens a chunk, an empty sequence, tokens outside
     (5, 65, 53, 53, 64, None, torch.bfloat16),                              # 530 on 512
     (1, 200, 260, 260, 64, [3, 60, 61, 200], torch.float16),                # 1300, packed
+    (1, 300, 140, 140, 256, [3, 66, 66, 67, 280], torch.bfloat16),          # 256 features: rows normalised a tile of q's at a time; tokens outside
+    (2, 130, 3, 9, 256, None, torch.float16),                               # ... three value heads each
 ])
 @pytest.mark.parametrize('l2', [False, True])
 def test_more_items_than_workgroups(B, T, H, HV, D, cu, dtype, l2):
