@@ -30,6 +30,11 @@ template <> struct Mma<bf16_t> {
     static __device__ __forceinline__ f32x4 run(V8 a, V8 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
     }
+    // (16 deep: lane (c16, g) holds the contraction indices 4g .. 4g+3)
+    static __device__ __forceinline__ f32x4 run16(V4 a, V4 b, f32x4 c) {
+        typedef short s16x4 __attribute__((ext_vector_type(4)));
+        return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
+    }
     // LDS transpose read: the 16 lanes of a group each pass the address of 4 consecutive
     // elements; lane L receives element L%4 of the runs addressed by lanes L/4, L/4+4, L/4+8, L/4+12.
     static __device__ __forceinline__ V4 tr_read(const bf16_t* p) {
@@ -42,6 +47,7 @@ template <> struct Mma<f16_t> {
     static __device__ __forceinline__ f32x4 run(V8 a, V8 b, f32x4 c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
     }
+    static __device__ __forceinline__ f32x4 run16(V4 a, V4 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }
     static __device__ __forceinline__ V4 tr_read(const f16_t* p) {
         return __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)p));
     }

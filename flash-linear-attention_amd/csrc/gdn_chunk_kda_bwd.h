@@ -17,13 +17,18 @@
 //   col side   dk_j  += sum_i (dPs_ij q_i + dL_ij beta_i k_i) e^(Gk_i - Gk_j)
 //   dGk_i += q_i dq_i + k_i (beta_i rk_i),   dGk_j -= k_j (col side)_j        (elementwise in the feature)
 // The exponent splits into a factor of row i and one of row j around a reference row R that lies between them: blocks of 16
-// rows, R = the row in front of i's block, e^(Gk_i - R) <= 1 on the results, e^(R - Gk_j) on the operand rows (<= 1 for earlier
-// blocks; inside the diagonal block >= 1, which the operand type holds as long as the block's total decay stays above a
-// bound - otherwise every pair of the diagonal block gets its own exponentials, as in the forward kernel and in the
-// reference's sub-chunks of 16, fla/ops/kda/chunk_intra.py).  All of it runs on the matrix cores: per block of rows an
-// operand k e^(R - Gk) for the row side, and for the column side one 32-deep step whose contraction index runs over the
-// block's 16 rows twice (dPs^T against q e^(Gk - R), dL^T against beta k e^(Gk - R)).
+// rows, R = the row in front of i's block, e^(Gk_i - R) <= 1.  For j in an earlier block t, whose last row is E_t, e^(R - Gk_j) is
+// e^(E_t - Gk_j) <= 1 times the decays across the blocks between, a factor per feature that goes onto the sums; inside the diagonal block
+// it is >= 1, which the operand type holds as long as the block's total decay stays above a bound - otherwise every pair of the
+// diagonal block gets its own exponentials, as in the forward kernel and in the reference's sub-chunks of 16,
+// fla/ops/kda/chunk_intra.py.  All of it runs on the matrix cores: per block of rows k e^(E - Gk) and k e^(R - Gk) for the row side, and
+// for the column side one 32-deep step whose contraction index runs over the block's 16 rows twice (dPs^T against q e^(Gk - R),
+// dL^T against beta k e^(Gk - R)).
 
+// x + the y of the first lane of its row of sixteen (row_newbcast)
+__device__ __forceinline__ float add_first_c16(float x, float y) {
+    return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, y), 0x150, 0xF, 0xF, true));
+}
 // x of this lane and of the lanes behind it in its row of sixteen, added up
 template <int N> __device__ __forceinline__ float add_behind(float x) {
     return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x100 + N, 0xF, 0xF, true));     // row_shl: N lanes on, zero past the row
@@ -36,9 +41,11 @@ __device__ __forceinline__ float suffix_sum_c16(float x) { return add_behind<8>(
 // L2: q and k are the rows before their l2 normalisation and dq, dk the gradients of those.
 // As two kernels of four waves this moved 530 KB per unit (dw, dPs, the first parts of dq, dk and dGk through memory, k, q and Gk twice) where
 // it now moves 280 KB, and the l2 normalisation was four passes over q and k around it.  8192 tokens, 96 heads: 1834 us + 320 us of passes ->
-// 1006 us (3.63 GB, 3.6 TB/s; bound by its chain of phases with two waves per SIMD, the longest of 3100 instructions and no barrier), the step
-// 4250 -> 3093 us.  The next unit's tiles are requested in the order of their use, the state's fragments last: earlier there
-// are no registers for them (112 bytes of scratch).
+// 1006 us, the step 4250 -> 3093 us.  Bound by the vector instructions of two waves per SIMD: with k e^(R - Gk) anew for every block of rows and
+// e^(R - Gk) for every tile of the column side (ten exponentials an element) 3100 of them a unit and wave; with three for operands and three for results,
+// block factors on the sums, e^Gk kept between the two phases that use it and the unit's place carried over from the request for its tiles 2600:
+// 1006 -> 885 us (3.63 GB, 4.1 TB/s), the step 2815 -> 2693.  The next unit's tiles are requested in the order of their use, the state's
+// fragments last.  (`pin`: the compiler moves sums down to their next use, here two phases on, and keeps their factors: 100 registers.)
 constexpr size_t BWD_UNIT_KDA_SMEM = (6 * 64 * P128 + 2 * 64 * P64) * 2 + (64 * PG + 3 * 64 + 8 * 64 + 4) * 4;
 
 template <typename T, bool L2>
@@ -97,13 +104,11 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
         }
         put_tile<BD, NTH>(s, P128, x, tid);
     };
+    UnitAt nx = unit_at(p, blockIdx.x);
     {
         const int tid = threadIdx.x;
-        const UnitAt at = unit_at(p, blockIdx.x);
+        const UnitAt& at = nx;
         fetch_qk(at, blockIdx.x, tid); fetch_out(at, blockIdx.x, tid); fetch_in(at, blockIdx.x, tid); fetch_state(at, blockIdx.x, tid);
-        // (the two tiles above the diagonal that a 32-wide step over the lower triangle reads stay zero)
-        const int t = tid >> 8, r = (tid >> 4) & 15, c = tid & 15;
-        sPs[(32 * t + r) * P64 + 32 * t + 16 + c] = (T)0.f;
     }
     for (int64_t u = blockIdx.x; u < units; u += gridDim.x) {
         // (everything derived from the lane number is derived again per unit from a copy the compiler cannot see through:
@@ -111,13 +116,13 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
         int tid_opaque = threadIdx.x;
         asm volatile("" : "+v"(tid_opaque));
         const int tid = tid_opaque, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = lane & 15, g = lane >> 4;
-        const UnitAt at = unit_at(p, u);
+        const UnitAt at = nx;
         const int hv = at.hv;
         const ChunkAt c = at.c;
         // (what comes next is requested in any case, the last time for nothing: behind a condition the registers of the last request
         // stay alive through the whole unit)
         const int64_t un = u + gridDim.x < units ? u + gridDim.x : u;
-        const UnitAt nx = unit_at(p, un);
+        nx = unit_at(p, un);
         const int n16 = 16 * w, f4 = n16 + 4 * g;                // this wave's features, this lane's four of them in a result
         put_tile<BD, NTH>(sDO, P128, rDO, tid);
         put_tile<BD, NTH>(sVn, P128, rVn, tid);
@@ -154,7 +159,7 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
             }
         }
         // dq, dk, dGk of the output and the state update, dw (kept until do is done with)
-        f32x4 dq[4], dk[4], dG[4];
+        f32x4 dq[4], dk[4], dG[4], eG[4];                       // (eG: e^Gk)
         float dbx[4] = {0.f, 0.f, 0.f, 0.f};                     // this lane's share of dbeta of token 16t + c16
         V4 dw[4];
         {
@@ -184,12 +189,14 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
                 const V4 q4 = *(const V4*)(sQ + x * P128 + f4), k4 = *(const V4*)(sK + x * P128 + f4);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    dq[t][r] = G1[t][r] * (p.scale * fast_exp2(Gx[r]));
+                    eG[t][r] = fast_exp2(Gx[r]);
+                    dq[t][r] = G1[t][r] * (p.scale * eG[t][r]);
                     dk[t][r] = dKS[t][r] * fast_exp2(Gl[r] - Gx[r]);
                     const float kdk = (float)k4[r] * dk[t][r];
                     last[r] += kdk;
                     dG[t][r] = (float)q4[r] * dq[t][r] - kdk;
                 }
+                pin(dq[t]); pin(dk[t]); pin(dG[t]); pin(eG[t]); // (sunk to their uses the sums would keep their factors alive)
             }
             // the chunk's last row also takes what goes through e^Gk_last
 #pragma unroll
@@ -197,6 +204,7 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
                 const float x = sum_over_c16(last[r] + (c16 == 4 * g + r ? fast_exp2(Gl[r]) * sd[r] : 0.f));
                 dG[3][r] += c16 == 15 ? x : 0.f;
             }
+            pin(dG[3]);
         }
 
         // dX's first term dv_new v^T (the same tiles as above), and dv = beta (A^T dv_new)
@@ -299,15 +307,14 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
                 const int j = 16 * t + c16;
                 const float bj = sBeta[j];
                 const V4 kp4 = *(const V4*)(sKp + j * P128 + f4);
-                const f32x4 Gj = *(const f32x4*)(sG + j * PG + f4);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const float x = ak[r] * (float)kp4[r];
                     dbx[t] += x;
                     dG[t][r] += bj * x;
-                    dk[t][r] += ak[r] * (bj * fast_exp2(Gj[r]));
+                    dk[t][r] += ak[r] * (bj * eG[t][r]);
                 }
-                pin(dbx[t]);
+                pin(dbx[t]); pin(dk[t]); pin(dG[t]);
             }
         }
         lds_barrier();
@@ -345,34 +352,75 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
         }
         lds_barrier();
 
-        // The two matrices with a decay per pair and feature, a block of 16 rows at a time; a wave on its own from here on.
-        // Operand layout: feature n16 + c16, tokens 8g + e of a 32-wide step.
+        // The two matrices with a decay per pair and feature, a block of 16 rows at a time from the last; a wave on its own from here on.
+        // E_t: the last row of block t, the reference row R of block t + 1.  Every element has three exponentials for its operands and three for
+        // results: f = e^(Gk - R) as a row, e^(E - Gk) as a column (or 1 / f in its own block); between blocks lies a factor per feature, D_t = e^(E_t - E_(t-1)),
+        // on the sums so far.  Operand layout: feature n16 + c16, tokens 4g + e of a block, two blocks or two matrices to a product.
+        V4 kn[3];                                                // k e^(E - Gk) of blocks 0 .. 2
+        f32x4 D[3], cs[3];                                       // (cs: what the later blocks' rows leave to the columns of block t, before e^(E_t - Gk))
+        {
+            int lane_opaque = tid & 63;
+            asm volatile("" : "+v"(lane_opaque));
+            const int lane = lane_opaque, c16 = lane & 15, g = lane >> 4, f4 = n16 + 4 * g;
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
+            for (int t = 0; t < 3; ++t) {
+                __builtin_amdgcn_sched_barrier(0);
+                const float* gt = sG + 16 * t * PG + n16 + c16;
+                const float E = gt[15 * PG];
+                kn[t] = tile_cols(sK, P128, 16 * t, n16, lane);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) kn[t][e] = (T)((float)kn[t][e] * fast_exp2(E - gt[(4 * g + e) * PG]));
+                if (t > 0) {
+                    const f32x4 E4 = *(const f32x4*)(sG + (16 * t + 15) * PG + f4), R4 = *(const f32x4*)(sG + (16 * t - 1) * PG + f4);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) D[t][r] = fast_exp2(E4[r] - R4[r]);
+                }
+                cs[t] = ZERO4;
+            }
+        }
+#pragma unroll
+        for (int a = 3; a >= 0; --a) {
             __builtin_amdgcn_sched_barrier(0);
             // (the lane number anew: what the four blocks read alike would stay in registers from the first to the last)
             int lane_opaque = tid & 63;
             asm volatile("" : "+v"(lane_opaque));
             const int lane = lane_opaque, c16 = lane & 15, g = lane >> 4, f4 = n16 + 4 * g;
-            const float Rc = a > 0 ? sG[(16 * a - 1) * PG + n16 + c16] : 0.f;        // the reference row, at the operand's feature ...
-            const f32x4 R4 = a > 0 ? *(const f32x4*)(sG + (16 * a - 1) * PG + f4) : ZERO4;     // ... and at the result's four
             const bool ok = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, sSpan[a]))) >= SpanOk<T>::value;
             const int x = 16 * a + c16;
             const float bx = sBeta[x];
-            // row side: k e^(R - Gk) of this and the earlier blocks
-            f32x4 rq = ZERO4, rk = ZERO4;                       // (rk: before the row's beta)
+            V4 qf = tile_cols(sQ, P128, 16 * a, n16, lane), kf = tile_cols(sK, P128, 16 * a, n16, lane), kd;      // q f, beta k f, k / f
+            {
+                const float* ga = sG + (16 * a + 4 * g) * PG + n16 + c16;
+                const float R = a > 0 ? sG[(16 * a - 1) * PG + n16 + c16] : 0.f;
+                const f32x4 b4 = *(const f32x4*)(sBeta + 16 * a + 4 * g);
 #pragma unroll
-            for (int s = 0; 32 * s < 16 * (a + 1); ++s) {
-                V8 kt = frag_cols(sK, P128, 32 * s, n16, lane);
-                const float* gj = sG + (32 * s + 8 * g) * PG + n16 + c16;
-                const int blk = 2 * s + (g >> 1);               // the block this lane's eight tokens lie in
-                const bool in = blk < a || (blk == a && ok);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) kt[e] = in ? (T)((float)kt[e] * fast_exp2(Rc - gj[e * PG])) : (T)0.f;
-                rq = Mma<T>::run(kt, frag_rows(sPs, P64, 16 * a, 32 * s, lane), rq);
-                rk = Mma<T>::run(kt, frag_rows(sDL, P64, 16 * a, 32 * s, lane), rk);
+                for (int e = 0; e < 4; ++e) {
+                    const float d = ga[e * PG] - R, f = fast_exp2(d), k = (float)kf[e];
+                    kd[e] = ok ? (T)(k * fast_exp2(-d)) : (T)0.f;
+                    qf[e] = (T)((float)qf[e] * f);
+                    kf[e] = (T)(k * (b4[e] * f));
+                }
             }
-            const f32x4 Gx = *(const f32x4*)(sG + x * PG + f4);
+            __builtin_amdgcn_sched_barrier(0);
+            // row side: against k of the earlier blocks and of this one
+            f32x4 rq = ZERO4, rk = ZERO4;                       // (rk: before the row's beta)
+            const T* prow = sPs + x * P64 + 4 * g; const T* lrow = sDL + x * P64 + 4 * g;
+#pragma unroll
+            for (int t = 0; t < a - 1; ++t) {
+                rq = Mma<T>::run16(kn[t], *(const V4*)(prow + 16 * t), rq);
+                rk = Mma<T>::run16(kn[t], *(const V4*)(lrow + 16 * t), rk);
+                rq *= D[t + 1]; rk *= D[t + 1];
+            }
+            if (a > 0) {
+                const V8 kk = join<V8>(kn[a > 0 ? a - 1 : 0], kd);
+                rq = Mma<T>::run(kk, join<V8>(*(const V4*)(prow + 16 * a - 16), *(const V4*)(prow + 16 * a)), rq);
+                rk = Mma<T>::run(kk, join<V8>(*(const V4*)(lrow + 16 * a - 16), *(const V4*)(lrow + 16 * a)), rk);
+            } else {
+                rq = Mma<T>::run16(kd, *(const V4*)prow, rq);
+                rk = Mma<T>::run16(kd, *(const V4*)lrow, rk);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const f32x4 Gx = *(const f32x4*)(sG + x * PG + f4), R4 = a > 0 ? *(const f32x4*)(sG + (16 * a - 1) * PG + f4) : ZERO4;
             const V4 qx = *(const V4*)(sQ + x * P128 + f4), kx = *(const V4*)(sK + x * P128 + f4);
             // dGk takes every product dPs_ij (q_i f_i) (k_j e^(R - Gk_j)) twice, once with each sign (row i, column j), and
             // the sums down the columns leave the difference: both sides form it from the same rounded operands
@@ -406,33 +454,32 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
                 dq[a][r] += rq[r];
             }
             __builtin_amdgcn_sched_barrier(0);
-            // column side: the block's rows (q in the lanes g < 2, beta k in the others) against the columns of this and the earlier blocks
-            V8 op = frag_cols(g < 2 ? sQ : sK, P128, g < 2 ? 16 * a : 16 * a - 16, n16, lane);
-            {
-                const int i0 = 16 * a + 8 * (g & 1);
-                const float* gi = sG + i0 * PG + n16 + c16;
-                f32x4 m[2];
+            // column side: the block's rows (q f against dPs, beta k f against dL) for the columns of the earlier blocks and of this one
+            const V8 op = join<V8>(qf, kf);
+            auto columns = [&](int t, const f32x4& acc) {
+                return Mma<T>::run(op, join<V8>(tile_cols(sPs, P64, 16 * a, 16 * t, lane), tile_cols(sDL, P64, 16 * a, 16 * t, lane)), acc);
+            };
+            auto into = [&](const f32x4& sum, int r, float e) {
+                dk[a][r] += sum[r] * e;
+                dG[a][r] -= (float)(T)((float)kx[r] * e) * sum[r];
+            };
 #pragma unroll
-                for (int h = 0; h < 2; ++h) m[h] = g < 2 ? f32x4{1.f, 1.f, 1.f, 1.f} : *(const f32x4*)(sBeta + i0 + 4 * h);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) op[e] = (T)((float)op[e] * (m[e >> 2][e & 3] * fast_exp2(gi[e * PG] - Rc)));
+            for (int t = 0; t < a; ++t) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (a < 3) cs[t] *= D[a];
+                cs[t] = columns(t, cs[t]);
             }
+            __builtin_amdgcn_sched_barrier(0);
+            if (a < 3) {
+                const f32x4 E4 = *(const f32x4*)(sG + (16 * a + 15) * PG + f4);
 #pragma unroll
-            for (int tj = 0; tj <= a; ++tj) {
-                if (tj == a && !ok) continue;
-                const V8 bm = frag_cols(g < 2 ? sPs : sDL, P64, g < 2 ? 16 * a : 16 * a - 16, 16 * tj, lane);
-                const f32x4 col = Mma<T>::run(op, bm, ZERO4);
-                const int xj = 16 * tj + c16;
-                const f32x4 Gj = *(const f32x4*)(sG + xj * PG + f4);
-                const V4 kj = *(const V4*)(sK + xj * P128 + f4);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float e = fast_exp2(R4[r] - Gj[r]);
-                    dk[tj][r] += col[r] * e;
-                    dG[tj][r] -= (float)(T)((float)kj[r] * e) * col[r];
-                }
+                for (int r = 0; r < 4; ++r) into(cs[a < 3 ? a : 0], r, fast_exp2(E4[r] - Gx[r]));
             }
-            if (!ok) {
+            if (ok) {
+                const f32x4 own = columns(a, ZERO4);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) into(own, r, fast_exp2(R4[r] - Gx[r]));
+            } else {
                 // ... and the column side for this lane's token x
 #pragma unroll 1
                 for (int il = 0; il < 16; ++il) {
@@ -466,8 +513,9 @@ __global__ __launch_bounds__(512, 2) void gdn_bwd_unit_kda_kernel(BwdParams p, i
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const float x = dG[t][r];
-                    dG[t][r] = suffix_sum_c16(x) + behind[r];
-                    behind[r] += sum_over_c16(x);
+                    const float sum = suffix_sum_c16(x);
+                    dG[t][r] = sum + behind[r];
+                    behind[r] = add_first_c16(behind[r], sum);
                 }
                 *(f32x4*)(sG + (16 * t + c16) * PG + f4) = dG[t];
             }

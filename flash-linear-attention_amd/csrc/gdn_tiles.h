@@ -159,6 +159,12 @@ __device__ __forceinline__ typename Mma<T>::V8 frag_cols(const T* s, int pitch, 
     const T* at = s + (r0 + 8 * (lane >> 4) + (a >> 2)) * pitch + c0 + 4 * (a & 3);
     return join<typename Mma<T>::V8>(Mma<T>::tr_read(at), Mma<T>::tr_read(at + 4 * pitch));
 }
+// ... of 16 rows and columns: column c0 + c16, rows r0 + 4g + e
+template <typename T>
+__device__ __forceinline__ typename Mma<T>::V4 tile_cols(const T* s, int pitch, int r0, int c0, int lane) {
+    const int a = lane & 15;
+    return Mma<T>::tr_read(s + (r0 + 4 * (lane >> 4) + (a >> 2)) * pitch + c0 + 4 * (a & 3));
+}
 // ---- tiles in blocks -----------------------------------------------------------------------
 // 64 rows of COLS elements without padding: blocks of four rows, in a block groups of sixteen 16-byte slots, group n the pieces (8 elements) 4n .. 4n+3 of its
 // rows; piece c of row 4j + r in slot 4r + ((c & 3) ^ block_flip(j)) of its group.  A CU's LDS serves 256 bytes a cycle: of a 16-byte read the lanes {0-3, 12-15,
