@@ -29,14 +29,25 @@ template <int VBT, int KD, int FORM> constexpr size_t bwd_dstate_smem() {
     return (2 * 64 * (KD + 8) + (FORM == FORM_GATED ? 64 * P64 + 64 * (VBT + 8) : 64 * (KD + 8)) + 64 * P64 + 2 * 64 * (VBT + 8) + KD * (VBT + 8)) * 2 + 128 * 4;
 }
 
+// How a step requests the next one's tiles.  EXACT: with the same loads whatever the chunk and the step (fetch_rows; the last step its own tiles once more, for
+// nothing), so that the compiler knows how many stores are younger and the wait for the loads leaves them in flight; and behind the state's stores, not before
+// them (which makes every step 5 % longer).  16000 packed tokens, 32 heads: the step 1007 -> 999 us; KDA, 8192 tokens, 96 heads: 2693 -> 2676.  Not where a step has little
+// to store and its instructions count (64 key features: 116.5 -> 118.8 us), nor where warm-up steps store nothing.
+template <bool SEG, int KD> constexpr bool scan_exact() { return !SEG && KD > 64; }
+template <bool EXACT, int NCOLS, int NTH, typename T>
+__device__ __forceinline__ void fetch_scan(TileRegs<NCOLS, NTH>& r, const T* g, int64_t stride, int valid, int tid) {
+    if constexpr (EXACT) fetch_rows<NCOLS, NTH>(r, g, stride, valid, tid);
+    else fetch_tile<NCOLS, NTH>(r, g, stride, valid, tid);
+}
+
 // Workgroups go to the 8 XCDs in turn: the slices of one (sequence, head) take the same residue, so that they share
 // an L2 for the rows of k, q, w and A that all of them read.  With time segments (nwg workgroups each) a segment's come in a row.
 struct ScanAt { bool out; int hv, hq, hg, vcol0; int64_t n; SeqAt sq; ScanPlan plan; };
-template <int VBT, int VD>
+template <bool SEG, int VBT, int VD>
 __device__ __forceinline__ ScanAt scan_at(const BwdParams& p, unsigned bid_all, unsigned nwg, int lane, int& seg) {
     constexpr int NVS = VD / VBT;
-    seg = p.nseg > 1 ? (int)(bid_all / (nwg / p.nseg)) : 0;
-    const unsigned bid = p.nseg > 1 ? bid_all % (nwg / p.nseg) : bid_all;
+    seg = SEG ? (int)(bid_all / (nwg / p.nseg)) : 0;
+    const unsigned bid = SEG ? bid_all % (nwg / p.nseg) : bid_all;
     const int64_t run = (int64_t)(bid / (8 * NVS)) * 8 + bid % 8;
     ScanAt at{};
     at.out = run >= p.N * p.HV;
@@ -45,7 +56,7 @@ __device__ __forceinline__ ScanAt scan_at(const BwdParams& p, unsigned bid_all, 
     at.n = seq_in_order(p, run / p.HV);
     at.sq = seq_at(p, at.n);
     at.vcol0 = ((bid / 8) % NVS) * VBT;
-    at.plan = scan_plan(p, at.sq, at.hg, seg, lane);
+    at.plan = SEG ? scan_plan(p, at.sq, at.hg, seg, lane) : ScanPlan{false, 0, at.sq.nc, 0, 0};
     return at;
 }
 // entry (key row kk, value column 0 of the workgroup's slice) of the caller's states [N, HV / nb, KD, nb VD]
@@ -54,13 +65,13 @@ __device__ __forceinline__ int64_t state_entry(const BwdParams& p, const ScanAt&
     return ((at.n * (p.HV / p.nb) + at.hg) * KD + kk) * (int64_t)(VD * p.nb) + (at.hv % p.nb) * VD + at.vcol0;
 }
 
-template <typename T, int VBT, int KD, int VD, int FORM, int NW>
+template <typename T, bool SEG, int VBT, int KD, int VD, int FORM, int NW>
 __device__ __forceinline__ void bwd_state_body(const BwdParams& p, char* smem, const int tid, const unsigned bid_all, const unsigned nwg) {
     typedef typename Mma<T>::V8 V8;
     typedef typename Mma<T>::V4 V4;
     // NW waves in groups of four: a group takes VBQ of the workgroup's value columns (NB tiles per wave), every wave NA key tiles
     constexpr int PV = VBT + 8, VBQ = VBT / (NW / 4), NB = VBQ / 16, PK = KD + 8, NA = KD / 64, NS = KD / 32, NTH = 64 * NW;
-    constexpr bool KDA = FORM == FORM_KDA, GATED = FORM == FORM_GATED, OUT_TILE = state_out_tile<VBT, KD, FORM>();
+    constexpr bool KDA = FORM == FORM_KDA, GATED = FORM == FORM_GATED, EXACT = scan_exact<SEG, KD>(), OUT_TILE = state_out_tile<VBT, KD, FORM>();
     T* sK = (T*)smem; T* sW = sK + 64 * PK;                      // (GATED: A in w's place)
     T* sR = sW + (GATED ? 64 * P64 : 64 * PK);                   // (GATED) beta (v - e^gam (k S))
     T* sS = sR + (GATED ? 64 * PV : 0); T* sVn = sS + KD * PV;
@@ -68,7 +79,7 @@ __device__ __forceinline__ void bwd_state_body(const BwdParams& p, char* smem, c
     float* sGam = (float*)(sOut + (OUT_TILE ? 64 * PV : 0)); float* sBet = sGam + 64;
     const int lane = tid & 63, w = (tid >> 6) & 3, vq0 = (tid >> 8) * VBQ, c16 = lane & 15, g = lane >> 4;
     int seg;
-    const ScanAt at = scan_at<VBT, VD>(p, bid_all, nwg, lane, seg);
+    const ScanAt at = scan_at<SEG, VBT, VD>(p, bid_all, nwg, lane, seg);
     if (at.out || (at.plan.whole && seg != 0)) return;
     const SeqAt& sq = at.sq;
     const int hv = at.hv, vcol0 = at.vcol0, HVg = p.HV / p.nb;
@@ -86,41 +97,46 @@ __device__ __forceinline__ void bwd_state_body(const BwdParams& p, char* smem, c
     TileRegs<CH, NTH> rA;
     V4 rU[NB];                                                   // u (GATED: v) of this lane's token
     float rGam = 0.f, rBet = 0.f, rE[NA];
+    int rvalid = CH;                                             // the chunk's tokens
     auto fetch = [&](int64_t ic) __attribute__((always_inline)) {
         const int64_t u = (sq.cbase + ic) * p.HV + hv, ug = (sq.cbase + ic) * HVg + at.hg, tok0 = sq.bos + ic * CH;
-        const int valid = (int)min((int64_t)CH, sq.len - ic * CH), i = 16 * w + c16;
+        const int64_t left = sq.len - ic * CH;
+        const int valid = (left >> 6) != 0 ? CH : (int)left, i = 16 * w + c16;
+        rvalid = valid;
         if constexpr (KDA) {
-            fetch_tile<KD, NTH>(rK, (const T*)p.ws.KG + u * 64 * KD, KD, 64, tid);
+            fetch_scan<EXACT, KD, NTH>(rK, (const T*)p.ws.KG + u * 64 * KD, KD, 64, tid);
 #pragma unroll
             for (int a2 = 0; a2 < NA; ++a2) rE[a2] = p.ws.EGL[u * KD + 16 * (NA * w + a2) + c16];
         } else {
-            fetch_tile<KD, NTH>(rK, (const T*)p.k + (tok0 * p.H + at.hq) * KD, (int64_t)p.H * KD, valid, tid);
-            if (tid < 64) rGam = p.ws.Gam[ug * 64 + tid];
+            fetch_scan<EXACT, KD, NTH>(rK, (const T*)p.k + (tok0 * p.H + at.hq) * KD, (int64_t)p.H * KD, valid, tid);
+            if (EXACT || tid < 64) rGam = p.ws.Gam[ug * 64 + lane];
         }
         if constexpr (GATED) {
-            fetch_tile<CH, NTH>(rA, (const T*)p.ws.Am + ug * 64 * 64, 64, 64, tid);
-            if (tid < 64) rBet = p.ws.Bet[ug * 64 + tid];
+            fetch_scan<EXACT, CH, NTH>(rA, (const T*)p.ws.Am + ug * 64 * 64, 64, 64, tid);
+            if (EXACT || tid < 64) rBet = p.ws.Bet[ug * 64 + lane];
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                rU[b] = V4{(T)0.f, (T)0.f, (T)0.f, (T)0.f};
-                if (i < valid) rU[b] = *(const V4*)((const T*)p.v + ((tok0 + i) * p.HV + hv) * VD + vcol0 + vq0 + 16 * b + 4 * g);
+                if constexpr (!EXACT) rU[b] = V4{(T)0.f, (T)0.f, (T)0.f, (T)0.f};
+                if (EXACT || i < valid) rU[b] = *(const V4*)((const T*)p.v + ((tok0 + (EXACT ? min(i, valid - 1) : i)) * p.HV + hv) * VD + vcol0 + vq0 + 16 * b + 4 * g);
             }
         } else {
-            fetch_tile<KD, NTH>(rW, (const T*)p.ws.Wm + u * 64 * KD, KD, 64, tid);
+            fetch_scan<EXACT, KD, NTH>(rW, (const T*)p.ws.Wm + u * 64 * KD, KD, 64, tid);
 #pragma unroll
             for (int b = 0; b < NB; ++b) rU[b] = *(const V4*)((const T*)p.ws.Um + (u * 64 + i) * VD + vcol0 + vq0 + 16 * b + 4 * g);
         }
     };
     auto step = [&](int64_t ic) __attribute__((always_inline)) {
         const int64_t u = (sq.cbase + ic) * p.HV + hv;
-        const bool keep = ic >= c_keep;                         // (chunks of the warm-up belong to another segment: nothing of them is stored)
+        const bool keep = !SEG || ic >= c_keep;                 // (chunks of the warm-up belong to another segment: nothing of them is stored)
+        const int valid = rvalid;
+        if constexpr (EXACT && !KDA) clear_rows<KD, NTH>(rK, valid, tid);
         put_tile<KD, NTH>(sK, PK, rK, tid);
         if constexpr (GATED) put_tile<CH, NTH>(sW, P64, rA, tid);
         else put_tile<KD, NTH>(sW, PK, rW, tid);
         if (tid < 64) { sGam[tid] = rGam; if constexpr (GATED) sBet[tid] = rBet; }
         V4 u4[NB];
 #pragma unroll
-        for (int b = 0; b < NB; ++b) u4[b] = rU[b];
+        for (int b = 0; b < NB; ++b) u4[b] = !EXACT || !GATED || 16 * w + c16 < valid ? rU[b] : V4{(T)0.f, (T)0.f, (T)0.f, (T)0.f};
         float egk[NA];
 #pragma unroll
         for (int a2 = 0; a2 < NA; ++a2) egk[a2] = rE[a2];
@@ -134,7 +150,7 @@ __device__ __forceinline__ void bwd_state_body(const BwdParams& p, char* smem, c
             }
         lds_barrier();
         if (keep) copy_state_out<KD, VBT, VD, NTH>(Hu, vcol0 / 32, sS, PV, tid);
-        if (ic + 1 < c_end) fetch(ic + 1);
+        if (EXACT || ic + 1 < c_end) fetch(ic + 1 < c_end ? ic + 1 : ic);
         const float glast = sGam[63];
         // transposed tiles: value columns on the rows, this wave's 16 tokens on the columns
         const int i = 16 * w + c16;
@@ -204,25 +220,26 @@ __device__ __forceinline__ void bwd_state_body(const BwdParams& p, char* smem, c
         lds_barrier();
     };
     if (c_end > c_first) fetch(c_first);
+    if constexpr (EXACT) __builtin_amdgcn_s_waitcnt(0x0f70);    // vmcnt(0): here no stores are younger, and the waits in the loop would allow for that
     for (int64_t ic = c_first; ic < c_end; ++ic) step(ic);
     // (side by side with the reverse scan in one workgroup: as many barriers as the longer of the two takes)
-    for (int64_t i = (c_end - c_first); i < pad_steps_of(at.plan); ++i)
+    if constexpr (SEG) for (int64_t i = (c_end - c_first); i < pad_steps_of(at.plan); ++i)
         for (int n = 0; n < (GATED ? 4 : 3); ++n) lds_barrier();
 }
 
-template <typename T, int VBT, int KD, int VD, int FORM, int NW>
+template <typename T, bool SEG, int VBT, int KD, int VD, int FORM, int NW>
 __device__ __forceinline__ void bwd_dstate_body(const BwdParams& p, char* smem, const int tid, const unsigned bid_all, const unsigned nwg) {
     typedef typename Mma<T>::V8 V8;
     typedef typename Mma<T>::V4 V4;
     constexpr int PV = VBT + 8, VBQ = VBT / (NW / 4), NB = VBQ / 16, PK = KD + 8, NA = KD / 64, NS = KD / 32, NTH = 64 * NW;
-    constexpr bool KDA = FORM == FORM_KDA, GATED = FORM == FORM_GATED;
+    constexpr bool KDA = FORM == FORM_KDA, GATED = FORM == FORM_GATED, EXACT = scan_exact<SEG, KD>();
     T* sK = (T*)smem; T* sQ = sK + 64 * PK; T* sW = sQ + 64 * PK;       // (GATED: A in w's place)
     T* sY = sW + (GATED ? 64 * P64 : 64 * PK);                          // (GATED) -beta e^gam (A^T dv_new)
     T* sP = sY + (GATED ? 64 * PV : 0); T* sDO = sP + 64 * P64; T* sDvn = sDO + 64 * PV; T* sDS = sDvn + 64 * PV;
     float* sGam = (float*)(sDS + KD * PV); float* sBet = sGam + 64;
     const int lane = tid & 63, w = (tid >> 6) & 3, vq0 = (tid >> 8) * VBQ, c16 = lane & 15, g = lane >> 4;
     int seg;
-    const ScanAt at = scan_at<VBT, VD>(p, bid_all, nwg, lane, seg);
+    const ScanAt at = scan_at<SEG, VBT, VD>(p, bid_all, nwg, lane, seg);
     if (at.out || (at.plan.whole && seg != 0)) return;
     const SeqAt& sq = at.sq;
     const int hv = at.hv, vcol0 = at.vcol0, HVg = p.HV / p.nb;
@@ -243,31 +260,37 @@ __device__ __forceinline__ void bwd_dstate_body(const BwdParams& p, char* smem, 
     TileRegs<CH, NTH> rA, rP;
     TileRegs<VBT, NTH> rDO;
     float rGam = 0.f, rBet = 0.f, rE[NA], rGq[QN];
+    int rvalid = CH;
     auto fetch = [&](int64_t ic) __attribute__((always_inline)) {
         const int64_t u = (sq.cbase + ic) * p.HV + hv, ug = (sq.cbase + ic) * HVg + at.hg, tok0 = sq.bos + ic * CH;
-        const int valid = (int)min((int64_t)CH, sq.len - ic * CH);
+        const int64_t left = sq.len - ic * CH;
+        const int valid = (left >> 6) != 0 ? CH : (int)left;
+        rvalid = valid;
         if constexpr (KDA) {
-            fetch_tile<KD, NTH>(rK, (const T*)p.ws.KG + u * 64 * KD, KD, 64, tid);
-            fetch_tile<KD, NTH>(rQ, (const T*)p.ws.QG + u * 64 * KD, KD, 64, tid);
+            fetch_scan<EXACT, KD, NTH>(rK, (const T*)p.ws.KG + u * 64 * KD, KD, 64, tid);
+            fetch_scan<EXACT, KD, NTH>(rQ, (const T*)p.ws.QG + u * 64 * KD, KD, 64, tid);
 #pragma unroll
             for (int a2 = 0; a2 < NA; ++a2) rE[a2] = p.ws.EGL[u * KD + 16 * (NA * w + a2) + c16];
         } else {
-            fetch_tile<KD, NTH>(rK, (const T*)p.k + (tok0 * p.H + at.hq) * KD, (int64_t)p.H * KD, valid, tid);
-            fetch_tile<KD, NTH>(rQ, (const T*)p.q + (tok0 * p.H + at.hq) * KD, (int64_t)p.H * KD, valid, tid);
-            if (tid < 64) rGam = p.ws.Gam[ug * 64 + tid];
+            fetch_scan<EXACT, KD, NTH>(rK, (const T*)p.k + (tok0 * p.H + at.hq) * KD, (int64_t)p.H * KD, valid, tid);
+            fetch_scan<EXACT, KD, NTH>(rQ, (const T*)p.q + (tok0 * p.H + at.hq) * KD, (int64_t)p.H * KD, valid, tid);
+            if (EXACT || tid < 64) rGam = p.ws.Gam[ug * 64 + lane];
 #pragma unroll
             for (int i = 0; i < QN; ++i) rGq[i] = p.ws.Gam[ug * 64 + tid / QPPR + QRPI * i];
         }
-        fetch_tile<CH, NTH>(rP, (const T*)(FORM == FORM_COMBA ? p.ws.PT : p.ws.Pm) + ug * 64 * 64, 64, 64, tid);
+        fetch_scan<EXACT, CH, NTH>(rP, (const T*)(FORM == FORM_COMBA ? p.ws.PT : p.ws.Pm) + ug * 64 * 64, 64, 64, tid);
         if constexpr (GATED) {
-            fetch_tile<CH, NTH>(rA, (const T*)p.ws.Am + ug * 64 * 64, 64, 64, tid);
-            if (tid < 64) rBet = p.ws.Bet[ug * 64 + tid];
-        } else fetch_tile<KD, NTH>(rW, (const T*)p.ws.Wm + u * 64 * KD, KD, 64, tid);
-        fetch_tile<VBT, NTH>(rDO, (const T*)p.dout + (tok0 * p.HV + hv) * VD + vcol0, (int64_t)p.HV * VD, valid, tid);
+            fetch_scan<EXACT, CH, NTH>(rA, (const T*)p.ws.Am + ug * 64 * 64, 64, 64, tid);
+            if (EXACT || tid < 64) rBet = p.ws.Bet[ug * 64 + lane];
+        } else fetch_scan<EXACT, KD, NTH>(rW, (const T*)p.ws.Wm + u * 64 * KD, KD, 64, tid);
+        fetch_scan<EXACT, VBT, NTH>(rDO, (const T*)p.dout + (tok0 * p.HV + hv) * VD + vcol0, (int64_t)p.HV * VD, valid, tid);
     };
     auto step = [&](int64_t ic) __attribute__((always_inline)) {
         const int64_t u = (sq.cbase + ic) * p.HV + hv;
-        const bool keep = ic < c_keep;                          // (chunks of the warm-up belong to another segment: nothing of them is stored)
+        const bool keep = !SEG || ic < c_keep;                  // (chunks of the warm-up belong to another segment: nothing of them is stored)
+        const int valid = rvalid;
+        if constexpr (EXACT && !KDA) { clear_rows<KD, NTH>(rK, valid, tid); clear_rows<KD, NTH>(rQ, valid, tid); }
+        if constexpr (EXACT) clear_rows<VBT, NTH>(rDO, valid, tid);
         put_tile<KD, NTH>(sK, PK, rK, tid);
         if constexpr (!KDA) {                                   // (KDA: the factors are on the rows of q already)
 #pragma unroll
@@ -303,7 +326,7 @@ __device__ __forceinline__ void bwd_dstate_body(const BwdParams& p, char* smem, 
             }
         lds_barrier();
         if (keep) copy_state_out<KD, VBT, VD, NTH>(dHu, at.vcol0 / 32, sDS, PV, tid);
-        if (ic >= c_lo + 1) fetch(ic - 1);
+        if (EXACT || ic > c_lo) fetch(ic > c_lo ? ic - 1 : ic);
         const float glast = sGam[63];
         const int j = 16 * w + c16;
         {
@@ -375,8 +398,9 @@ __device__ __forceinline__ void bwd_dstate_body(const BwdParams& p, char* smem, 
         lds_barrier();
     };
     if (c_top > c_lo) fetch(c_top - 1);
+    if constexpr (EXACT) __builtin_amdgcn_s_waitcnt(0x0f70);
     for (int64_t ic = c_top - 1; ic >= c_lo; --ic) step(ic);
-    for (int64_t i = (c_top - c_lo); i < pad_steps_of(at.plan); ++i)
+    if constexpr (SEG) for (int64_t i = (c_top - c_lo); i < pad_steps_of(at.plan); ++i)
         for (int n = 0; n < (GATED ? 4 : 3); ++n) lds_barrier();
     if (p.dh0 && c_lo == 0) {
 #pragma unroll
@@ -400,8 +424,8 @@ template <typename T, int VBT, int KD, int VD>
 __global__ __launch_bounds__(512) void gdn_bwd_scans_kernel(BwdParams p) {
     extern __shared__ __align__(16) char smem[];
     static_assert(bwd_state_smem<VBT, KD, FORM_GATED>() % 16 == 0, "the second set of tiles starts 16-byte aligned");
-    if (threadIdx.x < 256) bwd_state_body<T, VBT, KD, VD, FORM_GATED, 4>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
-    else bwd_dstate_body<T, VBT, KD, VD, FORM_GATED, 4>(p, smem + bwd_state_smem<VBT, KD, FORM_GATED>(), threadIdx.x - 256, blockIdx.x, gridDim.x);
+    if (threadIdx.x < 256) bwd_state_body<T, true, VBT, KD, VD, FORM_GATED, 4>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
+    else bwd_dstate_body<T, true, VBT, KD, VD, FORM_GATED, 4>(p, smem + bwd_state_smem<VBT, KD, FORM_GATED>(), threadIdx.x - 256, blockIdx.x, gridDim.x);
 }
 
 // Both scans in one launch, in workgroups of their own: the first `nrev` workgroups walk backwards (the longer steps) over VBR value
@@ -416,6 +440,6 @@ template <typename T, int VBT, int VBR, int KD, int VD, int FORM>
 __global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_scans_apart_kernel(BwdParams p, int64_t nrev) {
     extern __shared__ __align__(16) char smem[];
     static_assert(scan_waves<VBT>() == scan_waves<VBR>(), "workgroups of one size");
-    if (blockIdx.x < nrev) bwd_dstate_body<T, VBR, KD, VD, FORM, scan_waves<VBR>()>(p, smem, threadIdx.x, blockIdx.x, (unsigned)nrev);
-    else bwd_state_body<T, VBT, KD, VD, FORM, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x - (unsigned)nrev, gridDim.x - (unsigned)nrev);
+    if (blockIdx.x < nrev) bwd_dstate_body<T, false, VBR, KD, VD, FORM, scan_waves<VBR>()>(p, smem, threadIdx.x, blockIdx.x, (unsigned)nrev);
+    else bwd_state_body<T, false, VBT, KD, VD, FORM, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x - (unsigned)nrev, gridDim.x - (unsigned)nrev);
 }

@@ -97,6 +97,31 @@ __device__ __forceinline__ void fetch_tile(TileRegs<NCOLS, NTH>& r, const T* g, 
         }
     }
 }
+// The same for loops that keep stores in flight behind the next tile's loads: as many loads whatever `valid` (1 or more) is - behind a branch or a mask that leaves
+// some out the compiler no longer knows how many accesses are younger and waits for all of them.  Past the end they repeat the last row; cleared on their way to LDS.
+template <int NCOLS, int NTH, typename T>
+__device__ __forceinline__ void fetch_rows(TileRegs<NCOLS, NTH>& r, const T* g, int64_t stride, int valid, int tid) {
+    constexpr int PPR = NCOLS / 8, N = 64 * PPR / NTH, RPI = NTH / PPR;
+    static_assert(64 * PPR % NTH == 0, "whole rounds of the workgroup's threads");
+    const int row0 = tid / PPR;
+    const char* at = (const char*)(g + (int64_t)row0 * stride + tid % PPR * 8);
+    const int64_t step = (int64_t)RPI * stride * (int64_t)sizeof(T);
+    if (valid >= 64) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) r.x[i] = *(const u32x4*)(at + i * step);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) r.x[i] = *(const u32x4*)(at + (int64_t)min(RPI * i, valid - 1 - row0) * stride * (int64_t)sizeof(T));
+    }
+}
+template <int NCOLS, int NTH>
+__device__ __forceinline__ void clear_rows(TileRegs<NCOLS, NTH>& r, int valid, int tid) {
+    constexpr int PPR = NCOLS / 8, N = sizeof(r.x) / sizeof(r.x[0]), RPI = NTH / PPR;
+    if (valid >= 64) return;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        if (tid / PPR + RPI * i >= valid) r.x[i] = u32x4{0u, 0u, 0u, 0u};
+}
 template <int NCOLS, int NTH = 256, typename T>
 __device__ __forceinline__ void put_tile(T* s, int pitch, const TileRegs<NCOLS, NTH>& r, int tid) {
     constexpr int PPR = NCOLS / 8, TOTAL = 64 * PPR, N = TOTAL >= NTH ? TOTAL / NTH : 1, RPI = NTH / PPR;
@@ -121,7 +146,7 @@ __device__ __forceinline__ void copy_rows_out(T* g, int64_t stride, const T* s, 
 #pragma unroll
     for (int i = 0; i < N; ++i) {
         const int idx = tid + NTH * i;
-        if (idx / PPR < valid) *(u32x4*)(g + (int64_t)(idx / PPR) * stride + (idx % PPR) * 8) = x[i];
+        if (valid >= ROWS || idx / PPR < valid) *(u32x4*)(g + (int64_t)(idx / PPR) * stride + (idx % PPR) * 8) = x[i];
     }
 }
 // A state in the workspace lies as the operand fragments that its readers take from it: 16 key features (tile a) x 32 of VD value columns (step s) after one
