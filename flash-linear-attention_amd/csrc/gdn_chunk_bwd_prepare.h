@@ -8,7 +8,7 @@
 // left by the first of the value heads that share them.  The rows are loaded straight into matrix-core operand registers and serve as
 // both factors of k k^T; results go from registers to memory, four columns of a row per lane.  P is formed a column of tiles at a time and
 // on its way to memory before k k^T is begun, so that the rows of k stay in registers also at 256 features (128 registers, and two of q's
-// four row tiles, 64) and need no normalising pass before: memory bounds the kernel, 1.2 GB at 4.9 TB/s there.  Two waves per SIMD: three,
+// four row tiles, 64) and need no normalising pass before: memory bounds the kernel, 1.26 GB at 5.2 TB/s there.  Two waves per SIMD: three,
 // which 164 registers would let in at 128 features, only push one another's rows out of the caches (122 -> 136 us).
 // 16000 packed tokens, 16 q/k and 32 value heads of 128, normalisation inside: 122 us; as four waves per unit with row-major LDS tiles, which also formed
 // w = A (beta e^gam k) and u = A (beta v) - 32 KB per unit that the scans now do without - 264 us.

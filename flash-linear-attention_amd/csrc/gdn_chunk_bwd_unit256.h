@@ -1,10 +1,10 @@
 // The chunk-parallel end of the backward pass at 256 key features (included by gdn_chunk_bwd.hip, inside the namespace, after gdn_chunk_bwd_unit.h, which has the
 // mathematics).  Eight waves of 256 registers, one workgroup per CU: wave w owns the key features 32w .. of all 64 tokens, the tiles of the 64 x 64 lower triangles are
 // dealt out one by one; k and q of all features and one copy of every other tile fill the LDS, what comes next waits in registers.
-// 8 x 2048 tokens, 32 heads of 256 x 256: 1245 us (4.9 GB at 3.9 TB/s).  The sixteen waves of 128 registers that serve 64 and 128 features took 1440 us here: dq, dk and
+// 8 x 2048 tokens, 32 heads of 256 x 256: 1205 us (4.8 GB at 4.0 TB/s).  The sixteen waves of 128 registers that serve 64 and 128 features took 1440 us here: dq, dk and
 // both states' rows are 64 of a wave's registers before its first product, 30 more spill, and every spilled register that is read again waits for all that is under
 // way.  What it took at eight: the first feature tile's fragments requested in front of the dP phase and the products with the state one after the other (1642 us
-// with the three of them side by side, whose accumulators spilled); no sum's terms kept in registers (1570 us with those of dglast kept to the end of the products, 1290 with those of dq and dk kept to the end of the head); the next
+// with the three of them side by side, whose accumulators spilled); no sum's terms kept in registers (1570 us with those of dglast kept to the end of the products, 1250 with those of dq and dk kept to the end of the head); the next
 // head's tiles requested in three places, the last of them late (all at once behind the products 1400 us); the states as operand fragments (state_frag; 1330 us as rows).
 // The registers that are left over do not pay as a place for the next head's first state fragments: the step 3114 -> 3121 us.
 constexpr int UNIT256_NW = 8;
