@@ -1040,20 +1040,25 @@ static unsigned scan_grid(const BwdParams& p, int VD, int v) { return (unsigned)
 
 // Both scans of whole sequences in one launch, up to 128 runs every workgroup with a CU to itself, as many value columns each as that
 // allows.  What a CU moves per step bounds the step (some 22 GB/s per CU, loads and stores together, whatever shares the CU).
-template <typename T, int FORM>
-static BwdLaunch scans_128(const BwdParams& p) {
+template <typename T, int FORM, bool EXACT>
+static BwdLaunch scans_128_of(const BwdParams& p) {
     const int64_t runs = p.N * p.HV;
     auto apart = [&](const void* f, size_t smem, int v, int vr) {         // columns forwards, backwards
         const unsigned nrev = scan_grid(p, BD, vr);
         return BwdLaunch{f, smem, "gdn_bwd_scans_apart_kernel", nrev + scan_grid(p, BD, v), v >= 64 ? 512u : 256u, (int64_t)nrev};
     };
-    if (runs <= 32) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, BD, BD, FORM>, bwd_scans_apart_smem<32, 32, BD, FORM>(), 32, 32);
-    if (runs <= 64) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, BD, BD, FORM>, bwd_scans_apart_smem<64, 64, BD, FORM>(), 64, 64);
+    if (runs <= 32) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, BD, BD, FORM, EXACT>, bwd_scans_apart_smem<32, 32, BD, FORM>(), 32, 32);
+    if (runs <= 64) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, BD, BD, FORM, EXACT>, bwd_scans_apart_smem<64, 64, BD, FORM>(), 64, 64);
     // (65 to 80 runs: the longer, backward scan halves its columns where a workgroup each still has a CU to itself: 80 runs of 1500 tokens
     // 353 -> 325 us a step, 80 packed ones of 1600 456 -> 400, KDA, 72 runs of 4000 tokens, 1161 -> 1109)
     if (scan_grid(p, BD, 128) + scan_grid(p, BD, 64) <= 256)
-        return apart((const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, BD, BD, FORM>, bwd_scans_apart_smem<128, 64, BD, FORM>(), 128, 64);
-    return apart((const void*)gdn_bwd_scans_apart_kernel<T, 128, 128, BD, BD, FORM>, bwd_scans_apart_smem<128, 128, BD, FORM>(), 128, 128);
+        return apart((const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, BD, BD, FORM, EXACT>, bwd_scans_apart_smem<128, 64, BD, FORM>(), 128, 64);
+    return apart((const void*)gdn_bwd_scans_apart_kernel<T, 128, 128, BD, BD, FORM, EXACT>, bwd_scans_apart_smem<128, 128, BD, FORM>(), 128, 128);
+}
+// (EXACT requests pay once the sequences have some chunks: figures at fetch_scan)
+template <typename T, int FORM>
+static BwdLaunch scans_128(const BwdParams& p, int64_t num_chunks) {
+    return num_chunks >= (FORM == FORM_GATED ? 16 : 8) * p.N ? scans_128_of<T, FORM, true>(p) : scans_128_of<T, FORM, false>(p);
 }
 
 template <typename T, int KD, int VD>
@@ -1081,21 +1086,21 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
     if constexpr (KD <= BD) {
         if (p.nseg > 1)                                         // both scans side by side in a workgroup: every CU has one already
             ks[1] = {(const void*)gdn_bwd_scans_kernel<T, 32, KD, VD>, bwd_scans_smem<32, KD>(), "gdn_bwd_scans_kernel", scan_grid(p, VD, 32) * p.nseg, 512, 0};
-        else if constexpr (VD == BD) ks[1] = scans_128<T, FORM_GATED>(p);
+        else if constexpr (VD == BD) ks[1] = scans_128<T, FORM_GATED>(p, num_chunks);
         // (64 x 64: two workgroups fit a CU, so that 32-column slices pay up to twice as many runs.  They read every tile twice, which
         // costs once the tiles outgrow the caches: 80 heads, step with 32 / 64 columns at 1500 tokens 192.5 / 194.0 us, 2500 tokens
         // 333 / 322, 5000 tokens 625 / 596; 96 heads at 2000 tokens 331.7 / 333.6; 128 at 1000 tokens 177.0 / 175.9, 2000 tokens 371 / 351)
-        else if (runs <= 64 || (runs < 128 && units <= 3072)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
-        else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 64), 512, (int64_t)scan_grid(p, VD, 64)};
+        else if (runs <= 64 || (runs < 128 && units <= 3072)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
+        else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 64), 512, (int64_t)scan_grid(p, VD, 64)};
     } else {
         // 256 key features: the reverse scan's tiles leave room for 64 columns at most.  The forward scan takes 128 where a workgroup each
         // still has a CU to itself (72 runs, step with 64 / 128 columns: 477 / 462 us), and beyond 128 runs, where rounds follow one another anyway
         // and its workgroups fill up the last one of the reverse scan (in a launch of its own behind it / in one launch: 160 runs 1011 / 901 us, 256
         // runs 875 / 857, 336 packed runs 2661 / 2621, 512 runs equal); in between, 96 packed runs 820 / 838, 128 runs 660 / 699.
         const unsigned half = scan_grid(p, VD, 64), whole = scan_grid(p, VD, 128);
-        if (runs <= 32) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
-        else if (runs > 128 || (runs > 64 && half + whole <= 256)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<128, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", half + whole, 512, (int64_t)half};
-        else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * half, 512, (int64_t)half};
+        if (runs <= 32) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
+        else if (runs > 128 || (runs > 64 && half + whole <= 256)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<128, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", half + whole, 512, (int64_t)half};
+        else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * half, 512, (int64_t)half};
     }
     const int64_t items = num_chunks * p.H * p.parts;
     if constexpr (KD <= BD) {
@@ -1116,7 +1121,7 @@ static int launch_bwd_comba(const BwdParams& p, int64_t num_chunks, hipStream_t 
     const bool l2 = p.q_raw != nullptr;                         // (the entry has checked H == HV)
     const BwdLaunch ks[4] = {
         {l2 ? (const void*)gdn_bwd_prepare_comba_kernel<T, true> : (const void*)gdn_bwd_prepare_comba_kernel<T, false>, BWD_PREP_COMBA_SMEM, "gdn_bwd_prepare_comba_kernel", units < 512u ? units : 512u, 256, units},
-        scans_128<T, FORM_COMBA>(p),
+        scans_128<T, FORM_COMBA>(p, num_chunks),
         {l2 ? (const void*)gdn_bwd_dqkw_kernel<T, true> : (const void*)gdn_bwd_dqkw_kernel<T, false>, BWD_DQKW_SMEM, "gdn_bwd_dqkw_kernel", units < 256u ? units : 256u, 256, units},
         {l2 ? (const void*)gdn_bwd_wy2_kernel<T, true> : (const void*)gdn_bwd_wy2_kernel<T, false>, BWD_WY2_SMEM, "gdn_bwd_wy2_kernel", units < 512u ? units : 512u, 256, units},
     };

@@ -31,9 +31,12 @@ template <int VBT, int KD, int FORM> constexpr size_t bwd_dstate_smem() {
 
 // How a step requests the next one's tiles.  EXACT: with the same loads whatever the chunk and the step (fetch_rows; the last step its own tiles once more, for
 // nothing), so that the compiler knows how many stores are younger and the wait for the loads leaves them in flight; and behind the state's stores, not before
-// them (which makes every step 5 % longer).  16000 packed tokens, 32 heads: the step 1007 -> 999 us; KDA, 8192 tokens, 96 heads: 2693 -> 2676.  Not where a step has little
-// to store and its instructions count (64 key features: 116.5 -> 118.8 us), nor where warm-up steps store nothing.
-template <bool SEG, int KD> constexpr bool scan_exact() { return !SEG && KD > 64; }
+// them (which makes every step 5 % longer).  At 128 key features, for sequences of sixteen chunks or more on average, KDA and comba eight (scans_128): the step of 16000 packed
+// tokens in 12 sequences, 32 heads 1003 -> 997 us; KDA and comba, 64 heads of 4000 tokens, the launch 206 -> 188 us and 210 -> 201, 96 heads 287 -> 275 and 299 -> 295.  Short
+// sequences lose by what the last step requests and by the rows past their end: gated, one chunk of 32 tokens 735 -> 836 us, of 64 tokens 422 -> 444, four
+// chunks 327 -> 355, eight 319 -> 349; KDA and comba, one chunk of 32 tokens 365 -> 390 and 188 -> 209, of 64 tokens 196 -> 207 and 109 -> 115, two to four up to 1 and 6 %.
+// Nor where a step has little to store and its instructions count (64 key features: 116.5 -> 118.8 us), at 256 features, where nothing gains (8 x 2048 tokens, 32 heads
+// 3103 -> 3111 us, one chunk of 32 tokens 612 -> 691), or where warm-up steps store nothing.
 template <bool EXACT, int NCOLS, int NTH, typename T>
 __device__ __forceinline__ void fetch_scan(TileRegs<NCOLS, NTH>& r, const T* g, int64_t stride, int valid, int tid) {
     if constexpr (EXACT) fetch_rows<NCOLS, NTH>(r, g, stride, valid, tid);
@@ -65,13 +68,13 @@ __device__ __forceinline__ int64_t state_entry(const BwdParams& p, const ScanAt&
     return ((at.n * (p.HV / p.nb) + at.hg) * KD + kk) * (int64_t)(VD * p.nb) + (at.hv % p.nb) * VD + at.vcol0;
 }
 
-template <typename T, bool SEG, int VBT, int KD, int VD, int FORM, int NW>
+template <typename T, bool SEG, bool EXACT, int VBT, int KD, int VD, int FORM, int NW>
 __device__ __forceinline__ void bwd_state_body(const BwdParams& p, char* smem, const int tid, const unsigned bid_all, const unsigned nwg) {
     typedef typename Mma<T>::V8 V8;
     typedef typename Mma<T>::V4 V4;
     // NW waves in groups of four: a group takes VBQ of the workgroup's value columns (NB tiles per wave), every wave NA key tiles
     constexpr int PV = VBT + 8, VBQ = VBT / (NW / 4), NB = VBQ / 16, PK = KD + 8, NA = KD / 64, NS = KD / 32, NTH = 64 * NW;
-    constexpr bool KDA = FORM == FORM_KDA, GATED = FORM == FORM_GATED, EXACT = scan_exact<SEG, KD>(), OUT_TILE = state_out_tile<VBT, KD, FORM>();
+    constexpr bool KDA = FORM == FORM_KDA, GATED = FORM == FORM_GATED, OUT_TILE = state_out_tile<VBT, KD, FORM>();
     T* sK = (T*)smem; T* sW = sK + 64 * PK;                      // (GATED: A in w's place)
     T* sR = sW + (GATED ? 64 * P64 : 64 * PK);                   // (GATED) beta (v - e^gam (k S))
     T* sS = sR + (GATED ? 64 * PV : 0); T* sVn = sS + KD * PV;
@@ -227,12 +230,12 @@ __device__ __forceinline__ void bwd_state_body(const BwdParams& p, char* smem, c
         for (int n = 0; n < (GATED ? 4 : 3); ++n) lds_barrier();
 }
 
-template <typename T, bool SEG, int VBT, int KD, int VD, int FORM, int NW>
+template <typename T, bool SEG, bool EXACT, int VBT, int KD, int VD, int FORM, int NW>
 __device__ __forceinline__ void bwd_dstate_body(const BwdParams& p, char* smem, const int tid, const unsigned bid_all, const unsigned nwg) {
     typedef typename Mma<T>::V8 V8;
     typedef typename Mma<T>::V4 V4;
     constexpr int PV = VBT + 8, VBQ = VBT / (NW / 4), NB = VBQ / 16, PK = KD + 8, NA = KD / 64, NS = KD / 32, NTH = 64 * NW;
-    constexpr bool KDA = FORM == FORM_KDA, GATED = FORM == FORM_GATED, EXACT = scan_exact<SEG, KD>();
+    constexpr bool KDA = FORM == FORM_KDA, GATED = FORM == FORM_GATED;
     T* sK = (T*)smem; T* sQ = sK + 64 * PK; T* sW = sQ + 64 * PK;       // (GATED: A in w's place)
     T* sY = sW + (GATED ? 64 * P64 : 64 * PK);                          // (GATED) -beta e^gam (A^T dv_new)
     T* sP = sY + (GATED ? 64 * PV : 0); T* sDO = sP + 64 * P64; T* sDvn = sDO + 64 * PV; T* sDS = sDvn + 64 * PV;
@@ -424,8 +427,8 @@ template <typename T, int VBT, int KD, int VD>
 __global__ __launch_bounds__(512) void gdn_bwd_scans_kernel(BwdParams p) {
     extern __shared__ __align__(16) char smem[];
     static_assert(bwd_state_smem<VBT, KD, FORM_GATED>() % 16 == 0, "the second set of tiles starts 16-byte aligned");
-    if (threadIdx.x < 256) bwd_state_body<T, true, VBT, KD, VD, FORM_GATED, 4>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
-    else bwd_dstate_body<T, true, VBT, KD, VD, FORM_GATED, 4>(p, smem + bwd_state_smem<VBT, KD, FORM_GATED>(), threadIdx.x - 256, blockIdx.x, gridDim.x);
+    if (threadIdx.x < 256) bwd_state_body<T, true, false, VBT, KD, VD, FORM_GATED, 4>(p, smem, threadIdx.x, blockIdx.x, gridDim.x);
+    else bwd_dstate_body<T, true, false, VBT, KD, VD, FORM_GATED, 4>(p, smem + bwd_state_smem<VBT, KD, FORM_GATED>(), threadIdx.x - 256, blockIdx.x, gridDim.x);
 }
 
 // Both scans in one launch, in workgroups of their own: the first `nrev` workgroups walk backwards (the longer steps) over VBR value
@@ -436,10 +439,10 @@ __global__ __launch_bounds__(512) void gdn_bwd_scans_kernel(BwdParams p) {
 template <int VBT, int VBR, int KD, int FORM> constexpr size_t bwd_scans_apart_smem() {
     return bwd_state_smem<VBT, KD, FORM>() > bwd_dstate_smem<VBR, KD, FORM>() ? bwd_state_smem<VBT, KD, FORM>() : bwd_dstate_smem<VBR, KD, FORM>();
 }
-template <typename T, int VBT, int VBR, int KD, int VD, int FORM>
+template <typename T, int VBT, int VBR, int KD, int VD, int FORM, bool EXACT>
 __global__ __launch_bounds__(64 * scan_waves<VBT>()) void gdn_bwd_scans_apart_kernel(BwdParams p, int64_t nrev) {
     extern __shared__ __align__(16) char smem[];
     static_assert(scan_waves<VBT>() == scan_waves<VBR>(), "workgroups of one size");
-    if (blockIdx.x < nrev) bwd_dstate_body<T, false, VBR, KD, VD, FORM, scan_waves<VBR>()>(p, smem, threadIdx.x, blockIdx.x, (unsigned)nrev);
-    else bwd_state_body<T, false, VBT, KD, VD, FORM, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x - (unsigned)nrev, gridDim.x - (unsigned)nrev);
+    if (blockIdx.x < nrev) bwd_dstate_body<T, false, EXACT, VBR, KD, VD, FORM, scan_waves<VBR>()>(p, smem, threadIdx.x, blockIdx.x, (unsigned)nrev);
+    else bwd_state_body<T, false, EXACT, VBT, KD, VD, FORM, scan_waves<VBT>()>(p, smem, threadIdx.x, blockIdx.x - (unsigned)nrev, gridDim.x - (unsigned)nrev);
 }

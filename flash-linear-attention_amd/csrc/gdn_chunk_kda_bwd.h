@@ -574,7 +574,7 @@ static int launch_bwd_kda(const BwdParams& p, const KdaParams& kp, int64_t num_c
     const unsigned units = (unsigned)(num_chunks * p.HV), grid = units < 256u ? units : 256u;
     const bool l2 = kp.flags & GDN_FLAG_QK_L2NORM;
     const BwdLaunch ks[2] = {
-        scans_128<T, FORM_KDA>(p),
+        scans_128<T, FORM_KDA>(p, num_chunks),
         {l2 ? (const void*)gdn_bwd_unit_kda_kernel<T, true> : (const void*)gdn_bwd_unit_kda_kernel<T, false>, BWD_UNIT_KDA_SMEM, "gdn_bwd_unit_kda_kernel", grid, 512, units},
     };
     return launch_all(p, ks, 2, stream);
