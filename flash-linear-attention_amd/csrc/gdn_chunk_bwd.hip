@@ -1058,7 +1058,8 @@ static BwdLaunch scans_128_of(const BwdParams& p) {
 // (EXACT requests pay once the sequences have some chunks: figures at fetch_scan)
 template <typename T, int FORM>
 static BwdLaunch scans_128(const BwdParams& p, int64_t num_chunks) {
-    return num_chunks >= (FORM == FORM_GATED ? 16 : 8) * p.N ? scans_128_of<T, FORM, true>(p) : scans_128_of<T, FORM, false>(p);
+    const int64_t least = FORM == FORM_GATED && p.N * p.HV > 64 ? 16 : 8;
+    return num_chunks >= least * p.N ? scans_128_of<T, FORM, true>(p) : scans_128_of<T, FORM, false>(p);
 }
 
 template <typename T, int KD, int VD>
@@ -1098,7 +1099,10 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
         // and its workgroups fill up the last one of the reverse scan (in a launch of its own behind it / in one launch: 160 runs 1011 / 901 us, 256
         // runs 875 / 857, 336 packed runs 2661 / 2621, 512 runs equal); in between, 96 packed runs 820 / 838, 128 runs 660 / 699.
         const unsigned half = scan_grid(p, VD, 64), whole = scan_grid(p, VD, 128);
-        if (runs <= 32) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
+        // (EXACT requests: up to 32 runs, four chunks or more on average; figures at fetch_scan)
+        if (runs <= 32)
+            ks[1] = {num_chunks >= 4 * p.N ? (const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, true> : (const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, false>,
+                     bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
         else if (runs > 128 || (runs > 64 && half + whole <= 256)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<128, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", half + whole, 512, (int64_t)half};
         else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * half, 512, (int64_t)half};
     }

@@ -31,12 +31,14 @@ template <int VBT, int KD, int FORM> constexpr size_t bwd_dstate_smem() {
 
 // How a step requests the next one's tiles.  EXACT: with the same loads whatever the chunk and the step (fetch_rows; the last step its own tiles once more, for
 // nothing), so that the compiler knows how many stores are younger and the wait for the loads leaves them in flight; and behind the state's stores, not before
-// them (which makes every step 5 % longer).  At 128 key features, for sequences of sixteen chunks or more on average, KDA and comba eight (scans_128): the step of 16000 packed
-// tokens in 12 sequences, 32 heads 1003 -> 997 us; KDA and comba, 64 heads of 4000 tokens, the launch 206 -> 188 us and 210 -> 201, 96 heads 287 -> 275 and 299 -> 295.  Short
-// sequences lose by what the last step requests and by the rows past their end: gated, one chunk of 32 tokens 735 -> 836 us, of 64 tokens 422 -> 444, four
-// chunks 327 -> 355, eight 319 -> 349; KDA and comba, one chunk of 32 tokens 365 -> 390 and 188 -> 209, of 64 tokens 196 -> 207 and 109 -> 115, two to four up to 1 and 6 %.
-// Nor where a step has little to store and its instructions count (64 key features: 116.5 -> 118.8 us), at 256 features, where nothing gains (8 x 2048 tokens, 32 heads
-// 3103 -> 3111 us, one chunk of 32 tokens 612 -> 691), or where warm-up steps store nothing.
+// them (which makes every step 5 % longer).
+// At 128 key features for sequences of eight chunks or more on average, the gated form beyond 64 runs sixteen (scans_128): 16000 packed tokens in 12 sequences, 32 heads the step
+// 1003 -> 997 us; the launch, 30 heads of 1400 tokens 57.4 -> 55.9; KDA and comba, 64 heads of 4000 tokens 206 -> 188 and 210 -> 201, 96 heads 287 -> 275 and 299 -> 295.
+// Short sequences lose by what the last step requests and by the rows past their end: gated, one chunk of 32 tokens 735 -> 836 us, of 64 tokens 422 -> 444, four
+// chunks 327 -> 355, eight (992 runs) 319 -> 349; KDA and comba, one chunk of 32 tokens 365 -> 390 and 188 -> 209, of 64 tokens 196 -> 207 and 109 -> 115, two to four up to 1 and 6 %.
+// At 256 features where a workgroup has a CU to itself, up to 32 runs, four chunks or more on average: 4 heads of 1024 tokens 61.0 -> 59.1 us, of 1400 tokens 83.5 -> 79.8; one
+// chunk 13.7 and 14.0.  With more runs nothing gains: 33 to 64 equal within 3 % either way; 8 x 2048 tokens, 32 heads the step 3103 -> 3111 us, 250 sequences of 32 tokens, 16 heads
+// the launch 612 -> 691.  Nor where a step has little to store and its instructions count (64 features: 116.5 -> 118.8 us), or where warm-up steps store nothing.
 template <bool EXACT, int NCOLS, int NTH, typename T>
 __device__ __forceinline__ void fetch_scan(TileRegs<NCOLS, NTH>& r, const T* g, int64_t stride, int valid, int tid) {
     if constexpr (EXACT) fetch_rows<NCOLS, NTH>(r, g, stride, valid, tid);

@@ -1,5 +1,5 @@
-"""The backward scans at 128 key features ask for the next chunk's tiles in two ways, by the sequences' average length (sixteen chunks, KDA and comba eight): the same
-bits either way, at every split of the value columns, with sequences of one token, of no token and of ragged ends among them."""
+"""The backward scans at 128 and 256 key features ask for the next chunk's tiles in two ways, by the sequences' average length (eight chunks at 128 features, sixteen in
+the gated form beyond 64 runs; 256 features four, up to 32 runs): the same bits either way, at every split of the value columns, with sequences of one token, of no token and of ragged ends among them."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -16,13 +16,13 @@ def _grads(op, x, do, cu, h0, dht):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize('op', ['gdn', 'kda', 'comba'])
-@pytest.mark.parametrize('H', [2, 10, 14, 26])       # 10, 50, 70 and 130 runs: 32, 64, 128 and 64, 128 value columns to a workgroup
+@pytest.mark.parametrize('op,D,H', [(op, 128, H) for op in ('gdn', 'kda', 'comba') for H in (2, 10, 14, 26)]       # 10, 50, 70 and 130 runs: 32, 64, 128 and 64, 128 value columns to a workgroup
+                         + [('gdn', 256, 2)])                                                                       # 20 runs (24 with the sixth sequence): 32
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
-def test_both_ways_of_asking_give_the_same_bits(op, H, dtype):
-    # 1, 2, 0, 13 chunks and as many more as make the average: forty in five sequences, or eighty
-    cu = [3, 4, 69, 69, 900, 4996 if op == 'gdn' else 2436]
-    T, N, D = 5000 if op == 'gdn' else 2440, 5, 128
+def test_both_ways_of_asking_give_the_same_bits(op, D, H, dtype):
+    # 1, 2, 0, 13 chunks and as many more as make the average: eighty in five sequences, forty, or twenty
+    cu = [3, 4, 69, 69, 900, 1150 if D == 256 else 4996 if op == 'gdn' and H > 12 else 2436]
+    T, N = cu[-1] + 4, 5
     gen = torch.Generator(device='cuda').manual_seed(H)
     rn = lambda *s: torch.randn(*s, generator=gen, device='cuda')
     q, k, p, v, do = (rn(1, T, H, D).to(dtype) for _ in range(5))
