@@ -114,15 +114,17 @@ struct BwdParams {
     int split;
 };
 
-// How a q/k head's value heads (their blocks of columns, `nb` each) are dealt out to the workgroups of gdn_bwd_unit_kernel: all to one
-// where (chunk, q/k head) pairs fill the chip, in equal parts where they do not.  In units of what a block takes (9 us at 64 and 128 key
-// features, 20 us at 256), a workgroup spends 0.3 on its rows of q and k, and the pass over the parts costs a half.  It is a launch more
+// How a q/k head's value heads (their blocks of columns, `nb` each) are dealt out to the workgroups of the unit kernels: all to one
+// where (chunk, q/k head) pairs fill the chip, in equal parts where they do not.  In units of what a block takes (7 us at 64 and 128 key
+// features, 14 us at 256), a workgroup spends 0.3 on its rows of q and k, and the pass over the parts costs a half, at 64 and 128 features as much
+// again where the parts fill the chip: there memory bounds them, and fp32 rows are twice as long.  It is a launch more
 // too, which a call waits for on the host where its sequences are short (fewer than 8 chunks on average, of `num_seqs`): not for one
-// block saved.  (The workspace is sized as for one sequence: never smaller.)  Training step, one part -> the number chosen:
-//   1024 tokens, 2 q/k and 16 value heads of 128   202 -> 137 us (8 parts)     2 and 8 heads of 256        322 -> 218 us (8)
-//   2048 tokens, 4 and 32 heads of 128             270 -> 238 us (2; 4: 245)   2 and 16 heads of 64        177 -> 112 us (8)
-//   2048 tokens, 8 and 32 heads of 128 (256 pairs)       231 us (2: 245)       512 tokens, 16 and 32 heads 106 -> 103 us (2)
-//   256 tokens, 16 and 32 heads of 128              89.6 us (2: 93)            layer, 1000 tokens: the kernel 87 -> 56 + 9 us (2)
+// block saved.  (The workspace is sized as for one sequence: never smaller.)  Training step with one part, with the number chosen, with others:
+//   1024 tokens, 2 q/k and 16 value heads of 128   163, 125 us (8 parts; 4: 127)    2 and 8 heads of 256           275, 194 us (8; 4: 200)
+//   2048 tokens, 4 and 32 heads of 128             233, 218 us (2; 4: 225)          2 and 16 heads of 64           168, 129 us (8; 4: 132)
+//   2048 tokens, 8 and 32 heads of 128 (256 pairs) 211 us (2: 228)                  1000 tokens, 6 heads of 256 x 512   225, 207 us (2; 4: 218)
+//   4096 tokens, 2 and 4 heads of 128              169 us (2: 171)                  768 tokens, 10 and 30 heads of 128  117 us (3: 124)
+//   1024 tokens, 16 and 32 heads of 64             99.5 us (2: 101.5)               256 tokens, 16 and 32 heads of 128  89 us (2: 92)
 struct BwdParts {
     int parts = 1, split = 1;
     size_t row_bytes = 0, head_bytes = 0;        // of dq_part (dk_part), of dg_part (db_part); 0: none
@@ -136,7 +138,8 @@ inline BwdParts bwd_parts(int64_t num_chunks, int64_t num_seqs, int64_t tokens, 
     for (int64_t n = 1; n <= heads && items * n <= 2 * slots; ++n) {
         // whole value heads, or an equal share of one's blocks
         if (heads % n || !((heads / n) % nb == 0 || nb % (heads / n) == 0)) continue;
-        const double cost = (double)((items * n + slots - 1) / slots) * ((double)(heads / n) + 0.3) + (n == 1 ? 0.0 : num_chunks < 8 * num_seqs ? 1.2 : 0.5);
+        const double pass = (num_chunks < 8 * num_seqs ? 1.2 : 0.5) + (KD <= BD ? 0.5 * (double)(items * n) / (double)slots : 0.0);
+        const double cost = (double)((items * n + slots - 1) / slots) * ((double)(heads / n) + 0.3) + (n == 1 ? 0.0 : pass);
         if (cost < best) { best = cost; x.parts = (int)n; }
     }
     if (x.parts > 1) {

@@ -16,6 +16,11 @@ from oracle import gdn_oracle as O
     (16, 2, 16, 64, 64, 8),
     (4, 6, 6, 256, 512, 4),                     # the blocks of a head apart: dg and dbeta in four parts as well
     (4, 3, 6, 128, 384, 6),
+    (64, 2, 4, 128, 128, 1),                    # two parts would fill the chip: fp32 rows cost as much as the head saved
+    (16, 16, 32, 64, 64, 1),
+    (32, 4, 4, 256, 256, 2),                    # ... not at 256 features
+    (12, 10, 30, 128, 128, 1),
+    (10, 10, 50, 128, 128, 5),                  # more than fill it
 ])
 def test_parts_are_reserved_in_the_workspace(num_chunks, H, HV, K, V, parts):
     from fla_hip import _lib
