@@ -1092,9 +1092,10 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
             ks[1] = {(const void*)gdn_bwd_scans_kernel<T, 32, KD, VD>, bwd_scans_smem<32, KD>(), "gdn_bwd_scans_kernel", scan_grid(p, VD, 32) * p.nseg, 512, 0};
         else if constexpr (VD == BD) ks[1] = scans_128<T, FORM_GATED>(p, num_chunks);
         // (64 x 64: two workgroups fit a CU, so that 32-column slices pay up to twice as many runs.  They read every tile twice, which
-        // costs once the tiles outgrow the caches: 80 heads, step with 32 / 64 columns at 1500 tokens 192.5 / 194.0 us, 2500 tokens
-        // 333 / 322, 5000 tokens 625 / 596; 96 heads at 2000 tokens 331.7 / 333.6; 128 at 1000 tokens 177.0 / 175.9, 2000 tokens 371 / 351)
-        else if (runs <= 64 || (runs < 128 && units <= 3072)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
+        // costs once the tiles outgrow the caches, from some 2200 (chunk, head) pairs on, the step from 2600: the launch with 32 / 64 columns, 72 heads of 1500 tokens 50.1 / 53.2 us,
+        // of 2000 68.0 / 68.7, of 2500 90.8 / 87.1; 80 heads of 1800 tokens 64.2 / 63.7, of 2200 86.3 / 80.0; 96 heads of 1300 tokens 44.6 / 46.2, of 1500 56.2 / 53.8, of
+        // 2000 86.2 / 77.7; 112 heads of 1200 tokens 43.8 / 43.9, of 1300 51.9 / 49.1; 128 heads of 1000 tokens 37.6 / 37.5, of 2000 96.6 / 78.6; the step, 112 heads of 1300 tokens 211.8 / 213.1, 80 of 2200 276.6 / 272.8, 96 of 2000 286 / 276)
+        else if (runs <= 64 || (runs < 128 && units <= 2600)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
         else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 64), 512, (int64_t)scan_grid(p, VD, 64)};
     } else {
         // 256 key features: the reverse scan's tiles leave room for 64 columns at most.  The forward scan takes 128 where a workgroup each

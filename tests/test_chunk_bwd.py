@@ -542,7 +542,7 @@ def test_chunk_backward_time_segments(B, T, H, HV, gate_div, h0_std, forced, mon
 @pytest.mark.gpu
 @pytest.mark.parametrize('B,T,H,HV,l2', [(2, 70, 32, 64, True), (2, 2435, 20, 40, False), (3, 1, 44, 44, True)])
 def test_chunk_backward_64_columns_of_64_features(B, T, H, HV, l2, monkeypatch):
-    """64 x 64 heads, 128 runs or more, or more than 3072 pairs of a chunk and a head on more than 64 runs: the scans hold all 64 value
+    """64 x 64 heads, 128 runs or more, or more than 2600 pairs of a chunk and a head on more than 64 runs: the scans hold all 64 value
     columns in eight waves.  A sequence by itself has fewer runs and takes slices of 32 columns; the sums over features and tokens
     are the same ones in the same order, so that every gradient has the same bits."""
     monkeypatch.setenv('FLA_HIP_BWD_SCAN_MODE', 'wide')
