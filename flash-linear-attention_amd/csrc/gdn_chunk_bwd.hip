@@ -1098,16 +1098,17 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
         else if (runs <= 64 || (runs < 128 && units <= 2600)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
         else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 64), 512, (int64_t)scan_grid(p, VD, 64)};
     } else {
-        // 256 key features: the reverse scan's tiles leave room for 64 columns at most.  The forward scan takes 128 where a workgroup each
-        // still has a CU to itself (72 runs, step with 64 / 128 columns: 477 / 462 us), and beyond 128 runs, where rounds follow one another anyway
-        // and its workgroups fill up the last one of the reverse scan (in a launch of its own behind it / in one launch: 160 runs 1011 / 901 us, 256
-        // runs 875 / 857, 336 packed runs 2661 / 2621, 512 runs equal); in between, 96 packed runs 820 / 838, 128 runs 660 / 699.
+        // 256 key features: the reverse scan's tiles leave room for 64 columns at most, the forward scan can take 128: fewer workgroups, each 1.2 times as long.
+        // Up to 256 runs what counts are the rounds of 256 workgroups (one to a CU) that the launch takes: with 64 / 128 columns forwards, 80 runs of 500 tokens 53.2 / 44.2
+        // us, 96 64.2 / 77.7, 128 68.6 / 79.4, 144 91.7 / 84.9, 176 111.3 / 125.6, 192 112.7 / 126.0, 192 of 2000 449 / 508, 224 of 1000 277 / 270, 256 289 / 271.  With
+        // more runs rounds of sequences of different lengths fill one another up and 128 pays on the whole: 320 of 1500 560 / 545, 384 of 700 303 / 311, the step of 384
+        // packed runs 1638 / 1620, 512 of 1000 575 / 543.
         const unsigned half = scan_grid(p, VD, 64), whole = scan_grid(p, VD, 128);
         // (EXACT requests: up to 32 runs, four chunks or more on average; figures at fetch_scan)
         if (runs <= 32)
             ks[1] = {num_chunks >= 4 * p.N ? (const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, true> : (const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, false>,
                      bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
-        else if (runs > 128 || (runs > 64 && half + whole <= 256)) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<128, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", half + whole, 512, (int64_t)half};
+        else if (runs > 256 || (runs > 64 && 6 * ((half + whole + 255) / 256) < 5 * ((2 * half + 255) / 256))) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<128, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", half + whole, 512, (int64_t)half};
         else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * half, 512, (int64_t)half};
     }
     const int64_t items = num_chunks * p.H * p.parts;
