@@ -15,7 +15,11 @@ from oracle import gdn_oracle as O
     (5, 65, 53, 53, 64, None, torch.bfloat16),                              # 530 on 512
     (1, 200, 260, 260, 64, [3, 60, 61, 200], torch.float16),                # 1300, packed
     (1, 300, 140, 140, 256, [3, 66, 66, 67, 280], torch.bfloat16),          # 256 features: rows normalised a tile of q's at a time; tokens outside
-    (2, 130, 3, 9, 256, None, torch.float16),                               # ... three value heads each
+    (2, 130, 43, 129, 256, None, torch.float16),                            # ... three value heads each, 258 items
+    # groups in five parts (tests/test_chunk_bwd_parts.py), of which no round of workgroups is a multiple: from one item to the next the part wraps around, and with it head and chunk
+    (1, 630, 10, 50, 128, None, torch.bfloat16),                            # 500 items on 256
+    (1, 440, 10, 50, 128, [2, 70, 70, 71, 300, 430], torch.float16),        # ... packed
+    (2, 310, 20, 100, 64, None, torch.float16),                             # 1000 items on 512
 ])
 @pytest.mark.parametrize('l2', [False, True])
 def test_more_items_than_workgroups(B, T, H, HV, D, cu, dtype, l2):
@@ -29,9 +33,10 @@ def test_more_items_than_workgroups(B, T, H, HV, D, cu, dtype, l2):
     v, do = (torch.randn(B, T, HV, D, generator=gen).to(dtype) for _ in range(2))
     g, beta = F.logsigmoid(torch.randn(B, T, HV, generator=gen)) / 2, torch.rand(B, T, HV, generator=gen)
     h0, dht = 0.5 * torch.randn(N, HV, D, D, generator=gen), torch.randn(N, HV, D, D, generator=gen)
-    # (the oracle on heads apart from one another: the first, the last, and those where a round of workgroups ends)
     G = HV // H
-    heads = sorted({0, H - 1, *(i % H for i in (255, 256, 511, 512))})
+    # (the oracle on heads apart from one another: the first, the last, and those where a round of workgroups ends)
+    parts = 5 if G == 5 else 1
+    heads = sorted({0, H - 1, *(i // parts % H for i in (255, 256, 511, 512))})
     vheads = [h * G + i for h in heads for i in range(G)]
     ref = O.gated_delta_rule_grads(q[:, :, heads], k[:, :, heads], v[:, :, vheads], g[:, :, vheads], beta[:, :, vheads], do[:, :, vheads], dht[:, vheads],
                                    initial_state=h0[:, vheads], cu_seqlens=cu, use_qk_l2norm_in_kernel=l2, dtype=torch.float32)

@@ -20,7 +20,8 @@ from oracle import gdn_oracle as O
     (16, 16, 32, 64, 64, 1),
     (32, 4, 4, 256, 256, 2),                    # ... not at 256 features
     (12, 10, 30, 128, 128, 1),
-    (10, 10, 50, 128, 128, 5),                  # more than fill it
+    (10, 10, 50, 128, 128, 5),                  # more than fill it (tests/test_chunk_bwd_items.py)
+    (10, 20, 100, 64, 64, 5),
 ])
 def test_parts_are_reserved_in_the_workspace(num_chunks, H, HV, K, V, parts):
     from fla_hip import _lib
