@@ -106,7 +106,6 @@ struct BwdParams {
     // to `warm_cap` chunks outside its range where the chunks' transition bounds say that this is forgotten by the time its own
     // range begins (gdn_chunk_common.h, WARM_LOG2); a head with a segment that cannot is walked whole by the workgroups of segment 0.
     int nseg, seg_chunks, warm_cap;
-    int64_t tokens;                      // rows of q and k per head
     int parts;                           // dq and dk leave as this many partial rows per token and q/k head (a divisor of HV / H)
     // Partial rows that are added up here (BwdParts) leave in fp32 to these places instead of dq and dk (NULL: they do not), and where
     // the parts cut a value head's blocks of columns, `split` > 1 parts to a head, so do the partial sums of dg and dbeta.
@@ -1113,8 +1112,8 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
     }
     const int64_t items = num_chunks * p.H * p.parts;
     if constexpr (KD <= BD) {
-        const void* unit = p.dq_part ? (l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, VD, true, true> : (const void*)gdn_bwd_unit_kernel<T, KD, VD, false, true>)
-                                     : (l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, VD, true, false> : (const void*)gdn_bwd_unit_kernel<T, KD, VD, false, false>);
+        const void* unit = p.dq_part ? (l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, true, true> : (const void*)gdn_bwd_unit_kernel<T, KD, false, true>)
+                                     : (l2 ? (const void*)gdn_bwd_unit_kernel<T, KD, true, false> : (const void*)gdn_bwd_unit_kernel<T, KD, false, false>);
         ks[3] = {unit, bwd_unit_smem<KD>(), "gdn_bwd_unit_kernel", (unsigned)std::min<int64_t>(items, KD == 64 ? 512 : 256), 64 * bwd_unit_waves<KD>(), items};
     } else {
         const void* unit = l2 ? (const void*)gdn_bwd_unit256_kernel<T, true> : (const void*)gdn_bwd_unit256_kernel<T, false>;
@@ -1207,7 +1206,7 @@ static int chunk_bwd_entry(
     p.q = q; p.k = k; p.v = v; p.g = g; p.beta = beta; p.A_log = A_log; p.dt_bias = dt_bias; p.h0 = h0; p.dout = dout; p.dht = dht;
     p.dq = dq; p.dk = dk; p.dv = dv; p.dg = dg; p.dbeta = dbeta; p.dh0 = dh0; p.pk = pk; p.dp = dp;
     p.cu_seqlens = cu_seqlens; p.chunk_table = chunk_table; p.chunk_offsets = chunk_offsets;
-    p.T = T; p.H = (int)H; p.HV = (int)(HV * nb); p.nb = (int)nb; p.N = N; p.NT = (T + CH - 1) / CH; p.tokens = B * T;
+    p.T = T; p.H = (int)H; p.HV = (int)(HV * nb); p.nb = (int)nb; p.N = N; p.NT = (T + CH - 1) / CH;
     p.scale = scale; p.gb_dtype = gb_dtype & 255; p.beta_dtype = beta_dtype_of(gb_dtype); p.flags = flags;
     p.nseg = 1; p.seg_chunks = (int)p.NT; p.warm_cap = 0;
     p.parts = per_head ? parts.parts : (int)(HV / H);

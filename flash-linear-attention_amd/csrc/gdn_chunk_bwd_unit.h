@@ -6,8 +6,9 @@
 //   Y = dA A^T, dL = -stril(A^T Y), E = diag(beta) dL o D;   dk += E k + E^T k;   dbeta, dgam from every factor, dg = the reverse
 //   cumulative sum of dgam inside the chunk.
 //
-// One workgroup takes the value heads of a q/k head (or an equal share of them, BwdParts; with more value columns than VD their blocks
-// count as heads) of one chunk in turn, with k and q in LDS and dq, dk in fp32 registers over all of them: 168 KB per chunk and value head + 96 KB per q/k head.
+// One workgroup takes the value heads of a q/k head (or an equal share of them, BwdParts; with more value columns than key features their blocks
+// count as heads) of one chunk in turn, with k and q in LDS and dq, dk in fp32 registers over all of them; at 128 x 128 it moves
+// 152 KB per chunk and value head (S, dS, v_new, dv_new, do, v, dv, A) and 64 KB per chunk and q/k head (k, q, dq, dk; of several parts 96: fp32 rows).
 // 64 and 128 key features (256: gdn_chunk_bwd_unit256.h).
 //
 // What bounds it are chains - load, product, sum over lanes, barrier - and the rate at which a SIMD issues, so as many waves as there are registers for: sixteen of 128
@@ -48,15 +49,15 @@ __device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void pin(f32x4& x) { asm volatile("" : "+v"(x)); }
 
 // PARTS: rows and sums leave in fp32 to be added up (BwdParts); a choice inside one kernel cost 3 % (the step 1084 -> 1097 us at 16000 packed tokens, 32 heads).
-template <typename T, int KD, int VD, bool L2, bool PARTS>
+template <typename T, int KD, bool L2, bool PARTS>
 __global__ __launch_bounds__(64 * bwd_unit_waves<KD>(), 4) void gdn_bwd_unit_kernel(BwdParams p, int64_t items) {
     typedef typename Mma<T>::V8 V8;
     typedef typename Mma<T>::V4 V4;
     constexpr int NW = bwd_unit_waves<KD>(), NR = KD / 16, NTH = 64 * NW;
-    constexpr int SV = VD / 32, SK = KD / 32, NTRI = (10 + NW - 1) / NW;
+    constexpr int VD = KD, SV = VD / 32, SK = KD / 32, NTRI = (10 + NW - 1) / NW;      // (value columns: as many as key features)
     // (the tiles of the next head that have no place of their own wait in registers: A, at 64 features do, whose place dw and E take)
     constexpr bool ROOMY = KD == 128;
-    static_assert(2 * NR == NW && KD == VD, "a wave a feature tile of a side, or a value tile; dw fits the tile of do");
+    static_assert(2 * NR == NW, "a wave a feature tile of a side, or a value tile");
     extern __shared__ __align__(16) char smem[];
     T* sDO = (T*)smem; T* sVn = sDO + 64 * VD; T* sDvn0 = sVn + 64 * VD; T* sV = sDvn0 + 64 * VD; T* sK = sV + 64 * VD; T* sQ = sK + 64 * KD;
     T* sA = sQ + 64 * KD; T* sM1 = sA + 64 * CH; T* sRoom = sM1 + 64 * CH;
@@ -209,7 +210,7 @@ __global__ __launch_bounds__(64 * bwd_unit_waves<KD>(), 4) void gdn_bwd_unit_ker
             const int tid = tid_opaque, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = lane & 15, g = lane >> 4;
             const int wf = !qside ? w - NR : w, n16 = 16 * wf;            // this wave's features
             // this lane's shares of the addresses of operands by rows, by columns, of a result's four elements in a row, of a triangle tile's elements
-            const int ro_v = opaque(block_rows_lane<VD>(lane)), ro_k = KD == VD ? ro_v : opaque(block_rows_lane<KD>(lane)), ro_c = VD == CH ? ro_v : opaque(block_rows_lane<CH>(lane));
+            const int ro = opaque(block_rows_lane<KD>(lane)), ro_c = KD == CH ? ro : opaque(block_rows_lane<CH>(lane));
             auto cols_lane = [&](ColsLane x) { return ColsLane{opaque(x.a), opaque(x.b)}; };
             const ColsLane co_c = cols_lane(block_cols_lane<CH>(lane)), co_c1 = cols_lane(odd_tile(co_c));
             const int eo = opaque(block_lane<KD>(c16, 4 * g) ^ (32 * (wf & 1)));
@@ -232,12 +233,11 @@ __global__ __launch_bounds__(64 * bwd_unit_waves<KD>(), 4) void gdn_bwd_unit_ker
             const Item& to = last ? nx : at;
             const int to_hi = last ? 0 : hi + 1;
             lds_barrier();
-            // dv = beta (A^T dv_new), value columns 16 n ..
-            auto leave_dv = [&](int n) {
+            // dv = beta (A^T dv_new), value columns 16 wf ..
+            auto leave_dv = [&]() {
                 V8 f[2];
-                const ColsLane vk = block_cols_lane<VD>(lane), vo = KD == VD ? fo : n & 1 ? odd_tile(vk) : vk;
 #pragma unroll
-                for (int s = 0; s < 2; ++s) f[s] = block_cols<VD>(sDvn, 32 * s, 16 * n, vo);
+                for (int s = 0; s < 2; ++s) f[s] = block_cols<VD>(sDvn, 32 * s, 16 * wf, fo);
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     __builtin_amdgcn_sched_barrier(0);
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(64 * bwd_unit_waves<KD>(), 4) void gdn_bwd_unit_ker
                     for (int s = 0; s < 2; ++s)
                         if (32 * s + 31 >= 16 * t) av = Mma<T>::run(f[s], block_cols<CH>(sA, 32 * s, 16 * t, t % 2 ? co_c1 : co_c), av);     // A[i][j] = 0 for i < j
                     const int j = 16 * t + c16;
-                    if (j < at.c.valid) *(V4*)((T*)p.dv + (at.row0 + hi + (int64_t)j * p.HV) * VD + 16 * n + 4 * g) = pack4<T>(av * sBeta[j]);
+                    if (j < at.c.valid) *(V4*)((T*)p.dv + (at.row0 + hi + (int64_t)j * p.HV) * VD + n16 + 4 * g) = pack4<T>(av * sBeta[j]);
                 }
             };
             copy_blocks<VD, NW>(sDvn0 + (DVN_STEP - odd), unit_rows(p.ws.dVn, to, to_hi), VD, 64, w, lane);
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(64 * bwd_unit_waves<KD>(), 4) void gdn_bwd_unit_ker
                     for (int s = 0; s < SV; ++s) {
                         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                        for (int t = 0; t < 4; ++t) x[t] = Mma<T>::run(f[s], block_rows<VD>(rows, 16 * t, 32 * s, ro_v), x[t]);
+                        for (int t = 0; t < 4; ++t) x[t] = Mma<T>::run(f[s], block_rows<VD>(rows, 16 * t, 32 * s, ro), x[t]);
                         behind(s);
                     }
                     __builtin_amdgcn_sched_barrier(0);
@@ -329,13 +329,13 @@ __global__ __launch_bounds__(64 * bwd_unit_waves<KD>(), 4) void gdn_bwd_unit_ker
 #pragma unroll
                 for (int s = 0; s < SV; ++s) {
                     if (s % 2 == 0) __builtin_amdgcn_sched_barrier(0);
-                    d = Mma<T>::run(block_rows<VD>(sDO, 16 * ti, 32 * s, ro_v), block_rows<VD>(sVn, 16 * tj, 32 * s, ro_v), d);
+                    d = Mma<T>::run(block_rows<VD>(sDO, 16 * ti, 32 * s, ro), block_rows<VD>(sVn, 16 * tj, 32 * s, ro), d);
                 }
                 pin(d);
 #pragma unroll
                 for (int s = 0; s < SK; ++s) {
                     if (s % 2 == 0) __builtin_amdgcn_sched_barrier(0);
-                    qk = Mma<T>::run(block_rows<KD>(sQ, 16 * ti, 32 * s, ro_k), block_rows<KD>(sK, 16 * tj, 32 * s, ro_k), qk);
+                    qk = Mma<T>::run(block_rows<KD>(sQ, 16 * ti, 32 * s, ro), block_rows<KD>(sK, 16 * tj, 32 * s, ro), qk);
                 }
                 const int j = 16 * tj + c16;
                 const float gj = sGam[j];
@@ -406,14 +406,14 @@ __global__ __launch_bounds__(64 * bwd_unit_waves<KD>(), 4) void gdn_bwd_unit_ker
 #pragma unroll
                     for (int s = 0; s < SV; ++s) {
                         if (s % 2 == 0) __builtin_amdgcn_sched_barrier(0);
-                        dXv = Mma<T>::run(block_rows<VD>(sDvn, 16 * ti, 32 * s, ro_v), block_rows<VD>(sV, 16 * tj, 32 * s, ro_v), dXv);
+                        dXv = Mma<T>::run(block_rows<VD>(sDvn, 16 * ti, 32 * s, ro), block_rows<VD>(sV, 16 * tj, 32 * s, ro), dXv);
                     }
 #pragma unroll
                     for (int s = 0; s < SK; ++s) {
                         __builtin_amdgcn_sched_barrier(0);
-                        const V8 bk = block_rows<KD>(sK, 16 * tj, 32 * s, ro_k);
-                        dXw = Mma<T>::run(block_rows<KD>(sDW, 16 * ti, 32 * s, ro_k), bk, dXw);
-                        kk[n] = Mma<T>::run(block_rows<KD>(sK, 16 * ti, 32 * s, ro_k), bk, kk[n]);
+                        const V8 bk = block_rows<KD>(sK, 16 * tj, 32 * s, ro);
+                        dXw = Mma<T>::run(block_rows<KD>(sDW, 16 * ti, 32 * s, ro), bk, dXw);
+                        kk[n] = Mma<T>::run(block_rows<KD>(sK, 16 * ti, 32 * s, ro), bk, kk[n]);
                     }
                     const int j = 16 * tj + c16;
                     pin(kk[n]);
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(64 * bwd_unit_waves<KD>(), 4) void gdn_bwd_unit_ker
                 }
             }
             if constexpr (qside) {
-                leave_dv(w);
+                leave_dv();
                 // (a wave each for dg and dbeta)
                 if (w < 2) {
                     float x = 0.f;

@@ -393,8 +393,7 @@ __global__ __launch_bounds__(64 * UNIT256_NW, 2) void gdn_bwd_unit256_kernel(Bwd
                     }
                 }
             }
-            // (a wave each for dg and dbeta, while the others wait at the barrier.  One wave for both, with lane shuffles through the LDS: 16000
-            // packed tokens, 32 heads, the step 1087 us, now 1083; 4 x 2000 tokens, 32 heads of 64 315 and 311)
+            // (a wave each for dg and dbeta, while the others wait at the barrier)
             if (w < 2) {
                 const float* rows = w == 0 ? sDg : sDb;
                 float x = 0.f;
