@@ -1103,12 +1103,14 @@ static int launch_bwd(const BwdParams& p_in, int64_t num_chunks, hipStream_t str
         // more runs rounds of sequences of different lengths fill one another up and 128 pays on the whole: 320 of 1500 560 / 545, 384 of 700 303 / 311, the step of 384
         // packed runs 1638 / 1620, 512 of 1000 575 / 543.
         const unsigned half = scan_grid(p, VD, 64), whole = scan_grid(p, VD, 128);
-        // (EXACT requests: up to 32 runs, four chunks or more on average; figures at fetch_scan)
+        // (EXACT requests: up to 32 runs four chunks or more on average, where 64 columns go round more than once 32; figures at fetch_scan)
         if (runs <= 32)
             ks[1] = {num_chunks >= 4 * p.N ? (const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, true> : (const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, KD, VD, FORM_GATED, false>,
                      bwd_scans_apart_smem<32, 32, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * scan_grid(p, VD, 32), 256, (int64_t)scan_grid(p, VD, 32)};
         else if (runs > 256 || (runs > 64 && 6 * ((half + whole + 255) / 256) < 5 * ((2 * half + 255) / 256))) ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<128, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", half + whole, 512, (int64_t)half};
-        else ks[1] = {(const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED, false>, bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * half, 512, (int64_t)half};
+        else
+            ks[1] = {runs > 64 && num_chunks >= 32 * p.N ? (const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED, true> : (const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, KD, VD, FORM_GATED, false>,
+                     bwd_scans_apart_smem<64, 64, KD, FORM_GATED>(), "gdn_bwd_scans_apart_kernel", 2 * half, 512, (int64_t)half};
     }
     const int64_t items = num_chunks * p.H * p.parts;
     if constexpr (KD <= BD) {

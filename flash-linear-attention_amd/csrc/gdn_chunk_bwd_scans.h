@@ -37,8 +37,9 @@ template <int VBT, int KD, int FORM> constexpr size_t bwd_dstate_smem() {
 // Short sequences lose by what the last step requests and by the rows past their end: gated, one chunk of 32 tokens 735 -> 836 us, of 64 tokens 422 -> 444, four
 // chunks 327 -> 355, eight (992 runs) 319 -> 349; KDA and comba, one chunk of 32 tokens 365 -> 390 and 188 -> 209, of 64 tokens 196 -> 207 and 109 -> 115, two to four up to 1 and 6 %.
 // At 256 features where a workgroup has a CU to itself, up to 32 runs, four chunks or more on average: 4 heads of 1024 tokens 61.0 -> 59.1 us, of 1400 tokens 83.5 -> 79.8; one
-// chunk 13.7 and 14.0.  With more runs nothing gains: 33 to 64 equal within 3 % either way; 8 x 2048 tokens, 32 heads the step 3103 -> 3111 us, 250 sequences of 32 tokens, 16 heads
-// the launch 612 -> 691.  Nor where a step has little to store and its instructions count (64 features: 116.5 -> 118.8 us), or where warm-up steps store nothing.
+// chunk 13.7 and 14.0; and in the 64-column form beyond 64 runs 32 chunks or more: 48 heads of 3000 tokens 397 -> 390, 4 x 4096 tokens, 6 heads of 256 x 512 545 -> 528 (1500
+// tokens equal, 700 86.3 and 89.4; up to 64 runs 0.5 to 1.5 % longer).  Elsewhere nothing gains: 8 x 2048 tokens, 32 heads the step 3103 -> 3111 us, 250 sequences of 32 tokens, 16
+// heads the launch 612 -> 691.  Nor where a step has little to store and its instructions count (64 features: 116.5 -> 118.8 us), or where warm-up steps store nothing.
 template <bool EXACT, int NCOLS, int NTH, typename T>
 __device__ __forceinline__ void fetch_scan(TileRegs<NCOLS, NTH>& r, const T* g, int64_t stride, int valid, int tid) {
     if constexpr (EXACT) fetch_rows<NCOLS, NTH>(r, g, stride, valid, tid);

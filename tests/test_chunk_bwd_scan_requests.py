@@ -1,5 +1,5 @@
 """The backward scans at 128 and 256 key features ask for the next chunk's tiles in two ways, by the sequences' average length (eight chunks at 128 features, sixteen in
-the gated form beyond 64 runs; 256 features four, up to 32 runs): the same bits either way, at every split of the value columns, with sequences of one token, of no token and of ragged ends among them."""
+the gated form beyond 64 runs; 256 features four up to 32 runs, 32 with 64 columns beyond 64): the same bits either way, at every split of the value columns, with sequences of one token, of no token and of ragged ends among them."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -17,11 +17,12 @@ def _grads(op, x, do, cu, h0, dht):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize('op,D,H', [(op, 128, H) for op in ('gdn', 'kda', 'comba') for H in (2, 10, 14, 26)]       # 10, 50, 70 and 130 runs: 32, 64, 128 and 64, 128 value columns to a workgroup
-                         + [('gdn', 256, 2)])                                                                       # 20 runs (24 with the sixth sequence): 32
+                         + [('gdn', 256, 2), ('gdn', 256, 9)])                                                      # 20 and 90 runs: 32, 64
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
 def test_both_ways_of_asking_give_the_same_bits(op, D, H, dtype):
-    # 1, 2, 0, 13 chunks and as many more as make the average: eighty in five sequences, forty, or twenty
-    cu = [3, 4, 69, 69, 900, 1150 if D == 256 else 4996 if op == 'gdn' and H > 12 else 2436]
+    # 1, 2, 0, 13 chunks and as many more as make the average, in five sequences
+    chunks = 5 * ((32 if H == 9 else 4) if D == 256 else 16 if op == 'gdn' and H > 12 else 8)
+    cu = [3, 4, 69, 69, 900, 880 + 64 * (chunks - 16)]
     T, N = cu[-1] + 4, 5
     gen = torch.Generator(device='cuda').manual_seed(H)
     rn = lambda *s: torch.randn(*s, generator=gen, device='cuda')
