@@ -1051,8 +1051,8 @@ static BwdLaunch scans_128_of(const BwdParams& p) {
     };
     if (runs <= 32) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 32, 32, BD, BD, FORM, EXACT>, bwd_scans_apart_smem<32, 32, BD, FORM>(), 32, 32);
     if (runs <= 64) return apart((const void*)gdn_bwd_scans_apart_kernel<T, 64, 64, BD, BD, FORM, EXACT>, bwd_scans_apart_smem<64, 64, BD, FORM>(), 64, 64);
-    // (65 to 80 runs: the longer, backward scan halves its columns where a workgroup each still has a CU to itself: 80 runs of 1500 tokens
-    // 353 -> 325 us a step, 80 packed ones of 1600 456 -> 400, KDA, 72 runs of 4000 tokens, 1161 -> 1109)
+    // (65 to 80 runs: the longer, backward scan halves its columns where a workgroup each still has a CU to itself: the launch with 64 / 128 and 64 / 128 columns, 72 runs of
+    // 500 tokens 36.0 / 29.7 / 37.6 us, 80 of 1500 101.3 / 84.6 / 118.9, of 5000 342 / 277 / 388; 96 of 2000 175.9 / 207.9 / 164.3, 128 of 1000 92.5 / 107.1 / 89.5)
     if (scan_grid(p, BD, 128) + scan_grid(p, BD, 64) <= 256)
         return apart((const void*)gdn_bwd_scans_apart_kernel<T, 128, 64, BD, BD, FORM, EXACT>, bwd_scans_apart_smem<128, 64, BD, FORM>(), 128, 64);
     return apart((const void*)gdn_bwd_scans_apart_kernel<T, 128, 128, BD, BD, FORM, EXACT>, bwd_scans_apart_smem<128, 128, BD, FORM>(), 128, 128);
